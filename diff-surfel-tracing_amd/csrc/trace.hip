@@ -257,15 +257,6 @@ __device__ __forceinline__ uint32_t shift_in_any(uint32_t bits, uint64_t mask) {
     asm("s_cmp_lg_u64 %1, 0\n\ts_addc_u32 %0, %0, %0" : "+s"(bits) : "s"(mask) : "scc");
     return bits;
 }
-// The same for two masks at once: hit takes (a & b) != 0, ahead takes b != 0 (the and sets the carry itself).
-__device__ __forceinline__ void shift_in_near_far(uint32_t &hit, uint32_t &ahead, uint64_t a, uint64_t b) {
-    uint64_t both;
-    asm("s_and_b64 %2, %3, %4\n\ts_addc_u32 %0, %0, %0\n\ts_cmp_lg_u64 %4, 0\n\ts_addc_u32 %1, %1, %1"
-        : "+s"(hit), "+s"(ahead), "=&s"(both)
-        : "s"(a), "s"(b)
-        : "scc");
-}
-
 struct RaySlab {   // per-lane precomputation for the conservative slab test
     float ix, iy, iz;     // 1/d, with tiny components pushed away from zero
     float nx, ny, nz;     // -o * (1/d)
@@ -319,20 +310,6 @@ __device__ __forceinline__ uint64_t slab_hit_fast(const RaySlabFast &s, float nx
     return __builtin_amdgcn_fcmpf(tn, tf, 5);   // 5 = ordered <=
 }
 
-// The same test as two masks: `far` = lanes whose ray meets the box at all (at a distance >= 0), result = those of
-// them that meet it within tmax.  Lanes that are switched off carry slab constants that fail both (see packet_walk).
-__device__ __forceinline__ uint64_t slab_hit_near_far(const RaySlabFast &s, float nx, float ny, float nz, float fx,
-                                                      float fy, float fz, float tmax, uint64_t &far) {
-    const float a = __builtin_fmaf(nx, s.ix, s.cnx), b = __builtin_fmaf(ny, s.iy, s.cny),
-                c = __builtin_fmaf(nz, s.iz, s.cnz);
-    const float e = __builtin_fmaf(fx, s.ix, s.cfx), f = __builtin_fmaf(fy, s.iy, s.cfy),
-                g = __builtin_fmaf(fz, s.iz, s.cfz);
-    const float tn = __builtin_fmaxf(__builtin_fmaxf(a, b), __builtin_fmaxf(c, 0.0f));
-    const float tf = __builtin_fminf(__builtin_fminf(e, f), g);
-    far = __builtin_amdgcn_fcmpf(tn, tf, 5);   // 5 = ordered <=
-    return far & __builtin_amdgcn_fcmpf(tn, tmax, 5);
-}
-
 // The 16 nearest hits of a lane, ascending.  One entry = (bits of t) << 32 | idx: t is positive, so the
 // unsigned 64-bit order is the (t, idx) lexicographic order and the content does not depend on the order in
 // which the BVH delivers candidates (ties in t resolve to ascending primitive index).
@@ -348,20 +325,30 @@ __device__ __forceinline__ void kbuf_reset(KBuf &b) {
     for (int k = 0; k < kChunk; ++k) b.e[k] = kb_pack(kInfDepth, 0u);
 }
 
-// Sorted insert in place: slot k keeps its entry if that is smaller than the new one, else takes the new one
-// (if the slot above kept its entry) or the entry from the slot above.
+// Entries as doubles: an entry's upper word is the bits of a float between 0 and kInfDepth, so as a double it is a
+// finite number of the same sign whose order is that of the 64-bit integers (no NaN, and nothing that a double-precision
+// comparison would take for equal); kNoEntry is larger than all of them.  64-bit integer comparisons and selects cost
+// seven instructions per slot of a sorted insertion, minimum and maximum of doubles two.
+constexpr uint64_t kNoEntry = 0x7F000000FFFFFFFFull;
+__device__ __forceinline__ bool kb_less(uint64_t a, uint64_t b) {
+    return __builtin_bit_cast(double, a) < __builtin_bit_cast(double, b);
+}
+__device__ __forceinline__ uint64_t kb_min(uint64_t a, uint64_t b) {   // (written out: no canonicalising of operands)
+    uint64_t r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ uint64_t kb_max(uint64_t a, uint64_t b) {
+    uint64_t r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+// Sorted insert in place: slot k becomes the middle one of its entry, the entry above and the new one.
 __device__ __forceinline__ void kbuf_insert(KBuf &b, uint64_t x_in, bool on) {
-    // a lane that inserts nothing offers the largest key: every slot keeps its entry (no per-slot gating)
-    const uint64_t x = on ? x_in : ~0ull;
-    bool keep_k = b.e[kChunk - 1] < x;
+    const uint64_t x = on ? x_in : kNoEntry;   // a lane that inserts nothing offers what leaves every slot as it is
 #pragma unroll
-    for (int k = kChunk - 1; k >= 1; --k) {
-        const bool keep_up = b.e[k - 1] < x;
-        const uint64_t in = keep_up ? x : b.e[k - 1];
-        b.e[k] = keep_k ? b.e[k] : in;
-        keep_k = keep_up;
-    }
-    b.e[0] = keep_k ? b.e[0] : x;
+    for (int k = kChunk - 1; k >= 1; --k) b.e[k] = kb_max(b.e[k - 1], kb_min(b.e[k], x));
+    b.e[0] = kb_min(b.e[0], x);
 }
 
 #ifdef DST_STATS
@@ -396,12 +383,7 @@ __device__ __forceinline__ RayPre make_pre(F3 o, F3 d, float max_abs) {
 
 // The stand-in test of one quad for all lanes (about 28 instructions), as a lane mask: bit clear = that lane's ray
 // cannot pass the exact test (lanes that are switched off come back set or clear; the caller masks them).
-// FAR: also `far`, the same without the limit tmax (lanes whose ray may hit the quad at any distance ahead); for a
-// grazing ray, whose distance to the plane says nothing, the quad counts as ahead unless the sphere around it lies
-// behind the origin.
-template <bool FAR>
-__device__ __forceinline__ uint64_t quad_may_hit(const u32x16 &Q, const RayPre &rp, F3 o, F3 d, float tmax,
-                                                 uint64_t live, uint64_t &far) {
+__device__ __forceinline__ uint64_t quad_may_hit(const u32x16 &Q, const RayPre &rp, F3 o, F3 d, float tmax) {
 #define QF(k) __uint_as_float(Q[k])
     const float hx = QF(0) - o.x, hy = QF(1) - o.y, hz = QF(2) - o.z;
     const float qd = __builtin_fmaf(QF(5), d.z, __builtin_fmaf(QF(4), d.y, QF(3) * d.x));
@@ -414,17 +396,9 @@ __device__ __forceinline__ uint64_t quad_may_hit(const u32x16 &Q, const RayPre &
     const float lim = __builtin_fmaf(rp.padw, QF(12), QF(13));
     const float tpq = __builtin_fmaf(QF(14), rp.inv_dl, rp.tp);
     // every comparison is written so that a NaN keeps the ray in; the lane masks are combined without branches
-    uint64_t flat = wave_ballot(__builtin_fabsf(qd) < rp.graze);
+    const uint64_t flat = wave_ballot(__builtin_fabsf(qd) < rp.graze);
     const uint64_t out_base = wave_ballot(m > lim) | wave_ballot(t < -tpq);
     const uint64_t out_t = wave_ballot(__builtin_fmaf(t, 0.9999f, -tpq) > tmax);
-    if (FAR) {
-        if ((flat & live) != 0ull) {
-            // (centre - o).d < -(radius + slack) |d|: every point of the quad is behind the origin
-            const float hd = __builtin_fmaf(hz, d.z, __builtin_fmaf(hy, d.y, hx * d.x));
-            flat &= ~wave_ballot(hd < -(QF(15) + rp.padw) * (20.0f * rp.graze));
-        }
-        far = flat | ~out_base;
-    }
 #undef QF
     return flat | ~(out_base | out_t);
 }
@@ -445,7 +419,7 @@ __device__ __forceinline__ void quad_exact(const u32x16 &La, const u32x8 &Lb, F3
 #undef LF3
     const uint64_t x = kb_pack(t, 2u * LW(15) + tri);
 #undef LW
-    const bool adm = hit && (x < buf.e[kChunk - 1]);
+    const bool adm = hit && (kb_less(x, buf.e[kChunk - 1]));
     if (wave_ballot(adm) != 0ull) {
         STAT(ws.leaf_any++;)
         cnt += adm ? 1u : 0u;
@@ -455,17 +429,14 @@ __device__ __forceinline__ void quad_exact(const u32x16 &La, const u32x8 &Lb, F3
 
 // A leaf group (up to DST_GROUP quads, consecutive records) against all lanes' rays.  The stand-in records of
 // two quads are fetched together, then the exact records of those that some lane's ray may hit, again together:
-// one trip to memory per stage instead of one per quad.  FAR: returns whether some live lane's ray may hit a quad
-// of the group at any distance ahead (the group has to be looked at again when the ray's next chunk is traced).
-template <bool FAR>
-__device__ __forceinline__ bool test_group(const DstAccelView &acc, uint32_t first, uint32_t count, const RayPre &rp,
+// one trip to memory per stage instead of one per quad.
+__device__ __forceinline__ void test_group(const DstAccelView &acc, uint32_t first, uint32_t count, const RayPre &rp,
                                            F3 o, F3 d, bool active, KBuf &buf, uint32_t &cnt
 #ifdef DST_STATS
                                            , WaveStats &ws
 #endif
 ) {
     uint32_t q0 = 0;   // count >= 1
-    bool again = false;
 #pragma unroll 1
     do {
         const bool two = q0 + 1u < count;
@@ -475,10 +446,8 @@ __device__ __forceinline__ bool test_group(const DstAccelView &acc, uint32_t fir
         STAT(ws.leaves += two ? 2 : 1;)
         const float tmax = kb_t(buf.e[kChunk - 1]);
         const uint64_t live = wave_ballot(active);
-        uint64_t f0 = 0ull, f1 = 0ull;
-        const uint64_t k0 = quad_may_hit<FAR>(Q0, rp, o, d, tmax, live, f0) & live;
-        const uint64_t k1 = two ? (quad_may_hit<FAR>(Q1, rp, o, d, tmax, live, f1) & live) : 0ull;
-        if (FAR) again = again || (((f0 | (two ? f1 : 0ull)) & live) != 0ull);
+        const uint64_t k0 = quad_may_hit(Q0, rp, o, d, tmax) & live;
+        const uint64_t k1 = two ? (quad_may_hit(Q1, rp, o, d, tmax) & live) : 0ull;
         uint32_t todo = (k0 != 0ull ? 1u : 0u) | (k1 != 0ull ? 2u : 0u);
 #pragma unroll 1
         while (todo != 0u) {
@@ -491,27 +460,7 @@ __device__ __forceinline__ bool test_group(const DstAccelView &acc, uint32_t fir
         }
         q0 += 2;
     } while (DST_GROUP > 2 && q0 < count);   // groups of at most two quads: one pass, no loop
-    return again;
 }
-
-// Work list of a walk that can be resumed.  The rays of a wave are traced in chunks of 16 hits, each chunk from an
-// origin moved up to the last hit of the one before.  Instead of walking down from the root again, a walk writes
-// down what the next chunk can still need - the nodes it left with children that lie ahead of some ray but beyond
-// its 16th hit so far (with the children concerned), and the leaf groups it tested that hold a quad ahead of some
-// ray - and the next walk starts from that list.  What is ahead of a ray from the moved origin was ahead of it
-// before, and both tests have margins far above the rounding of the moved origin, so the list is a superset of
-// what a walk from the root would reach; the buffer's content does not depend on the order or on extra candidates.
-// An item is a leaf-group reference, or a node index with the children NOT to look at in bits 27..30.
-constexpr uint32_t kListCap = 512;            // items per list (a multiple of the wave size); a longer list is dropped
-constexpr uint32_t kListFresh = 0xFFFFFFFFu;  // n_in: no list, walk from the root
-constexpr uint32_t kListIndexBits = 27;       // node indices must fit below the excluded-children bits
-struct WalkList {
-    lds_u32 in, out;   // kListCap words each (LDS of this wave)
-    uint32_t n_in;     // items in `in`, or kListFresh
-    bool record;       // write `out` (false: plain walks from the root)
-    uint32_t limit;    // steps this walk may take at most (0: as many as the hierarchy can need)
-    bool spent;        // set by a walk that ran into its limit: its buffer is not to be used
-};
 
 // One traversal for the whole wave: every active lane ends with its own 16 nearest hits (t relative
 // to its origin, 0 < t < 1e16) and the number of admissions.  Wave-uniform control flow: nodes and quads
@@ -521,14 +470,14 @@ struct WalkList {
 // the build measures; nodes that open one level at a time only over hierarchies measured to be at most 42 deep).  A
 // stack that is full all the same loses the entry (no fault; checked on the builder's side, not here).
 // All active lanes share the direction signs `sgn` (bit a set = axis a negative), see slab_hit_fast.
-template <bool RESUME, bool HAND>
+// (The backward trace without a hit record: its LDS is taken by the gradient table, which leaves none for the lists
+// of the bundle walk.)
 __device__ __forceinline__ void packet_walk(const DstAccelView &acc, const RaySlab &slab, uint32_t sgn, F3 o, F3 d,
-                                            bool active, int rep, KBuf &buf, uint32_t &cnt, WalkList &wl
+                                            bool active, KBuf &buf, uint32_t &cnt
 #ifdef DST_STATS
                                             , WaveStats &ws
 #endif
 ) {
-    const uint32_t lane = __lane_id();
     const RayPre rp = make_pre(o, d, slab.max_abs);
     RaySlabFast fs;
     // byte offsets of the near / far face arrays inside a wide node (lox 0, loy 16, loz 32, hix 48, hiy 64, hiz 80)
@@ -536,11 +485,6 @@ __device__ __forceinline__ void packet_walk(const DstAccelView &acc, const RaySl
     fs.ix = slab.ix; fs.iy = slab.iy; fs.iz = slab.iz;
     fs.cnx = slab.nx - slab.wx; fs.cny = slab.ny - slab.wy; fs.cnz = slab.nz - slab.wz;
     fs.cfx = slab.nx + slab.wx; fs.cfy = slab.ny + slab.wy; fs.cfz = slab.nz + slab.wz;
-    const bool recording = RESUME && wl.record;
-    if (RESUME && !active) {   // a lane that is switched off meets no box: exit distance -inf on every axis
-        fs.ix = fs.iy = fs.iz = 0.f;
-        fs.cfx = fs.cfy = fs.cfz = -INFINITY;
-    }
     if (sgn & 1u) { onx = 48; ofx = 0; }
     if (sgn & 2u) { ony = 64; ofy = 16; }
     if (sgn & 4u) { onz = 80; ofz = 32; }
@@ -552,39 +496,15 @@ __device__ __forceinline__ void packet_walk(const DstAccelView &acc, const RaySl
     // copies of the buffer's 32 registers and moved them back and forth at every leaf group).
     constexpr uint32_t kEnd = 0xFFFFFFFFu;   // not a reference: leaf bit set, impossible position
     uint32_t budget = 2u * acc.n_leaves + 8u;
-    if constexpr (RESUME && HAND) {
-        if (wl.limit != 0u) budget = min(budget, wl.limit);
-    }
-    // The work lists are read and written a page of 64 items at a time: lane k of a page register holds item k.
-    uint32_t in_page = 0u, out_page = 0u, in_pos = 0u, n_out = 0u;
-    const uint32_t n_in = (RESUME && wl.n_in != kListFresh) ? wl.n_in : 0u;
-    auto next_input = [&]() -> uint32_t {
-        if (!RESUME || in_pos >= n_in) return kEnd;
-        if ((in_pos & 63u) == 0u) in_page = wl.in[in_pos + lane];
-        const uint32_t v = __builtin_amdgcn_readlane(in_page, in_pos & 63u);
-        ++in_pos;
-        return v;
-    };
-    auto record = [&](uint32_t v) {
-        if (n_out < kListCap) {
-            out_page = (uint32_t)dst_writelane((int)v, n_out & 63u, (int)out_page);
-            if ((n_out & 63u) == 63u) wl.out[(n_out & ~63u) + lane] = out_page;
-        }
-        n_out = min(n_out + 1u, kListCap + 1u);
-    };
     auto pop = [&]() -> uint32_t {
-        if (sp == 0) return next_input();
+        if (sp == 0) return kEnd;
         --sp;
         const uint32_t a = __builtin_amdgcn_readlane(stack0, sp & 63), b = __builtin_amdgcn_readlane(stack1, sp & 63);
         return sp < 64 ? a : b;
     };
-    // node items of a list carry the children to leave out; plain references (stack, root) leave out none
-    const bool packed = RESUME && acc.n_leaves <= (1u << kListIndexBits);
-    uint32_t ref = (RESUME && wl.n_in != kListFresh) ? next_input() : acc.root;
+    uint32_t ref = acc.root;
     for (;;) {
         while ((ref & DST_LEAF_BIT) == 0u) {
-            const uint32_t excl = packed ? (ref >> kListIndexBits) : 0u;
-            if (packed) ref &= (1u << kListIndexBits) - 1u;
             if (budget == 0u || ref + 1u >= acc.n_leaves) {   // spent, or not a node of this hierarchy
                 ref = kEnd;
                 break;
@@ -595,36 +515,17 @@ __device__ __forceinline__ void packet_walk(const DstAccelView &acc, const RaySl
             const float tmax = active ? kb_t(buf.e[kChunk - 1]) : -1.0f;
             uint32_t tail[5];
             uint32_t hit = 0u;                     // bit k: some lane enters child k
-            uint32_t ahead = 0u;                   // bit k: child k lies ahead of some lane's ray, at any distance
             {
                 u32x4 NX, NY, NZ, FX, FY, FZ, refs;
                 load_node(node, onx, ony, onz, ofx, ofy, ofz, NX, NY, NZ, FX, FY, FZ, refs, tail[4]);
                 tail[0] = refs[0]; tail[1] = refs[1]; tail[2] = refs[2]; tail[3] = refs[3];
 #pragma unroll
                 for (int k = DST_WIDE - 1; k >= 0; --k) {   // last child first: its bit is shifted up the furthest
-                    const float a = __builtin_fmaf(__uint_as_float(NX[k]), fs.ix, fs.cnx),
-                                b = __builtin_fmaf(__uint_as_float(NY[k]), fs.iy, fs.cny),
-                                c = __builtin_fmaf(__uint_as_float(NZ[k]), fs.iz, fs.cnz);
-                    const float e = __builtin_fmaf(__uint_as_float(FX[k]), fs.ix, fs.cfx),
-                                f = __builtin_fmaf(__uint_as_float(FY[k]), fs.iy, fs.cfy),
-                                g = __builtin_fmaf(__uint_as_float(FZ[k]), fs.iz, fs.cfz);
-                    const float tn = __builtin_fmaxf(__builtin_fmaxf(a, b), __builtin_fmaxf(c, 0.0f));
-                    if (RESUME) {
-                        // met at all (at a distance >= 0) / met within tmax; lanes that are switched off fail both
-                        const float tf = __builtin_fminf(__builtin_fminf(e, f), g);
-                        shift_in_near_far(hit, ahead, __builtin_amdgcn_fcmpf(tn, tmax, 5), __builtin_amdgcn_fcmpf(tn, tf, 5));
-                    } else {
-                        const float tf = __builtin_fminf(__builtin_fminf(e, f), __builtin_fminf(g, tmax));
-                        hit = shift_in_any(hit, __builtin_amdgcn_fcmpf(tn, tf, 5));   // 5 = ordered <=
-                    }
+                    float tn;
+                    hit = shift_in_any(hit, slab_hit_fast(fs, __uint_as_float(NX[k]), __uint_as_float(NY[k]), __uint_as_float(NZ[k]),
+                                                          __uint_as_float(FX[k]), __uint_as_float(FY[k]), __uint_as_float(FZ[k]), tmax, tn));
                 }
-                const uint32_t valid = ((1u << tail[4]) - 1u) & ~excl;   // unused slots are never entered
-                hit &= valid;
-                ahead &= valid;
-            }
-            if (recording) {
-                const uint32_t later = ahead & ~hit;   // beyond every ray's 16th hit so far: the next chunk's business
-                if (later != 0u) record(ref | ((~later & 15u) << kListIndexBits));
+                hit &= (1u << tail[4]) - 1u;   // unused slots are never entered
             }
             if (hit != 0u) {
                 // Children are taken in stored order: the first one that is hit next, the others deferred (last
@@ -661,25 +562,8 @@ __device__ __forceinline__ void packet_walk(const DstAccelView &acc, const RaySl
         --budget;
         const uint32_t first = ref & DST_REF_FIRST_MASK, count = ((ref >> 28) & 7u) + 1u;
         if (first + count > acc.n_leaves) break;   // not a leaf group of this hierarchy
-        const bool again = test_group<RESUME>(acc, first, count, rp, o, d, active, buf, cnt WSP);
-        if (recording && again) record(ref);
+        test_group(acc, first, count, rp, o, d, active, buf, cnt WSP);
         ref = pop();
-    }
-    if (RESUME) {
-        if constexpr (HAND) {
-            if (wl.limit != 0u && budget == 0u) wl.spent = true;
-        }
-        if (recording) {
-            // a walk that stopped early (budget, damaged structure) or a list that overflowed leaves no list
-            const bool whole = n_out <= kListCap && budget != 0u && ref == kEnd;
-            if (whole && (n_out & 63u) != 0u) wl.out[(n_out & ~63u) + lane] = out_page;
-            wl.n_in = whole ? n_out : kListFresh;
-            const lds_u32 t = wl.in;
-            wl.in = wl.out;
-            wl.out = t;
-        } else {
-            wl.n_in = kListFresh;
-        }
     }
 }
 
@@ -777,7 +661,7 @@ __device__ __attribute__((noinline)) void lane_walk(const LaneWalkAccel acc_in, 
         const bool hit = ray_quad(o, d, f3(w0.x, w0.y, w0.z), AB, AC, AD, cross_f(AB, AC), n1, cross_f(AC, AD),        \
                                   dot_f(n1, AB), t, tri);                                                              \
         const uint64_t x = kb_pack(t, 2u * __float_as_uint(w3.w) + tri);                                               \
-        if (hit && (x < buf.e[kChunk - 1])) {                                                                          \
+        if (hit && (kb_less(x, buf.e[kChunk - 1]))) {                                                                          \
             cnt += 1u;                                                                                                 \
             kbuf_insert(buf, x, true);                                                                                 \
         }                                                                                                              \
@@ -835,6 +719,8 @@ __device__ __attribute__((noinline)) void lane_walk(const LaneWalkAccel acc_in, 
     cnt_mem = cnt;
 }
 
+#include "bundle.inc"
+
 // Packet or per-lane walk for the rays of this wave?  A packet pays off when the rays run side by side: every
 // live ray is compared with the first live one (origins as given by the caller, not advanced along the ray).
 __device__ __forceinline__ bool rays_run_together(F3 o, F3 d, bool active, float max_abs) {
@@ -857,17 +743,18 @@ __device__ __forceinline__ bool rays_run_together(F3 o, F3 d, bool active, float
     return wave_ballot(apart) == 0ull;
 }
 
-template <bool MIXED, bool SHELF, bool RESUME, bool HAND>
-__device__ __forceinline__ void packet_knn(const DstAccelView &acc, float max_abs, F3 o, F3 d, bool active, KBuf &buf,
-                                           uint32_t &cnt, bool as_packet, WalkList &wl, uint32_t *shelf
+// `bw`: the bundle walk's state (forward), carried from chunk to chunk of a bounce.
+template <bool BWD, bool MIXED, bool SHELF, bool HAND>
+__device__ __forceinline__ void wave_knn(const DstAccelView &acc, float max_abs, F3 ro, F3 o, F3 d, float pay, bool active,
+                                         KBuf &buf, uint32_t &cnt, bool as_packet, BundleWalk &bw, uint32_t *shelf
 #ifdef DST_STATS
-                                           , WaveStats &ws
+                                         , WaveStats &ws
 #endif
 ) {
     const uint64_t live = wave_ballot(active);
     if (live == 0ull) return;
-    const RaySlab slab = make_slab(o, d, max_abs);
     if (MIXED && !as_packet) {
+        const RaySlab slab = make_slab(o, d, max_abs);
         KBuf mine = buf;   // a copy the call may keep in memory; the caller's buffer stays in registers
         uint32_t n = cnt;
         // forward kernels (one wave per workgroup, no other LDS) give the walk an LDS shelf for its stacks
@@ -877,23 +764,21 @@ __device__ __forceinline__ void packet_knn(const DstAccelView &acc, float max_ab
         cnt = n;
         return;
     }
-    // The walk assumes one set of direction signs per packet (the near face of every box is then the same for
-    // all lanes).  A wave whose rays straddle an axis plane (about 1 % of the tiles of a pinhole image) is
-    // walked once per sign class present, each time with the lanes of that class only.
-    const uint32_t my_sgn = (slab.ix < 0.f ? 1u : 0u) | (slab.iy < 0.f ? 2u : 0u) | (slab.iz < 0.f ? 4u : 0u);
-    uint64_t todo = live;
-    if (RESUME) {
-        // a work list serves one walk per chunk: waves with several sign classes walk from the root every time
-        const uint32_t sgn0 = __builtin_amdgcn_readlane(my_sgn, __builtin_ctzll(live));
-        wl.record = wave_ballot(active && my_sgn != sgn0) == 0ull && acc.n_leaves <= (1u << kListIndexBits);
-        if (!wl.record) wl.n_in = kListFresh;
-    }
-    while (todo != 0ull) {
-        const int rep = __builtin_ctzll(todo);   // also the lane whose entry distances order the children
-        const uint32_t sgn = __builtin_amdgcn_readlane(my_sgn, rep);
-        const bool mine = active && my_sgn == sgn;
-        todo &= ~wave_ballot(mine);
-        packet_walk<RESUME, HAND>(acc, slab, sgn, o, d, mine, rep, buf, cnt, wl WSP);
+    if constexpr (!BWD) {
+        bundle_knn<HAND>(acc, max_abs, ro, o, d, pay, active, buf, cnt, bw WSP);
+    } else {
+        // The walk assumes one set of direction signs per packet (the near face of every box is then the same for
+        // all lanes).  A wave whose rays straddle an axis plane (about 1 % of the tiles of a pinhole image) is
+        // walked once per sign class present, each time with the lanes of that class only.
+        const RaySlab slab = make_slab(o, d, max_abs);
+        const uint32_t my_sgn = (slab.ix < 0.f ? 1u : 0u) | (slab.iy < 0.f ? 2u : 0u) | (slab.iz < 0.f ? 4u : 0u);
+        uint64_t todo = live;
+        while (todo != 0ull) {
+            const uint32_t sgn = __builtin_amdgcn_readlane(my_sgn, __builtin_ctzll(todo));
+            const bool mine = active && my_sgn == sgn;
+            todo &= ~wave_ballot(mine);
+            packet_walk(acc, slab, sgn, o, d, mine, buf, cnt WSP);
+        }
     }
 }
 
@@ -1547,24 +1432,18 @@ __device__ __forceinline__ bool walk_bounce(const DstParams &p, const DstAccelVi
     // kernels built without the per-lane walk (MIXED false) take every wave as a packet
     const bool as_packet = (!MIXED || (REC && BWD)) ? true
                                                     : (HAND && first_walk == kWalkPerLane ? false : rays_run_together(ro, rd, lane_on, max_abs));
-    // Forward: the walks of a bounce's later chunks resume from the list the walk before left (the backward
-    // re-trace has its LDS taken by the gradient table and walks from the root).
-    constexpr bool RESUME = !BWD;
-    // One LDS area per wave serves the packet walk's two lists or the per-lane walk's stack shelf: all chunks of
-    // a bounce use the same walk, and a bounce starts without a list.
+    // Forward: one LDS area per wave serves the bundle walk's lists or the per-lane walk's stack shelf (all chunks of a
+    // bounce use the same walk, and a bounce starts without a list).
     constexpr bool SHELF = MIXED && !BWD;
-    constexpr uint32_t kListWords = 2u * kListCap;
-    constexpr uint32_t kWaveLds = (SHELF && (uint32_t)(kLaneShelf * DST_WAVE) > kListWords) ? (uint32_t)(kLaneShelf * DST_WAVE)
-                                                                                            : (RESUME ? kListWords : 1u);
-    __shared__ uint32_t s_list[(RESUME || SHELF) ? kFwdWavesPerBlock * kWaveLds : 1];
-    uint32_t *const wave_lds = s_list + ((RESUME || SHELF) ? (threadIdx.x / DST_WAVE) * kWaveLds : 0);
-    WalkList wl;
-    wl.in = (lds_u32)wave_lds;
-    wl.out = wl.in + (RESUME ? kListCap : 0);
-    wl.n_in = kListFresh;
-    wl.record = false;
-    wl.limit = (HAND && first_walk != kWalkPerLane) ? first_walk : 0u;
-    wl.spent = false;
+    constexpr uint32_t kWaveLds = BWD ? 1u : (SHELF ? (uint32_t)(kLaneShelf * DST_WAVE) : kBwWords);
+    static_assert(kBwWords <= (uint32_t)(kLaneShelf * DST_WAVE), "the lists fit where the shelf is");
+    __shared__ uint32_t s_walk[BWD ? 1u : (uint32_t)kFwdWavesPerBlock * kWaveLds];
+    uint32_t *const wave_lds = s_walk + (BWD ? 0u : (threadIdx.x / DST_WAVE) * kWaveLds);
+    BundleWalk bw;
+    bw.lds.base = (lds_u32)wave_lds;
+    bw.da = bw.uoff = 0.f;
+    bw.kept = bw.spent = false;
+    bw.limit = (HAND && first_walk != kWalkPerLane) ? first_walk : 0u;
     uint32_t rec_pos = (REC && BWD) ? (rv.dir[bounce] & kRecDirBlockMask) : 0xFFFFFFFFu;   // replay: next block + 1; record: previous block
     uint32_t rec_chunks = 0u;   // forward with a record: chunks stored for this bounce
     for (;;) {
@@ -1593,10 +1472,10 @@ __device__ __forceinline__ bool walk_bounce(const DstParams &p, const DstAccelVi
             }
         } else {
             kbuf_reset(buf);
-            packet_knn<MIXED, SHELF, RESUME, HAND>(acc, max_abs, ot, rd, live, buf, cnt, as_packet, wl, wave_lds WSP);
+            wave_knn<BWD, MIXED, SHELF, HAND>(acc, max_abs, ro, ot, rd, pay_dpt, live, buf, cnt, as_packet, bw, wave_lds WSP);
             if constexpr (HAND) {
-                if (wl.spent) return true;   // only a bounce's first walk has a limit: nothing has been written yet
-                wl.limit = 0u;
+                if (bw.spent) return true;   // only a bounce's first walk has a limit: nothing has been written yet
+                bw.limit = 0u;
             }
             if (REC && !BWD) {
                 rec_colours = rec_store(rv, bounce, rec_pos, buf, cnt);
