@@ -50,7 +50,7 @@ struct alignas(16) DstLeaf {
     uint32_t g;
     float n0[3], n2[3];
     float c1;
-    uint32_t pad;
+    float edge;           // largest |coordinate| of AB, AC, AD
 };
 static_assert(sizeof(DstLeaf) == 96, "leaf records are 24 dwords");
 

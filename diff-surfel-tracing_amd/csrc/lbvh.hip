@@ -605,7 +605,9 @@ __device__ __forceinline__ void write_leaf(const float (&c)[4][3], uint32_t g, u
     }
     out[15] = __uint_as_float(g);
     out[22] = c1;
-    out[23] = 0.f;
+    out[23] = 0.f;   // largest coordinate of an edge vector
+#pragma unroll
+    for (int a = 0; a < 3; ++a) out[23] = fmaxf(out[23], fmaxf(fmaxf(fabsf(e1[a]), fabsf(e2[a])), fabsf(e3[a])));
     float4 *dst = reinterpret_cast<float4 *>(&leaves[i]);
 #pragma unroll
     for (int k = 0; k < 6; ++k) dst[k] = make_float4(out[4 * k], out[4 * k + 1], out[4 * k + 2], out[4 * k + 3]);

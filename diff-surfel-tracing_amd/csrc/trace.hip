@@ -205,6 +205,18 @@ __device__ __forceinline__ bool ray_quad(F3 o, F3 d, F3 A, F3 AB, F3 AC, F3 AD, 
 // v_writelane_b32: value (uniform) into lane `lane` (uniform) of `old`; the compiler offers no builtin for it.
 __device__ int dst_writelane(int value, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
 
+// The kernel's parameter block where the hardware put it.  Read through a pointer the compiler cannot follow
+// (fresh_params), the block's pointers are scalar loads at their place of use, in every step of a loop anew; read
+// through the kernel's argument they are loaded once, far too many for the scalar registers, and every use in a loop
+// brings them back from lanes of a vector register, one vector instruction per word: a quarter of the compositing
+// loop's instructions.
+typedef const __attribute__((address_space(4))) DstParams *const_params;
+__device__ __forceinline__ const_params fresh_params() {
+    const_params p = (const_params)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
 // ---- wave-uniform fetches ---------------------------------------------------------------------------------
 typedef const __attribute__((address_space(4))) uint32_t *const_u32_ptr;
 typedef __attribute__((address_space(3))) uint32_t *lds_u32;
@@ -346,9 +358,13 @@ __device__ __forceinline__ uint64_t kb_max(uint64_t a, uint64_t b) {
 // Sorted insert in place: slot k becomes the middle one of its entry, the entry above and the new one.
 __device__ __forceinline__ void kbuf_insert(KBuf &b, uint64_t x_in, bool on) {
     const uint64_t x = on ? x_in : kNoEntry;   // a lane that inserts nothing offers what leaves every slot as it is
+    // (two slots at a time: a double-precision result is not ready for the very next instruction)
 #pragma unroll
-    for (int k = kChunk - 1; k >= 1; --k) b.e[k] = kb_max(b.e[k - 1], kb_min(b.e[k], x));
-    b.e[0] = kb_min(b.e[0], x);
+    for (int k = kChunk - 1; k >= 1; k -= 2) {
+        const uint64_t m1 = kb_min(b.e[k], x), m0 = kb_min(b.e[k - 1], x);
+        b.e[k] = kb_max(b.e[k - 1], m1);
+        b.e[k - 1] = k >= 2 ? kb_max(b.e[k - 2], m0) : m0;
+    }
 }
 
 #ifdef DST_STATS
@@ -1540,8 +1556,9 @@ __device__ __forceinline__ bool walk_bounce(const DstParams &p, const DstAccelVi
             F3 R[3] = {f3(1, 0, 0), f3(0, 1, 0), f3(0, 0, 1)};
             float col[3] = {0.f, 0.f, 0.f};
             bool neg[3] = {false, false, false};
-            const float *sh = p.shs;   // valid address for lanes that sit phase 2 out
+            const float *sh = nullptr;
             do {
+                const const_params kp = fresh_params();
                 if (!on) break;
                 g = (int)(e_i >> 1);
                 if (g == last_g) break;
@@ -1552,10 +1569,10 @@ __device__ __forceinline__ bool walk_bounce(const DstParams &p, const DstAccelVi
                     sx = cur.s[0]; sy = cur.s[1];
                     q0 = cur.q[0]; q1 = cur.q[1]; q2 = cur.q[2]; q3 = cur.q[3];
                 } else {
-                    mean = ld3(p.means3D + 3 * (size_t)g);
-                    sx = p.scales[2 * (size_t)g];
-                    sy = p.scales[2 * (size_t)g + 1];
-                    const float *qp = p.rotations + 4 * (size_t)g;
+                    mean = ld3(kp->means3D + 3 * (size_t)g);
+                    sx = kp->scales[2 * (size_t)g];
+                    sy = kp->scales[2 * (size_t)g + 1];
+                    const float *qp = kp->rotations + 4 * (size_t)g;
                     q0 = qp[0]; q1 = qp[1]; q2 = qp[2]; q3 = qp[3];
                 }
                 quat_rows(q0, q1, q2, q3, R);
@@ -1574,7 +1591,7 @@ __device__ __forceinline__ bool walk_bounce(const DstParams &p, const DstAccelVi
                 if (dpt < min_depth) break;
                 const float power = -0.5f * rho;
                 if (power > 0.0f) break;
-                opac = (REC && BWD) ? cur.o : p.opacities[g];
+                opac = (REC && BWD) ? cur.o : kp->opacities[g];
                 G = exp_det(power);
                 alpha = opac * G;
                 alpha = (alpha < 0.99f) ? alpha : 0.99f;
@@ -1590,19 +1607,19 @@ __device__ __forceinline__ bool walk_bounce(const DstParams &p, const DstAccelVi
                     for (int ch = 0; ch < 3; ++ch) {
                         col[ch] = cur.c[ch];
                         // -0: clamped (a colour evaluated from SH is never negative; given colours may be)
-                        neg[ch] = p.colors_precomp == nullptr && (__float_as_uint(col[ch]) >> 31) != 0u;
+                        neg[ch] = kp->colors_precomp == nullptr && (__float_as_uint(col[ch]) >> 31) != 0u;
                     }
-                } else if (p.colors_precomp == nullptr) {
-                    sh = p.shs + (size_t)g * p.M * 3;
+                } else if (kp->colors_precomp == nullptr) {
+                    sh = kp->shs + (size_t)g * kp->M * 3;
                     // (the binary16 source lives in the forward kernels that carry the rarely used options; a backward
                     // trace is given the widened values as shs)
-                    const F3 c = (!BWD && DET && (p.flags & DST_FLAG_SH_HALF)) ? sh_color_half(p, g, rd, neg)
-                                                                              : sh_color(p.D, ShF32{sh}, rd, neg);
+                    const F3 c = (!BWD && DET && (kp->flags & DST_FLAG_SH_HALF)) ? sh_color_half(p, g, rd, neg)
+                                                                              : sh_color(kp->D, ShF32{sh}, rd, neg);
                     col[0] = c.x; col[1] = c.y; col[2] = c.z;
                 } else {
-                    col[0] = p.colors_precomp[3 * (size_t)g];
-                    col[1] = p.colors_precomp[3 * (size_t)g + 1];
-                    col[2] = p.colors_precomp[3 * (size_t)g + 2];
+                    col[0] = kp->colors_precomp[3 * (size_t)g];
+                    col[1] = kp->colors_precomp[3 * (size_t)g + 1];
+                    col[2] = kp->colors_precomp[3 * (size_t)g + 2];
                 }
                 if (REC && !BWD && rec_colours != nullptr) {
                     float *cs = rec_colours + it * 3 * DST_WAVE + lane_;
@@ -1612,12 +1629,12 @@ __device__ __forceinline__ bool walk_bounce(const DstParams &p, const DstAccelVi
                 run.C[0] += w * col[0];
                 run.C[1] += w * col[1];
                 run.C[2] += w * col[2];
-                if (p.others_precomp != nullptr) {
+                if (kp->others_precomp != nullptr) {
 #pragma unroll
                     for (int ch = 0; ch < AUXM; ++ch)
-                        if (ch < p.aux) run.O[ch] += w * p.others_precomp[(size_t)p.aux * g + ch];
+                        if (ch < kp->aux) run.O[ch] += w * kp->others_precomp[(size_t)kp->aux * g + ch];
                 }
-                if (!BWD && DET && (p.flags & DST_FLAG_DISTORTION)) {
+                if (!BWD && DET && (kp->flags & DST_FLAG_DISTORTION)) {
                     // depth distortion of 2DGS with its running moments (x = distortion, y = M1, z = M2); the
                     // reference declares the three and leaves the computation open (forward.cu:286)
                     const float A_before = 1 - Tp;
@@ -1638,9 +1655,10 @@ __device__ __forceinline__ bool walk_bounce(const DstParams &p, const DstAccelVi
                 Tp = Tn;
             } while (false);
             if (REC && BWD) fetch_geometry(want_next);
-            if (!BWD && p.training && p.a_weights != nullptr) {
-                if (!MIXED && !DET) wet_add(tab_keys, tab_rows, p.a_weights, did, (uint32_t)g, w);   // the wave's LDS table
-                else wave_add_grouped(p.a_weights, (DET && (p.flags & DST_FLAG_DETERMINISTIC)) ? p.det_workspace : nullptr, did,
+            const const_params kp = fresh_params();
+            if (!BWD && kp->training && kp->a_weights != nullptr) {
+                if (!MIXED && !DET) wet_add(tab_keys, tab_rows, kp->a_weights, did, (uint32_t)g, w);   // the wave's LDS table
+                else wave_add_grouped(kp->a_weights, (DET && (kp->flags & DST_FLAG_DETERMINISTIC)) ? kp->det_workspace : nullptr, did,
                                       (uint32_t)g, w);
             }
             // ---- phase 2 (whole wave, backward only): gradients of the hits composited above -----------
@@ -2112,7 +2130,10 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
 // The two entry kernels differ only in the occupancy the register allocator is told to aim for: both are
 // bound by the latency of dependent fetches, so waves in flight matter more than a few spilled values.
 #ifndef DST_FWD_WAVES
-#define DST_FWD_WAVES 4
+#define DST_FWD_WAVES 3
+#endif
+#ifndef DST_MIXED_WAVES
+#define DST_MIXED_WAVES 4
 #endif
 #ifndef DST_BWD_WAVES
 #define DST_BWD_WAVES 3
@@ -2120,7 +2141,7 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
 // EXTRAS: the rarely used forward options (DstParams.flags: fixed-point blending weights, distortion output) live in
 // a kernel of their own, so that the usual one does not carry their registers.
 template <int AUXM, bool REC, bool MIXED, bool EXTRAS>
-__global__ __launch_bounds__(kFwdWavesPerBlock *DST_WAVE) __attribute__((amdgpu_waves_per_eu(DST_FWD_WAVES, DST_FWD_WAVES)))
+__global__ __launch_bounds__(kFwdWavesPerBlock *DST_WAVE) __attribute__((amdgpu_waves_per_eu(MIXED ? DST_MIXED_WAVES : DST_FWD_WAVES, MIXED ? DST_MIXED_WAVES : DST_FWD_WAVES)))
 void k_trace_fwd(const DstParams p, const DstAccelView acc, int tw_log2, int th_log2, uint32_t tiles_x,
                  uint32_t tiles_y, uint32_t btiles_x, const uint32_t *ray_order, uint32_t strip_width, uint32_t *handover,
                  uint32_t hand_arg) {
