@@ -29,6 +29,9 @@ constexpr int kWavesPerBlock = 4;
 #define DST_FWD_WPB 1
 #endif
 constexpr int kFwdWavesPerBlock = DST_FWD_WPB;   // 1 or kWavesPerBlock
+#ifndef DST_BWD_WAVES
+#define DST_BWD_WAVES 2
+#endif
 #ifndef DST_STRIP_FWD
 #define DST_STRIP_FWD 8   // width of the column strips the blocks of an image grid are walked in (0: row-major)
 #endif
@@ -809,28 +812,22 @@ __device__ __forceinline__ void aadd(float *p, float v) { unsafeAtomicAdd(p, v);
 #define DST_TABLE_FLUSH_NUM 3   // the table is emptied between rounds once this many eighths of its rows are in use
                                 // (measured 1..6: a fuller table sends more hits past it, straight to memory)
 #endif
-#ifndef DST_TABLE_ROWS_LOG2
-#define DST_TABLE_ROWS_LOG2 7
-#endif
 constexpr uint32_t kEmptyKey = 0xFFFFFFFFu;
 constexpr int kMaxProbe = 8;
-// row columns: colour 0-2, opacity 3, scales 4-5, rotation 6-9, mean 10-12, densification mean 13-15, SH coefficient
-// j channel c at 16+3j+c (16..63), aux 64..64+AUXM-1.  The auxiliary channels come last so that a scene without
-// them (the usual one) fills exactly four 16-column tiles of the group reduction and skips the fifth.
+// Row columns: colour 0-2, opacity 3, scales 4-5, rotation 6-9, mean 10-12, densification mean 13-15, SH coefficient
+// j channel c at 16+16c+j (16..63: what sixteen lanes add together lies together), aux 64..64+AUXM-1.
 constexpr int kColColor = 0, kColOpac = 3, kColScale = 4, kColRot = 6, kColMean = 10, kColGrad = 13, kColSh = 16,
               kColAux = 64;
+// The sums are doubles (deterministic mode: 64-bit fixed point).  Not for their precision: an LDS addition of floats
+// takes its lanes one after the other (measured: 3 cycles a lane, 192 for a wave, whatever the addresses), one of
+// doubles or of integers takes 8.
+constexpr int kStageBytes = kWavesPerBlock * DST_WAVE * 17 * 4;   // the waves' staging areas (GradSink)
 template <int AUXM> struct RowLayout {
-    static constexpr int sh0 = kColSh;
     static constexpr int cols = kColAux + AUXM;
-    static constexpr int stride = cols | 1;     // odd: rows spread over all LDS banks
-    // rows of the block's table: with more auxiliary channels the rows are longer, and three blocks must fit a CU
-    static constexpr int rows_log2 = AUXM <= 2 ? DST_TABLE_ROWS_LOG2 : DST_TABLE_ROWS_LOG2 - 1;
-    static constexpr int rows = 1 << rows_log2;
-};
-// The deterministic mode keeps 64-bit fixed-point sums in the table: half as many rows in the same memory.
-template <int AUXM, bool DET> struct TableRows {
-    static constexpr int rows_log2 = RowLayout<AUXM>::rows_log2 - (DET ? 1 : 0);
-    static constexpr int rows = 1 << rows_log2;
+    static constexpr int stride = cols | 1;     // 8-byte words of a table row; odd: rows spread over all LDS banks
+    // Rows of the block's table, one more taking what belongs nowhere: what three blocks leave each other of a CU's
+    // 160 KB, which is given out in pieces of 1280 bytes.
+    static constexpr int rows = ((128 / DST_BWD_WAVES) * 1280 - kStageBytes - 1024) / (8 * stride) - 1;
 };
 
 // ---- deterministic mode: sums in 64-bit fixed point ------------------------------------------------------
@@ -849,9 +846,10 @@ __device__ __forceinline__ long long to_fixed(float v, int shift) {
 }
 __device__ __forceinline__ float from_fixed(long long q, int shift) { return (float)__builtin_ldexp((double)q, -shift); }
 
+// (P: DstParams, wherever it lies.)
 // Address in the caller's gradient tensors of column `col` of surfel g (nullptr: nothing to write).
-template <int AUXM>
-__device__ __forceinline__ float *tensor_address(const DstParams &p, uint32_t g, int col) {
+template <int AUXM, class P>
+__device__ __forceinline__ float *tensor_address(const P &p, uint32_t g, int col) {
     if (col < kColOpac) return p.dL_dcolors + 3 * (size_t)g + col;
     if (col < kColScale) return p.dL_dopacities + g;
     if (col < kColRot) return p.dL_dscales + 2 * (size_t)g + (col - kColScale);
@@ -862,20 +860,20 @@ __device__ __forceinline__ float *tensor_address(const DstParams &p, uint32_t g,
         const int ch = col - kColAux;
         return (p.others_precomp != nullptr && ch < p.aux) ? p.dL_dothers + (size_t)p.aux * g + ch : nullptr;
     }
-    const int k = col - kColSh;   // 3j + c
-    return (p.colors_precomp == nullptr && k < 3 * p.M) ? p.dL_dshs + (size_t)g * p.M * 3 + k : nullptr;
+    const int c = (col - kColSh) >> 4, j = (col - kColSh) & 15;
+    return (p.colors_precomp == nullptr && j < p.M) ? p.dL_dshs + (size_t)g * p.M * 3 + 3 * j + c : nullptr;
 }
 // Is column `col` in use?  (no auxiliary input: no aux columns; colours given: no SH columns; SH degree < 3: fewer)
-template <int AUXM>
-__device__ __forceinline__ bool column_live(const DstParams &p, int col) {
+template <int AUXM, class P>
+__device__ __forceinline__ bool column_live(const P &p, int col) {
     if (col < kColSh) return true;
     if (col >= kColAux) return p.others_precomp != nullptr && col - kColAux < p.aux;
-    return p.colors_precomp == nullptr && col - kColSh < 3 * p.M;
+    return p.colors_precomp == nullptr && ((col - kColSh) & 15) < p.M;
 }
 // Where the kernels add column `col` of surfel g: the row of g in the caller's gradient rows if there are any
 // (all columns of a surfel side by side; a closing kernel adds the rows to the tensors), else the tensors.
-template <int AUXM>
-__device__ __forceinline__ float *grad_address(const DstParams &p, uint32_t g, int col) {
+template <int AUXM, class P>
+__device__ __forceinline__ float *grad_address(const P &p, uint32_t g, int col) {
     if (p.grad_rows == nullptr) return tensor_address<AUXM>(p, g, col);
     return column_live<AUXM>(p, col) ? p.grad_rows + (size_t)g * RowLayout<AUXM>::cols + col : nullptr;
 }
@@ -922,10 +920,10 @@ __device__ __forceinline__ void wave_add_grouped(float *base, unsigned long long
 
 // The blending weights of an image wave (forward, training): a wave composites the same two hundred or so surfels over
 // and over (64 neighbouring rays, some 37 hits each), so their weights are first summed in a small hash table in LDS
-// (surfel id -> running sum, LDS atomics) and go to memory once per surfel and wave when the wave ends - a sixteenth of
+// (surfel id -> running sum, LDS atomics on doubles: those on floats take a lane at a time) and go to memory once per surfel and wave when the wave ends - a sixteenth of
 // the global atomics.  A surfel that finds no slot within a few probes adds straight to memory.
 constexpr int kWetSlotsLog2 = 8, kWetSlots = 1 << kWetSlotsLog2, kWetProbes = 4;
-__device__ __forceinline__ void wet_add(uint32_t *keys, float *vals, float *a_weights, bool on, uint32_t g, float w) {
+__device__ __forceinline__ void wet_add(uint32_t *keys, double *vals, float *a_weights, bool on, uint32_t g, float w) {
     if (!on) return;
     uint32_t slot = (g * 2654435761u) >> (32 - kWetSlotsLog2);
 #pragma unroll 1
@@ -938,7 +936,7 @@ __device__ __forceinline__ void wet_add(uint32_t *keys, float *vals, float *a_we
             k = expected == 0xFFFFFFFFu ? g : expected;
         }
         if (k == g) {
-            __hip_atomic_fetch_add(vals + slot, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __hip_atomic_fetch_add(vals + slot, (double)w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             return;
         }
         slot = (slot + 1u) & (uint32_t)(kWetSlots - 1);
@@ -948,9 +946,9 @@ __device__ __forceinline__ void wet_add(uint32_t *keys, float *vals, float *a_we
 
 // Find or claim the table row of surfel g; -1 if none is free within a few probes.  keys[rows] counts the
 // rows claimed since the table was last emptied.
-template <int ROWS_LOG2>
+template <int ROWS>
 __device__ __forceinline__ int table_slot(uint32_t *keys, uint32_t g) {
-    uint32_t slot = (g * 2654435761u) >> (32 - ROWS_LOG2);
+    uint32_t slot = __umulhi(g * 2654435761u, (uint32_t)ROWS);
 #pragma unroll 1
     for (int probe = 0; probe < kMaxProbe; ++probe) {
         uint32_t k = __hip_atomic_load(keys + slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -960,161 +958,199 @@ __device__ __forceinline__ int table_slot(uint32_t *keys, uint32_t g) {
                                                  __HIP_MEMORY_SCOPE_WORKGROUP);
             if (expected == kEmptyKey) {
                 k = g;
-                __hip_atomic_fetch_add(keys + (1u << ROWS_LOG2), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                __hip_atomic_fetch_add(keys + ROWS, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             } else {
                 k = expected;
             }
         }
         if (k == g) return (int)slot;
-        slot = (slot + 1) & ((1u << ROWS_LOG2) - 1u);
+        slot = slot + 1u == (uint32_t)ROWS ? 0u : slot + 1u;
     }
     return -1;
 }
 
-// Where one step's per-surfel gradients go.  Neighbouring rays mostly composite the same few surfels in the
-// same step, so the wave first sums the lanes of each surfel and only the sums go to the table.  That sum is
-// a matrix product: (columns x rays) times (rays x surfel groups, entries 0 or 1).  The lanes stage their
-// column values in LDS, sixteen columns at a time, and sixteen 16x16x4 fp32 MFMAs per tile produce the sums
-// of up to sixteen groups at once; lanes of further groups (rare) add their values directly.
-constexpr int kStageCols = 16;                 // columns per tile
-constexpr int kStageStride = DST_WAVE + 1;     // floats per staged column: conflict-free writes and reads
-constexpr int kStageWords = kStageCols * kStageStride;
+// The SH basis in direction d up to degree `deg`, zero beyond (gradient algebra; reference backward.cu:68-166).
+__device__ __forceinline__ void sh_basis(int deg, F3 d, float (&basis)[16]) {
+#pragma clang fp contract(fast)
+    const float x = d.x, y = d.y, z = d.z;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) basis[j] = 0.f;
+    basis[0] = SH0;
+    if (deg > 0) {
+        basis[1] = -SH1 * y;
+        basis[2] = SH1 * z;
+        basis[3] = -SH1 * x;
+        if (deg > 1) {
+            const float xx = x * x, yy = y * y, zz = z * z, xy = x * y, yz = y * z, xz = x * z;
+            basis[4] = SH2[0] * xy;
+            basis[5] = SH2[1] * yz;
+            basis[6] = SH2[2] * (2.f * zz - xx - yy);
+            basis[7] = SH2[3] * xz;
+            basis[8] = SH2[4] * (xx - yy);
+            if (deg > 2) {
+                basis[9] = SH3[0] * y * (3.f * xx - yy);
+                basis[10] = SH3[1] * xy * z;
+                basis[11] = SH3[2] * y * (4.f * zz - xx - yy);
+                basis[12] = SH3[3] * z * (2.f * zz - 3.f * xx - 3.f * yy);
+                basis[13] = SH3[4] * x * (4.f * zz - xx - yy);
+                basis[14] = SH3[5] * z * (xx - yy);
+                basis[15] = SH3[6] * x * (xx - 3.f * yy);
+            }
+        }
+    }
+}
+
+// Value of lane m of this lane's row of sixteen.
+template <int M>
+__device__ __forceinline__ uint32_t row_bcast(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + M, 0xf, 0xf, true); }
+template <int M>
+__device__ __forceinline__ float row_bcast(float v) { return __uint_as_float(row_bcast<M>(__float_as_uint(v))); }
+
+// One hit's columns to memory, for the lanes with `on`: lane%16 has the geometric column of that number and the three
+// channels of that SH coefficient.  The slow way, column by column: for the
+// deterministic mode, and for callers without gradient rows.
+template <int AUXM, bool DET>
+__device__ __attribute__((noinline)) void put_columns(const DstParams *p_in, uint32_t g, bool on, float geo, F3 sh) {
+    const DstParams &p = *uniform_ptr(p_in);
+    const int i = (int)(__lane_id() & 15u);
+    auto put = [&](int col, float v) {
+        if (DET) {
+            if (column_live<AUXM>(p, col))
+                atomicAdd(p.det_workspace + (size_t)g * RowLayout<AUXM>::cols + col, (unsigned long long)to_fixed(v, det_shift(col)));
+        } else {
+            float *dst = grad_address<AUXM>(p, g, col);
+            if (dst != nullptr) aadd(dst, v);
+        }
+    };
+    if (!on) return;
+    if (geo != 0.f) put(i, geo);
+    if (sh.x != 0.f) put(kColSh + i, sh.x);
+    if (sh.y != 0.f) put(kColSh + 16 + i, sh.y);
+    if (sh.z != 0.f) put(kColSh + 32 + i, sh.z);
+}
+
+// Where one step's per-surfel gradients go: into the block's table, row of the hit's surfel, columns 0..15 geometry,
+// 16..63 SH (basis_j(ray) * colour gradient_c), 64.. auxiliary channels.  A row of sixteen lanes takes the hits of its
+// own sixteen rays one after the other, a lane per column (and per SH coefficient): four hits at a time, sixteen
+// rounds.  The geometric columns come through LDS ([ray][column], an odd stride); the basis belongs to the ray, so
+// each lane keeps its coefficient's values for its row's sixteen rays in registers for the whole bounce, and the hit's
+// colour gradient is broadcast along the row by the multiplication itself.  Hits of the same surfel meet in the LDS
+// atomics, and it does not matter how many different surfels a step composites.
+// (Before, the lanes of a surfel were summed by matrix products over up to sixteen groups a step, the 64 columns staged
+// in LDS.  Grouping cost more than it saved: a step of these scenes composites 6 to 20 different surfels, over half the
+// steps of two of them more than sixteen, and what did not fit went column by column.)
+constexpr int kGeoCols = 16;
 template <int AUXM, bool DET>
 struct GradSink {
-    const DstParams *p;
-    float *rows;         // the block's table
-    float *stage;        // this wave's staging tile: [column in tile][lane]
+    static constexpr int stride = kGeoCols + 1;   // four rays sixteen apart start in different quarters of the banks
+    static constexpr int words = DST_WAVE * stride;
+    static_assert(kWavesPerBlock * words * 4 == kStageBytes, "the table's size counts on the staging areas'");
+    double *rows;        // the block's table; its last row takes what belongs nowhere
+    float *stage;        // this wave's staging area
     bool did;            // this lane composited a hit in this step
     uint32_t g;          // its surfel
     int own_slot;        // table row of g, -1: none
-    bool stray;          // hit, but not in one of the sixteen groups
-    bool any_stray;      // wave-uniform: some lane is a stray
-    uint32_t members;    // bit m: the ray of lane 16*(lane/16)+m belongs to group lane%16
-    bool out_on;         // lane%16 is a group of this step
-    int out_slot;        // table row of group lane%16, -1: write through to global memory
-    uint32_t out_g;      // surfel of group lane%16
-    int limit;           // columns in use
     uint64_t wt;         // wave-uniform: lanes whose surfel has no table row (their values go to global memory)
 
-    // Wave-uniform; every lane of the wave must be active.
     __device__ __forceinline__ void plan(uint32_t *keys) {
-        const uint32_t lane = __lane_id();
-        uint64_t rem = wave_ballot(did);
-        int n_groups = 0;
-        bool grouped = false;
-        uint32_t leader = 0u;
-        members = 0u;
-#pragma unroll 1
-        while (rem != 0ull && n_groups < kStageCols) {
-            const int first = __builtin_ctzll(rem);
-            const uint32_t k0 = __builtin_amdgcn_readlane(g, first);
-            const bool same = did && g == k0;
-            const uint64_t grp = wave_ballot(same);
-            if ((lane & 15u) == (uint32_t)n_groups) {
-                members = (uint32_t)(grp >> (lane & 48u)) & 0xFFFFu;
-                leader = (uint32_t)first;
-            }
-            grouped = grouped || same;
-            ++n_groups;
-            rem &= ~grp;
+        own_slot = did ? table_slot<RowLayout<AUXM>::rows>(keys, g) : -1;
+        wt = wave_ballot(did && own_slot < 0);
+    }
+    // Column `col` of this lane's hit (every lane; a lane without a hit may pass anything).
+    __device__ __forceinline__ void set(int col, float v) const { stage[__lane_id() * stride + col] = v; }
+
+    // v into column `col` (in the table's memory: word `at`).
+    __device__ __forceinline__ void put(uint32_t at, int shift, float v) const {
+        if (DET) __hip_atomic_fetch_add(reinterpret_cast<long long *>(rows) + at, to_fixed(v, shift), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        else __hip_atomic_fetch_add(rows + at, (double)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+
+    template <int M>
+    __device__ __forceinline__ void round(const_params p, uint32_t slot, uint32_t ray0, const float (&basis)[16], F3 gc, bool sh) const {
+        const uint32_t i = __lane_id() & 15u;
+        const uint32_t at = row_bcast<M>(slot) + i;
+        const float geo = stage[ray0 + M * stride];
+        const float x = row_bcast<M>(gc.x) * basis[M], y = row_bcast<M>(gc.y) * basis[M], z = row_bcast<M>(gc.z) * basis[M];
+        put(at, det_shift((int)i), geo);
+        if (sh) {
+            put(at + kColSh, kDetShiftOther, x);
+            put(at + kColSh + 16u, kDetShiftOther, y);
+            put(at + kColSh + 32u, kDetShiftOther, z);
         }
-        stray = did && !grouped;
-        any_stray = wave_ballot(stray) != 0ull;
-        out_on = (lane & 15u) < (uint32_t)n_groups;
-        own_slot = did ? table_slot<TableRows<AUXM, DET>::rows_log2>(keys, g) : -1;
-        out_slot = __builtin_amdgcn_ds_bpermute((int)(leader << 2), own_slot);
-        out_g = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(leader << 2), (int)g);
-        // (deterministic mode: a group's sum must be rounded to fixed point as one number whether or not it finds
-        // a table row, which depends on timing; so only the lanes outside the groups take this route there)
-        wt = wave_ballot(did && own_slot < 0 && (!DET || stray));
-    }
-
-    __device__ __forceinline__ void put_global(uint32_t surfel, int col, float v) const {
-        if (DET) {
-            if (column_live<AUXM>(*p, col))
-                atomicAdd(p->det_workspace + (size_t)surfel * RowLayout<AUXM>::cols + col,
-                          (unsigned long long)to_fixed(v, det_shift(col)));
-        } else {
-            float *dst = grad_address<AUXM>(*p, surfel, col);
-            if (dst != nullptr) aadd(dst, v);
-        }
-    }
-
-    // Add v to column `col` of table row `slot` (>= 0).
-    __device__ __forceinline__ void put(int slot, int col, float v) const {
-        if (DET)
-            __hip_atomic_fetch_add(reinterpret_cast<long long *>(rows) + (size_t)slot * RowLayout<AUXM>::stride + col,
-                                   to_fixed(v, det_shift(col)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        else
-            __hip_atomic_fetch_add(rows + (size_t)slot * RowLayout<AUXM>::stride + col, v, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-
-    // The staged tile's values of the lanes in `wt`, added to global memory.  Sixteen lanes take the sixteen
-    // columns of one such lane's hit, so that one instruction adds to four runs of consecutive addresses (four hits)
-    // instead of to one address in each of up to 64 surfels' rows: the memory system works on whole cache lines.
-    __device__ __forceinline__ void write_through(int tile) const {
-        const uint32_t lane = __lane_id();
-        const int c = (int)(lane & 15u), k = (int)(lane >> 4);
-        const int col = tile * kStageCols + c;
-        uint64_t m = wt;
-#pragma unroll 1
-        while (m != 0ull) {
-            int h = -1;   // quarter k of the wave takes the k-th of the next four hits
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                if (m != 0ull) {
-                    const int hq = __builtin_ctzll(m);
-                    m &= m - 1ull;
-                    if (k == q) h = hq;
+        if (((wt >> M) & 0x0001000100010001ull) != 0ull) {
+            const uint32_t gm = row_bcast<M>(g);
+            const bool on = ((wt >> ((__lane_id() & 48u) + M)) & 1ull) != 0ull;
+            float *const grad_rows = p->grad_rows;
+            if (DET || grad_rows == nullptr) {
+                put_columns<AUXM, DET>((const DstParams *)p, gm, on, geo, sh ? f3(x, y, z) : f3(0, 0, 0));
+            } else if (on) {
+                float *dst = grad_rows + (size_t)gm * RowLayout<AUXM>::cols + i;
+                aadd(dst, geo);
+                if (sh) {
+                    aadd(dst + kColSh, x);
+                    aadd(dst + kColSh + 16, y);
+                    aadd(dst + kColSh + 32, z);
                 }
             }
-            const int src = h < 0 ? 0 : h;
-            const uint32_t gh = (uint32_t)__builtin_amdgcn_ds_bpermute(src << 2, (int)g);   // every lane is active here
-            const float v = stage[c * kStageStride + src];
-            if (h >= 0 && col < limit && v != 0.f) put_global(gh, col, v);
         }
     }
 
-    // Sums of the staged tile per group, added to the groups' rows.  Wave-uniform.
-    __device__ __forceinline__ void flush(int tile) const {
+    // After the columns: everything into the table.  Wave-uniform call.
+    __device__ __forceinline__ void commit(const_params p, const float (&basis)[16], F3 gc, bool sh, bool aux, const float (&aux_v)[AUXM]) const {
         const uint32_t lane = __lane_id();
-        const float *a = stage + (lane & 15u) * kStageStride + (lane & 48u);
-        v4f acc = {0.f, 0.f, 0.f, 0.f};
-        // all sixteen operands are asked for before the first product: left alone, the compiler reads two, waits,
-        // multiplies, reads the next two, ... - eight trips to LDS one after the other per tile
-        float av[16];
+        const uint32_t slot = (own_slot >= 0 ? (uint32_t)own_slot : (uint32_t)RowLayout<AUXM>::rows) * RowLayout<AUXM>::stride;
+        const uint32_t ray0 = (lane & 48u) * stride + (lane & 15u);
+        round<0>(p, slot, ray0, basis, gc, sh); round<1>(p, slot, ray0, basis, gc, sh);
+        round<2>(p, slot, ray0, basis, gc, sh); round<3>(p, slot, ray0, basis, gc, sh);
+        round<4>(p, slot, ray0, basis, gc, sh); round<5>(p, slot, ray0, basis, gc, sh);
+        round<6>(p, slot, ray0, basis, gc, sh); round<7>(p, slot, ray0, basis, gc, sh);
+        round<8>(p, slot, ray0, basis, gc, sh); round<9>(p, slot, ray0, basis, gc, sh);
+        round<10>(p, slot, ray0, basis, gc, sh); round<11>(p, slot, ray0, basis, gc, sh);
+        round<12>(p, slot, ray0, basis, gc, sh); round<13>(p, slot, ray0, basis, gc, sh);
+        round<14>(p, slot, ray0, basis, gc, sh); round<15>(p, slot, ray0, basis, gc, sh);
+        if (aux) {   // the few auxiliary channels ray by ray; past the table, a ray's channels together
+            if (own_slot >= 0) {
 #pragma unroll
-        for (int m = 0; m < 16; ++m) av[m] = a[m];
-        __builtin_amdgcn_sched_barrier(0);
+                for (int ch = 0; ch < AUXM; ++ch) put(slot + kColAux + ch, kDetShiftOther, aux_v[ch]);
+            }
+            if (wt != 0ull) {
 #pragma unroll
-        for (int m = 0; m < 16; ++m)
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[m], ((members >> m) & 1u) ? 1.0f : 0.0f, acc, 0, 0, 0);
-        // acc[r] = column 16*tile + 4*(lane/16) + r summed over the rays of group lane%16
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int col = tile * kStageCols + 4 * (int)(lane >> 4) + r;
-            if (out_on && col < limit && acc[r] != 0.f) {
-                if (out_slot >= 0) put(out_slot, col, acc[r]);
-                else if (DET) put_global(out_g, col, acc[r]);
+                for (int ch = 0; ch < AUXM; ++ch) set(ch, aux_v[ch]);
+                constexpr uint32_t kRays = DST_WAVE / AUXM;   // rays a round takes
+                const uint32_t ch = lane % AUXM, k = lane / AUXM;
+                uint64_t m = wt;
+#pragma unroll 1
+                while (m != 0ull) {
+                    // lane's ray: the k-th of those left
+                    uint64_t mine = m;
+                    for (uint32_t q = 0; q < kRays - 1u; ++q)
+                        if (q < k) mine &= mine - 1ull;
+                    const int src = mine != 0ull ? __builtin_ctzll(mine) : -1;
+                    const uint32_t gs = (uint32_t)__builtin_amdgcn_ds_bpermute((src & 63) << 2, (int)g);
+                    const float v = stage[(src & 63) * stride + ch];
+                    if (src >= 0 && (int)ch < p->aux && v != 0.f) {
+                        if (DET) atomicAdd(p->det_workspace + (size_t)gs * RowLayout<AUXM>::cols + kColAux + ch, (unsigned long long)to_fixed(v, kDetShiftOther));
+                        else aadd(p->grad_rows != nullptr ? p->grad_rows + (size_t)gs * RowLayout<AUXM>::cols + kColAux + ch
+                                                          : p->dL_dothers + (size_t)p->aux * gs + ch, v);
+                    }
+                    for (uint32_t q = 0; q < kRays; ++q) m &= m - 1ull;
+                }
             }
         }
-        if (wt != 0ull) write_through(tile);   // groups and further lanes without a table row
-    }
-
-    // Wave-uniform calls in ascending column order (every lane reaches them); `col` is a constant after
-    // inlining.  The tile is reduced when its last column arrives; finish() reduces a partly filled last tile.
-    __device__ __forceinline__ void add(int col, float v) const {
-        stage[(col & (kStageCols - 1)) * kStageStride + __lane_id()] = did ? v : 0.f;
-        if (any_stray) {   // rare: more than sixteen surfels in one step
-            if (stray && own_slot >= 0 && col < limit) put(own_slot, col, v);
-        }
-        if ((col & (kStageCols - 1)) == kStageCols - 1) flush(col / kStageCols);
-    }
-    __device__ __forceinline__ void finish(int next_col) const {
-        if ((next_col & (kStageCols - 1)) != 0) flush(next_col / kStageCols);
     }
 };
+// The basis values as GradSink wants them: basis[m] = coefficient lane%16 of ray m of this lane's row.  Once per bounce;
+// `stage` is free then.
+template <int STRIDE>
+__device__ __forceinline__ void sh_operand(float *stage, int deg, F3 rd, float (&basis)[16]) {
+    float b[16];
+    sh_basis(deg, rd, b);
+    const uint32_t lane = __lane_id();
+#pragma unroll
+    for (int j = 0; j < 16; ++j) stage[lane * STRIDE + j] = b[j];
+#pragma unroll
+    for (int m = 0; m < 16; ++m) basis[m] = stage[((lane & 48u) + m) * STRIDE + (lane & 15u)];
+}
 
 template <int AUXM>
 struct BounceIn {  // backward: saved results of the bounce and the gradients flowing into them
@@ -1169,13 +1205,13 @@ __device__ __forceinline__ F3 sh_direction_gradient(int deg, const SH &sh, F3 rd
 // Gradient of one composited hit (reference backward.cu:528-640 and 201-287, 68-166).
 // Pure gradient algebra: nothing here feeds a decision, so contraction is allowed.
 template <int AUXM, bool DET>
-__device__ __forceinline__ void hit_backward(const DstParams &p, const BounceIn<AUXM> &in, const BounceAcc<AUXM> &run,
+__device__ __forceinline__ void hit_backward(const const_params p, const BounceIn<AUXM> &in, const BounceAcc<AUXM> &run,
                                              int g, uint32_t pidx, float Tp, float alpha, float G, float w, float dpt,
                                              F3 xyz, const F3 (&R)[3], float u, float v, float sx, float sy, F3 mean,
                                              float q0, float q1, float q2, float q3, float opac, float nsign,
                                              F3 normal, const float (&col)[3], const bool (&neg)[3], F3 ro, F3 rd,
-                                             const float *__restrict__ sh, F3 &g_ro, F3 &g_rd,
-                                             const GradSink<AUXM, DET> &sink, bool did, LastShHit &last) {
+                                             F3 &g_ro, F3 &g_rd,
+                                             const GradSink<AUXM, DET> &sink, const float (&basis)[16], bool did, LastShHit &last) {
 #pragma clang fp contract(fast)
     // gradient algebra only: divisions become multiplications by a hardware reciprocal (1 ulp)
     const float num = 1.0f - alpha, inv_num = __builtin_amdgcn_rcpf(num);
@@ -1186,15 +1222,15 @@ __device__ __forceinline__ void hit_backward(const DstParams &p, const BounceIn<
     for (int ch = 0; ch < 3; ++ch) {
         g_col[ch] = in.g_rgb[ch] * w;
         g_alpha += in.g_rgb[ch] * (Tp * col[ch] - (in.rgb[ch] - run.C[ch]) * inv_num);
-        g_alpha += in.g_rgb[ch] * p.background[ch] * (-T_final * inv_num);
+        g_alpha += in.g_rgb[ch] * p->background[ch] * (-T_final * inv_num);
     }
 #pragma unroll
     for (int ch = 0; ch < AUXM; ++ch) g_aux_w[ch] = 0.f;
-    if (p.others_precomp != nullptr) {
+    if (p->others_precomp != nullptr) {
 #pragma unroll
         for (int ch = 0; ch < AUXM; ++ch) {
-            if (ch < p.aux) {
-                float o = p.others_precomp[(size_t)p.aux * g + ch];
+            if (ch < p->aux) {
+                float o = p->others_precomp[(size_t)p->aux * g + ch];
                 g_aux_w[ch] = in.g_aux[ch] * w;
                 g_alpha += in.g_aux[ch] * (Tp * o - (in.aux[ch] - run.O[ch]) * inv_num);
             }
@@ -1211,7 +1247,7 @@ __device__ __forceinline__ void hit_backward(const DstParams &p, const BounceIn<
     const float pc = (opac * G) > 0.99f ? 0.0f : 1.0f;
 
     // triangle that was hit, with its corner coordinates in splat units (backward.cu:583-602)
-    const float *V = p.vertices + (size_t)g * 12;
+    const float *V = p->vertices + (size_t)g * 12;
     const bool second = (pidx & 1u) != 0u;
     const F3 v1 = ld3(second ? V + 3 : V), v2 = ld3(second ? V + 6 : V + 3), v3 = ld3(second ? V + 9 : V + 6);
     const float k = g_G * pc;
@@ -1266,56 +1302,20 @@ __device__ __forceinline__ void hit_backward(const DstParams &p, const BounceIn<
         g_rot[0] = r0; g_rot[1] = r1; g_rot[2] = r2; g_rot[3] = r3;
     }
     STAT(last.t_alg += __builtin_readcyclecounter() - last.t0; last.t0 = __builtin_readcyclecounter();)
-    // the table columns, in ascending order
-    sink.add(kColColor + 0, g_col[0]); sink.add(kColColor + 1, g_col[1]); sink.add(kColColor + 2, g_col[2]);
-    sink.add(kColOpac, g_alpha * G * pc);
-    sink.add(kColScale + 0, g_sx);
-    sink.add(kColScale + 1, g_sy);
-    sink.add(kColRot + 0, g_rot[0]); sink.add(kColRot + 1, g_rot[1]); sink.add(kColRot + 2, g_rot[2]); sink.add(kColRot + 3, g_rot[3]);
-    sink.add(kColMean + 0, g_mean.x); sink.add(kColMean + 1, g_mean.y); sink.add(kColMean + 2, g_mean.z);
+    sink.set(kColColor + 0, g_col[0]); sink.set(kColColor + 1, g_col[1]); sink.set(kColColor + 2, g_col[2]);
+    sink.set(kColOpac, g_alpha * G * pc);
+    sink.set(kColScale + 0, g_sx);
+    sink.set(kColScale + 1, g_sy);
+    sink.set(kColRot + 0, g_rot[0]); sink.set(kColRot + 1, g_rot[1]); sink.set(kColRot + 2, g_rot[2]); sink.set(kColRot + 3, g_rot[3]);
+    sink.set(kColMean + 0, g_mean.x); sink.set(kColMean + 1, g_mean.y); sink.set(kColMean + 2, g_mean.z);
     const float hd = 0.5f * dpt;
-    sink.add(kColGrad + 0, g_mean.x * hd); sink.add(kColGrad + 1, g_mean.y * hd); sink.add(kColGrad + 2, g_mean.z * hd);
-    // (the first tile, columns 0..15, has just been reduced: its last column triggers that)
-
-    STAT(last.t_sh += __builtin_readcyclecounter() - last.t0;)   // first tile done
-    if (p.colors_precomp == nullptr) {
-        // SH backward (backward.cu:68-166); the direction gradient REPLACES the ray's (backward.cu:165)
-        const int deg = p.D;
-        F3 gc = f3(neg[0] ? 0.f : g_col[0], neg[1] ? 0.f : g_col[1], neg[2] ? 0.f : g_col[2]);
-        auto put = [&](int j, float basis) {
-            sink.add(RowLayout<AUXM>::sh0 + 3 * j + 0, basis * gc.x);
-            sink.add(RowLayout<AUXM>::sh0 + 3 * j + 1, basis * gc.y);
-            sink.add(RowLayout<AUXM>::sh0 + 3 * j + 2, basis * gc.z);
-        };
-        const float x = rd.x, y = rd.y, z = rd.z;
-        float basis[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) basis[j] = 0.f;
-        basis[0] = SH0;
-        if (deg > 0) {
-            basis[1] = -SH1 * y;
-            basis[2] = SH1 * z;
-            basis[3] = -SH1 * x;
-            if (deg > 1) {
-                const float xx = x * x, yy = y * y, zz = z * z, xy = x * y, yz = y * z, xz = x * z;
-                basis[4] = SH2[0] * xy;
-                basis[5] = SH2[1] * yz;
-                basis[6] = SH2[2] * (2.f * zz - xx - yy);
-                basis[7] = SH2[3] * xz;
-                basis[8] = SH2[4] * (xx - yy);
-                if (deg > 2) {
-                    basis[9] = SH3[0] * y * (3.f * xx - yy);
-                    basis[10] = SH3[1] * xy * z;
-                    basis[11] = SH3[2] * y * (4.f * zz - xx - yy);
-                    basis[12] = SH3[3] * z * (2.f * zz - 3.f * xx - 3.f * yy);
-                    basis[13] = SH3[4] * x * (4.f * zz - xx - yy);
-                    basis[14] = SH3[5] * z * (xx - yy);
-                    basis[15] = SH3[6] * x * (xx - 3.f * yy);
-                }
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 16; ++j) put(j, basis[j]);   // columns 16..63: three full tiles
+    sink.set(kColGrad + 0, g_mean.x * hd); sink.set(kColGrad + 1, g_mean.y * hd); sink.set(kColGrad + 2, g_mean.z * hd);
+    const bool sh = p->colors_precomp == nullptr;
+    // SH backward (backward.cu:68-166); the direction gradient REPLACES the ray's (backward.cu:165)
+    const F3 gc = f3(neg[0] ? 0.f : g_col[0], neg[1] ? 0.f : g_col[1], neg[2] ? 0.f : g_col[2]);
+    sink.commit(p, basis, gc, sh, p->others_precomp != nullptr, g_aux_w);
+    STAT(last.t_sh += __builtin_readcyclecounter() - last.t0;)
+    if (sh) {
         // The reference overwrites the ray-direction gradient with the SH term at every hit (backward.cu:165), so
         // only the last composited hit's term survives: remember it, walk_bounce computes it once per bounce.
         if (did) {
@@ -1323,11 +1323,6 @@ __device__ __forceinline__ void hit_backward(const DstParams &p, const BounceIn<
             last.gc = gc;
             last.any = true;
         }
-    }
-    if (p.others_precomp != nullptr) {   // the fifth tile only where there are auxiliary channels
-#pragma unroll
-        for (int ch = 0; ch < AUXM; ++ch) sink.add(kColAux + ch, g_aux_w[ch]);
-        sink.finish(RowLayout<AUXM>::cols);
     }
 }
 
@@ -1388,9 +1383,9 @@ __device__ __forceinline__ const uint64_t *rec_open(const RecView &rv, uint32_t 
 // consecutive columns of a row, so the 48 SH columns of a surfel go out as contiguous atomics.  The caller
 // puts barriers around it.
 template <int AUXM, bool DET>
-__device__ __forceinline__ void table_flush(const DstParams &p, uint32_t *keys, float *rows) {
-    constexpr int stride = RowLayout<AUXM>::stride, n_rows = TableRows<AUXM, DET>::rows;
-    for (int k = threadIdx.x; k < n_rows * stride; k += kWavesPerBlock * DST_WAVE) {
+__device__ __forceinline__ void table_flush(const DstParams &p, uint32_t *keys, double *rows) {
+    constexpr int stride = RowLayout<AUXM>::stride;
+    for (int k = threadIdx.x; k < RowLayout<AUXM>::rows * stride; k += kWavesPerBlock * DST_WAVE) {
         const int row = k / stride, col = k - row * stride;
         const uint32_t g = keys[row];
         if (g == kEmptyKey || col >= RowLayout<AUXM>::cols) continue;
@@ -1402,18 +1397,18 @@ __device__ __forceinline__ void table_flush(const DstParams &p, uint32_t *keys, 
             if (column_live<AUXM>(p, col))
                 atomicAdd(p.det_workspace + (size_t)g * RowLayout<AUXM>::cols + col, (unsigned long long)q);
         } else {
-            const float v = rows[k];
-            if (v == 0.f) continue;
-            rows[k] = 0.f;
+            const double v = rows[k];
+            if (v == 0.0) continue;
+            rows[k] = 0.0;
             float *dst = grad_address<AUXM>(p, g, col);
-            if (dst != nullptr) aadd(dst, v);
+            if (dst != nullptr) aadd(dst, (float)v);
         }
     }
 }
 template <int AUXM, bool DET>
 __device__ __forceinline__ void table_clear_keys(uint32_t *keys) {
-    for (int k = threadIdx.x; k <= TableRows<AUXM, DET>::rows; k += kWavesPerBlock * DST_WAVE)
-        keys[k] = (k < TableRows<AUXM, DET>::rows) ? kEmptyKey : 0u;
+    for (int k = threadIdx.x; k <= RowLayout<AUXM>::rows; k += kWavesPerBlock * DST_WAVE)
+        keys[k] = (k < RowLayout<AUXM>::rows) ? kEmptyKey : 0u;
 }
 
 // One bounce: chunked 16-nearest traversal + front-to-back compositing (reference forward.cu:136-315),
@@ -1427,7 +1422,7 @@ template <bool BWD, int AUXM, bool REC, bool MIXED, bool DET, bool HAND>
 __device__ __forceinline__ bool walk_bounce(const DstParams &p, const DstAccelView &acc, float max_abs, bool lane_on,
                                             F3 ro, F3 rd, float min_depth, BounceAcc<AUXM> &run,
                                             const BounceIn<AUXM> &in, F3 &g_ro, F3 &g_rd, uint32_t &n_proc,
-                                            uint32_t &n_con, uint32_t *tab_keys, float *tab_rows, float *stage,
+                                            uint32_t &n_con, uint32_t *tab_keys, double *tab_rows, float *stage,
                                             const RecView &rv, int bounce, F3 &dist_acc, uint32_t first_walk
 #ifdef DST_STATS
                                             , WaveStats &ws
@@ -1461,6 +1456,10 @@ __device__ __forceinline__ bool walk_bounce(const DstParams &p, const DstAccelVi
     bw.kept = bw.spent = false;
     bw.limit = (HAND && first_walk != kWalkPerLane) ? first_walk : 0u;
     uint32_t rec_pos = (REC && BWD) ? (rv.dir[bounce] & kRecDirBlockMask) : 0xFFFFFFFFu;   // replay: next block + 1; record: previous block
+    // (the re-tracing kernel, short of registers, brings it into place in every step)
+    float basis[16];
+    constexpr bool KEEP_BASIS = BWD && REC;
+    if (KEEP_BASIS && p.colors_precomp == nullptr) sh_operand<GradSink<AUXM, DET>::stride>(stage, p.D, rd, basis);
     uint32_t rec_chunks = 0u;   // forward with a record: chunks stored for this bounce
     for (;;) {
         // Backward: the four waves of the block take their chunks in step, so that between two rounds nobody
@@ -1664,19 +1663,18 @@ __device__ __forceinline__ bool walk_bounce(const DstParams &p, const DstAccelVi
             // ---- phase 2 (whole wave, backward only): gradients of the hits composited above -----------
             if (BWD && wave_ballot(did) != 0ull) {
                 GradSink<AUXM, DET> sink;
-                sink.p = &p;
                 sink.rows = tab_rows;
                 sink.stage = stage;
                 sink.did = did;
                 sink.g = (uint32_t)g;
-                sink.limit = RowLayout<AUXM>::cols;   // dead columns (no SH, no aux) are never staged
                 STAT(unsigned long long d0 = __builtin_readcyclecounter();)
+                if (!KEEP_BASIS && p.colors_precomp == nullptr) sh_operand<GradSink<AUXM, DET>::stride>(stage, p.D, rd, basis);
                 sink.plan(tab_keys);
                 STAT(last_sh.t0 = __builtin_readcyclecounter();)
                 STAT(unsigned long long d1 = __builtin_readcyclecounter(); ws.t_plan += d1 - d0; ws.steps++;
                      ws.leaf_any += __popcll(wave_ballot(did));)
-                hit_backward<AUXM, DET>(p, in, run, did ? g : 0, e_i, Tp_hit, alpha, G, w, dpt_hit, xyz, R, u, v, sx, sy, mean,
-                                   q0, q1, q2, q3, opac, nsign, normal, col, neg, ro, rd, sh, g_ro, g_rd, sink, did, last_sh);
+                hit_backward<AUXM, DET>(fresh_params(), in, run, did ? g : 0, e_i, Tp_hit, alpha, G, w, dpt_hit, xyz, R, u, v, sx, sy, mean,
+                                   q0, q1, q2, q3, opac, nsign, normal, col, neg, ro, rd, g_ro, g_rd, sink, basis, did, last_sh);
                 STAT(ws.t_hb += __builtin_readcyclecounter() - d1;)
             }
         }
@@ -1695,7 +1693,7 @@ __device__ __forceinline__ bool walk_bounce(const DstParams &p, const DstAccelVi
         } while (false);
         if (BWD) {
             __syncthreads();   // every wave's additions of this round are in the table
-            if (tab_keys[TableRows<AUXM, DET>::rows] > (uint32_t)(DST_TABLE_FLUSH_NUM * TableRows<AUXM, DET>::rows / 8)) {
+            if (tab_keys[RowLayout<AUXM>::rows] > (uint32_t)(DST_TABLE_FLUSH_NUM * RowLayout<AUXM>::rows / 8)) {
                 table_flush<AUXM, DET>(p, tab_keys, tab_rows);
                 __syncthreads();
                 table_clear_keys<AUXM, DET>(tab_keys);   // the barrier at the top of the next round publishes it
@@ -1820,21 +1818,23 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
     // is what the block's gradient table and the caches live on
     constexpr int kTableRows = RowLayout<AUXM>::rows;
     __shared__ uint32_t s_keys[BWD ? kTableRows + 1 : 1];   // + the count of claimed rows
-    __shared__ __attribute__((aligned(8))) float s_rows[BWD ? kTableRows * RowLayout<AUXM>::stride : 1];   // DET: half the rows, 8 bytes each
+    constexpr int kTableWords = (kTableRows + 1) * RowLayout<AUXM>::stride;
+    __shared__ double s_rows[BWD ? kTableWords : 1];
+    constexpr int kStageWords = GradSink<AUXM, DET>::words;
     __shared__ float s_stage[BWD ? kWavesPerBlock * kStageWords : 1];
     uint32_t *tab_keys = s_keys;
-    float *tab_rows = s_rows;
+    double *tab_rows = s_rows;
     // forward of an image at depth 0: the wave's table of blending weights (wet_add; in the kernels that carry the
     // per-lane walk it measured no gain and would take the LDS to the limit of 16 waves per CU)
     constexpr bool WET = !BWD && !MIXED && !DET;
     __shared__ uint32_t s_wet_keys[WET ? kFwdWavesPerBlock * kWetSlots : 1];
-    __shared__ float s_wet_vals[WET ? kFwdWavesPerBlock * kWetSlots : 1];
+    __shared__ double s_wet_vals[WET ? kFwdWavesPerBlock * kWetSlots : 1];
     uint32_t *const wet_keys = s_wet_keys + (WET ? (threadIdx.x / DST_WAVE) * kWetSlots : 0);
-    float *const wet_vals = s_wet_vals + (WET ? (threadIdx.x / DST_WAVE) * kWetSlots : 0);
+    double *const wet_vals = s_wet_vals + (WET ? (threadIdx.x / DST_WAVE) * kWetSlots : 0);
     if (WET) {   // (a wave's LDS accesses keep their order: no barrier between this and the first use)
         for (int e = threadIdx.x % DST_WAVE; e < kWetSlots; e += DST_WAVE) {
             wet_keys[e] = 0xFFFFFFFFu;
-            wet_vals[e] = 0.f;
+            wet_vals[e] = 0.0;
         }
     }
     // Backward with a hit record: the launcher starts the replaying kernel and the re-tracing kernel one after
@@ -1846,8 +1846,7 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
     }
     if (BWD) {
         table_clear_keys<AUXM, DET>(s_keys);
-        for (int k = threadIdx.x; k < kTableRows * RowLayout<AUXM>::stride; k += kWavesPerBlock * DST_WAVE)
-            s_rows[k] = 0.f;
+        for (int k = threadIdx.x; k < kTableWords; k += kWavesPerBlock * DST_WAVE) s_rows[k] = 0.0;
         __syncthreads();
     }
     // Backward: a block is the four waves of a 16x16 pixel tile (they share the gradient table).  Forward: the
@@ -2012,7 +2011,7 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
         if (WET && p.training && p.a_weights != nullptr) {   // the wave's blending weights: one addition per surfel
             for (int e = (int)lane; e < kWetSlots; e += DST_WAVE) {
                 const uint32_t k = wet_keys[e];
-                const float v = wet_vals[e];
+                const float v = (float)wet_vals[e];
                 if (k != 0xFFFFFFFFu && v != 0.f) aadd(p.a_weights + k, v);
             }
         }
@@ -2134,9 +2133,6 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
 #endif
 #ifndef DST_MIXED_WAVES
 #define DST_MIXED_WAVES 4
-#endif
-#ifndef DST_BWD_WAVES
-#define DST_BWD_WAVES 3
 #endif
 // EXTRAS: the rarely used forward options (DstParams.flags: fixed-point blending weights, distortion output) live in
 // a kernel of their own, so that the usual one does not carry their registers.
