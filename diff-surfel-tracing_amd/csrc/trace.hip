@@ -1042,6 +1042,9 @@ __device__ __attribute__((noinline)) void put_columns(const DstParams *p_in, uin
 constexpr int kGeoCols = 16;
 template <int AUXM, bool DET>
 struct GradSink {
+    // basis value of this lane's coefficient for ray M of its row (rows of one ray: the same for all)
+    template <int M> static __device__ __forceinline__ float basis_of(const float (&b)[16]) { return b[M]; }
+    template <int M> static __device__ __forceinline__ float basis_of(const float &b) { return b; }
     static constexpr int stride = kGeoCols + 1;   // four rays sixteen apart start in different quarters of the banks
     static constexpr int words = DST_WAVE * stride;
     static_assert(kWavesPerBlock * words * 4 == kStageBytes, "the table's size counts on the staging areas'");
@@ -1065,12 +1068,13 @@ struct GradSink {
         else __hip_atomic_fetch_add(rows + at, (double)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
 
-    template <int M>
-    __device__ __forceinline__ void round(const_params p, uint32_t slot, uint32_t ray0, const float (&basis)[16], F3 gc, bool sh) const {
+    template <int M, class B>
+    __device__ __forceinline__ void round(const_params p, uint32_t slot, uint32_t ray0, const B &basis, F3 gc, bool sh) const {
         const uint32_t i = __lane_id() & 15u;
         const uint32_t at = row_bcast<M>(slot) + i;
         const float geo = stage[ray0 + M * stride];
-        const float x = row_bcast<M>(gc.x) * basis[M], y = row_bcast<M>(gc.y) * basis[M], z = row_bcast<M>(gc.z) * basis[M];
+        const float b = basis_of<M>(basis);
+        const float x = row_bcast<M>(gc.x) * b, y = row_bcast<M>(gc.y) * b, z = row_bcast<M>(gc.z) * b;
         put(at, det_shift((int)i), geo);
         if (sh) {
             put(at + kColSh, kDetShiftOther, x);
@@ -1096,7 +1100,8 @@ struct GradSink {
     }
 
     // After the columns: everything into the table.  Wave-uniform call.
-    __device__ __forceinline__ void commit(const_params p, const float (&basis)[16], F3 gc, bool sh, bool aux, const float (&aux_v)[AUXM]) const {
+    template <class B>
+    __device__ __forceinline__ void commit(const_params p, const B &basis, F3 gc, bool sh, bool aux, const float (&aux_v)[AUXM]) const {
         const uint32_t lane = __lane_id();
         const uint32_t slot = (own_slot >= 0 ? (uint32_t)own_slot : (uint32_t)RowLayout<AUXM>::rows) * RowLayout<AUXM>::stride;
         const uint32_t ray0 = (lane & 48u) * stride + (lane & 15u);
@@ -1204,14 +1209,14 @@ __device__ __forceinline__ F3 sh_direction_gradient(int deg, const SH &sh, F3 rd
 
 // Gradient of one composited hit (reference backward.cu:528-640 and 201-287, 68-166).
 // Pure gradient algebra: nothing here feeds a decision, so contraction is allowed.
-template <int AUXM, bool DET>
+template <int AUXM, bool DET, class B>
 __device__ __forceinline__ void hit_backward(const const_params p, const BounceIn<AUXM> &in, const BounceAcc<AUXM> &run,
                                              int g, uint32_t pidx, float Tp, float alpha, float G, float w, float dpt,
                                              F3 xyz, const F3 (&R)[3], float u, float v, float sx, float sy, F3 mean,
                                              float q0, float q1, float q2, float q3, float opac, float nsign,
                                              F3 normal, const float (&col)[3], const bool (&neg)[3], F3 ro, F3 rd,
                                              F3 &g_ro, F3 &g_rd,
-                                             const GradSink<AUXM, DET> &sink, const float (&basis)[16], bool did, LastShHit &last) {
+                                             const GradSink<AUXM, DET> &sink, const B &basis, bool did, LastShHit &last) {
 #pragma clang fp contract(fast)
     // gradient algebra only: divisions become multiplications by a hardware reciprocal (1 ulp)
     const float num = 1.0f - alpha, inv_num = __builtin_amdgcn_rcpf(num);
@@ -1330,7 +1335,8 @@ __device__ __forceinline__ void hit_backward(const const_params p, const BounceI
 // them instead of walking the BVH again.  Layout of the caller's buffer, in 8-byte words:
 //   [0] blocks requested so far (the forward kernel counts on past the capacity, which is how overflow shows)
 //   [1] chains that a replay found broken (stays 0 for a record written by a forward trace with a zeroed header)
-//   [2 ...) directory: one uint32 per (wave, bounce slot): low 26 bits = 1 + first block of that wave's bounce (0 =
+//   [2] 0, or the count of pieces of a record written ray by ray (row.inc)
+//   [3 ...) directory: one uint32 per (wave, bounce slot): low 26 bits = 1 + first block of that wave's bounce (0 =
 //           none), high 6 bits = the number of chunks the wave stored for that bounce (what its replay will cost)
 //   then `capacity` blocks of kRecBlockWords words: 16x64 entries ([slot][lane]), 64 uint32 counts, next+1, and
 //   the colour of every composited hit as the forward evaluated it ([slot][channel][lane] floats; a channel clamped
@@ -1338,6 +1344,12 @@ __device__ __forceinline__ void hit_backward(const const_params p, const BounceI
 constexpr uint32_t kRecDirBlockBits = 26, kRecDirBlockMask = (1u << kRecDirBlockBits) - 1u;
 constexpr uint32_t kRecColourWord = kChunk * DST_WAVE + DST_WAVE / 2 + 8;   // first word of the colours
 constexpr uint32_t kRecBlockWords = kRecColourWord + kChunk * 3 * DST_WAVE / 2;
+// Words in front of the first block: the three of the header and the directory, of the wave layout (one entry per wave and
+// bounce slot) or of the row layout (one per ray and slot, row.inc), whichever is longer.
+__host__ __device__ static inline uint64_t record_header_words(uint64_t rays, uint32_t slots, uint64_t waves) {
+    const uint64_t entries = (rays > waves ? rays : waves) * slots;
+    return 3u + ((entries + 1u) / 2u + 1u) / 2u * 2u + 1u;   // even: blocks start on 16-byte boundaries where the record does
+}
 struct RecView {
     uint64_t *base;      // nullptr: not recording / not replaying
     uint64_t *blocks;    // first block
@@ -1842,7 +1854,7 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
     // the two does the work: the host never has to wait for the forward trace to learn whether its record is complete.
     if (BWD && p.hit_record != nullptr) {
         const bool complete = p.hit_record[0] <= (uint64_t)p.hit_record_blocks;
-        if (REC != complete) return;
+        if (REC != complete || (REC && (uint32_t)p.hit_record[2] != 0u)) return;
     }
     if (BWD) {
         table_clear_keys<AUXM, DET>(s_keys);
@@ -1896,10 +1908,9 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
     RecView rv = {nullptr, nullptr, nullptr, 0u};
     if (REC) {
         const uint32_t n_waves = btiles_x * ((tiles_y + 1u) / 2u) * kWavesPerBlock, slots_ = (uint32_t)p.mtd_alloc + 1u;
-        const uint64_t dir_words = ((uint64_t)n_waves * slots_ + 1u) / 2u;
         rv.base = p.hit_record;
-        rv.dir = reinterpret_cast<uint32_t *>(p.hit_record + 2) + (size_t)((by * btiles_x + bx) * kWavesPerBlock + wv) * slots_;
-        rv.blocks = p.hit_record + 2 + dir_words;
+        rv.dir = reinterpret_cast<uint32_t *>(p.hit_record + 3) + (size_t)((by * btiles_x + bx) * kWavesPerBlock + wv) * slots_;
+        rv.blocks = p.hit_record + record_header_words((uint64_t)p.H * p.W, slots_, n_waves);
         rv.capacity = p.hit_record_blocks;
     }
     const uint32_t ty = flat ? 0u : 2u * by + (wv >> 1), tx = flat ? 4u * bx + wv : 2u * bx + (wv & 1u);
@@ -2160,6 +2171,8 @@ void k_trace_bwd(const DstParams p, const DstAccelView acc, int tw_log2, int th_
     trace_body<true, AUXM, REC, MIXED, DET, false>(p, acc, tw_log2, th_log2, tiles_x, tiles_y, btiles_x, ray_order, strip_width, block_order, nullptr, 0u);
 }
 
+#include "row.inc"
+
 // Closing kernels of the deterministic mode: fixed point -> fp32, added to the caller's (zero-filled) tensors.
 template <int AUXM>
 __global__ void k_det_finish_grads(const DstParams p, uint32_t *out_of_range) {
@@ -2324,6 +2337,57 @@ void launch(const DstParams &p, const DstAccelView &acc, const TileGrid &t, cons
 #undef DST_LAUNCH
 }
 
+// Are the rays of this grid traced by the row kernels (sixteen lanes per ray), and how are they dealt out?
+// Unrelated rays - lists, and whatever is traced beyond its first bounce - always; images traced to depth 0 where waves of
+// 64 rays would leave most of the chip idle.
+#ifndef DST_ROW_MAX_WAVES
+#define DST_ROW_MAX_WAVES 400
+#endif
+bool row_grid(const DstParams &p, const TileGrid &t, RowGrid &g) {
+    const uint64_t rays = (uint64_t)p.H * p.W, waves = (rays + 63u) / 64u;
+    if (t.th_log2 == 3 && p.max_trace_depth == 0 && waves > DST_ROW_MAX_WAVES) return false;
+    g.record_header = record_header_words(rays, (uint32_t)p.mtd_alloc + 1u, (uint64_t)t.btiles_x * t.btiles_y * kWavesPerBlock);
+    g.batch_log2 = rays >= 16384u ? 4u : 2u;   // sixteen rays a wave once that leaves a thousand waves
+    if (t.th_log2 == 0) {
+        g.side_log2 = 0u;
+        g.tiles_x = g.n_waves = (uint32_t)((rays + (1u << g.batch_log2) - 1u) >> g.batch_log2);
+        g.tiles_y = 0u;
+    } else {
+        g.side_log2 = g.batch_log2 / 2u;
+        g.tiles_x = ((uint32_t)p.W + (1u << g.side_log2) - 1u) >> g.side_log2;
+        g.tiles_y = ((uint32_t)p.H + (1u << g.side_log2) - 1u) >> g.side_log2;
+        g.n_waves = g.tiles_x * g.tiles_y;
+    }
+    return true;
+}
+template <bool REC>
+void launch_row_fwd(const DstParams &p, const DstAccelView &acc, const RowGrid &g, const uint32_t *ray_order, hipStream_t stream) {
+    const dim3 grid((g.n_waves + 31u) / 32u * 32u), block(DST_WAVE);
+    const uint32_t grab = g.batch_log2 == 4u ? 4u : 1u;
+#define DST_ROW(AUX)                                                                                                       \
+    do {                                                                                                                   \
+        if (p.flags != 0u) hipLaunchKernelGGL((k_row_fwd<AUX, REC, true>), grid, block, 0, stream, p, acc, g, ray_order, grab); \
+        else hipLaunchKernelGGL((k_row_fwd<AUX, REC, false>), grid, block, 0, stream, p, acc, g, ray_order, grab);          \
+    } while (0)
+    if (p.aux <= 2) DST_ROW(2);
+    else if (p.aux <= 4) DST_ROW(4);
+    else DST_ROW(8);
+#undef DST_ROW
+}
+void launch_row_bwd(const DstParams &p, const RowGrid &g, const uint32_t *ray_order, hipStream_t stream) {
+    const dim3 grid((g.n_waves + kWavesPerBlock - 1u) / kWavesPerBlock), block(kWavesPerBlock * DST_WAVE);
+    const bool det = (p.flags & DST_FLAG_DETERMINISTIC) != 0u;
+#define DST_ROW(AUX)                                                                                        \
+    do {                                                                                                    \
+        if (det) hipLaunchKernelGGL((k_row_bwd<AUX, true>), grid, block, 0, stream, p, g, ray_order);       \
+        else hipLaunchKernelGGL((k_row_bwd<AUX, false>), grid, block, 0, stream, p, g, ray_order);          \
+    } while (0)
+    if (p.aux <= 2) DST_ROW(2);
+    else if (p.aux <= 4) DST_ROW(4);
+    else DST_ROW(8);
+#undef DST_ROW
+}
+
 }  // namespace
 
 int dst_launch_pack_half(const float *src, uint16_t *dst, uint64_t n, hipStream_t stream) {
@@ -2348,7 +2412,7 @@ uint64_t dst_hit_record_layout(int32_t H, int32_t W, int32_t mtd_alloc, uint32_t
     }
     const TileGrid t = tile_grid(H, W);
     const uint64_t waves = (uint64_t)t.btiles_x * t.btiles_y * kWavesPerBlock;
-    const uint64_t header = 2 + (waves * (uint64_t)(mtd_alloc + 1) + 1) / 2;
+    const uint64_t header = record_header_words((uint64_t)H * W, (uint32_t)mtd_alloc + 1u, waves);
     if (header_words) *header_words = header;
     if (n_waves) *n_waves = (uint32_t)waves;
     return header + (uint64_t)blocks * kRecBlockWords;
@@ -2400,8 +2464,12 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
     const bool rec = p.hit_record != nullptr;
     const bool det = (p.flags & DST_FLAG_DETERMINISTIC) != 0u;
     uint32_t *const out_of_range = ctx->handover + kDstHandoverOutOfRange;   // (a spare word of the list's header)
+    RowGrid rows;
+    const bool by_rows = row_grid(p, t, rows);
     if (backward) {
         const uint32_t n_blocks = t.btiles_x * t.btiles_y;
+        // the kernel that fits the record (complete, written ray by ray or wave by wave; incomplete) does the work
+        if (rec && by_rows) launch_row_bwd(p, rows, ray_order, stream);
         if (rec && n_blocks < kOrderMinBlocks) {
             launch<true, true>(p, acc, t, ray_order, stream);
         } else if (rec) {
@@ -2415,7 +2483,7 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
             }
             const uint32_t strip = t.th_log2 != 0 ? (uint32_t)DST_STRIP_BWD : 0u;
             hipLaunchKernelGGL(k_block_order, dim3(1), dim3(1024), 0, stream,
-                               reinterpret_cast<const uint32_t *>(p.hit_record + 2), (uint32_t)p.mtd_alloc + 1u, t.btiles_x,
+                               reinterpret_cast<const uint32_t *>(p.hit_record + 3), (uint32_t)p.mtd_alloc + 1u, t.btiles_x,
                                t.btiles_y, strip, t.th_log2 != 0 ? 1 : 0, n_blocks, ctx->block_order);
             launch<true, true>(p, acc, t, ray_order, stream, ctx->block_order);   // does the work if the record is complete,
         }
@@ -2442,9 +2510,14 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
                 ctx->small_quads_asked = true;
             }
         }
+        const uint32_t steps = std::max<uint32_t>(ctx->handover_steps, 1u);
         // the second launch of each pair traces the tiles the first one handed over (usually none: it leaves at once)
         uint32_t *const list = (kFwdWavesPerBlock == 1 && dst_handover_active(ctx)) ? ctx->handover : nullptr;
-        const uint32_t steps = std::max<uint32_t>(ctx->handover_steps, 1u);
+        // (a context told never to hand tiles over keeps the rays of an image's tile together)
+        if (by_rows && list == nullptr && (ctx->handover_mode != DST_HANDOVER_OFF || p.max_trace_depth > 0 || t.th_log2 < 3)) {
+            if (rec) launch_row_fwd<true>(p, acc, rows, ray_order, stream);
+            else launch_row_fwd<false>(p, acc, rows, ray_order, stream);
+        } else
         for (int pass = 0; pass < (list != nullptr ? 2 : 1); ++pass) {
             const uint32_t arg = pass == 0 ? steps : 0u;
             if (rec) launch<false, true>(p, acc, t, ray_order, stream, nullptr, list, arg);
