@@ -28,14 +28,17 @@ struct alignas(64) DstNode {
 };
 
 // Traversal node, indexed like the binary node it was collapsed from: up to four children (the binary
-// node's grandchildren, or a child itself where that child is a leaf group), boxes stored by coordinate.
-// One 128-byte wave-uniform fetch decides four descents.
+// node's grandchildren, or a child itself where that child is a leaf group), 32 bytes each: a lane that looks at one
+// child reads two 16-byte words (boxes stored by coordinate took it seven 4-byte loads), a whole node is 128 bytes.
+// An unused slot has an empty box, which nothing meets, and the reference of a one-quad group.
+struct DstWideChild {
+    float lo[3];
+    uint32_t ref;             // wide node index, or leaf-group reference
+    float hi[3];
+    uint32_t used;            // 1, or 0 for an unused slot
+};
 struct alignas(128) DstWideNode {
-    float lox[DST_WIDE], loy[DST_WIDE], loz[DST_WIDE];
-    float hix[DST_WIDE], hiy[DST_WIDE], hiz[DST_WIDE];
-    uint32_t ref[DST_WIDE];   // wide node index, or leaf-group reference
-    uint32_t count;           // children in use (2..4)
-    uint32_t pad[3];
+    DstWideChild child[DST_WIDE];
 };
 
 // Leaf = one surfel quad in leaf order (triangles ABC and BCD), as the hit test wants it: corner A, the edge vectors

@@ -972,9 +972,11 @@ __global__ void k_widen(const DstNode *__restrict__ nodes, DstWideNode *__restri
     DstWideNode w;
     uint32_t k = 0;
     auto put = [&](const float *lo, const float *hi, uint32_t ref) {
-        w.lox[k] = lo[0]; w.loy[k] = lo[1]; w.loz[k] = lo[2];
-        w.hix[k] = hi[0]; w.hiy[k] = hi[1]; w.hiz[k] = hi[2];
-        w.ref[k] = ref;
+        DstWideChild &c = w.child[k];
+        c.lo[0] = lo[0]; c.lo[1] = lo[1]; c.lo[2] = lo[2];
+        c.hi[0] = hi[0]; c.hi[1] = hi[1]; c.hi[2] = hi[2];
+        c.ref = ref;
+        c.used = 1u;
         ++k;
     };
     uint32_t own[2];
@@ -1038,13 +1040,13 @@ __global__ void k_widen(const DstNode *__restrict__ nodes, DstWideNode *__restri
         }
         for (int c = 0; c < m; ++c) put(lo[c], hi[c], ref[c]);
     }
-    w.count = k;
-    for (; k < DST_WIDE; ++k) {   // unused slots: the traversal masks them by `count`
-        w.lox[k] = w.loy[k] = w.loz[k] = 0.f;
-        w.hix[k] = w.hiy[k] = w.hiz[k] = 0.f;
-        w.ref[k] = DST_LEAF_BIT;  // would be a harmless one-quad group, never another node
+    for (; k < DST_WIDE; ++k) {
+        DstWideChild &c = w.child[k];
+        c.lo[0] = c.lo[1] = c.lo[2] = INFINITY;
+        c.hi[0] = c.hi[1] = c.hi[2] = -INFINITY;
+        c.ref = DST_LEAF_BIT;   // would be a harmless one-quad group, never another node
+        c.used = 0u;
     }
-    w.pad[0] = w.pad[1] = w.pad[2] = 0u;
     wide[i] = w;
 }
 

@@ -230,27 +230,7 @@ __device__ __forceinline__ void load_uniform(const void *p, uint32_t (&out)[N]) 
     for (int k = 0; k < N; ++k) out[k] = c[k];
 }
 
-// A whole traversal node in one trip: the six face arrays picked by byte offset (scalar-register offsets, so no
-// address arithmetic per array), the child references and the child count, and one wait for all of them.
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void load_node(const void *node, uint32_t onx, uint32_t ony, uint32_t onz, uint32_t ofx,
-                                          uint32_t ofy, uint32_t ofz, u32x4 &NX, u32x4 &NY, u32x4 &NZ, u32x4 &FX,
-                                          u32x4 &FY, u32x4 &FZ, u32x4 &refs, uint32_t &count) {
-    asm volatile(
-        "s_load_dwordx4 %0, %8, %9\n\t"
-        "s_load_dwordx4 %1, %8, %10\n\t"
-        "s_load_dwordx4 %2, %8, %11\n\t"
-        "s_load_dwordx4 %3, %8, %12\n\t"
-        "s_load_dwordx4 %4, %8, %13\n\t"
-        "s_load_dwordx4 %5, %8, %14\n\t"
-        "s_load_dwordx4 %6, %8, 0x60\n\t"
-        "s_load_dword %7, %8, 0x70\n\t"
-        "s_waitcnt lgkmcnt(0)"
-        : "=&s"(NX), "=&s"(NY), "=&s"(NZ), "=&s"(FX), "=&s"(FY), "=&s"(FZ), "=&s"(refs), "=&s"(count)
-        : "s"(node), "s"(onx), "s"(ony), "s"(onz), "s"(ofx), "s"(ofy), "s"(ofz)
-        : "memory");
-}
 // Two consecutive 64-byte records (the stand-ins of a leaf group's two quads), or one 96-byte quad record, in one
 // trip: left to itself the compiler splits these fetches and waits for the first part before asking for the rest.
 typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
@@ -272,6 +252,9 @@ __device__ __forceinline__ uint32_t shift_in_any(uint32_t bits, uint64_t mask) {
     asm("s_cmp_lg_u64 %1, 0\n\ts_addc_u32 %0, %0, %0" : "+s"(bits) : "s"(mask) : "scc");
     return bits;
 }
+// A whole traversal node in one trip, and one wait for all of it.
+__device__ __forceinline__ void load_node(const void *node, u32x16 &a, u32x16 &b) { load_record_pair(node, a, b); }
+
 struct RaySlab {   // per-lane precomputation for the conservative slab test
     float ix, iy, iz;     // 1/d, with tiny components pushed away from zero
     float nx, ny, nz;     // -o * (1/d)
@@ -499,14 +482,10 @@ __device__ __forceinline__ void packet_walk(const DstAccelView &acc, const RaySl
 ) {
     const RayPre rp = make_pre(o, d, slab.max_abs);
     RaySlabFast fs;
-    // byte offsets of the near / far face arrays inside a wide node (lox 0, loy 16, loz 32, hix 48, hiy 64, hiz 80)
-    uint32_t onx = 0, ony = 16, onz = 32, ofx = 48, ofy = 64, ofz = 80;
     fs.ix = slab.ix; fs.iy = slab.iy; fs.iz = slab.iz;
     fs.cnx = slab.nx - slab.wx; fs.cny = slab.ny - slab.wy; fs.cnz = slab.nz - slab.wz;
     fs.cfx = slab.nx + slab.wx; fs.cfy = slab.ny + slab.wy; fs.cfz = slab.nz + slab.wz;
-    if (sgn & 1u) { onx = 48; ofx = 0; }
-    if (sgn & 2u) { ony = 64; ofy = 16; }
-    if (sgn & 4u) { onz = 80; ofz = 32; }
+    const bool sx = (sgn & 1u) != 0u, sy = (sgn & 2u) != 0u, sz = (sgn & 4u) != 0u;
     uint32_t stack0 = 0u, stack1 = 0u;
     int sp = 0;
     // A well-formed hierarchy is walked in at most one step per node and per leaf group; the cap makes the
@@ -532,19 +511,19 @@ __device__ __forceinline__ void packet_walk(const DstAccelView &acc, const RaySl
             const char *node = reinterpret_cast<const char *>(&acc.wide[ref]);
             STAT(ws.nodes++;)
             const float tmax = active ? kb_t(buf.e[kChunk - 1]) : -1.0f;
-            uint32_t tail[5];
+            uint32_t tail[4];
             uint32_t hit = 0u;                     // bit k: some lane enters child k
             {
-                u32x4 NX, NY, NZ, FX, FY, FZ, refs;
-                load_node(node, onx, ony, onz, ofx, ofy, ofz, NX, NY, NZ, FX, FY, FZ, refs, tail[4]);
-                tail[0] = refs[0]; tail[1] = refs[1]; tail[2] = refs[2]; tail[3] = refs[3];
+                u32x16 n0, n1;                     // children 0 and 1, children 2 and 3
+                load_node(node, n0, n1);
 #pragma unroll
                 for (int k = DST_WIDE - 1; k >= 0; --k) {   // last child first: its bit is shifted up the furthest
-                    float tn;
-                    hit = shift_in_any(hit, slab_hit_fast(fs, __uint_as_float(NX[k]), __uint_as_float(NY[k]), __uint_as_float(NZ[k]),
-                                                          __uint_as_float(FX[k]), __uint_as_float(FY[k]), __uint_as_float(FZ[k]), tmax, tn));
+                    auto word = [&](int w) { return __uint_as_float(k < 2 ? n0[8 * k + w] : n1[8 * (k - 2) + w]); };
+                    tail[k] = __float_as_uint(word(3));
+                    float tn;   // (the box of an unused slot is empty)
+                    hit = shift_in_any(hit, slab_hit_fast(fs, sx ? word(4) : word(0), sy ? word(5) : word(1), sz ? word(6) : word(2),
+                                                          sx ? word(0) : word(4), sy ? word(1) : word(5), sz ? word(2) : word(6), tmax, tn));
                 }
-                hit &= (1u << tail[4]) - 1u;   // unused slots are never entered
             }
             if (hit != 0u) {
                 // Children are taken in stored order: the first one that is hit next, the others deferred (last
@@ -690,19 +669,18 @@ __device__ __attribute__((noinline)) void lane_walk(const LaneWalkAccel acc_in, 
 #undef DST_LANE_QUAD
                 // (groups of more than two quads do not occur: DST_GROUP = 2; a longer one would lose its tail)
             } else {
-                // lox r0, loy r1, loz r2, hix r3, hiy r4, hiz r5, child references r6, child count r7.x
-                const uint32_t n_child = __float_as_uint(r7.x);
+                // a child is two words: low corner and reference, high corner and whether the slot is used
                 const float tmax = kb_t(buf.e[kChunk - 1]);
                 uint32_t key[DST_WIDE], cref[DST_WIDE];
 #pragma unroll
                 for (int k = 0; k < DST_WIDE; ++k) {
+                    const v4f lo = k == 0 ? r0 : (k == 1 ? r2 : (k == 2 ? r4 : r6)), hi = k == 0 ? r1 : (k == 1 ? r3 : (k == 2 ? r5 : r7));
                     float tn;
-                    const uint64_t h = slab_hit_fast(fs, neg_x ? r3[k] : r0[k], neg_y ? r4[k] : r1[k], neg_z ? r5[k] : r2[k],
-                                                     neg_x ? r0[k] : r3[k], neg_y ? r1[k] : r4[k], neg_z ? r2[k] : r5[k],
-                                                     tmax, tn);
-                    const bool mine = ((h >> __lane_id()) & 1ull) != 0ull && (uint32_t)k < n_child;
+                    const uint64_t h = slab_hit_fast(fs, neg_x ? hi.x : lo.x, neg_y ? hi.y : lo.y, neg_z ? hi.z : lo.z,
+                                                     neg_x ? lo.x : hi.x, neg_y ? lo.y : hi.y, neg_z ? lo.z : hi.z, tmax, tn);
+                    const bool mine = ((h >> __lane_id()) & 1ull) != 0ull && __float_as_uint(hi.w) != 0u;
                     key[k] = mine ? __float_as_uint(tn) : 0xFFFFFFFFu;   // entry distance (non-negative: bits order like the value)
-                    cref[k] = __float_as_uint(r6[k]);
+                    cref[k] = __float_as_uint(lo.w);
                 }
 #define CSWAP(a, b)                                                            \
     {                                                                          \
@@ -1040,7 +1018,8 @@ __device__ __attribute__((noinline)) void put_columns(const DstParams *p_in, uin
 // in LDS.  Grouping cost more than it saved: a step of these scenes composites 6 to 20 different surfels, over half the
 // steps of two of them more than sixteen, and what did not fit went column by column.)
 constexpr int kGeoCols = 16;
-template <int AUXM, bool DET>
+// TABLE = false: every hit's columns go straight to memory (the row kernels, whose hits hardly ever share a surfel).
+template <int AUXM, bool DET, bool TABLE = true>
 struct GradSink {
     // basis value of this lane's coefficient for ray M of its row (rows of one ray: the same for all)
     template <int M> static __device__ __forceinline__ float basis_of(const float (&b)[16]) { return b[M]; }
@@ -1056,7 +1035,7 @@ struct GradSink {
     uint64_t wt;         // wave-uniform: lanes whose surfel has no table row (their values go to global memory)
 
     __device__ __forceinline__ void plan(uint32_t *keys) {
-        own_slot = did ? table_slot<RowLayout<AUXM>::rows>(keys, g) : -1;
+        own_slot = TABLE && did ? table_slot<RowLayout<AUXM>::rows>(keys, g) : -1;
         wt = wave_ballot(did && own_slot < 0);
     }
     // Column `col` of this lane's hit (every lane; a lane without a hit may pass anything).
@@ -1064,6 +1043,7 @@ struct GradSink {
 
     // v into column `col` (in the table's memory: word `at`).
     __device__ __forceinline__ void put(uint32_t at, int shift, float v) const {
+        if (!TABLE) return;
         if (DET) __hip_atomic_fetch_add(reinterpret_cast<long long *>(rows) + at, to_fixed(v, shift), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         else __hip_atomic_fetch_add(rows + at, (double)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
@@ -1209,14 +1189,14 @@ __device__ __forceinline__ F3 sh_direction_gradient(int deg, const SH &sh, F3 rd
 
 // Gradient of one composited hit (reference backward.cu:528-640 and 201-287, 68-166).
 // Pure gradient algebra: nothing here feeds a decision, so contraction is allowed.
-template <int AUXM, bool DET, class B>
+template <int AUXM, class SINK, class B>
 __device__ __forceinline__ void hit_backward(const const_params p, const BounceIn<AUXM> &in, const BounceAcc<AUXM> &run,
                                              int g, uint32_t pidx, float Tp, float alpha, float G, float w, float dpt,
                                              F3 xyz, const F3 (&R)[3], float u, float v, float sx, float sy, F3 mean,
                                              float q0, float q1, float q2, float q3, float opac, float nsign,
                                              F3 normal, const float (&col)[3], const bool (&neg)[3], F3 ro, F3 rd,
                                              F3 &g_ro, F3 &g_rd,
-                                             const GradSink<AUXM, DET> &sink, const B &basis, bool did, LastShHit &last) {
+                                             const SINK &sink, const B &basis, bool did, LastShHit &last) {
 #pragma clang fp contract(fast)
     // gradient algebra only: divisions become multiplications by a hardware reciprocal (1 ulp)
     const float num = 1.0f - alpha, inv_num = __builtin_amdgcn_rcpf(num);
@@ -1685,7 +1665,7 @@ __device__ __forceinline__ bool walk_bounce(const DstParams &p, const DstAccelVi
                 STAT(last_sh.t0 = __builtin_readcyclecounter();)
                 STAT(unsigned long long d1 = __builtin_readcyclecounter(); ws.t_plan += d1 - d0; ws.steps++;
                      ws.leaf_any += __popcll(wave_ballot(did));)
-                hit_backward<AUXM, DET>(fresh_params(), in, run, did ? g : 0, e_i, Tp_hit, alpha, G, w, dpt_hit, xyz, R, u, v, sx, sy, mean,
+                hit_backward<AUXM>(fresh_params(), in, run, did ? g : 0, e_i, Tp_hit, alpha, G, w, dpt_hit, xyz, R, u, v, sx, sy, mean,
                                    q0, q1, q2, q3, opac, nsign, normal, col, neg, ro, rd, g_ro, g_rd, sink, basis, did, last_sh);
                 STAT(ws.t_hb += __builtin_readcyclecounter() - d1;)
             }
@@ -2375,7 +2355,7 @@ void launch_row_fwd(const DstParams &p, const DstAccelView &acc, const RowGrid &
 #undef DST_ROW
 }
 void launch_row_bwd(const DstParams &p, const RowGrid &g, const uint32_t *ray_order, hipStream_t stream) {
-    const dim3 grid((g.n_waves + kWavesPerBlock - 1u) / kWavesPerBlock), block(kWavesPerBlock * DST_WAVE);
+    const dim3 grid((g.n_waves + 31u) / 32u * 32u), block(DST_WAVE);
     const bool det = (p.flags & DST_FLAG_DETERMINISTIC) != 0u;
 #define DST_ROW(AUX)                                                                                        \
     do {                                                                                                    \
