@@ -1927,7 +1927,9 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
         float s_prod = 1.0f;
         bool on = inside;
         uint32_t first_walk = (HAND && handover != nullptr) ? hand_arg : 0u;
-        for (int i = 0; i <= mtd; ++i) {
+        // (kernels without the per-lane walk trace the first bounce; k_row_fwd goes on from there)
+        const int last = MIXED ? mtd : 0;
+        for (int i = 0; i <= last; ++i) {
             const float min_depth = (i == 0) ? (p.start_from_first ? kNear : 0.0f) : kStartOffset;
             F3 dist_acc = f3(0, 0, 0);
             const bool gave_up = walk_bounce<false, AUXM, REC, MIXED, DET, HAND>(p, acc, max_abs, on, ot, dt, min_depth, run, in, g_ro, g_rd, n_proc, n_con, WET ? wet_keys : nullptr, WET ? wet_vals : nullptr, nullptr, rv, i, dist_acc, taker ? kWalkPerLane : (i == 0 ? first_walk : 0u) WS_ARG);
@@ -1993,7 +1995,7 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
             }
         }
         if (inside) {
-            if (on)
+            if (on && last == mtd)
                 for (int k = (mtd + 1) * MID; k < slots * MID; ++k) mid[k] = 0.f;
             p.out_rgb[3 * r + 0] = out_rgb[0];
             p.out_rgb[3 * r + 1] = out_rgb[1];
@@ -2267,7 +2269,7 @@ TileGrid tile_grid(int H, int W) {
 // `handover` / `hand_arg`: see trace_body (forward only; hand_arg steps = 0 launches the takers of the listed tiles).
 template <bool BWD, bool REC>
 void launch(const DstParams &p, const DstAccelView &acc, const TileGrid &t, const uint32_t *ray_order, hipStream_t stream,
-            const uint32_t *block_order = nullptr, uint32_t *handover = nullptr, uint32_t hand_arg = 0u) {
+            const uint32_t *block_order = nullptr, uint32_t *handover = nullptr, uint32_t hand_arg = 0u, bool first_bounce = false) {
     const uint32_t n_blocks = t.btiles_x * t.btiles_y;
     dim3 grid(n_blocks), block(kWavesPerBlock * DST_WAVE);
     const bool takers = !BWD && handover != nullptr && hand_arg == 0u;
@@ -2285,7 +2287,7 @@ void launch(const DstParams &p, const DstAccelView &acc, const TileGrid &t, cons
     // The backward trace gains 1 to 3 % from strips of 8 on every grid measured.
     uint32_t strip = 0u;
     if (t.th_log2 != 0) strip = BWD ? (uint32_t)DST_STRIP_BWD : (n_blocks >= kStripMinBlocks ? (uint32_t)DST_STRIP_FWD : 0u);
-    const bool mixed = takers || p.max_trace_depth > 0 || t.th_log2 < 3;
+    const bool mixed = takers || (p.max_trace_depth > 0 && !first_bounce) || t.th_log2 < 3;   // first_bounce: forward, nothing beyond it
     const bool det = (p.flags & DST_FLAG_DETERMINISTIC) != 0u;
 #define DST_LAUNCH_M(AUX, MIXED)                                                                                   \
     do {                                                                                                           \
@@ -2317,16 +2319,24 @@ void launch(const DstParams &p, const DstAccelView &acc, const TileGrid &t, cons
 #undef DST_LAUNCH
 }
 
-// Are the rays of this grid traced by the row kernels (sixteen lanes per ray), and how are they dealt out?
-// Unrelated rays - lists, and whatever is traced beyond its first bounce - always; images traced to depth 0 where waves of
-// 64 rays would leave most of the chip idle.
+// How the rays of this grid are traced.  Tiles: a wave per 64 rays.  Rows (sixteen lanes per ray): lists, whose rays
+// are unrelated, and images so small that waves of 64 rays leave most of the chip idle.  TilesThenRows: images with
+// reflections - the primary rays as tiles, the bounces beyond as rows.
 #ifndef DST_ROW_MAX_WAVES
 #define DST_ROW_MAX_WAVES 400
 #endif
-bool row_grid(const DstParams &p, const TileGrid &t, RowGrid &g) {
+enum class TraceBy { Tiles, Rows, TilesThenRows };
+TraceBy row_grid(const DstParams &p, const TileGrid &t, RowGrid &g) {
     const uint64_t rays = (uint64_t)p.H * p.W, waves = (rays + 63u) / 64u;
-    if (t.th_log2 == 3 && p.max_trace_depth == 0 && waves > DST_ROW_MAX_WAVES) return false;
     g.record_header = record_header_words(rays, (uint32_t)p.mtd_alloc + 1u, (uint64_t)t.btiles_x * t.btiles_y * kWavesPerBlock);
+    if (t.th_log2 == 3 && waves > DST_ROW_MAX_WAVES) {
+        g.batch_log2 = 4u;
+        g.side_log2 = 3u;
+        g.tiles_x = t.btiles_x;
+        g.tiles_y = t.btiles_y;
+        g.n_waves = t.btiles_x * t.btiles_y * kWavesPerBlock;
+        return p.max_trace_depth == 0 ? TraceBy::Tiles : TraceBy::TilesThenRows;
+    }
     g.batch_log2 = rays >= 16384u ? 4u : 2u;   // sixteen rays a wave once that leaves a thousand waves
     if (t.th_log2 == 0) {
         g.side_log2 = 0u;
@@ -2338,16 +2348,16 @@ bool row_grid(const DstParams &p, const TileGrid &t, RowGrid &g) {
         g.tiles_y = ((uint32_t)p.H + (1u << g.side_log2) - 1u) >> g.side_log2;
         g.n_waves = g.tiles_x * g.tiles_y;
     }
-    return true;
+    return TraceBy::Rows;
 }
-template <bool REC>
+template <bool REC, bool BEYOND>
 void launch_row_fwd(const DstParams &p, const DstAccelView &acc, const RowGrid &g, const uint32_t *ray_order, hipStream_t stream) {
-    const dim3 grid((g.n_waves + 31u) / 32u * 32u), block(DST_WAVE);
+    const dim3 grid(BEYOND ? g.n_waves : (g.n_waves + 31u) / 32u * 32u), block(BEYOND ? kWavesPerBlock * DST_WAVE : DST_WAVE);
     const uint32_t grab = g.batch_log2 == 4u ? 4u : 1u;
 #define DST_ROW(AUX)                                                                                                       \
     do {                                                                                                                   \
-        if (p.flags != 0u) hipLaunchKernelGGL((k_row_fwd<AUX, REC, true>), grid, block, 0, stream, p, acc, g, ray_order, grab); \
-        else hipLaunchKernelGGL((k_row_fwd<AUX, REC, false>), grid, block, 0, stream, p, acc, g, ray_order, grab);          \
+        if (p.flags != 0u) hipLaunchKernelGGL((k_row_fwd<AUX, REC, true, BEYOND>), grid, block, 0, stream, p, acc, g, ray_order, grab); \
+        else hipLaunchKernelGGL((k_row_fwd<AUX, REC, false, BEYOND>), grid, block, 0, stream, p, acc, g, ray_order, grab);  \
     } while (0)
     if (p.aux <= 2) DST_ROW(2);
     else if (p.aux <= 4) DST_ROW(4);
@@ -2445,11 +2455,11 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
     const bool det = (p.flags & DST_FLAG_DETERMINISTIC) != 0u;
     uint32_t *const out_of_range = ctx->handover + kDstHandoverOutOfRange;   // (a spare word of the list's header)
     RowGrid rows;
-    const bool by_rows = row_grid(p, t, rows);
+    const TraceBy by = row_grid(p, t, rows);
     if (backward) {
         const uint32_t n_blocks = t.btiles_x * t.btiles_y;
         // the kernel that fits the record (complete, written ray by ray or wave by wave; incomplete) does the work
-        if (rec && by_rows) launch_row_bwd(p, rows, ray_order, stream);
+        if (rec && by == TraceBy::Rows) launch_row_bwd(p, rows, ray_order, stream);
         if (rec && n_blocks < kOrderMinBlocks) {
             launch<true, true>(p, acc, t, ray_order, stream);
         } else if (rec) {
@@ -2494,9 +2504,17 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
         // the second launch of each pair traces the tiles the first one handed over (usually none: it leaves at once)
         uint32_t *const list = (kFwdWavesPerBlock == 1 && dst_handover_active(ctx)) ? ctx->handover : nullptr;
         // (a context told never to hand tiles over keeps the rays of an image's tile together)
-        if (by_rows && list == nullptr && (ctx->handover_mode != DST_HANDOVER_OFF || p.max_trace_depth > 0 || t.th_log2 < 3)) {
-            if (rec) launch_row_fwd<true>(p, acc, rows, ray_order, stream);
-            else launch_row_fwd<false>(p, acc, rows, ray_order, stream);
+        if (by == TraceBy::Rows && list == nullptr && (ctx->handover_mode != DST_HANDOVER_OFF || p.max_trace_depth > 0 || t.th_log2 < 3)) {
+            if (rec) launch_row_fwd<true, false>(p, acc, rows, ray_order, stream);
+            else launch_row_fwd<false, false>(p, acc, rows, ray_order, stream);
+        } else if (by == TraceBy::TilesThenRows && list == nullptr) {
+            if (rec) {
+                launch<false, true>(p, acc, t, ray_order, stream, nullptr, nullptr, 0u, true);
+                launch_row_fwd<true, true>(p, acc, rows, ray_order, stream);
+            } else {
+                launch<false, false>(p, acc, t, ray_order, stream, nullptr, nullptr, 0u, true);
+                launch_row_fwd<false, true>(p, acc, rows, ray_order, stream);
+            }
         } else
         for (int pass = 0; pass < (list != nullptr ? 2 : 1); ++pass) {
             const uint32_t arg = pass == 0 ? steps : 0u;
