@@ -38,6 +38,8 @@ int check_common(dst_ctx *ctx, const DstParams *p) {
     if (p->flags & ~(DST_FLAG_DETERMINISTIC | DST_FLAG_DISTORTION | DST_FLAG_SH_HALF))
         return dst_fail(ctx, DST_E_INVALID, "unknown bits in flags");
 
+    if (p->dist_channels != 0 && p->dist_channels != 1 && p->dist_channels != 3)
+        return dst_fail(ctx, DST_E_INVALID, "dist_channels must be 1 or 3");
     if (p->hit_record && (reinterpret_cast<uintptr_t>(p->hit_record) & 7u))
         return dst_fail(ctx, DST_E_INVALID, "hit_record must be 8-byte aligned");
     if (p->H > 0 && p->W > 0 &&
@@ -88,6 +90,7 @@ void dst_destroy(dst_ctx *ctx) {
     if (ctx->bounds) (void)hipFree(ctx->bounds);
     if (ctx->core_box) (void)hipFree(ctx->core_box);
     if (ctx->bounds_host) (void)hipHostFree(ctx->bounds_host);
+    if (ctx->det_host) (void)hipHostFree(ctx->det_host);
     if (ctx->ploc_host) (void)hipHostFree(ctx->ploc_host);
     delete ctx;
 }
@@ -173,11 +176,14 @@ int dst_trace_backward(dst_ctx *ctx, const DstParams *p, void *stream) {
     if (p->H > 0 && p->W > 0 &&
         (!p->dL_drgb || !p->dL_ddpt || !p->dL_dacc || !p->dL_dnorm || !p->dL_daux || !p->dL_dray_o || !p->dL_dray_d))
         return dst_fail(ctx, DST_E_INVALID, "upstream gradients or ray gradient buffers missing");
-    if (!p->dL_dmeans3D || !p->dL_dgrads3D || !p->dL_dcolors || !p->dL_dopacities || !p->dL_dscales ||
+    const bool writes = p->grad_touched != nullptr;   // the closing kernel writes what is there and adds to nothing
+    if (writes && !(p->flags & DST_FLAG_DETERMINISTIC) && !p->grad_rows)
+        return dst_fail(ctx, DST_E_INVALID, "grad_touched goes with grad_rows or the deterministic mode");
+    if (!p->dL_dmeans3D || !p->dL_dgrads3D || (!p->dL_dcolors && !writes) || !p->dL_dopacities || !p->dL_dscales ||
         !p->dL_drotations)
         return dst_fail(ctx, DST_E_INVALID, "per-surfel gradient buffers missing");
     if (p->shs && !p->dL_dshs) return dst_fail(ctx, DST_E_INVALID, "dL_dshs missing");
-    if (p->others_precomp && !p->dL_dothers) return dst_fail(ctx, DST_E_INVALID, "dL_dothers missing");
+    if (p->others_precomp && !p->dL_dothers && !writes) return dst_fail(ctx, DST_E_INVALID, "dL_dothers missing");
     return dst_launch_trace(ctx, *p, true, (hipStream_t)stream);
 }
 
@@ -194,6 +200,16 @@ int dst_trace_info(dst_ctx *ctx, DstTraceInfo *info) {
     info->handover_active = dst_handover_active(ctx) ? 1u : 0u;
     info->det_out_of_range = words[kDstHandoverOutOfRange];
     info->tiles_handed_over = words[2];
+    return DST_OK;
+}
+
+int dst_det_out_of_range(dst_ctx *ctx, uint32_t *count, void *stream) {
+    if (!ctx || !count) return DST_E_INVALID;
+    if (!ctx->det_host) DST_HIP(ctx, hipHostMalloc((void **)&ctx->det_host, sizeof(uint32_t)));
+    DST_HIP(ctx, hipMemcpyAsync(ctx->det_host, ctx->handover + kDstHandoverOutOfRange, sizeof(uint32_t), hipMemcpyDeviceToHost,
+                                (hipStream_t)stream));
+    DST_HIP(ctx, hipStreamSynchronize((hipStream_t)stream));
+    *count = *ctx->det_host;
     return DST_OK;
 }
 

@@ -37,8 +37,32 @@ struct DstWideChild {
     float hi[3];
     uint32_t used;            // 1, or 0 for an unused slot
 };
+// The same words by coordinate, for the checks of a finished hierarchy (host only: the kernels read whole children).
+template <typename T, int WORD>
+struct DstWideColumn {
+    uint32_t word0;
+    const T &operator[](uint32_t k) const { return reinterpret_cast<const T *>(this)[8u * k + WORD]; }
+};
+struct DstWideCount {
+    uint32_t words[8 * DST_WIDE];
+    operator uint32_t() const {
+        uint32_t n = 0;
+        for (int k = 0; k < DST_WIDE; ++k) n += words[8 * k + 7];
+        return n;
+    }
+};
 struct alignas(128) DstWideNode {
-    DstWideChild child[DST_WIDE];
+    union {
+        DstWideChild child[DST_WIDE];
+        DstWideColumn<float, 0> lox;
+        DstWideColumn<float, 1> loy;
+        DstWideColumn<float, 2> loz;
+        DstWideColumn<uint32_t, 3> ref;
+        DstWideColumn<float, 4> hix;
+        DstWideColumn<float, 5> hiy;
+        DstWideColumn<float, 6> hiz;
+        DstWideCount count;
+    };
 };
 
 // Leaf = one surfel quad in leaf order (triangles ABC and BCD), as the hit test wants it: corner A, the edge vectors
@@ -159,6 +183,7 @@ struct dst_ctx {
     bool small_quads_asked = false;    // a copy of the device's count into bounds_host has been enqueued since the build
     DstBounds *bounds = nullptr;       // device (allocated by dst_create together with the hand-over list)
     DstBounds *bounds_host = nullptr;  // pinned host copy
+    uint32_t *det_host = nullptr;      // pinned host copy of the deterministic mode's out-of-range count
     void *core_box = nullptr;          // device: the box the two-level Morton keys are laid over (lbvh.hip)
     float scene_lo[3] = {0, 0, 0}, scene_hi[3] = {0, 0, 0}, max_abs = 0;
 };

@@ -38,7 +38,8 @@ class DstParams(C.Structure):
         + [(n, _FP) for n in ("dL_drgb", "dL_ddpt", "dL_dacc", "dL_ddist", "dL_dnorm", "dL_daux")]
         + [(n, _FP) for n in ("dL_dray_o", "dL_dray_d", "dL_dmeans3D", "dL_dgrads3D", "dL_dshs", "dL_dcolors",
                               "dL_dothers", "dL_dopacities", "dL_dscales", "dL_drotations")]
-        + [("shs_half", _FP)]
+        + [("shs_half", _FP), ("grad_touched", _FP), ("hit_record_asked", _FP), ("dist_channels", C.c_int32),
+           ("reserved", C.c_int32)]
     )
 
 
@@ -61,7 +62,7 @@ HANDOVER_OFF, HANDOVER_AUTO, HANDOVER_ALWAYS = 0, 1, 2
 EXPORTS = ("dst_create", "dst_destroy", "dst_build_accel", "dst_trace_forward", "dst_trace_backward",
            "dst_last_error", "dst_accel_info", "dst_accel_download", "dst_version", "dst_sizeof_params",
            "dst_hit_record_layout", "dst_refit_accel_static", "dst_refit_from_surfels",
-           "dst_det_workspace_words", "dst_pack_sh_half", "dst_trace_info", "dst_set_handover")
+           "dst_det_workspace_words", "dst_pack_sh_half", "dst_trace_info", "dst_set_handover", "dst_det_out_of_range")
 
 _lib = None
 
@@ -90,6 +91,7 @@ def load_library():
     L.dst_accel_info.argtypes = [C.c_void_p, C.POINTER(DstAccelInfo)]
     L.dst_accel_download.argtypes = [C.c_void_p] * 7
     L.dst_trace_info.argtypes = [C.c_void_p, C.POINTER(DstTraceInfo)]
+    L.dst_det_out_of_range.argtypes = [C.c_void_p, C.POINTER(C.c_uint32), C.c_void_p]
     L.dst_set_handover.argtypes = [C.c_void_p, C.c_int, C.c_uint32]
     L.dst_det_workspace_words.restype = C.c_uint64
     L.dst_det_workspace_words.argtypes = [C.c_int32, C.c_int32, C.c_int]
@@ -105,8 +107,22 @@ def load_library():
     return L
 
 
+_streams = {}
+
+
+def _current_stream():
+    """torch.cuda.current_stream(), from a small cache of the objects (building one costs more than a launch)."""
+    key = torch._C._cuda_getCurrentStream(torch._C._cuda_getDevice())
+    s = _streams.get(key)
+    if s is None:
+        if len(_streams) >= 64:
+            _streams.clear()
+        s = _streams[key] = torch.cuda.Stream(stream_id=key[0], device_index=key[1], device_type=key[2])
+    return s
+
+
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
 
 def _check(ctx, rc):
@@ -123,7 +139,7 @@ def _cuda_f32(t, name):
         raise RuntimeError("%s must be a CUDA tensor" % name)
     if t.dtype != torch.float32:
         t = t.float()
-    return t.contiguous()
+    return t if t.is_contiguous() else t.contiguous()
 
 
 def _ptr(t):
@@ -135,16 +151,25 @@ class HitRecord:
     replay them instead of walking the BVH again (see `hit_record` in include/dst_api.h).  `storage` is a
     caller- or pool-owned int64 tensor that is at least `words_needed(...)` long."""
 
-    @staticmethod
-    def layout(H, W, mtd_alloc, blocks_per_wave):
+    _layouts = {}   # (H, W, mtd_alloc) -> (header words, waves, words of a block)
+    _slots = []     # free words of pinned host memory for the request counts (note_request)
+    _late = []      # words given up before their copy had come: looked at again when new ones are needed
+
+    @classmethod
+    def layout(cls, H, W, mtd_alloc, blocks_per_wave):
         """(words of the whole buffer, header words, blocks, waves) for an (H,W) ray grid."""
-        header, waves = C.c_uint64(0), C.c_uint32(0)
-        lib = load_library()
-        lib.dst_hit_record_layout(H, W, mtd_alloc, 0, C.byref(header), C.byref(waves))
-        n_waves = max(1, waves.value)
+        known = cls._layouts.get((H, W, mtd_alloc))
+        if known is None:
+            header, waves = C.c_uint64(0), C.c_uint32(0)
+            lib = load_library()
+            words = lib.dst_hit_record_layout(H, W, mtd_alloc, 0, C.byref(header), C.byref(waves))
+            per_block = lib.dst_hit_record_layout(H, W, mtd_alloc, 1, None, None) - words
+            if len(cls._layouts) >= 256:
+                cls._layouts.clear()
+            known = cls._layouts[(H, W, mtd_alloc)] = (int(header.value), max(1, waves.value), int(per_block))
+        header, n_waves, per_block = known
         blocks = max(1, int(n_waves * blocks_per_wave) + 1)
-        words = lib.dst_hit_record_layout(H, W, mtd_alloc, blocks, None, None)
-        return int(words), int(header.value), blocks, n_waves
+        return (header + blocks * per_block if per_block else 0), header, blocks, n_waves
 
     def __init__(self, H, W, mtd_alloc, blocks_per_wave, device, storage=None):
         words, header, self.blocks, self.n_waves = self.layout(H, W, mtd_alloc, blocks_per_wave)
@@ -154,26 +179,43 @@ class HitRecord:
             raise RuntimeError("hit record storage must be a CUDA int64 tensor of at least %d elements" % words)
         self.words = storage
         self.words[:header].zero_()
-        self._asked_host = None
-        self._asked_event = None
+        self._slot = None          # (numpy view, index, address) of a pinned word
+        self._slot_stream = None
 
     def note_request(self):
-        """Stream-ordered, non-blocking copy of word 0 (blocks the forward trace asked for) to pinned host
-        memory; `asked()` reads it once the copy has happened."""
-        self._asked_host = torch.empty(1, dtype=torch.int64, pin_memory=True)
-        self._asked_host.copy_(self.words[:1], non_blocking=True)
-        self._asked_event = torch.cuda.Event()
-        self._asked_event.record()
+        """Address of a pinned host word that the forward trace about to be launched copies word 0 (the blocks it asked
+        for) to, stream-ordered and without anybody waiting; `asked()` reads it once the copy has happened."""
+        if self._slot is None:
+            try:
+                self._slot = HitRecord._slots.pop()
+            except IndexError:   # pinned memory by the page: a few hundred words at a time
+                late, HitRecord._late = HitRecord._late, []
+                HitRecord._slots.extend(s for s in late if s[0][s[1]] != -1)
+                HitRecord._late.extend(s for s in late if s[0][s[1]] == -1)
+                page = torch.empty(256, dtype=torch.int64, pin_memory=True)
+                view, at = page.numpy(), page.data_ptr()
+                HitRecord._slots.extend((view, k, at + 8 * k, page) for k in range(1, 256))
+                self._slot = (view, 0, at, page)
+        self._slot[0][self._slot[1]] = -1
+        self._slot_stream = _current_stream()
+        return self._slot[2]
+
+    def __del__(self):
+        # a word whose copy may still be under way is not handed to anybody else
+        slot, self._slot = getattr(self, "_slot", None), None
+        if slot is not None:
+            (HitRecord._late if slot[0][slot[1]] == -1 else HitRecord._slots).append(slot)
 
     def asked(self, wait=False):
         """Blocks requested by the forward trace, or None while that is not known yet (never waits unless told to)."""
-        if self._asked_event is None:
+        if self._slot is None:
             return int(self.words[0].item()) if wait else None
-        if wait:
-            self._asked_event.synchronize()
-        elif not self._asked_event.query():
-            return None
-        return int(self._asked_host[0])
+        view, k = self._slot[:2]
+        if view[k] == -1:
+            if not wait:
+                return None
+            self._slot_stream.synchronize()
+        return int(view[k])
 
     def requested_blocks(self):
         """Blocks the forward trace asked for (waits for it to finish)."""
@@ -226,6 +268,8 @@ class OptiXStateWrapper:
         self._record_events = {}            # id(storage) -> event recorded when the storage came back
         self._record_fixed = False          # True: only caller-provided storage is used, nothing is allocated
         self._record_watch = []             # records whose request count has not been read yet
+        self.single_dist = False            # set by the autograd wrapper: the next forward call's dist has one channel
+        self._row_pool = []                 # (rows, marks, stream, event): per-surfel sums of backward calls, all zero
 
     # ---- hit-record storage ---------------------------------------------------------------------------
     def use_record_storage(self, storage):
@@ -279,7 +323,7 @@ class OptiXStateWrapper:
             # the backward trace that last read this storage may still be running on another stream
             done = self._record_events.pop(id(storage), None)
             if done is not None:
-                torch.cuda.current_stream().wait_event(done)
+                _current_stream().wait_event(done)
         elif self._record_fixed:
             return None
         else:
@@ -297,7 +341,7 @@ class OptiXStateWrapper:
             return
         if rec.words.is_cuda:
             done = torch.cuda.Event()
-            done.record()
+            done.record(_current_stream())
             self._record_events[id(rec.words)] = done
         self._record_pool.append(rec.words)
         rec.words = None
@@ -309,6 +353,37 @@ class OptiXStateWrapper:
             smallest = min(self._record_pool, key=lambda t: t.numel())
             self._record_pool = [t for t in self._record_pool if t is not smallest]
             self._record_events.pop(id(smallest), None)
+
+    # ---- per-surfel sums of the backward traces -------------------------------------------------------
+    ROW_POOL_SIZE = 2
+
+    def acquire_rows(self, P, words, dtype, device):
+        """A zeroed buffer of at least `words` sums and one of at least P marks (DstParams.grad_touched).  The closing
+        kernel of a backward trace leaves both zero, so they are filled once, not per call; at most ROW_POOL_SIZE pairs
+        are kept, with the context."""
+        if not torch.cuda.is_current_stream_capturing():   # (a captured fill has not run yet)
+            for _ in range(self.ROW_POOL_SIZE):
+                try:   # taken out first: another thread may be looking too
+                    rows, marks, stream, event = self._row_pool.pop(0)
+                except IndexError:
+                    break
+                if rows.dtype != dtype or rows.numel() < words or marks.numel() < P or rows.device != device:
+                    self._row_pool.append((rows, marks, stream, event))
+                    continue
+                now = _current_stream()
+                if stream is not now:   # its last user may still be running there
+                    now.wait_event(event)
+                return rows, marks
+        return (torch.zeros(words, dtype=dtype, device=device), torch.zeros(P, dtype=torch.uint8, device=device))
+
+    def release_rows(self, rows, marks):
+        """Back to the pool, behind a backward trace that has been launched (after a failed call they are dropped)."""
+        if torch.cuda.is_current_stream_capturing():
+            return
+        stream, event = _current_stream(), torch.cuda.Event()
+        event.record(stream)
+        self._row_pool.insert(0, (rows, marks, stream, event))
+        del self._row_pool[self.ROW_POOL_SIZE:]
 
     def accel_info(self):
         info = DstAccelInfo()
@@ -326,8 +401,10 @@ class OptiXStateWrapper:
     def check_deterministic_range(self):
         """Warn if sums of the deterministic mode have left their fixed-point range since the last look (gradients
         beyond about 6.7e7 for scales, rotations and means, 4.2e6 for the rest: they come out clamped or wrapped).
-        Waits for the device.  Returns the number of such sums."""
-        seen = int(self.trace_info().det_out_of_range)
+        Waits for the current stream.  Returns the number of such sums."""
+        count = C.c_uint32(0)
+        _check(self, load_library().dst_det_out_of_range(self.handle, C.byref(count), _stream()))
+        seen = count.value
         new, self._det_out_of_range = (seen - self._det_out_of_range) & 0xFFFFFFFF, seen
         if new:
             warnings.warn("deterministic mode: %d per-surfel sums left the fixed-point range and are wrong; scale the "
@@ -442,15 +519,20 @@ def trace_surfels(ctx, training, start_from_first, ray_o, ray_d, vertices, backg
     Extras for measurement: `counters` (2 int64 on the device) receives the evaluated / composited hit totals;
     `events` (two torch.cuda.Event) are recorded on the launch stream right around the kernel launch;
     `hit_record` (a HitRecord) receives the hit buffers for a later replay by trace_surfels_backward."""
+    single = getattr(ctx, "single_dist", False)
+    if single:
+        ctx.single_dist = False
     p, keep = _common_params(ray_o, ray_d, vertices, background, means3D, shs, degree, colors_precomp,
                              others_precomp, opacities, scales, scale_modifier, rotations, max_trace_depth,
                              specular_threshold, start_from_first)
     H, W, P, dev = p.H, p.W, p.P, means3D.device
     mid_ch = (14 + p.aux) * (p.mtd_alloc + 1)
-    new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=dev)  # noqa: E731 (kernel writes every element)
-    out_rgb, out_dpt, out_acc = new(H, W, NUM_CHANNELS), new(H, W, 1), new(H, W, 1)
-    out_norm, out_dist, out_aux, mid_val = new(H, W, 3), new(H, W, 3), new(H, W, p.aux), new(H, W, mid_ch)
-    a_weights = torch.zeros((P, 1), dtype=torch.float32, device=dev) if training else None
+    p.dist_channels = 1 if single else 3
+    new = keep["means3D"].new_empty   # (the kernel writes every element)
+    out_rgb, out_dpt, out_acc = new((H, W, NUM_CHANNELS)), new((H, W, 1)), new((H, W, 1))
+    out_norm, out_dist, out_aux, mid_val = (new((H, W, 3)), new((H, W, 1 if single else 3)), new((H, W, p.aux)),
+                                            new((H, W, mid_ch)))
+    a_weights = keep["means3D"].new_zeros((P, 1)) if training else None
     p.training = int(bool(training))
     p.out_rgb, p.out_dpt, p.out_acc = out_rgb.data_ptr(), out_dpt.data_ptr(), out_acc.data_ptr()
     p.out_norm, p.out_dist, p.out_aux = out_norm.data_ptr(), out_dist.data_ptr(), out_aux.data_ptr()
@@ -459,6 +541,7 @@ def trace_surfels(ctx, training, start_from_first, ray_o, ray_d, vertices, backg
     p.counters = _ptr(counters)
     if hit_record is not None:
         p.hit_record, p.hit_record_blocks = hit_record.words.data_ptr(), hit_record.blocks
+        p.hit_record_asked = hit_record.note_request()
     det_ws = None
     if getattr(ctx, "deterministic", False) and training:
         det_ws = torch.zeros(load_library().dst_det_workspace_words(P, p.aux, 0), dtype=torch.int64, device=dev)
@@ -472,7 +555,6 @@ def trace_surfels(ctx, training, start_from_first, ray_o, ray_d, vertices, backg
     if events is not None:
         events[1].record()
     if hit_record is not None:
-        hit_record.note_request()
         ctx._record_watch.append(hit_record)
     del keep
     return out_rgb, out_dpt, out_acc, out_norm, out_dist, out_aux, mid_val, a_weights
@@ -483,10 +565,11 @@ def trace_surfels_backward(ctx, start_from_first, ray_o, ray_d, vertices, backgr
                            transMat_precomp, viewmatrix, projmatrix, campos, prefiltered, debug, max_trace_depth,
                            specular_threshold, out_rgb, out_dpt, out_acc, out_norm, out_dist, out_aux, mid_val,
                            dL_dout_rgb, dL_dout_dpt, dL_dout_acc, dL_dout_norm, dL_dout_dist, dL_dout_aux,
-                           events=None, hit_record=None, counters=None):
+                           events=None, hit_record=None, counters=None, wanted_only=False):
     """Reference TraceSurfelsBackwardCUDA (trace_surfels.cpp:307-464): returns (dL_dray_o, dL_dray_d, dL_dmeans3D,
     dL_dgrads3D, dL_dgrads3D_abs, dL_dshs, dL_dcolors, dL_dothers, dL_dopacities, dL_dscales, dL_drotations,
-    dL_dtransMat_precomp)."""
+    dL_dtransMat_precomp).  `wanted_only`: None for the gradients of inputs that were not given, and for the two that are
+    always zero."""
     p, keep = _common_params(ray_o, ray_d, vertices, background, means3D, shs, degree, colors_precomp,
                              others_precomp, opacities, scales, scale_modifier, rotations, max_trace_depth,
                              specular_threshold, start_from_first)
@@ -507,16 +590,24 @@ def trace_surfels_backward(ctx, start_from_first, ray_o, ray_d, vertices, backgr
             raise RuntimeError("upstream gradient of %s has the wrong size" % n)
     p.dL_drgb, p.dL_ddpt, p.dL_dacc, p.dL_dnorm, p.dL_ddist, p.dL_daux = (
         ups[0].data_ptr(), ups[1].data_ptr(), ups[2].data_ptr(), ups[3].data_ptr(), _ptr(ups[4]), ups[5].data_ptr())
-    zeros = lambda *shape: torch.zeros(shape, dtype=torch.float32, device=dev)  # noqa: E731 (atomically accumulated)
-    dL_dray_o = torch.empty((H, W, 3), dtype=torch.float32, device=dev)
-    dL_dray_d = torch.empty((H, W, 3), dtype=torch.float32, device=dev)
-    dL_dmeans3D, dL_dgrads3D, dL_dgrads3D_abs = zeros(P, 3), zeros(P, 3), zeros(P, 3)
-    dL_dshs, dL_dcolors, dL_dothers = zeros(P, p.M, 3), zeros(P, NUM_CHANNELS), zeros(P, p.aux)
-    dL_dopacities, dL_dscales, dL_drotations = zeros(P, 1), zeros(P, 2), zeros(P, 4)
-    dL_dtransMat = zeros(P, 9)
+    det = bool(getattr(ctx, "deterministic", False))
+    # The per-surfel gradients are summed in a buffer of their own first (a surfel's columns side by side; fixed point in
+    # the deterministic mode), and a closing kernel writes them to the tensors; without it they are added to the tensors.
+    by_rows = det or getattr(ctx, "gradient_rows", True)
+    like = keep["means3D"]
+    new = like.new_empty if by_rows else like.new_zeros
+    dL_dray_o, dL_dray_d = like.new_empty((H, W, 3)), like.new_empty((H, W, 3))
+    dL_dmeans3D, dL_dgrads3D = new((P, 3)), new((P, 3))
+    dL_dshs = new((P, p.M, 3))
+    lean = wanted_only and by_rows
+    dL_dcolors = None if lean and not p.colors_precomp else new((P, NUM_CHANNELS))
+    dL_dothers = None if lean and not p.others_precomp else new((P, p.aux))
+    dL_dopacities, dL_dscales, dL_drotations = new((P, 1)), new((P, 2)), new((P, 4))
+    dL_dgrads3D_abs = None if wanted_only else like.new_zeros((P, 3))
+    dL_dtransMat = None if wanted_only else like.new_zeros((P, 9))
     p.dL_dray_o, p.dL_dray_d = dL_dray_o.data_ptr(), dL_dray_d.data_ptr()
     p.dL_dmeans3D, p.dL_dgrads3D, p.dL_dshs = dL_dmeans3D.data_ptr(), dL_dgrads3D.data_ptr(), _ptr(dL_dshs)
-    p.dL_dcolors, p.dL_dothers = dL_dcolors.data_ptr(), dL_dothers.data_ptr()
+    p.dL_dcolors, p.dL_dothers = _ptr(dL_dcolors), _ptr(dL_dothers)
     p.dL_dopacities, p.dL_dscales, p.dL_drotations = (dL_dopacities.data_ptr(), dL_dscales.data_ptr(),
                                                       dL_drotations.data_ptr())
     if hit_record is not None:
@@ -524,14 +615,14 @@ def trace_surfels_backward(ctx, start_from_first, ray_o, ray_d, vertices, backgr
         # nothing here waits for the forward trace
         p.hit_record, p.hit_record_blocks = hit_record.words.data_ptr(), hit_record.blocks
     p.counters = _ptr(counters)
-    det_ws = None
-    if getattr(ctx, "deterministic", False):
-        det_ws = torch.zeros(load_library().dst_det_workspace_words(P, p.aux, 1), dtype=torch.int64, device=dev)
-        p.flags, p.det_workspace = FLAG_DETERMINISTIC, det_ws.data_ptr()
-    elif getattr(ctx, "gradient_rows", True):
-        # the per-surfel gradients are summed in rows of one buffer first (a surfel's columns side by side)
-        det_ws = torch.zeros(load_library().dst_det_workspace_words(P, p.aux, 1), dtype=torch.float32, device=dev)
-        p.grad_rows = det_ws.data_ptr()
+    if by_rows:
+        rows, marks = ctx.acquire_rows(P, load_library().dst_det_workspace_words(P, p.aux, 1),
+                                       torch.int64 if det else torch.float32, like.device)
+        p.grad_touched = marks.data_ptr()
+        if det:
+            p.flags, p.det_workspace = FLAG_DETERMINISTIC, rows.data_ptr()
+        else:
+            p.grad_rows = rows.data_ptr()
     if getattr(ctx, "sh_half", False) and keep["shs"].numel() != 0:
         # the backward trace reads fp32 coefficients: the values the forward trace used
         keep["shs"] = pack_sh_half(keep["shs"]).float()
@@ -541,6 +632,8 @@ def trace_surfels_backward(ctx, start_from_first, ray_o, ray_d, vertices, backgr
     _check(ctx, load_library().dst_trace_backward(ctx.handle, C.byref(p), _stream()))
     if events is not None:
         events[1].record()
+    if by_rows:
+        ctx.release_rows(rows, marks)
     if p.flags & FLAG_DETERMINISTIC and getattr(ctx, "deterministic_check", False):
         ctx.check_deterministic_range()   # (the mode waits for the device elsewhere too: record sizes)
     del keep

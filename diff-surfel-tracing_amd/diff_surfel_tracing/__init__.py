@@ -37,6 +37,17 @@ class SurfelTracingSettings(NamedTuple):
     specular_threshold: float = 0.0
 
 
+_placeholders = {}
+
+
+def _placeholder(device):
+    t = _placeholders.get(device)
+    if t is None:
+        with torch.inference_mode(False):   # (it may be saved for a backward pass later)
+            t = _placeholders[device] = torch.empty(0, dtype=torch.float32, device=device)
+    return t
+
+
 def _settings_args(s):
     """The settings fields in the order the launcher takes them after `rotations, cov3Ds_precomp`."""
     return (s.viewmatrix, s.projmatrix, s.campos, s.prefiltered, s.debug, s.max_trace_depth, s.specular_threshold)
@@ -52,6 +63,13 @@ def _guarded(fn, args, debug, dump_name, what):
         torch.save(snapshot, dump_name)
         print("\nAn error occured in %s. Please forward %s for debugging." % (what, dump_name))
         raise
+
+
+def _results(out_rgb, out_dpt, out_acc, out_norm, out_dist, out_aux, mid_val, a_weights, means3D):
+    # per-surfel accumulated blending weight (training) or zeros of shape (P,) (evaluation)
+    acc_wet = a_weights if a_weights is not None else means3D.new_zeros(means3D.size(0))
+    dist = out_dist if out_dist.size(-1) == 1 else out_dist[..., :1].clone()
+    return out_rgb, out_dpt, out_acc, out_norm, dist, out_aux, mid_val, acc_wet
 
 
 class _TraceSurfels(torch.autograd.Function):
@@ -70,6 +88,7 @@ class _TraceSurfels(torch.autograd.Function):
             record = optix_context.acquire_record(ray_o.size(0), ray_o.size(1),
                                                   max(_C.DEFAULT_MAX_TRACE_DEPTH, s.max_trace_depth), ray_o.device,
                                                   max_trace_depth=s.max_trace_depth)
+        optix_context.single_dist = True
         try:
             out_rgb, out_dpt, out_acc, out_norm, out_dist, out_aux, mid_val, a_weights = _guarded(
                 lambda *a: _C.trace_surfels(*a, hit_record=record), args, s.debug, "snapshot_fw.dump", "forward")
@@ -84,9 +103,7 @@ class _TraceSurfels(torch.autograd.Function):
         ctx.save_for_backward(ray_o, ray_d, vertices, means3D, shs, colors_precomp, others_precomp, opacities, scales,
                               rotations, cov3Ds_precomp, out_rgb, out_dpt, out_acc, out_norm, out_dist, out_aux,
                               mid_val)
-        # per-surfel accumulated blending weight (training) or zeros of shape (P,) (evaluation)
-        acc_wet = a_weights if a_weights is not None else torch.zeros_like(means3D[:, 0])
-        return out_rgb, out_dpt, out_acc, out_norm, out_dist[..., :1].clone(), out_aux, mid_val, acc_wet
+        return _results(out_rgb, out_dpt, out_acc, out_norm, out_dist, out_aux, mid_val, a_weights, means3D)
 
     @staticmethod
     def backward(ctx, grad_out_rgb, grad_out_dpt, grad_out_acc, grad_out_norm, grad_out_dist, grad_out_aux,
@@ -103,7 +120,7 @@ class _TraceSurfels(torch.autograd.Function):
         try:
             (g_ray_o, g_ray_d, g_means3D, g_grads3D, _g_grads3D_abs, g_shs, g_colors, g_others, g_opacities,
              g_scales, g_rotations, g_cov3Ds) = _guarded(
-                 lambda *a: _C.trace_surfels_backward(*a, hit_record=record), args, s.debug, "snapshot_bw.dump",
+                 lambda *a: _C.trace_surfels_backward(*a, hit_record=record, wanted_only=True), args, s.debug, "snapshot_bw.dump",
                  "backward")
         finally:
             # the storage goes back to the pool (stream-ordered reuse); a second backward through the same graph
@@ -126,6 +143,14 @@ def trace_surfels(optix_context, training, start_from_first, ray_o, ray_d, verti
     optix_context.record_wanted = torch.is_grad_enabled() and any(
         isinstance(t, torch.Tensor) and t.requires_grad
         for t in (ray_o, ray_d, means3D, grads3D, shs, colors_precomp, others_precomp, opacities, scales, rotations))
+    if not optix_context.record_wanted:
+        # nothing to differentiate: the launcher without the autograd function around it
+        s = tracer_settings
+        args = (optix_context, training, start_from_first, ray_o, ray_d, vertices, s.bg, means3D, shs, s.sh_degree,
+                colors_precomp, others_precomp, opacities, scales, s.scale_modifier, rotations,
+                cov3Ds_precomp) + _settings_args(s)
+        optix_context.single_dist = True
+        return _results(*_guarded(_C.trace_surfels, args, s.debug, "snapshot_fw.dump", "forward"), means3D)
     return _TraceSurfels.apply(optix_context, training, start_from_first, ray_o, ray_d, vertices, means3D, grads3D,
                                shs, colors_precomp, others_precomp, opacities, scales, rotations, cov3Ds_precomp,
                                tracer_settings)
@@ -195,15 +220,14 @@ class SurfelTracer(nn.Module):
         if ((scales is None or rotations is None) and not has_cov) or (has_sr and has_cov):
             raise Exception('Please provide exactly one of either scale/rotation pair or precomputed 3D covariance!')
 
-        dev = means3D.device
-        empty = lambda: torch.empty(0, dtype=torch.float32, device=dev)  # noqa: E731 placeholder for an absent input
-        shs = empty() if shs is None else shs
-        colors_precomp = empty() if colors_precomp is None else colors_precomp
-        others_precomp = empty() if others_precomp is None else others_precomp
-        scales = empty() if scales is None else scales
-        rotations = empty() if rotations is None else rotations
-        cov3D_precomp = empty() if cov3D_precomp is None else cov3D_precomp
-        vertices = empty() if vertices is None else vertices
+        empty = _placeholder(means3D.device)   # stands for an absent input
+        shs = empty if shs is None else shs
+        colors_precomp = empty if colors_precomp is None else colors_precomp
+        others_precomp = empty if others_precomp is None else others_precomp
+        scales = empty if scales is None else scales
+        rotations = empty if rotations is None else rotations
+        cov3D_precomp = empty if cov3D_precomp is None else cov3D_precomp
+        vertices = empty if vertices is None else vertices
 
         return trace_surfels(self.optix_context, self.training, start_from_first, ray_o, ray_d, vertices, means3D,
                              grads3D, shs, colors_precomp, others_precomp, opacities, scales, rotations,

@@ -136,9 +136,20 @@ typedef struct DstParams {
     float *dL_dopacities;         /* (P,1) */
     float *dL_dscales;            /* (P,2) */
     float *dL_drotations;         /* (P,4) */
-    /* forward, DST_FLAG_SH_HALF: binary16 copy of shs, same shape (P,M,3); NULL otherwise (last in the block: the
+    /* forward, DST_FLAG_SH_HALF: binary16 copy of shs, same shape (P,M,3); NULL otherwise (at the end of the block: the
      * kernels fetch their arguments in groups, and a field in the middle would move the others) */
     const uint16_t *shs_half;
+    /* backward, optional, together with grad_rows or the deterministic mode's workspace: P bytes, zero before the call.
+     * The trace marks the surfels it adds to, and the closing kernel then WRITES the per-surfel gradient tensors (they
+     * need not be zero-filled; dL_dcolors and dL_dothers may be NULL where their gradient is not wanted), reads the rows
+     * of the marked surfels only, and leaves the rows and the marks all zero again: a caller that keeps both between
+     * calls never fills them, and fills no gradient tensor. */
+    uint8_t *grad_touched;
+    /* forward, optional: HOST memory (pinned) that receives word 0 of hit_record behind the trace (a copy on the stream
+     * that nobody waits for) */
+    uint64_t *hit_record_asked;
+    int32_t dist_channels;        /* forward: channels of out_dist: 1 (the distortion alone), or 3 (also 0: three) */
+    int32_t reserved;
 } DstParams;
 
 /* Shape of the current acceleration structure, for tests and tools. */
@@ -208,6 +219,10 @@ int dst_trace_forward(dst_ctx *ctx, const DstParams *params, void *stream);
 /* Backward re-trace: fills dL_dray_o/d, accumulates the per-surfel gradients.
  * Replaces TraceSurfelsBackwardCUDA (trace_surfels.cpp:307-464); stream-ordered, no wait. */
 int dst_trace_backward(dst_ctx *ctx, const DstParams *params, void *stream);
+
+/* Sums of the deterministic mode found out of range so far (DstTraceInfo.det_out_of_range), as of the work enqueued on
+ * `stream`; waits for that stream only. */
+int dst_det_out_of_range(dst_ctx *ctx, uint32_t *count, void *stream);
 
 /* Message of the last failure on this context (never NULL).  The reference
  * prints CUDA/OptiX failures and carries on (optix_tracer/common.h:38-50). */
