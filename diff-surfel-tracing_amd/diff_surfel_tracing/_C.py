@@ -323,7 +323,9 @@ class OptiXStateWrapper:
             # the backward trace that last read this storage may still be running on another stream
             done = self._record_events.pop(id(storage), None)
             if done is not None:
-                _current_stream().wait_event(done)
+                now = _current_stream()
+                now.wait_event(done)
+                storage.record_stream(now)   # (its allocator knows the stream it was made on, and no other)
         elif self._record_fixed:
             return None
         else:
@@ -340,8 +342,9 @@ class OptiXStateWrapper:
         if rec is None or rec.words is None:
             return
         if rec.words.is_cuda:
-            done = torch.cuda.Event()
-            done.record(_current_stream())
+            done, now = torch.cuda.Event(), _current_stream()
+            done.record(now)
+            rec.words.record_stream(now)
             self._record_events[id(rec.words)] = done
         self._record_pool.append(rec.words)
         rec.words = None
@@ -371,8 +374,10 @@ class OptiXStateWrapper:
                     self._row_pool.append((rows, marks, stream, event))
                     continue
                 now = _current_stream()
-                if stream is not now:   # its last user may still be running there
+                if stream is not now:   # its last user may still be running there, and when the pair is dropped, this one
                     now.wait_event(event)
+                    rows.record_stream(now)
+                    marks.record_stream(now)
                 return rows, marks
         return (torch.zeros(words, dtype=dtype, device=device), torch.zeros(P, dtype=torch.uint8, device=device))
 

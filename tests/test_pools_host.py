@@ -1,0 +1,109 @@
+"""The buffers a context keeps between calls (hit records, rows of gradient sums), without a GPU: stand-ins for tensors,
+streams and events that note what is asked of them."""
+import pytest
+import torch
+
+from diff_surfel_tracing import _C
+
+
+class _Stream:
+    def __init__(self):
+        self.waited = []
+
+    def wait_event(self, event):
+        self.waited.append(event)
+
+
+class _Event:
+    def record(self, stream):
+        self.stream = stream
+
+
+class _Buffer:
+    """A device tensor as the caching allocator sees it: `home` is the stream it was made on, `users` the streams the
+    allocator has been told of.  Once it is dropped the memory is free for `home` as soon as those are done with it."""
+
+    def __init__(self, n, dtype, device, home):
+        self.n, self.dtype, self.device, self.home, self.users, self.is_cuda = n, dtype, device, home, [], True
+
+    def numel(self):
+        return self.n
+
+    def element_size(self):
+        return {torch.float32: 4, torch.int64: 8, torch.uint8: 1}[self.dtype]
+
+    def record_stream(self, stream):
+        if stream is not self.home:
+            self.users.append(stream)
+
+
+class _Device:
+    """What the pools ask of torch.cuda, with a current stream that the test sets."""
+
+    def __init__(self, monkeypatch):
+        self.now = _Stream()
+        make = lambda n, dtype=torch.float32, device=None: _Buffer(n, dtype, device, self.now)  # noqa: E731
+        monkeypatch.setattr(_C, "_current_stream", lambda: self.now)
+        monkeypatch.setattr(_C.torch.cuda, "Event", _Event)
+        monkeypatch.setattr(_C.torch.cuda, "current_device", lambda: 0)
+        monkeypatch.setattr(_C.torch.cuda, "is_current_stream_capturing", lambda: False)
+        monkeypatch.setattr(_C.torch, "zeros", make)
+        monkeypatch.setattr(_C.torch, "empty", make)
+
+
+@pytest.fixture
+def device(monkeypatch):
+    return _Device(monkeypatch)
+
+
+def _context():
+    ctx = _C.OptiXStateWrapper.__new__(_C.OptiXStateWrapper)
+    ctx.handle = None
+    ctx._row_pool, ctx._record_pool, ctx._record_fixed, ctx._record_events, ctx._record_watch = [], [], False, {}, []
+    ctx.record_blocks_per_wave, ctx.deterministic, ctx.records_skipped = 4.0, False, 0
+    ctx.record_max_bytes, ctx.record_pool_max_bytes = 1 << 40, 1 << 40
+    return ctx
+
+
+def test_gradient_rows_tell_the_allocator_of_every_stream_they_serve(device):
+    """A pair made on one stream and used on another may be dropped while that other one still works on it (P grew, the
+    mode changed, the tracer went away): the allocator has to know."""
+    ctx = _context()
+    a, b = device.now, _Stream()
+    pair = ctx.acquire_rows(10, 660, torch.float32, "cuda:0")
+    ctx.release_rows(*pair)
+    device.now = b
+    again = ctx.acquire_rows(10, 660, torch.float32, "cuda:0")
+    assert again[0] is pair[0] and again[1] is pair[1]
+    assert len(b.waited) == 1 and b.waited[0].stream is a
+    assert pair[0].users == [b] and pair[1].users == [b]
+    ctx.release_rows(*again)
+    device.now = a                              # and back: nothing new to be told of, but b has to be waited for
+    assert ctx.acquire_rows(10, 660, torch.float32, "cuda:0")[0] is pair[0]
+    assert a.waited[-1].stream is b and pair[0].users == [b]
+
+
+class _Record:
+    """HitRecord without the library behind it."""
+
+    def __init__(self, H, W, mtd_alloc, blocks_per_wave, device, storage=None):
+        self.words, self.blocks = storage, 1
+
+    @classmethod
+    def layout(cls, H, W, mtd_alloc, blocks_per_wave):
+        return H * W, 4, 1, 1
+
+
+def test_hit_records_tell_the_allocator_of_every_stream_they_serve(device, monkeypatch):
+    monkeypatch.setattr(_C, "HitRecord", _Record)
+    ctx = _context()
+    a, b, c = device.now, _Stream(), _Stream()
+    rec = ctx.acquire_record(8, 8, 1, torch.device("cuda", 0))
+    storage = rec.words
+    ctx.release_record(rec)
+    device.now = b                              # a forward trace there, whose graph may go without a backward pass
+    rec = ctx.acquire_record(8, 8, 1, torch.device("cuda", 0))
+    assert rec.words is storage and b.waited[0].stream is a and storage.users == [b]
+    device.now = c                              # a backward trace on a stream of its own
+    ctx.release_record(rec)
+    assert c in storage.users
