@@ -9,6 +9,7 @@ from typing import NamedTuple
 
 import torch
 import torch.nn as nn
+from torch.autograd import forward_ad
 
 from . import _C
 
@@ -136,6 +137,14 @@ class _TraceSurfels(torch.autograd.Function):
                 like(g_cov3Ds, cov3Ds_precomp), None)
 
 
+def _transforms_active():
+    """Whether more goes on than the call shows: inputs that may carry tangents of forward-mode differentiation or
+    functorch's levels (the autograd function refuses what it has no rule for), or a trace being recorded (the autograd
+    function is a node of it; its launches alone would leave only the empty output tensors there)."""
+    return (forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active()
+            or torch._C._get_tracing_state() is not None)
+
+
 def trace_surfels(optix_context, training, start_from_first, ray_o, ray_d, vertices, means3D, grads3D, shs,
                   colors_precomp, others_precomp, opacities, scales, rotations, cov3Ds_precomp, tracer_settings):
     # a hit record only pays off when a backward pass can follow: not under torch.no_grad(), not for inputs
@@ -143,7 +152,7 @@ def trace_surfels(optix_context, training, start_from_first, ray_o, ray_d, verti
     optix_context.record_wanted = torch.is_grad_enabled() and any(
         isinstance(t, torch.Tensor) and t.requires_grad
         for t in (ray_o, ray_d, means3D, grads3D, shs, colors_precomp, others_precomp, opacities, scales, rotations))
-    if not optix_context.record_wanted:
+    if not optix_context.record_wanted and not _transforms_active():
         # nothing to differentiate: the launcher without the autograd function around it
         s = tracer_settings
         args = (optix_context, training, start_from_first, ray_o, ray_d, vertices, s.bg, means3D, shs, s.sh_degree,

@@ -218,3 +218,67 @@ def test_record_pool_takes_back_records_of_any_size():
     pool.record_pool_max_bytes = 8
     pool.release_record(_Rec(4))
     assert [t.numel() for t in pool._record_pool] == [11]
+
+
+def _call_args(P=5, H=4, W=4):
+    import diff_surfel_tracing as dst
+    eye = torch.eye(4)
+    st = dst.SurfelTracingSettings(H, W, 1.0, 1.0, torch.zeros(3), 1.0, eye, eye, 3, torch.zeros(3), False, False)
+    return [_FakeContext(), True, True, torch.zeros(H, W, 3), torch.zeros(H, W, 3), torch.zeros(4 * P, 3), torch.zeros(P, 3),
+            torch.zeros(P, 3), torch.zeros(P, 16, 3), torch.empty(0), torch.empty(0), torch.zeros(P, 1), torch.ones(P, 2),
+            torch.zeros(P, 4), torch.empty(0), st]
+
+
+def _fake_launcher(ctx, training, sff, ray_o, *rest, hit_record=None):
+    H, W = ray_o.shape[:2]
+    z = lambda c: torch.zeros(H, W, c)  # noqa: E731
+    return z(3), z(1), z(1), z(3), z(1), z(2), z(32), None
+
+
+def test_forward_mode_tangents_are_refused(monkeypatch):
+    """A dual tensor made from a plain one does not require a gradient; without a rule for its tangent the call has to
+    raise, not to return outputs that have none."""
+    import torch.autograd.forward_ad as fwad
+
+    import diff_surfel_tracing as dst
+    from diff_surfel_tracing import _C
+    monkeypatch.setattr(_C, "trace_surfels", _fake_launcher)
+    for k in (3, 6, 8, 11):
+        args = _call_args()
+        with fwad.dual_level():
+            args[k] = fwad.make_dual(args[k], torch.ones_like(args[k]))
+            with pytest.raises(NotImplementedError):
+                dst.trace_surfels(*args)
+    with fwad.dual_level():            # no tangent among the inputs: a plain evaluation
+        assert dst.trace_surfels(*_call_args())[0].shape == (4, 4, 3)
+
+
+def test_functorch_transforms_are_refused(monkeypatch):
+    import diff_surfel_tracing as dst
+    from diff_surfel_tracing import _C
+    monkeypatch.setattr(_C, "trace_surfels", _fake_launcher)
+    args = _call_args()
+
+    def rgb(means):
+        return dst.trace_surfels(*args[:6], means, *args[7:])[0]
+    with pytest.raises(RuntimeError):
+        torch.func.jvp(rgb, (args[6],), (torch.ones_like(args[6]),))
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(rgb)(torch.zeros(2, 5, 3))
+
+
+def test_a_recorded_trace_launches_again(monkeypatch):
+    """torch.jit.trace of an evaluation: the call is a node of the trace, run whenever the traced function is."""
+    import diff_surfel_tracing as dst
+    from diff_surfel_tracing import _C
+    launches = []
+
+    def launcher(*a, **k):
+        launches.append(1)
+        return _fake_launcher(*a, **k)
+    monkeypatch.setattr(_C, "trace_surfels", launcher)
+    args = _call_args()
+    traced = torch.jit.trace(lambda means: dst.trace_surfels(*args[:6], means, *args[7:])[0], (args[6],), check_trace=False)
+    n = len(launches)
+    traced(args[6])
+    assert len(launches) == n + 1
