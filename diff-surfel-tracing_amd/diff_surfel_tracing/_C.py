@@ -268,7 +268,6 @@ class OptiXStateWrapper:
         self._record_events = {}            # id(storage) -> event recorded when the storage came back
         self._record_fixed = False          # True: only caller-provided storage is used, nothing is allocated
         self._record_watch = []             # records whose request count has not been read yet
-        self.single_dist = False            # set by the autograd wrapper: the next forward call's dist has one channel
         self._row_pool = []                 # (rows, marks, stream, event): per-surfel sums of backward calls, all zero
 
     # ---- hit-record storage ---------------------------------------------------------------------------
@@ -518,24 +517,22 @@ def _common_params(ray_o, ray_d, vertices, background, means3D, shs, degree, col
 def trace_surfels(ctx, training, start_from_first, ray_o, ray_d, vertices, background, means3D, shs, degree,
                   colors_precomp, others_precomp, opacities, scales, scale_modifier, rotations, transMat_precomp,
                   viewmatrix, projmatrix, campos, prefiltered, debug, max_trace_depth, specular_threshold,
-                  counters=None, events=None, hit_record=None):
+                  counters=None, events=None, hit_record=None, dist_channels=3):
     """Reference TraceSurfelsCUDA (trace_surfels.cpp:162-304): returns
     (out_rgb, out_dpt, out_acc, out_norm, out_dist, out_aux, mid_val, a_weights or None).
     Extras for measurement: `counters` (2 int64 on the device) receives the evaluated / composited hit totals;
     `events` (two torch.cuda.Event) are recorded on the launch stream right around the kernel launch;
-    `hit_record` (a HitRecord) receives the hit buffers for a later replay by trace_surfels_backward."""
-    single = getattr(ctx, "single_dist", False)
-    if single:
-        ctx.single_dist = False
+    `hit_record` (a HitRecord) receives the hit buffers for a later replay by trace_surfels_backward.
+    `dist_channels`: 3 as the reference's launcher returns them, 1 for the distortion alone."""
     p, keep = _common_params(ray_o, ray_d, vertices, background, means3D, shs, degree, colors_precomp,
                              others_precomp, opacities, scales, scale_modifier, rotations, max_trace_depth,
                              specular_threshold, start_from_first)
     H, W, P, dev = p.H, p.W, p.P, means3D.device
     mid_ch = (14 + p.aux) * (p.mtd_alloc + 1)
-    p.dist_channels = 1 if single else 3
+    p.dist_channels = int(dist_channels)
     new = keep["means3D"].new_empty   # (the kernel writes every element)
     out_rgb, out_dpt, out_acc = new((H, W, NUM_CHANNELS)), new((H, W, 1)), new((H, W, 1))
-    out_norm, out_dist, out_aux, mid_val = (new((H, W, 3)), new((H, W, 1 if single else 3)), new((H, W, p.aux)),
+    out_norm, out_dist, out_aux, mid_val = (new((H, W, 3)), new((H, W, p.dist_channels)), new((H, W, p.aux)),
                                             new((H, W, mid_ch)))
     a_weights = keep["means3D"].new_zeros((P, 1)) if training else None
     p.training = int(bool(training))

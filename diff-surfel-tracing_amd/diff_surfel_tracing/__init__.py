@@ -89,10 +89,9 @@ class _TraceSurfels(torch.autograd.Function):
             record = optix_context.acquire_record(ray_o.size(0), ray_o.size(1),
                                                   max(_C.DEFAULT_MAX_TRACE_DEPTH, s.max_trace_depth), ray_o.device,
                                                   max_trace_depth=s.max_trace_depth)
-        optix_context.single_dist = True
         try:
             out_rgb, out_dpt, out_acc, out_norm, out_dist, out_aux, mid_val, a_weights = _guarded(
-                lambda *a: _C.trace_surfels(*a, hit_record=record), args, s.debug, "snapshot_fw.dump", "forward")
+                lambda *a: _C.trace_surfels(*a, None, None, record, 1), args, s.debug, "snapshot_fw.dump", "forward")
         except Exception:
             optix_context.release_record(record)
             raise
@@ -158,8 +157,8 @@ def trace_surfels(optix_context, training, start_from_first, ray_o, ray_d, verti
         args = (optix_context, training, start_from_first, ray_o, ray_d, vertices, s.bg, means3D, shs, s.sh_degree,
                 colors_precomp, others_precomp, opacities, scales, s.scale_modifier, rotations,
                 cov3Ds_precomp) + _settings_args(s)
-        optix_context.single_dist = True
-        return _results(*_guarded(_C.trace_surfels, args, s.debug, "snapshot_fw.dump", "forward"), means3D)
+        return _results(*_guarded(lambda *a: _C.trace_surfels(*a, None, None, None, 1), args, s.debug, "snapshot_fw.dump",
+                                  "forward"), means3D)
     return _TraceSurfels.apply(optix_context, training, start_from_first, ray_o, ray_d, vertices, means3D, grads3D,
                                shs, colors_precomp, others_precomp, opacities, scales, rotations, cov3Ds_precomp,
                                tracer_settings)

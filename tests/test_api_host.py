@@ -282,3 +282,25 @@ def test_a_recorded_trace_launches_again(monkeypatch):
     n = len(launches)
     traced(args[6])
     assert len(launches) == n + 1
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_a_failed_call_leaves_nothing_for_the_next_one(monkeypatch, grad):
+    """Everything a forward call is asked for travels with the call: after one that fails before the launcher (here: in
+    the debug mode's snapshot) the context is what it was, and a direct launcher call gets the reference's outputs."""
+    import inspect
+
+    import diff_surfel_tracing as dst
+    from diff_surfel_tracing import _C
+
+    def broken(args):
+        raise OSError("no room for the snapshot")
+    monkeypatch.setattr(dst, "cpu_deep_copy_tuple", broken)
+    args = _call_args()
+    args[6].requires_grad_(grad)
+    args[-1] = args[-1]._replace(debug=True)
+    before = dict(vars(args[0]), record_wanted=grad, acquired=int(grad), released=int(grad))
+    with pytest.raises(OSError):
+        dst.trace_surfels(*args)
+    assert vars(args[0]) == before
+    assert inspect.signature(_C.trace_surfels).parameters["dist_channels"].default == 3
