@@ -100,8 +100,10 @@ class _TraceSurfels(torch.autograd.Function):
         ctx.tracer_settings = s
         ctx.optix_context = optix_context
         ctx.start_from_first = start_from_first
+        # (the backward trace takes the distortion's memory and reads nothing of it: the caller may change what it was
+        # returned in place, so what is saved does not share its version)
         ctx.save_for_backward(ray_o, ray_d, vertices, means3D, shs, colors_precomp, others_precomp, opacities, scales,
-                              rotations, cov3Ds_precomp, out_rgb, out_dpt, out_acc, out_norm, out_dist, out_aux,
+                              rotations, cov3Ds_precomp, out_rgb, out_dpt, out_acc, out_norm, out_dist.data, out_aux,
                               mid_val)
         return _results(out_rgb, out_dpt, out_acc, out_norm, out_dist, out_aux, mid_val, a_weights, means3D)
 

@@ -304,3 +304,23 @@ def test_a_failed_call_leaves_nothing_for_the_next_one(monkeypatch, grad):
         dst.trace_surfels(*args)
     assert vars(args[0]) == before
     assert inspect.signature(_C.trace_surfels).parameters["dist_channels"].default == 3
+
+
+def test_the_returned_dist_may_be_changed_in_place(monkeypatch):
+    """No gradient flows from it and the backward trace does not read it."""
+    import diff_surfel_tracing as dst
+    from diff_surfel_tracing import _C
+    P = 5
+
+    def backward(ctx, *a, **k):
+        z = lambda *s: torch.zeros(*s)  # noqa: E731
+        return (z(4, 4, 3), z(4, 4, 3), torch.full((P, 3), 2.0), z(P, 3), None, z(P, 16, 3), None, None, z(P, 1), z(P, 2), z(P, 4),
+                None)
+    monkeypatch.setattr(_C, "trace_surfels", _fake_launcher)
+    monkeypatch.setattr(_C, "trace_surfels_backward", backward)
+    args = _call_args(P)
+    args[6].requires_grad_(True)
+    out = dst.trace_surfels(*args)
+    out[4].mul_(3.0)
+    out[0].sum().backward()
+    assert torch.equal(args[6].grad, torch.full((P, 3), 2.0))
