@@ -5,6 +5,7 @@
 """
 import ctypes as C
 import os
+import threading
 import warnings
 
 import torch
@@ -269,6 +270,7 @@ class OptiXStateWrapper:
         self._record_fixed = False          # True: only caller-provided storage is used, nothing is allocated
         self._record_watch = []             # records whose request count has not been read yet
         self._row_pool = []                 # (rows, marks, stream, event): per-surfel sums of backward calls, all zero
+        self.row_pool_max_bytes = 8 << 30   # of them kept for reuse; 2M surfels, aux 4: 0.55 GB a pair, deterministic 1.1
 
     # ---- hit-record storage ---------------------------------------------------------------------------
     def use_record_storage(self, storage):
@@ -358,36 +360,51 @@ class OptiXStateWrapper:
 
     # ---- per-surfel sums of the backward traces -------------------------------------------------------
     ROW_POOL_SIZE = 2
+    _pool_lock = threading.Lock()   # of all contexts: held for a few list operations, and nothing waits inside
 
     def acquire_rows(self, P, words, dtype, device):
         """A zeroed buffer of at least `words` sums and one of at least P marks (DstParams.grad_touched).  The closing
         kernel of a backward trace leaves both zero, so they are filled once, not per call; at most ROW_POOL_SIZE pairs
-        are kept, with the context."""
+        and `row_pool_max_bytes` are kept between calls.  A pair that this call's scene or mode has no use for is let
+        go: the one made in its place is kept."""
+        found, now = None, _current_stream()
         if not torch.cuda.is_current_stream_capturing():   # (a captured fill has not run yet)
-            for _ in range(self.ROW_POOL_SIZE):
-                try:   # taken out first: another thread may be looking too
-                    rows, marks, stream, event = self._row_pool.pop(0)
-                except IndexError:
-                    break
-                if rows.dtype != dtype or rows.numel() < words or marks.numel() < P or rows.device != device:
-                    self._row_pool.append((rows, marks, stream, event))
-                    continue
-                now = _current_stream()
-                if stream is not now:   # its last user may still be running there, and when the pair is dropped, this one
-                    now.wait_event(event)
-                    rows.record_stream(now)
-                    marks.record_stream(now)
-                return rows, marks
-        return (torch.zeros(words, dtype=dtype, device=device), torch.zeros(P, dtype=torch.uint8, device=device))
+            with self._pool_lock:
+                fits = [p for p in self._row_pool if p[0].dtype == dtype and p[0].numel() >= words and
+                        p[1].numel() >= P and p[0].device == device]
+                found = next((p for p in fits if p[2] is now), fits[0] if fits else None)   # (nothing to wait for)
+                self._row_pool = [p for p in fits if p is not found]
+        if found is None:
+            return torch.zeros(words, dtype=dtype, device=device), torch.zeros(P, dtype=torch.uint8, device=device)
+        rows, marks, stream, event = found
+        if stream is not now:   # its last user may still be running there, and when the pair is dropped, this one
+            now.wait_event(event)
+            rows.record_stream(now)
+            marks.record_stream(now)
+        return rows, marks
 
     def release_rows(self, rows, marks):
         """Back to the pool, behind a backward trace that has been launched (after a failed call they are dropped)."""
-        if torch.cuda.is_current_stream_capturing():
+        size = rows.numel() * rows.element_size() + marks.numel()
+        if torch.cuda.is_current_stream_capturing() or size > self.row_pool_max_bytes:
             return
         stream, event = _current_stream(), torch.cuda.Event()
         event.record(stream)
-        self._row_pool.insert(0, (rows, marks, stream, event))
-        del self._row_pool[self.ROW_POOL_SIZE:]
+        with self._pool_lock:
+            kept = [(rows, marks, stream, event)]
+            for p in self._row_pool[:self.ROW_POOL_SIZE - 1]:
+                size += p[0].numel() * p[0].element_size() + p[1].numel()
+                if size <= self.row_pool_max_bytes:
+                    kept.append(p)
+            self._row_pool = kept
+
+    def release_memory(self):
+        """Give back what is kept between calls for reuse (hit records, rows of gradient sums; not a caller's own record
+        storage).  The next training step allocates again."""
+        with self._pool_lock:
+            self._row_pool = []
+        if not self._record_fixed:
+            self._record_pool, self._record_events = [], {}
 
     def accel_info(self):
         info = DstAccelInfo()

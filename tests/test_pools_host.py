@@ -61,7 +61,7 @@ def _context():
     ctx.handle = None
     ctx._row_pool, ctx._record_pool, ctx._record_fixed, ctx._record_events, ctx._record_watch = [], [], False, {}, []
     ctx.record_blocks_per_wave, ctx.deterministic, ctx.records_skipped = 4.0, False, 0
-    ctx.record_max_bytes, ctx.record_pool_max_bytes = 1 << 40, 1 << 40
+    ctx.record_max_bytes, ctx.record_pool_max_bytes, ctx.row_pool_max_bytes = 1 << 40, 1 << 40, 1 << 40
     return ctx
 
 
@@ -107,3 +107,35 @@ def test_hit_records_tell_the_allocator_of_every_stream_they_serve(device, monke
     device.now = c                              # a backward trace on a stream of its own
     ctx.release_record(rec)
     assert c in storage.users
+
+
+def _held(ctx):
+    return sum(r.n * r.element_size() + m.n for r, m, _, _ in ctx._row_pool)
+
+
+def test_gradient_rows_kept_between_calls_are_bounded_and_given_back(device):
+    ctx = _context()
+    pairs = [ctx.acquire_rows(10, 660, torch.float32, "cuda:0") for _ in range(3)]
+    assert len({id(p[0]) for p in pairs}) == 3
+    one = 4 * 660 + 10
+    for p in pairs:
+        ctx.release_rows(*p)
+    assert _held(ctx) == 2 * one                       # ROW_POOL_SIZE pairs
+    ctx.row_pool_max_bytes = 2 * one - 1
+    ctx.release_rows(*ctx.acquire_rows(10, 660, torch.float32, "cuda:0"))
+    assert _held(ctx) == one                           # and a limit in bytes
+    # the mode changed, or the scene grew: what no longer fits is not held beside what does
+    det = ctx.acquire_rows(10, 660, torch.int64, "cuda:0")
+    assert _held(ctx) == 0
+    ctx.row_pool_max_bytes = 8 * 660
+    ctx.release_rows(*det)
+    assert _held(ctx) == 0                             # 8 * 660 + 10: more than the limit, not kept at all
+    ctx.row_pool_max_bytes = 1 << 30
+    ctx.release_rows(*ctx.acquire_rows(10, 660, torch.int64, "cuda:0"))
+    grown = ctx.acquire_rows(20, 1320, torch.int64, "cuda:0")
+    assert _held(ctx) == 0
+    ctx.release_rows(*grown)
+    assert ctx.acquire_rows(10, 660, torch.int64, "cuda:0")[0] is grown[0]   # larger than needed: serves
+    ctx.release_rows(*grown)
+    ctx.release_memory()
+    assert _held(ctx) == 0
