@@ -240,6 +240,8 @@ class OptiXStateWrapper:
     fails, is not made and the backward pass walks the BVH again (`records_skipped` counts those calls, the first
     one warns)."""
 
+    _pool_lock = threading.Lock()   # of the pools of all contexts: held for a few list operations, and nothing waits inside
+
     RECORD_POOL_SIZE = 4
     RECORD_FIRST_BLOCKS = 5.0   # blocks per wave and bounce before a forward trace has said what it needs
     RECORD_HEADROOM = 1.08      # a record is sized this much above the largest request seen so far
@@ -316,13 +318,13 @@ class OptiXStateWrapper:
         device = torch.device(device)
         if device.index is None:
             device = torch.device(device.type, torch.cuda.current_device())
-        fit = [t for t in self._record_pool if t.numel() >= words and t.device == device]
-        storage = None
-        if fit:
-            storage = min(fit, key=lambda t: t.numel())
+        with self._pool_lock:
+            fit = [t for t in self._record_pool if t.numel() >= words and t.device == device]
+            storage = min(fit, key=lambda t: t.numel()) if fit else None
             self._record_pool = [t for t in self._record_pool if t is not storage]
-            # the backward trace that last read this storage may still be running on another stream
             done = self._record_events.pop(id(storage), None)
+        if storage is not None:
+            # the backward trace that last read this storage may still be running on another stream
             if done is not None:
                 now = _current_stream()
                 now.wait_event(done)
@@ -342,25 +344,25 @@ class OptiXStateWrapper:
         marked with an event that the next user waits for, whatever stream that user runs on."""
         if rec is None or rec.words is None:
             return
-        if rec.words.is_cuda:
+        words, rec.words = rec.words, None
+        done = None
+        if words.is_cuda:
             done, now = torch.cuda.Event(), _current_stream()
             done.record(now)
-            rec.words.record_stream(now)
-            self._record_events[id(rec.words)] = done
-        self._record_pool.append(rec.words)
-        rec.words = None
-        if self._record_fixed:
-            return
-        # by identity: list.remove() would compare tensors element-wise
-        while len(self._record_pool) > 1 and (len(self._record_pool) > self.RECORD_POOL_SIZE or
-                                              8 * sum(t.numel() for t in self._record_pool) > self.record_pool_max_bytes):
-            smallest = min(self._record_pool, key=lambda t: t.numel())
-            self._record_pool = [t for t in self._record_pool if t is not smallest]
-            self._record_events.pop(id(smallest), None)
+            words.record_stream(now)
+        with self._pool_lock:
+            pool = self._record_pool + [words]
+            if done is not None:
+                self._record_events[id(words)] = done
+            while not self._record_fixed and len(pool) > 1 and (
+                    len(pool) > self.RECORD_POOL_SIZE or 8 * sum(t.numel() for t in pool) > self.record_pool_max_bytes):
+                smallest = min(pool, key=lambda t: t.numel())
+                pool = [t for t in pool if t is not smallest]   # (list.remove() would compare tensors element-wise)
+                self._record_events.pop(id(smallest), None)
+            self._record_pool = pool
 
     # ---- per-surfel sums of the backward traces -------------------------------------------------------
     ROW_POOL_SIZE = 2
-    _pool_lock = threading.Lock()   # of all contexts: held for a few list operations, and nothing waits inside
 
     def acquire_rows(self, P, words, dtype, device):
         """A zeroed buffer of at least `words` sums and one of at least P marks (DstParams.grad_touched).  The closing
@@ -403,8 +405,8 @@ class OptiXStateWrapper:
         storage).  The next training step allocates again."""
         with self._pool_lock:
             self._row_pool = []
-        if not self._record_fixed:
-            self._record_pool, self._record_events = [], {}
+            if not self._record_fixed:
+                self._record_pool, self._record_events = [], {}
 
     def accel_info(self):
         info = DstAccelInfo()

@@ -139,3 +139,43 @@ def test_gradient_rows_kept_between_calls_are_bounded_and_given_back(device):
     ctx.release_rows(*grown)
     ctx.release_memory()
     assert _held(ctx) == 0
+
+
+def test_threads_never_share_a_buffer(device, monkeypatch):
+    """Several threads that draw from one context's pools and give back: nobody holds what somebody else holds."""
+    import sys
+    import threading
+    monkeypatch.setattr(_C, "HitRecord", _Record)
+    ctx = _context()
+    held, clashes, guard = set(), [], threading.Lock()
+
+    def hold(*buffers):
+        with guard:
+            clashes.extend(b for b in buffers if id(b) in held)
+            held.update(id(b) for b in buffers)
+
+    def let_go(*buffers):
+        with guard:
+            held.difference_update(id(b) for b in buffers)
+
+    def work():
+        for _ in range(3000):
+            rows, marks = ctx.acquire_rows(4, 264, torch.float32, torch.device("cuda", 0))
+            rec = ctx.acquire_record(8, 8, 1, torch.device("cuda", 0))
+            words = rec.words
+            hold(rows, marks, words)
+            let_go(rows, marks, words)
+            ctx.release_rows(rows, marks)
+            ctx.release_record(rec)
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1e-6)
+    try:
+        threads = [threading.Thread(target=work) for _ in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        sys.setswitchinterval(interval)
+    assert not clashes
+    assert len(ctx._record_pool) <= ctx.RECORD_POOL_SIZE and len(ctx._record_events) <= ctx.RECORD_POOL_SIZE
