@@ -1,0 +1,76 @@
+"""Images large enough to be traced by tiles, whose reflections are traced ray by ray (k_row_fwd<BEYOND>), against the
+oracle: per-ray outputs bit-identical, gradients within the usual bar.  The oracle follows a window of the image; upstream
+gradients are zero outside of it, so that the per-surfel sums are the window's alone."""
+import numpy as np
+import pytest
+import torch
+
+import dst_scenes as S
+from helpers import GRAD_REL, assert_forward_exact, assert_gradients, gpu_trace, oracle_scene, upstream
+
+pytestmark = pytest.mark.gpu
+H, W = 152, 176          # 418 waves: above the sizes that are traced ray by ray from the start
+
+
+def window_reference(oracle, sc, o, d, aux, rows, cols, **kw):
+    ug = upstream(o.shape[0], o.shape[1], aux)
+    inside = torch.zeros(o.shape[0], o.shape[1], 1)
+    inside[rows, cols] = 1.0
+    ug = {k: v * inside for k, v in ug.items()}
+    s = oracle_scene(oracle, sc, o[rows, cols].contiguous(), d[rows, cols].contiguous(), **kw)
+    ref = oracle.forward(s, oracle.HITS_BVH_LEXI)
+    ugn = {k: v[rows, cols].contiguous().numpy() for k, v in ug.items()}
+    return ug, ref, oracle.backward(s, ref, ugn, oracle.HITS_BVH_LEXI), oracle.backward(s, ref, ugn, oracle.HITS_BVH_LEXI, noise=True)
+
+
+def check_window(out, g, ref, refg, refg64, rows, cols, tag):
+    assert_forward_exact({k: v[rows, cols] for k, v in out.items() if k != "wet"}, ref)
+    got = dict(g)
+    for k in ("ray_o", "ray_d"):
+        got[k] = g[k][rows, cols]
+    assert_gradients(got, refg, refg64, GRAD_REL, tag)
+
+
+def translucent_corridor(n=720, seed=5):
+    """A mirror in front of the camera and, behind the camera, a stack of quads as wide as the view: seven in ten too
+    faint to count at all, the others a per cent or two.  A reflected ray meets them all."""
+    gen = torch.Generator().manual_seed(seed)
+    x = torch.cat([torch.tensor([4.0]), -1.0 - 6.0 * torch.rand(n, generator=gen)])
+    means = torch.stack([x, 0.2 * torch.randn(n + 1, generator=gen), 0.2 * torch.randn(n + 1, generator=gen)], dim=-1)
+    scales = torch.full((n + 1, 2), 1.6)
+    nn = torch.tensor([1.0, 0.0, 0.0]) + torch.cat([torch.zeros(1, 3), 0.05 * torch.randn(n, 3, generator=gen)])
+    nn = torch.nn.functional.normalize(nn, dim=-1)
+    rotations = torch.stack([1 + nn[:, 2], -nn[:, 1], nn[:, 0], torch.zeros(n + 1)], dim=-1)   # z into the normal
+    rotations = torch.nn.functional.normalize(rotations, dim=-1)
+    faint = torch.rand(n + 1, generator=gen) < 0.7
+    opacities = torch.where(faint, torch.full((n + 1,), 0.003), 0.01 + 0.01 * torch.rand(n + 1, generator=gen))
+    opacities[0] = 0.999
+    others = 0.1 * torch.rand(n + 1, 2, generator=gen)
+    others[0, 0] = 0.9
+    sc = {"means3D": means, "scales": scales, "rotations": rotations.contiguous(), "opacities": opacities[:, None].contiguous(),
+          "shs": 0.3 * torch.randn(n + 1, 16, 3, generator=gen), "others_precomp": others}
+    sc["vertices"], sc["faces"] = S.get_triangles(sc["means3D"], sc["scales"], sc["rotations"])
+    return sc
+
+
+def test_a_long_way_through_translucent_surfels_is_recorded(oracle):
+    """Some fifty chunks of sixteen entries behind the mirror: the record of the second step has room for them all, is
+    complete, and stays the size it is; replay and re-trace both give the oracle's gradients."""
+    import diff_surfel_tracing as dst
+    sc = translucent_corridor()
+    o, d = S.pinhole_rays(H, W, 40.0, (0.0, 0.0, 0.0), (1.0, 0.0, 0.0))
+    rows, cols = slice(60, 76), slice(70, 94)
+    kw = dict(max_trace_depth=1, specular_threshold=0.4)
+    ug, ref, refg, refg64 = window_reference(oracle, sc, o, d, 2, rows, cols, **kw)
+    assert ref["n_proc"].max() > 16 * 40 and ref["n_con"].mean() > 100
+    tracer = dst.SurfelTracer()
+    ctx = tracer.optix_context
+    sizes = []
+    for step in range(4):
+        out, g = gpu_trace(tracer, sc, o, d, upstream=ug, build=(step == 0), **kw)
+        rec = ctx._record_watch[-1]
+        sizes.append(rec.blocks)
+        assert rec.complete() == (step > 0), (step, rec.requested_blocks(), rec.blocks)
+        assert rec.requested_blocks() > 40 * rec.n_waves / 2
+        check_window(out, g, ref, refg, refg64, rows, cols, "step %d " % step)
+    assert sizes[1] == sizes[2] == sizes[3]
