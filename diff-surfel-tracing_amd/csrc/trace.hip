@@ -1325,10 +1325,17 @@ __device__ __forceinline__ void hit_backward(const const_params p, const BounceI
 constexpr uint32_t kRecDirBlockBits = 26, kRecDirBlockMask = (1u << kRecDirBlockBits) - 1u;
 constexpr uint32_t kRecColourWord = kChunk * DST_WAVE + DST_WAVE / 2 + 8;   // first word of the colours
 constexpr uint32_t kRecBlockWords = kRecColourWord + kChunk * 3 * DST_WAVE / 2;
+// Are images of this many rays small enough to be traced ray by ray?  (Ray lists, th_log2 < 3, always may be.)
+#ifndef DST_ROW_MAX_WAVES
+#define DST_ROW_MAX_WAVES 400
+#endif
+__host__ __device__ static inline bool rows_may_trace(uint64_t rays, int th_log2) {
+    return th_log2 < 3 || (rays + 63u) / 64u <= DST_ROW_MAX_WAVES;
+}
 // Words in front of the first block: the three of the header and the directory, of the wave layout (one entry per wave and
-// bounce slot) or of the row layout (one per ray and slot, row.inc), whichever is longer.
-__host__ __device__ static inline uint64_t record_header_words(uint64_t rays, uint32_t slots, uint64_t waves) {
-    const uint64_t entries = (rays > waves ? rays : waves) * slots;
+// bounce slot) or, on grids that may be traced ray by ray, of the row layout (one per ray and slot, row.inc) if it is longer.
+__host__ __device__ static inline uint64_t record_header_words(uint64_t rays, int th_log2, uint32_t slots, uint64_t waves) {
+    const uint64_t entries = (rows_may_trace(rays, th_log2) && rays > waves ? rays : waves) * slots;
     return 3u + ((entries + 1u) / 2u + 1u) / 2u * 2u + 1u;   // even: blocks start on 16-byte boundaries where the record does
 }
 struct RecView {
@@ -1892,7 +1899,7 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
         const uint32_t n_waves = btiles_x * ((tiles_y + 1u) / 2u) * kWavesPerBlock, slots_ = (uint32_t)p.mtd_alloc + 1u;
         rv.base = p.hit_record;
         rv.dir = reinterpret_cast<uint32_t *>(p.hit_record + 3) + (size_t)((by * btiles_x + bx) * kWavesPerBlock + wv) * slots_;
-        rv.blocks = p.hit_record + record_header_words((uint64_t)p.H * p.W, slots_, n_waves);
+        rv.blocks = p.hit_record + record_header_words((uint64_t)p.H * p.W, th_log2, slots_, n_waves);
         rv.capacity = p.hit_record_blocks;
     }
     const uint32_t ty = flat ? 0u : 2u * by + (wv >> 1), tx = flat ? 4u * bx + wv : 2u * bx + (wv & 1u);
@@ -2381,14 +2388,11 @@ void launch(const DstParams &p, const DstAccelView &acc, const TileGrid &t, cons
 // How the rays of this grid are traced.  Tiles: a wave per 64 rays.  Rows (sixteen lanes per ray): lists, whose rays
 // are unrelated, and images so small that waves of 64 rays leave most of the chip idle.  TilesThenRows: images with
 // reflections - the primary rays as tiles, the bounces beyond as rows.
-#ifndef DST_ROW_MAX_WAVES
-#define DST_ROW_MAX_WAVES 400
-#endif
 enum class TraceBy { Tiles, Rows, TilesThenRows };
 TraceBy row_grid(const DstParams &p, const TileGrid &t, RowGrid &g) {
-    const uint64_t rays = (uint64_t)p.H * p.W, waves = (rays + 63u) / 64u;
-    g.record_header = record_header_words(rays, (uint32_t)p.mtd_alloc + 1u, (uint64_t)t.btiles_x * t.btiles_y * kWavesPerBlock);
-    if (t.th_log2 == 3 && waves > DST_ROW_MAX_WAVES) {
+    const uint64_t rays = (uint64_t)p.H * p.W;
+    g.record_header = record_header_words(rays, t.th_log2, (uint32_t)p.mtd_alloc + 1u, (uint64_t)t.btiles_x * t.btiles_y * kWavesPerBlock);
+    if (!rows_may_trace(rays, t.th_log2)) {
         g.batch_log2 = 4u;
         g.side_log2 = 3u;
         g.tiles_x = t.btiles_x;
@@ -2476,7 +2480,7 @@ uint64_t dst_hit_record_layout(int32_t H, int32_t W, int32_t mtd_alloc, uint32_t
     }
     const TileGrid t = tile_grid(H, W);
     const uint64_t waves = (uint64_t)t.btiles_x * t.btiles_y * kWavesPerBlock;
-    const uint64_t header = record_header_words((uint64_t)H * W, (uint32_t)mtd_alloc + 1u, waves);
+    const uint64_t header = record_header_words((uint64_t)H * W, t.th_log2, (uint32_t)mtd_alloc + 1u, waves);
     if (header_words) *header_words = header;
     if (n_waves) *n_waves = (uint32_t)waves;
     return header + (uint64_t)blocks * kRecBlockWords;

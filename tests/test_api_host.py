@@ -324,3 +324,13 @@ def test_the_returned_dist_may_be_changed_in_place(monkeypatch):
     out[4].mul_(3.0)
     out[0].sum().backward()
     assert torch.equal(args[6].grad, torch.full((P, 3), 2.0))
+
+
+@pytest.mark.parametrize("H,W", [(1080, 1920), (2160, 3840), (152, 176)])
+def test_record_headers_hold_the_directory_in_use(binding, H, W):
+    """Images above 25,600 rays are recorded by waves of 64 rays: their directory has an entry per wave and slot, and no
+    room for one per ray, which every training step would clear.  Smaller images and lists may be recorded ray by ray."""
+    words, header, _, waves = binding.HitRecord.layout(H, W, 1, 4.0)
+    assert header <= 4 + waves + 2 and words > header
+    assert binding.HitRecord.layout(160, 160, 1, 4.0)[1] >= 3 + 160 * 160
+    assert binding.HitRecord.layout(1, 131072, 1, 4.0)[1] >= 3 + 131072
