@@ -74,3 +74,44 @@ def test_a_long_way_through_translucent_surfels_is_recorded(oracle):
         assert rec.requested_blocks() > 40 * rec.n_waves / 2
         check_window(out, g, ref, refg, refg64, rows, cols, "step %d " % step)
     assert sizes[1] == sizes[2] == sizes[3]
+
+
+@pytest.mark.parametrize("depth,aux,mode", [(1, 2, "plain"), (1, 4, "det"), (2, 8, "norec"), (3, 2, "plain"), (3, 4, "colors"),
+                                            (1, 3, "colors_det"), (2, 2, "half"), (1, 8, "distortion"), (3, 8, "det"),
+                                            (2, 4, "norows")])
+def test_reflections_of_images_traced_by_tiles(oracle, depth, aux, mode):
+    import diff_surfel_tracing as dst
+    from test_gpu_parity import check_case
+    sc = S.scene_room(P=12000, seed=depth + aux, aux=aux, half=1.5)
+    sc["others_precomp"][:, 0] = sc["others_precomp"][:, 0] * 0.8 + 0.1    # the reference divides by the specular
+    if mode.startswith("colors"):
+        sc["colors_precomp"] = torch.rand(12000, 3, generator=torch.Generator().manual_seed(3))
+        del sc["shs"]
+    o, d = S.pinhole_rays(H, W, 70.0, (-0.6, -0.3, 0.15), (0.9, 0.45, -0.15))
+    kw = dict(max_trace_depth=depth, specular_threshold=0.0 if depth == 3 else 0.1, bg=(0.3, 0.1, 0.2))
+    tracer = dst.SurfelTracer()
+    ctx = tracer.optix_context
+    tracer.deterministic = mode.endswith("det")
+    seen, call = sc, tracer
+    if mode == "half":
+        from test_gpu_tiles import _HalfSeen
+        tracer.sh_half = True
+        seen, call = dict(sc, shs=sc["shs"].half().float()), _HalfSeen(tracer, sc["shs"])
+    elif mode == "norec":
+        ctx.record_max_bytes = 0
+    elif mode == "norows":
+        ctx.gradient_rows = False
+    if mode == "distortion":
+        tracer.distortion = True
+        out, _ = gpu_trace(tracer, sc, o, d, **kw)
+        ref = oracle.forward(oracle_scene(oracle, sc, o, d, **kw), oracle.HITS_BVH_LEXI, compute_dist=True)
+        np.testing.assert_array_equal(out["dist"].view(np.uint32), ref["dist"][..., :1].view(np.uint32))
+        assert out["dist"].max() > 1e-6
+        tracer.distortion = False
+    runs = [check_case(oracle, call, seen, o, d, **kw) for _ in range(3 if tracer.deterministic else 2)]
+    assert mode == "norec" or ctx._record_watch[-1].complete()
+    assert (runs[0][0]["mid"][..., (14 + aux) * depth + 3:(14 + aux) * depth + 6] != 0).any()    # the last bounce is reached
+    if tracer.deterministic:
+        for k, v in runs[1][0]["grads_gpu"].items():
+            assert v is None or np.array_equal(v.view(np.uint32), runs[2][0]["grads_gpu"][k].view(np.uint32)), k
+        assert np.array_equal(runs[0][1]["wet"], runs[1][1]["wet"])

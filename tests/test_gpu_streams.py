@@ -1,0 +1,55 @@
+"""Training steps of one context on two streams in turn, without the host waiting in between: the buffers kept between
+calls (records, rows of gradient sums and marks) go from stream to stream, grow with the scene and change with the
+mode, and every step's gradients are those of the step on its own."""
+import pytest
+import torch
+
+import dst_scenes as S
+from helpers import GRAD_REL, PARAM_NAMES, assert_same_sums, settings
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def step(tracer, st, g, o, d, ug, leaf):
+    out = tracer(o, d, g["vertices"], leaf["means3D"], torch.zeros_like(leaf["means3D"]), shs=leaf["shs"],
+                 others_precomp=leaf["others_precomp"], opacities=leaf["opacities"], scales=leaf["scales"],
+                 rotations=leaf["rotations"], tracer_settings=st)
+    names = [k for k in PARAM_NAMES if k in leaf]
+    losses = [out[0], out[1], out[2], out[3], out[5]]
+    return dict(zip(names, torch.autograd.grad(losses, [leaf[k] for k in names], [ug[k] for k in ("rgb", "dpt", "acc", "norm", "aux")])))
+
+
+@pytest.mark.parametrize("size", [(48, 64), (152, 176)])
+def test_two_streams_in_turn(size):
+    import diff_surfel_tracing as dst
+    H, W = size
+    tracer = dst.SurfelTracer()
+    st = settings(dst, H, W, DEV)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    views = [tuple(t.to(DEV) for t in S.rays_cube(H, W, view=v)) for v in range(4)]
+    ups = [{k: t.to(DEV) for k, t in S.upstream_grads(H, W, 2, seed=v).items()} for v in range(4)]
+    for P in (3000, 7000, 16000):                    # each scene needs larger rows than the one before
+        g = {k: v.to(DEV) for k, v in S.scene_cube(P=P, seed=P, aux=2).items()}
+        tracer.build_acceleration_structure(g["vertices"], g["faces"], True)
+        leaf = {k: g[k].clone().requires_grad_(True) for k in PARAM_NAMES if k in g}
+        fresh = dst.SurfelTracer()
+        fresh.build_acceleration_structure(g["vertices"], g["faces"], True)
+        want = [step(fresh, st, g, *views[v], ups[v], leaf) for v in range(4)]
+        torch.cuda.synchronize()
+        for det in (False, True, False):
+            tracer.deterministic = det
+            tracer.optix_context.deterministic_check = False     # (it waits)
+            got, noise = [], []
+            for v in range(4):
+                with torch.cuda.stream(streams[v % 2]):
+                    got.append(step(tracer, st, g, *views[v], ups[v], leaf))
+                    # what the allocator has free on either stream is taken and written over at once
+                    noise.append([torch.full((n,), 7.0, device=DEV) for n in (P * 66, P, P // 4)])
+            torch.cuda.synchronize()
+            for v in range(4):
+                for k in want[v]:
+                    assert_same_sums(got[v][k].cpu().numpy(), want[v][k].cpu().numpy(), GRAD_REL, "view %d %s" % (v, k))
+            del noise
+    tracer.optix_context.release_memory()
+    assert not tracer.optix_context._row_pool and not tracer.optix_context._record_pool

@@ -1,0 +1,108 @@
+"""Images traced by tiles of 8x8 rays (the bundle walk) without the tile hand-over, against the oracle: the degenerate
+scenes of the random sweep, whose own images are small enough to be traced ray by ray, and the options of the forward
+trace.  152 x 176 rays are 418 tiles; HANDOVER_OFF keeps the walk whatever the scene holds."""
+import warnings
+
+import numpy as np
+import pytest
+import torch
+
+import dst_scenes as S
+import helpers
+from helpers import assert_forward_exact, gpu_trace, oracle_scene
+from test_gpu_parity import _with_scales, check_case
+from test_gpu_sweep import TRAITS, _apply_trait
+
+pytestmark = pytest.mark.gpu
+H, W = 152, 176
+
+
+def tile_tracer(**options):
+    import diff_surfel_tracing as dst
+    from diff_surfel_tracing import _C
+    t = dst.SurfelTracer()
+    t.optix_context.set_handover(_C.HANDOVER_OFF)
+    for k, v in options.items():
+        setattr(t, k, v)
+    return t
+
+
+def view(kind):
+    if kind == "room":
+        return S.pinhole_rays(H, W, 70.0, (-0.6, -0.3, 0.15), (0.9, 0.45, -0.15))
+    if kind == "lidar":
+        return S.pinhole_rays(H, W, 80.0, (0.0, 0.0, 1.8), (30.0, 10.0, 0.0))
+    return S.rays_cube(H, W, view=1)
+
+
+@pytest.mark.parametrize("fine", [False, True])
+@pytest.mark.parametrize("trait", sorted(set(TRAITS)))
+def test_degenerate_scenes(oracle, monkeypatch, trait, fine):
+    """As in the sweep: its shares of elements that may lean on the rounding allowance."""
+    seed = 100 * sorted(set(TRAITS)).index(trait) + 7 * fine
+    kind = ("cube", "room", "lidar")[seed % 3]
+    P = 300 if trait == "samepoint" else 4000
+    sc = {"cube": lambda: S.scene_cube(P=P, seed=seed, aux=2), "room": lambda: S.scene_room(P=P, seed=seed, aux=4, half=1.5),
+          "lidar": lambda: S.scene_lidar(P=P, seed=seed, aux=0)}[kind]()
+    if fine:
+        sc = _with_scales(sc, 1.0 / 30.0)
+    sc = {k: v.clone() for k, v in sc.items()}
+    move, zoom = _apply_trait(sc, trait, torch.Generator().manual_seed(seed + 77))
+    o, d = view(kind)
+    o = (o * zoom + (0.0 if move is None else move)).contiguous()
+    monkeypatch.setattr(helpers, "MAX_LOUD", 1.0)
+    monkeypatch.setattr(helpers, "MAX_NOISY", 2e-2)
+    monkeypatch.setattr(helpers, "MIN_NOISY", 8)
+    tracer = tile_tracer()
+    check_case(oracle, tracer, sc, o, d, bg=(0.1, 0.3, 0.2), start_from_first=not fine)
+    info = tracer.optix_context.trace_info()
+    assert info.handover_active == 0 and info.tiles_handed_over == 0
+
+
+@pytest.mark.parametrize("aux,colors,sh", [(0, False, 1), (2, True, 3), (3, False, 0), (8, False, 3)])
+def test_deterministic_mode(oracle, aux, colors, sh):
+    """Fixed-point sums: the oracle's gradients, and the same bits on every run (after the first, which sizes the
+    record)."""
+    sc = S.scene_room(P=9000, seed=aux, aux=aux, half=1.5)
+    if colors:
+        sc["colors_precomp"] = torch.rand(9000, 3, generator=torch.Generator().manual_seed(3))
+        del sc["shs"]
+    tracer = tile_tracer(deterministic=True)
+    runs = []
+    with warnings.catch_warnings():
+        warnings.simplefilter("error", RuntimeWarning)
+        for _ in range(3):
+            ref, out = check_case(oracle, tracer, sc, *view("room"), **({} if colors else {"sh_degree": sh}))
+            runs.append((out["wet"], ref["grads_gpu"]))
+    for k, v in runs[1][1].items():
+        assert v is None or np.array_equal(v.view(np.uint32), runs[2][1][k].view(np.uint32)), k
+    assert np.array_equal(runs[0][0], runs[1][0]) and np.array_equal(runs[1][0], runs[2][0])
+
+
+@pytest.mark.parametrize("det", [False, True])
+def test_half_coefficients_and_distortion(oracle, det):
+    sc = S.scene_cube(P=8000, seed=4)
+    o, d = view("cube")
+    seen = dict(sc)
+    seen["shs"] = sc["shs"].half().float()               # what the kernels read
+    tracer = tile_tracer(sh_half=True, distortion=True, deterministic=det)
+    out, _ = gpu_trace(tracer, sc, o, d)
+    ref = oracle.forward(oracle_scene(oracle, seen, o, d), oracle.HITS_BVH_LEXI, compute_dist=True)
+    assert_forward_exact({**out, "dist": 0 * out["dist"]}, {**ref, "dist": 0 * ref["dist"]})
+    np.testing.assert_array_equal(out["dist"].view(np.uint32), ref["dist"][..., :1].view(np.uint32))
+    assert out["dist"].max() > 1e-6
+    tracer.distortion = False
+    check_case(oracle, _HalfSeen(tracer, sc["shs"]), seen, o, d)
+
+
+class _HalfSeen:
+    """The tracer, given the fp32 coefficients where the oracle is given their binary16 values."""
+
+    def __init__(self, tracer, shs):
+        self._tracer, self._shs = tracer, shs
+
+    def __getattr__(self, name):
+        return getattr(self._tracer, name)
+
+    def __call__(self, *a, shs=None, **k):
+        return self._tracer(*a, shs=shs + (self._shs.to(shs.device) - shs.detach()), **k)
