@@ -70,23 +70,39 @@ def workloads():
     }
 
 
-def traffic_of(workload, which):
-    """HBM bytes per launch from the committed counter runs (not measured by this run)."""
+def traffic_of(workload, which, kernel):
+    """HBM bytes per call from the committed counter runs (not measured by this run), if those were of the kernels that
+    run now."""
     tpath = os.path.join(ROOT, "profiles", "hbm_traffic.json")
     if os.path.exists(tpath):
         rec = json.load(open(tpath)).get("%s/%s" % (workload, which))
-        if rec:
+        if rec and rec["kernels"] == kernel:
             return rec["bytes_per_launch"]
     return None
 
 
+def kernels_of(H, W, aux, depth, handover):
+    """Names of the kernels that do a step's work with a complete hit record: (forward, backward, backward without a
+    record).  Lists (fewer than eight rows of rays) and images of up to 25,600 rays are traced ray by ray, larger images
+    by tiles of 64 rays, their reflections ray by ray; a context that can hand tiles over traces everything by tiles."""
+    a = 2 if aux <= 2 else (4 if aux <= 4 else 8)
+    lists, mixed = H < 8, "true" if depth > 0 or H < 8 else "false"
+    retrace = "k_trace_bwd<%d,false,%s,false>" % (a, mixed)
+    if handover:
+        return "k_trace_fwd<%d,true,%s,false>" % (a, mixed), "k_trace_bwd<%d,true,false,false> + k_close_gradients<%d,false>" % (a, a), retrace
+    if lists or (H * W + 63) // 64 <= 400:
+        return "k_row_fwd<%d,true,false,false>" % a, "k_row_bwd<%d,false> + k_close_gradients<%d,false>" % (a, a), retrace
+    fwd = "k_trace_fwd_plain<%d,true>" % a + (" + k_row_fwd<%d,true,false,true>" % a if depth > 0 else "")
+    return fwd, "k_trace_bwd<%d,true,false,false> + k_close_gradients<%d,false>" % (a, a), retrace
+
+
 def roofline_of(workload, which, kernel, a_bytes, ms, basis):
     achieved = a_bytes / (ms * 1e-3) / 1e9
-    traffic = traffic_of(workload, which)
+    traffic = traffic_of(workload, which, kernel)
     r = {"bound": "hbm", "kernel": kernel, "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
          "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic,
          # `traffic` is not measured by this run: it is the FETCH_SIZE + WRITE_SIZE figure of the committed
-         # counter runs of the same command (profiles/), which goes stale when the kernels change
+         # counter runs of the same command (profiles/), quoted only for kernels of the same names
          "traffic_source": None if traffic is None else "profiles/hbm_traffic.json (rocprofv3 --pmc runs of this command)",
          "algorithmic_bytes_per_launch": int(a_bytes), "algorithmic_bytes_basis": basis, "avg_launch_ms": round(ms, 4)}
     if traffic is not None:   # what actually crossed the HBM interface, as a share of its peak
@@ -289,21 +305,17 @@ def run_workload(key, steps, warmup, main, args):
                             aux)
     rays_per_s = R / (ms_per_step * 1e-3)
 
-    aux_max = 2 if aux_out <= 2 else (4 if aux_out <= 4 else 8)
-    mixed = "true" if (depth > 0 or H < 8) else "false"   # kernels with the per-lane walk built in
-    # (image grids at depth 0 run the kernels without the tile hand-over unless the scene has many small quads)
-    fwd_name = ("k_trace_fwd_plain<%d,true>" % aux_max if mixed == "false" and not trace_info.handover_active
-                else "k_trace_fwd<%d,true,%s,false>" % (aux_max, mixed))
+    fwd_name, bwd_name, retrace_name = kernels_of(H, W, aux_out, depth, bool(trace_info.handover_active))
     fwd_roof = roofline_of(key, "forward", fwd_name, A_fwd, fwd_ms,
                            "per ray / evaluated entry / composited hit, reference-shaped")
-    bwd_roof = roofline_of(key, "backward", "k_trace_bwd<%d,true,false,false>" % aux_max, A_replay, bwd_ms,
+    bwd_roof = roofline_of(key, "backward", bwd_name, A_replay, bwd_ms,
                            "what the replaying kernel moves by design: record, per-hit geometry, gradient rows")
     # the reference-shaped count (66 atomics and an SH gather per hit) describes the work the kernel stands in for,
     # not bytes it moves: above the HBM peak it is no utilisation figure
     bwd_roof["reference_equivalent"] = {"algorithmic_bytes_per_launch": int(A_bwd),
                                         "GB/s": round(A_bwd / (bwd_ms * 1e-3) / 1e9, 2)}
-    retrace_roof = roofline_of(key, "backward_retrace", "k_trace_bwd<%d,false,%s,false>" % (aux_max, mixed), A_bwd,
-                               bwd_retrace_ms, "per ray / evaluated entry / composited hit, reference-shaped")
+    retrace_roof = roofline_of(key, "backward_retrace", retrace_name, A_bwd, bwd_retrace_ms,
+                               "per ray / evaluated entry / composited hit, reference-shaped")
     per_kernel = {"forward": fwd_roof, "backward": bwd_roof, "backward_retrace": retrace_roof}
 
     result = {
@@ -317,7 +329,7 @@ def run_workload(key, steps, warmup, main, args):
         "hits_evaluated_per_ray": round(n_proc / R, 3), "hits_composited_per_ray": round(n_con / R, 3),
         "hit_record": {"blocks_used": info.get("blocks"), "complete": info.get("complete"),
                        "allocated_bytes": info.get("record_bytes")},
-        # forward tiles whose packet walk ran into the step limit and were traced ray by ray by the second launch
+        # forward tiles whose first walk ran into the step limit and were traced ray by ray by the second launch
         "tile_handover": {"active": bool(trace_info.handover_active), "small_quads": trace_info.small_quads,
                           "step_limit": trace_info.handover_steps, "tiles_per_forward": round(handed, 2)},
         "algorithmic_bytes": int(A_total),

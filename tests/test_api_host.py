@@ -334,3 +334,16 @@ def test_record_headers_hold_the_directory_in_use(binding, H, W):
     assert header <= 4 + waves + 2 and words > header
     assert binding.HitRecord.layout(160, 160, 1, 4.0)[1] >= 3 + 160 * 160
     assert binding.HitRecord.layout(1, 131072, 1, 4.0)[1] >= 3 + 131072
+
+
+def test_bench_quotes_traffic_for_the_kernels_that_run_only():
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("bench", os.path.join(ROOT, "bench.py"))
+    bench = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bench)
+    source = open(os.path.join(ROOT, "diff-surfel-tracing_amd", "csrc", "trace.hip")).read()
+    assert re.search(r"#define DST_ROW_MAX_WAVES 400\b", source)      # kernels_of states the same line
+    for key, grid in (("config3", (1080, 1920, 2, 0)), ("config4", (720, 1280, 8, 2)), ("config5", (1, 131072, 4, 0))):
+        fwd, bwd, _ = bench.kernels_of(*grid, False)
+        assert bench.traffic_of(key, "forward", fwd) and bench.traffic_of(key, "backward", bwd)
+        assert bench.traffic_of(key, "forward", bench.kernels_of(*grid, True)[0]) is None
