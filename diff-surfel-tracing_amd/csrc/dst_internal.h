@@ -101,7 +101,7 @@ struct DstBounds {          // device-resident reduction targets, order-preservi
     uint32_t equal_keys;    // neighbours in Morton order with equal keys, counted while the hierarchy is made
     uint32_t max_depth;     // nodes above the deepest leaf (builds with two-level keys only)
     uint32_t scale;         // raw bits of a float: size of the scene's bulk (set by a build, kept by refits); what ray
-                            // origins are compared with (packets, ray keys) - not a bound on anything
+                            // origins are compared with (rays_run_together, ray keys) - not a bound on anything
     uint32_t small_quads;   // quads with edges below kDstSmallQuad of that size, counted by every build and refit
 };
 // Quads this much smaller than the scene are smaller than a pixel at usual resolutions (a 1080p pixel at half the
@@ -174,7 +174,7 @@ struct dst_ctx {
     uint32_t ray_capacity = 0;
     uint32_t *block_order = nullptr;   // dispatch order of a replaying backward trace (longest blocks first), grow-only
     uint32_t block_order_capacity = 0;
-    // forward traces: tiles whose packet walk ran long, handed over to waves that walk every ray on its own (trace.hip)
+    // forward traces: tiles whose first walk ran long, handed over to waves that walk every ray on its own (trace.hip)
     uint32_t *handover = nullptr;      // device, behind `bounds`: kDstHandoverHeader words + kDstHandoverCap entries, zeroed at creation
     uint32_t handover_steps = kDstHandoverSteps;   // limit of a tile's first walk
     int handover_mode = DST_HANDOVER_AUTO;         // auto: only for scenes with many small quads

@@ -1,10 +1,14 @@
 // Forward trace and backward re-trace kernels.
 //
-// One wavefront (64 lanes) carries an 8x8 tile of rays as a PACKET: the BVH walk is wave-uniform
-// (node and leaf records are fetched once per wave through the scalar path, the traversal stack
-// is two VGPRs indexed by lane), every lane tests its own ray against the shared node / quad,
-// and each lane keeps its own 16-entry nearest-hit buffer in registers.  Replaces the raygen /
-// any-hit programs of the reference (optix_tracer/forward.cu, optix_tracer/backward.cu).
+// Four ways to the sixteen nearest hits of a ray, which all give the same hits bit for bit:
+//   bundle walk (bundle.inc)  images: a wave carries an 8x8 tile of rays; its lanes take boxes, then quads, against
+//                             the planes around the whole tile, and what survives is tested exactly, a ray per lane
+//   row walk (row.inc)        ray lists, small images, reflections: sixteen lanes per ray
+//   per-lane walk             tiles handed over by the bundle walk, and rays that go apart in the kernels that carry
+//                             the hand-over or trace without a record: a ray per lane, each on its own
+//   packet walk               the backward trace without a hit record: a wave goes down with all its rays at once
+// Tiles keep the buffer of a ray in a lane's registers, rows across sixteen lanes; compositing follows chunk by chunk.
+// Replaces the raygen / any-hit programs of the reference (optix_tracer/forward.cu, optix_tracer/backward.cu).
 //
 // Arithmetic that feeds a decision (hit test, hit order, uv, alpha, transmittance, reflection)
 // is plain fp32 evaluated as written: this file is compiled with -ffp-contract=off, rsqrt is
@@ -38,8 +42,10 @@ constexpr int kFwdWavesPerBlock = DST_FWD_WPB;   // 1 or kWavesPerBlock
 #ifndef DST_STRIP_BWD
 #define DST_STRIP_BWD 8
 #endif
-constexpr uint32_t kOrderMinBlocks = 1536;   // replay: blocks are taken longest first on grids of at least two rounds of blocks
-                                             // (768 fit the chip at once; below that the order kernel costs more than it saves)
+constexpr uint32_t kOrderMinBlocks = 1536;   // replay: blocks are taken longest first on grids of at least three rounds of
+                                             // blocks (512 fit the chip at once).  Training steps with / without: 8160 blocks
+                                             // (1080p room) 10.74 / 10.91 ms, 2500 (800x800 sphere) 3.70 / 3.78; at 405 blocks
+                                             // (233x417) no difference beyond the noise, and one kernel less
 constexpr uint32_t kStripMinBlocks = 4096;   // forward: strips only for grids of at least this many blocks (see launch())
 
 __device__ const float SH0 = 0.28209479177387814f;
@@ -581,11 +587,13 @@ constexpr float kPacketDirSpread = DST_PACKET_DIR_SPREAD;   // largest direction
 constexpr float kPacketOrgSpread = DST_PACKET_ORG_SPREAD;   // largest origin difference, relative to the scene extent
 constexpr int kLaneStack = 2 * 64;        // as deep as the packet's two lane-indexed registers
 constexpr uint32_t kWalkDone = 0xFFFFFFFFu;   // not a reference: leaf bit set with an impossible position
-// A real call on purpose: inlined, its register needs would spill the packet walk that nearly every wave takes.
+// A real call on purpose: inlined, its register needs would spill the bundle walk that nearly every wave takes.
 // The walk is a real function, so the compiler cannot see where its pointers lead: say it (global memory, LDS).
 typedef const __attribute__((address_space(1))) float *global_f32;
 typedef const __attribute__((address_space(1))) uint32_t *global_u32;
 #define LD3(p, k) f3((p)[(k)], (p)[(k) + 1], (p)[(k) + 2])
+// (Four waves per SIMD, DST_MIXED_WAVES, spill some hundred registers around this call: 20,000 unrelated rays among
+// small quads take 813 us at four, 791 at three, 734 at two waves.  The row walk takes 290 for the same list.)
 // `shelf`: optional LDS for the first kLaneShelf stack entries of every lane ([entry][lane], conflict-free);
 // deeper entries, or all of them without a shelf, live in private memory.
 constexpr int kLaneShelf = 32;
@@ -718,8 +726,9 @@ __device__ __attribute__((noinline)) void lane_walk(const LaneWalkAccel acc_in, 
 
 #include "bundle.inc"
 
-// Packet or per-lane walk for the rays of this wave?  A packet pays off when the rays run side by side: every
-// live ray is compared with the first live one (origins as given by the caller, not advanced along the ray).
+// One walk for the rays of this wave, or one per lane (kernels that carry both)?  Walking together pays off when the rays
+// run side by side: every live ray is compared with the first live one (origins as given by the caller, not advanced
+// along the ray).
 __device__ __forceinline__ bool rays_run_together(F3 o, F3 d, bool active, float max_abs) {
     const uint64_t live = wave_ballot(active);
     if (live == 0ull) return true;
@@ -788,7 +797,9 @@ __device__ __forceinline__ void aadd(float *p, float v) { unsafeAtomicAdd(p, v);
 // few probes goes straight to global atomics, so the table can never be wrong, only less effective.
 #ifndef DST_TABLE_FLUSH_NUM
 #define DST_TABLE_FLUSH_NUM 3   // the table is emptied between rounds once this many eighths of its rows are in use
-                                // (measured 1..6: a fuller table sends more hits past it, straight to memory)
+                                // (a fuller table sends more hits past it, straight to memory.  Training steps at 1 / 2 / 3
+                                // / 5 eighths: 1080p room 10.69 / 10.66 / 10.74 / 10.85 ms, 800x800 sphere 3.67 / 3.68 /
+                                // 3.70 / 3.66, 233x417 room in fixed point 0.566 / 0.557 / 0.559 / 0.595)
 #endif
 constexpr uint32_t kEmptyKey = 0xFFFFFFFFu;
 constexpr int kMaxProbe = 8;
@@ -803,8 +814,8 @@ constexpr int kStageBytes = kWavesPerBlock * DST_WAVE * 17 * 4;   // the waves' 
 template <int AUXM> struct RowLayout {
     static constexpr int cols = kColAux + AUXM;
     static constexpr int stride = cols | 1;     // 8-byte words of a table row; odd: rows spread over all LDS banks
-    // Rows of the block's table, one more taking what belongs nowhere: what three blocks leave each other of a CU's
-    // 160 KB, which is given out in pieces of 1280 bytes.
+    // Rows of the block's table, one more taking what belongs nowhere: what DST_BWD_WAVES blocks (two: 117 rows with two
+    // auxiliary channels) leave each other of a CU's 160 KB, which is given out in pieces of 1280 bytes.
     static constexpr int rows = ((128 / DST_BWD_WAVES) * 1280 - kStageBytes - 1024) / (8 * stride) - 1;
 };
 
@@ -1414,7 +1425,7 @@ __device__ __forceinline__ void table_clear_keys(uint32_t *keys) {
 
 // One bounce: chunked 16-nearest traversal + front-to-back compositing (reference forward.cu:136-315),
 // and for BWD the per-hit gradients of the re-trace (reference backward.cu:332-655).
-// `first_walk` (forward): 0, or the number of steps the packet walk of the bounce's first chunk may take before the
+// `first_walk` (forward): 0, or the number of steps the bundle walk of the bounce's first chunk may take before the
 // wave gives its tile up (returns true, nothing written yet: see the tile hand-over in trace_body), or kWalkPerLane:
 // every ray of the wave walks on its own whatever the rays look like (the waves that take such tiles over).
 // HAND: kernels without the hand-over do not contain its code at all (first_walk is ignored).
@@ -1441,7 +1452,7 @@ __device__ __forceinline__ bool walk_bounce(const DstParams &p, const DstAccelVi
     KBuf buf;
     LastShHit last_sh = {0, f3(0, 0, 0), false};
     STAT(last_sh.t_alg = 0; last_sh.t_sh = 0;)
-    // kernels built without the per-lane walk (MIXED false) take every wave as a packet
+    // kernels built without the per-lane walk (MIXED false) walk once for every wave
     const bool as_packet = (!MIXED || (REC && BWD)) ? true
                                                     : (HAND && first_walk == kWalkPerLane ? false : rays_run_together(ro, rd, lane_on, max_abs));
     // Forward: one LDS area per wave serves the bundle walk's lists or the per-lane walk's stack shelf (all chunks of a
@@ -1797,10 +1808,11 @@ __global__ __launch_bounds__(1024) void k_block_order(const uint32_t *__restrict
     }
 }
 
-// Tile hand-over (forward).  A packet walk visits what any of its 64 rays needs, one dependent fetch after the other.
-// Over geometry much finer than the ray spacing (a dense cloud of surfels far smaller than a pixel) that is the whole
-// content of the tile's frustum, wanted by one ray at best, and a single wave walks for milliseconds while the chip
-// idles.  So the first walk of a tile may take `hand_arg` steps and no more: a wave that runs into that limit has
+// Tile hand-over (forward).  A bundle walk lists and tests what any of its 64 rays may need, one candidate after the
+// other.  Over geometry much finer than the ray spacing (a dense cloud of surfels far smaller than a pixel) that is the
+// whole content of the tile's frustum, wanted by one ray at best, and a single wave walks for milliseconds while the chip
+// idles (150,000 quads of 2 mm in a ball of 12 cm, 64x64 pixels: 29.9 ms; handed over 2.8).  So the first walk of a tile
+// may take `hand_arg` steps (nodes and candidates) and no more: a wave that runs into that limit has
 // written nothing yet, puts its tile on the context's list and leaves, and a second, small launch right behind
 // (kernels with the per-lane walk, hand_arg = 0: the takers) traces the listed tiles with every ray walking on its
 // own - the same buffer content, so the same results bit for bit.  List: word 0 = tiles listed by this trace, word 1 =
@@ -1858,14 +1870,11 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
         bid = (blockIdx.x >> 5) * 8u + (blockIdx.x & 7u);
         wv = (blockIdx.x >> 3) & 3u;
     }
-    // (Measured slower than the strips below, on the 1080p room scene: a band or whole rows of the image per XCD,
-    // +15 % / +8 % forward - eight distant image regions in flight, eight times more distinct BVH data in the shared
-    // last-level cache - and compact patches of 2x4 to 8x16 blocks per XCD inside super-tiles, +1 % to +13 %.)
     // Image grids are walked in column strips eight blocks wide, row by row inside a strip.  Workgroups go to the
     // eight XCDs in turn, so in a full strip XCD q works its way down column q: the tiles an XCD has in flight are
     // vertical neighbours and meet the same BVH nodes in that XCD's own L2 (row-major order over a 120-block-wide image
-    // gave an XCD blocks eight columns apart: forward 8.5 -> 8.1 ms on the 1080p room scene).  The last strip may be
-    // narrower; its blocks are spread over all XCDs like the others.  The launcher chooses the width (launch()).
+    // gives an XCD blocks eight columns apart).  The last strip may be narrower; its blocks are spread over all XCDs
+    // like the others.  The launcher chooses the width, and has the figures (launch()).
     if (BWD && block_order != nullptr) bid = block_order[bid];   // replay: the longest blocks first (k_block_order)
     uint32_t bx, by;
     static_assert(!HAND || (!BWD && kFwdWavesPerBlock == 1), "tiles are handed over by forward kernels of one wave per workgroup");
@@ -2132,8 +2141,10 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
     }
 }
 
-// The two entry kernels differ only in the occupancy the register allocator is told to aim for: both are
-// bound by the latency of dependent fetches, so waves in flight matter more than a few spilled values.
+// Occupancy the register allocator is told to aim for, waves per SIMD: enough in flight to cover the fetches, few enough
+// for the working set to stay in registers.  1080p room, evaluated, at 2 / 3 / 4 forward waves: 5.09 / 3.81 / 5.23 ms,
+// 800x800 sphere 2.16 / 1.85 / 2.12.  The kernels with the per-lane walk: see there.  Backward, training steps at 2 / 3
+// waves (a table of 117 / 64 rows): room 10.7 / 12.7 ms, sphere 3.70 / 4.68, 233x417 room in fixed point 0.56 / 0.68.
 #ifndef DST_FWD_WAVES
 #define DST_FWD_WAVES 3
 #endif
@@ -2150,8 +2161,8 @@ void k_trace_fwd(const DstParams p, const DstAccelView acc, int tw_log2, int th_
     trace_body<false, AUXM, REC, MIXED, EXTRAS, kFwdWavesPerBlock == 1>(p, acc, tw_log2, th_log2, tiles_x, tiles_y, btiles_x, ray_order, strip_width, nullptr, handover, hand_arg);
 }
 // The forward kernel of image grids at depth 0 without the tile hand-over: what scenes without many small quads are
-// traced with (the hand-over's few extra live values cost the walk 1 to 4 % of its time through the register
-// allocation, whether a tile is ever handed over or not).
+// traced with (the hand-over's counting and its few extra live values cost the walk 9 % on the 1080p room and 16 % on the
+// 800x800 sphere, whether a tile is ever handed over or not: 3.80 -> 4.13 ms, 1.84 -> 2.13).
 template <int AUXM, bool REC>
 __global__ __launch_bounds__(kFwdWavesPerBlock *DST_WAVE) __attribute__((amdgpu_waves_per_eu(DST_FWD_WAVES, DST_FWD_WAVES)))
 void k_trace_fwd_plain(const DstParams p, const DstAccelView acc, int tw_log2, int th_log2, uint32_t tiles_x,
@@ -2344,13 +2355,13 @@ void launch(const DstParams &p, const DstAccelView &acc, const TileGrid &t, cons
         block = dim3(DST_WAVE);
         if (takers) grid = dim3(std::min<uint32_t>(n_blocks * (uint32_t)kWavesPerBlock, kHandCap));
     }
-    // The per-lane walk is built into the kernels used where waves of unrelated rays are to be expected:
-    // reflection bounces and ray lists (thin grids).  Image-shaped grids traced to depth 0 get the pure packet kernels.
-    // Order of the blocks of an image grid (trace_body): column strips put vertical neighbours on one XCD.  Measured
-    // forward, strips of 8 / 16 / 24 blocks / row-major: 8.12 / 8.20 / 8.53 / 8.48 ms on 120 x 68 blocks (1080p, 1M
-    // surfels), but 4.68 / 4.37 / 4.19 / 4.28 ms on 50 x 50 blocks (a sphere in front of an empty background): with only
-    // two or three rounds of workgroups on the chip the order decides more about the last round than about the caches.
-    // The backward trace gains 1 to 3 % from strips of 8 on every grid measured.
+    // The per-lane walk is built into the kernels that meet waves of unrelated rays: reflection bounces and ray lists
+    // (thin grids) of contexts that can hand tiles over, and of the backward trace without a record.
+    // Order of the blocks of an image grid (trace_body): column strips put vertical neighbours on one XCD.  Evaluated,
+    // strips of 8 / 16 blocks / row-major: 3.81 / 3.80 / 4.08 ms on 120 x 68 blocks (1080p, 1M surfels); strips of 8 /
+    // row-major 1.87 / 1.85 ms on 50 x 50 blocks (a sphere in front of an empty background): with only two or three rounds
+    // of workgroups on the chip the order decides more about the last round than about the caches.  Training steps with
+    // strips of 8 / 16 / none in both directions: 10.74 / 10.66 / 10.99 ms and 3.70 / 3.67 / 3.67.
     uint32_t strip = 0u;
     if (t.th_log2 != 0) strip = BWD ? (uint32_t)DST_STRIP_BWD : (n_blocks >= kStripMinBlocks ? (uint32_t)DST_STRIP_FWD : 0u);
     const bool mixed = takers || (p.max_trace_depth > 0 && !first_bounce) || t.th_log2 < 3;   // first_bounce: forward, nothing beyond it
@@ -2388,6 +2399,11 @@ void launch(const DstParams &p, const DstAccelView &acc, const TileGrid &t, cons
 // How the rays of this grid are traced.  Tiles: a wave per 64 rays.  Rows (sixteen lanes per ray): lists, whose rays
 // are unrelated, and images so small that waves of 64 rays leave most of the chip idle.  TilesThenRows: images with
 // reflections - the primary rays as tiles, the bounces beyond as rows.
+// The line between small images and the others (400 waves: 25,600 rays), rows / tiles in us: training steps 128x128 cube
+// of 10,000 surfels 914 / 1367, 160x160 1022 / 1204, 192x192 1155 / 1138, 256x256 1761 / 1083; room of 200,000 surfels
+// 160x160 620 / 780, 192x192 725 / 675.  Evaluated, rows would still pay beyond it, with four rays a wave (below):
+// 192x192 189 / 482 and 113 / 382, 256x256 262 / 455 and 162 / 284; a record has one layout for both directions of a step,
+// and calls without one follow the same line.
 enum class TraceBy { Tiles, Rows, TilesThenRows };
 TraceBy row_grid(const DstParams &p, const TileGrid &t, RowGrid &g) {
     const uint64_t rays = (uint64_t)p.H * p.W;
@@ -2400,7 +2416,12 @@ TraceBy row_grid(const DstParams &p, const TileGrid &t, RowGrid &g) {
         g.n_waves = t.btiles_x * t.btiles_y * kWavesPerBlock;
         return p.max_trace_depth == 0 ? TraceBy::Tiles : TraceBy::TilesThenRows;
     }
-    g.batch_log2 = rays >= 16384u ? 4u : 2u;   // sixteen rays a wave once that leaves a thousand waves
+    // Sixteen rays a wave once that leaves a thousand waves, four below: a wave's record pieces and the tail of its batch
+    // are then shared by more rays.  Four / sixteen rays a wave, us: training steps of lidar lists of 131,072 rays 1409 /
+    // 1079, 65,536 883 / 772, 32,768 584 / 624, 16,384 476 / 539; 128x128 images 546 / 909 (cube) and 363 / 506 (room);
+    // evaluated lists of 16,384 rays 204 / 310, 131,072 467 / 540.  So the line is right for training lists of some 50,000
+    // rays and more, and too low for everything else.
+    g.batch_log2 = rays >= 16384u ? 4u : 2u;
     if (t.th_log2 == 0) {
         g.side_log2 = 0u;
         g.tiles_x = g.n_waves = (uint32_t)((rays + (1u << g.batch_log2) - 1u) >> g.batch_log2);
@@ -2416,6 +2437,9 @@ TraceBy row_grid(const DstParams &p, const TileGrid &t, RowGrid &g) {
 template <bool REC, bool BEYOND>
 void launch_row_fwd(const DstParams &p, const DstAccelView &acc, const RowGrid &g, const uint32_t *ray_order, hipStream_t stream) {
     const dim3 grid(BEYOND ? g.n_waves : (g.n_waves + 31u) / 32u * 32u), block(BEYOND ? kWavesPerBlock * DST_WAVE : DST_WAVE);
+    // Pieces of a record a wave takes at a time (an addition to one counter that all waves share): four where a wave has
+    // sixteen rays.  One / four / sixteen, training steps of lidar lists: 131,072 rays 1576 / 1078 / 1056 us, 32,768
+    // 717 / 625 / 626.
     const uint32_t grab = g.batch_log2 == 4u ? 4u : 1u;
 #define DST_ROW(AUX)                                                                                                       \
     do {                                                                                                                   \
@@ -2578,7 +2602,11 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
         const uint32_t steps = std::max<uint32_t>(ctx->handover_steps, 1u);
         // the second launch of each pair traces the tiles the first one handed over (usually none: it leaves at once)
         uint32_t *const list = (kFwdWavesPerBlock == 1 && dst_handover_active(ctx)) ? ctx->handover : nullptr;
-        // (a context told never to hand tiles over keeps the rays of an image's tile together)
+        // A hand-over mode is about tiles, so contexts that can hand them over (list != nullptr) and, for images without
+        // reflections, contexts told not to (DST_HANDOVER_OFF) trace by tiles: OFF against AUTO shows what the hand-over is
+        // worth, tile by tile.  Rows need none and would be faster for all of these: the ball of small quads above, 64x64,
+        // takes 29.9 ms with OFF, 2.8 with the hand-over and 0.24 by rows, a list of 20,000 rays there 813 and 290 us, a
+        // 637x1013 room with one reflection 5.5 ms against 3.5.
         if (by == TraceBy::Rows && list == nullptr && (ctx->handover_mode != DST_HANDOVER_OFF || p.max_trace_depth > 0 || t.th_log2 < 3)) {
             if (rec) launch_row_fwd<true, false>(p, acc, rows, ray_order, stream);
             else launch_row_fwd<false, false>(p, acc, rows, ray_order, stream);

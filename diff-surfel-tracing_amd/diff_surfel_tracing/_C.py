@@ -436,7 +436,7 @@ class OptiXStateWrapper:
 
     def set_handover(self, mode, steps=0):
         """HANDOVER_OFF / HANDOVER_AUTO (only for scenes with many quads far smaller than the scene) / HANDOVER_ALWAYS;
-        `steps`: what a tile's first packet walk may take before its rays are walked one by one (0: unchanged)."""
+        `steps`: what a tile's first walk may take before its rays are walked one by one (0: unchanged)."""
         _check(self, load_library().dst_set_handover(self.handle, int(mode), int(steps)))
 
     def __del__(self):

@@ -241,17 +241,18 @@ int dst_accel_download(dst_ctx *ctx, void *nodes, void *leaves, uint32_t *node_p
  * hardware: optix_tracer/forward.cu:318).  The trace kernels walk the BVH once for the 64 rays of an 8x8 pixel tile.
  * Over geometry much finer than the ray spacing (a dense cloud of surfels far smaller than a pixel) that walk visits
  * everything inside the tile's frustum for the sake of one ray at a time, and one wave runs for milliseconds.  A tile
- * whose first walk takes more than `handover_steps` steps (nodes and leaf groups; default 2048, a few hundred on
+ * whose first walk takes more than `handover_steps` steps (nodes and candidate quads; default 2048, a few hundred on
  * ordinary scenes) is therefore put on a list and traced by a second launch in which every ray walks on its own: same
  * results bit for bit.  At most `handover_capacity` tiles per call are handed over; further ones are traced the usual
- * way.  The kernels that can hand over are 1 to 4 % slower than those that cannot, so by default (DST_HANDOVER_AUTO)
+ * way.  The kernels that can hand over are 9 to 16 % slower on ordinary scenes than those that cannot, and trace ray lists,
+ * small images and reflections by tiles too, which the others trace ray by ray; so by default (DST_HANDOVER_AUTO)
  * a context uses them only while its last build or refit counted at least 2048 quads with edges below 1/2048 of the scene's
  * size (`small_quads`; refits count too, and their count reaches the host behind the first forward trace that follows,
  * so it serves from the second one on); DST_HANDOVER_ALWAYS and DST_HANDOVER_OFF decide regardless of the
- * scene.  dst_set_handover: steps = 0 keeps the current limit.  DST_HANDOVER=off|auto|always and DST_HANDOVER_STEPS=n
- * in the environment of dst_create set the initial values.  The list is emptied on the device by the second launch, so
- * a forward call recorded into a graph can be replayed.  dst_trace_info waits for the device; tiles_handed_over
- * counts since the context was created (a 32-bit count). */
+ * scene (OFF also keeps small images without reflections on tiles).  dst_set_handover: steps = 0 keeps the current
+ * limit.  DST_HANDOVER=off|auto|always and DST_HANDOVER_STEPS=n in the environment of dst_create set the initial values.
+ * The list is emptied on the device by the second launch, so a forward call recorded into a graph can be replayed.
+ * dst_trace_info waits for the device; tiles_handed_over counts since the context was created (a 32-bit count). */
 #define DST_HANDOVER_OFF 0
 #define DST_HANDOVER_AUTO 1
 #define DST_HANDOVER_ALWAYS 2
