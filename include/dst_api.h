@@ -241,8 +241,8 @@ int dst_accel_download(dst_ctx *ctx, void *nodes, void *leaves, uint32_t *node_p
  * hardware: optix_tracer/forward.cu:318).  The trace kernels walk the BVH once for the 64 rays of an 8x8 pixel tile.
  * Over geometry much finer than the ray spacing (a dense cloud of surfels far smaller than a pixel) that walk visits
  * everything inside the tile's frustum for the sake of one ray at a time, and one wave runs for milliseconds.  A tile
- * whose first walk takes more than `handover_steps` steps (nodes and candidate quads; default 2048, a few hundred on
- * ordinary scenes) is therefore put on a list and traced by a second launch in which every ray walks on its own: same
+ * whose first walk takes more than `handover_steps` steps (nodes and candidate quads; default 2048, a few hundred to a
+ * thousand on ordinary scenes) is therefore put on a list and traced by a second launch in which every ray walks on its own: same
  * results bit for bit.  At most `handover_capacity` tiles per call are handed over; further ones are traced the usual
  * way.  The kernels that can hand over are 9 to 16 % slower on ordinary scenes than those that cannot, and trace ray lists,
  * small images and reflections by tiles too, which the others trace ray by ray; so by default (DST_HANDOVER_AUTO)
