@@ -318,8 +318,10 @@ class OptiXStateWrapper:
         device = torch.device(device)
         if device.index is None:
             device = torch.device(device.type, torch.cuda.current_device())
+        # (what a graph being captured writes must belong to that graph: a pooled storage would go on to other calls)
+        captured = not self._record_fixed and torch.cuda.is_current_stream_capturing()
         with self._pool_lock:
-            fit = [t for t in self._record_pool if t.numel() >= words and t.device == device]
+            fit = [] if captured else [t for t in self._record_pool if t.numel() >= words and t.device == device]
             storage = min(fit, key=lambda t: t.numel()) if fit else None
             self._record_pool = [t for t in self._record_pool if t is not storage]
             done = self._record_events.pop(id(storage), None)
@@ -347,6 +349,8 @@ class OptiXStateWrapper:
         words, rec.words = rec.words, None
         done = None
         if words.is_cuda:
+            if not self._record_fixed and torch.cuda.is_current_stream_capturing():
+                return
             done, now = torch.cuda.Event(), _current_stream()
             done.record(now)
             words.record_stream(now)
@@ -560,9 +564,12 @@ def trace_surfels(ctx, training, start_from_first, ray_o, ray_d, vertices, backg
     p.mid_val = mid_val.data_ptr()
     p.a_weights = _ptr(a_weights)
     p.counters = _ptr(counters)
+    # (a captured copy of the request count would be made on every replay, long after the word has another owner)
+    watch = hit_record is not None and not torch.cuda.is_current_stream_capturing()
     if hit_record is not None:
         p.hit_record, p.hit_record_blocks = hit_record.words.data_ptr(), hit_record.blocks
-        p.hit_record_asked = hit_record.note_request()
+        if watch:
+            p.hit_record_asked = hit_record.note_request()
     det_ws = None
     if getattr(ctx, "deterministic", False) and training:
         det_ws = torch.zeros(load_library().dst_det_workspace_words(P, p.aux, 0), dtype=torch.int64, device=dev)
@@ -575,7 +582,7 @@ def trace_surfels(ctx, training, start_from_first, ray_o, ray_d, vertices, backg
     _check(ctx, load_library().dst_trace_forward(ctx.handle, C.byref(p), _stream()))
     if events is not None:
         events[1].record()
-    if hit_record is not None:
+    if watch:
         ctx._record_watch.append(hit_record)
     del keep
     return out_rgb, out_dpt, out_acc, out_norm, out_dist, out_aux, mid_val, a_weights

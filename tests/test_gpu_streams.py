@@ -53,3 +53,48 @@ def test_two_streams_in_turn(size):
             del noise
     tracer.optix_context.release_memory()
     assert not tracer.optix_context._row_pool and not tracer.optix_context._record_pool
+
+
+@pytest.mark.parametrize("size,depth", [((48, 64), 0), ((152, 176), 1)])
+def test_a_captured_training_step_can_be_replayed(size, depth):
+    """Forward and backward recorded into a graph: every replay gives the eager gradients, with eager training steps in
+    between, one of them in two halves around the replay (the graph's record and rows are its own)."""
+    import diff_surfel_tracing as dst
+    H, W = size
+    tracer = dst.SurfelTracer()
+    st = settings(dst, H, W, DEV, max_trace_depth=depth, specular_threshold=0.1)
+    g = {k: v.to(DEV) for k, v in S.scene_room(P=6000, seed=1, aux=2, half=1.5).items()}
+    g["others_precomp"][:, 0] = g["others_precomp"][:, 0] * 0.8 + 0.1
+    tracer.build_acceleration_structure(g["vertices"], g["faces"], True)
+    o, d = (t.to(DEV) for t in S.pinhole_rays(H, W, 70.0, (-0.6, -0.3, 0.15), (0.9, 0.45, -0.15)))
+    o2, d2 = (t.to(DEV) for t in S.pinhole_rays(H, W, 50.0, (0.6, 0.3, 0.15), (-0.9, 0.45, -0.15)))
+    ug = {k: t.to(DEV) for k, t in S.upstream_grads(H, W, 2, seed=2).items()}
+    leaf = {k: g[k].clone().requires_grad_(True) for k in PARAM_NAMES if k in g}
+    own = lambda grads: {k: v.clone() for k, v in grads.items()}  # noqa: E731
+    for _ in range(3):                                   # the record's size settles
+        want, want2 = own(step(tracer, st, g, o, d, ug, leaf)), own(step(tracer, st, g, o2, d2, ug, leaf))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step(tracer, st, g, o, d, ug, leaf)              # warm-up on a side stream, as torch asks before a capture
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step(tracer, st, g, o, d, ug, leaf)
+    for k in range(4):
+        for t in got.values():
+            t.fill_(-7.0)
+        out = tracer(o2, d2, g["vertices"], leaf["means3D"], torch.zeros_like(leaf["means3D"]), shs=leaf["shs"],
+                     others_precomp=leaf["others_precomp"], opacities=leaf["opacities"], scales=leaf["scales"],
+                     rotations=leaf["rotations"], tracer_settings=st)
+        graph.replay()
+        half = torch.autograd.grad([out[0], out[1], out[2], out[3], out[5]], list(leaf.values()),
+                                   [ug[n] for n in ("rgb", "dpt", "acc", "norm", "aux")])
+        torch.cuda.synchronize()
+        for name, eager in zip(leaf, half):
+            assert_same_sums(got[name].cpu().numpy(), want[name].cpu().numpy(), GRAD_REL, "replay %d %s" % (k, name))
+            assert_same_sums(eager.cpu().numpy(), want2[name].cpu().numpy(), GRAD_REL, "around replay %d %s" % (k, name))
+        if k == 1:
+            tracer.optix_context.release_memory()
+            torch.cuda.empty_cache()

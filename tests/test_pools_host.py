@@ -41,12 +41,12 @@ class _Device:
     """What the pools ask of torch.cuda, with a current stream that the test sets."""
 
     def __init__(self, monkeypatch):
-        self.now = _Stream()
+        self.now, self.capturing = _Stream(), False
         make = lambda n, dtype=torch.float32, device=None: _Buffer(n, dtype, device, self.now)  # noqa: E731
         monkeypatch.setattr(_C, "_current_stream", lambda: self.now)
         monkeypatch.setattr(_C.torch.cuda, "Event", _Event)
         monkeypatch.setattr(_C.torch.cuda, "current_device", lambda: 0)
-        monkeypatch.setattr(_C.torch.cuda, "is_current_stream_capturing", lambda: False)
+        monkeypatch.setattr(_C.torch.cuda, "is_current_stream_capturing", lambda: self.capturing)
         monkeypatch.setattr(_C.torch, "zeros", make)
         monkeypatch.setattr(_C.torch, "empty", make)
 
@@ -179,3 +179,27 @@ def test_threads_never_share_a_buffer(device, monkeypatch):
         sys.setswitchinterval(interval)
     assert not clashes
     assert len(ctx._record_pool) <= ctx.RECORD_POOL_SIZE and len(ctx._record_events) <= ctx.RECORD_POOL_SIZE
+
+
+def test_a_captured_step_keeps_its_buffers_to_itself(device, monkeypatch):
+    """A graph writes to the same memory on every replay: what a captured call takes is its own, not the pool's, and does
+    not go on to other calls."""
+    monkeypatch.setattr(_C, "HitRecord", _Record)
+    ctx = _context()
+    dev = torch.device("cuda", 0)
+    rec, pair = ctx.acquire_record(8, 8, 1, dev), ctx.acquire_rows(10, 660, torch.float32, dev)
+    pooled = [rec.words, pair[0], pair[1]]
+    ctx.release_record(rec)
+    ctx.release_rows(*pair)
+    device.capturing = True
+    rec, pair = ctx.acquire_record(8, 8, 1, dev), ctx.acquire_rows(10, 660, torch.float32, dev)
+    taken = [rec.words, pair[0], pair[1]]
+    assert not any(t is p for t in taken for p in pooled)
+    ctx.release_record(rec)
+    ctx.release_rows(*pair)
+    assert rec.words is None
+    device.capturing = False
+    rec, pair = ctx.acquire_record(8, 8, 1, dev), ctx.acquire_rows(10, 660, torch.float32, dev)
+    assert [rec.words, pair[0], pair[1]] == pooled
+    rec, pair = ctx.acquire_record(8, 8, 1, dev), ctx.acquire_rows(10, 660, torch.float32, dev)
+    assert not any(t is x for t in (rec.words, *pair) for x in taken)
