@@ -260,7 +260,6 @@ class OptiXStateWrapper:
                                             # of the 1M-surfel room scene needs 13 GB, of the card's 288
         self.record_pool_max_bytes = 48 << 30   # free storages kept for reuse, all together
         self.records_skipped = 0            # forward calls that made no record because of the two limits above
-        self.record_wanted = True           # set by the autograd wrapper for the call that follows
         self.deterministic = False          # True: a_weights and per-surfel gradients are bitwise reproducible
         self.deterministic_check = True     # with `deterministic`: warn after a backward trace whose sums left the range
         self._det_out_of_range = 0          # the library's count when last looked at

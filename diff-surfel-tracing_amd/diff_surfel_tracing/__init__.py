@@ -5,6 +5,7 @@ Public names, argument order, defaults and return tuples follow the reference pa
 `SurfelTracer`, `SurfelTracingSettings`, `trace_surfels`, `_TraceSurfels`.  The work happens in
 hand-written HIP kernels behind the C ABI of libdst.so (see `_C.py`); there is no fallback path.
 """
+import threading
 from typing import NamedTuple
 
 import torch
@@ -73,6 +74,9 @@ def _results(out_rgb, out_dpt, out_acc, out_norm, out_dist, out_aux, mid_val, a_
     return out_rgb, out_dpt, out_acc, out_norm, dist, out_aux, mid_val, acc_wet
 
 
+_call = threading.local()   # .record_wanted: whether a backward pass can follow the call this thread is making
+
+
 class _TraceSurfels(torch.autograd.Function):
     @staticmethod
     def forward(ctx, optix_context, training, start_from_first, ray_o, ray_d, vertices, means3D, grads3D, shs,
@@ -85,7 +89,7 @@ class _TraceSurfels(torch.autograd.Function):
         # says whether one can follow (gradient mode is always off in here, and needs_input_grad stays set
         # under torch.no_grad())
         record = None
-        if optix_context.record_wanted and any(ctx.needs_input_grad) and ray_o.dim() == 3 and ray_o.numel() > 0:
+        if getattr(_call, "record_wanted", True) and any(ctx.needs_input_grad) and ray_o.dim() == 3 and ray_o.numel() > 0:
             record = optix_context.acquire_record(ray_o.size(0), ray_o.size(1),
                                                   max(_C.DEFAULT_MAX_TRACE_DEPTH, s.max_trace_depth), ray_o.device,
                                                   max_trace_depth=s.max_trace_depth)
@@ -150,10 +154,10 @@ def trace_surfels(optix_context, training, start_from_first, ray_o, ray_d, verti
                   colors_precomp, others_precomp, opacities, scales, rotations, cov3Ds_precomp, tracer_settings):
     # a hit record only pays off when a backward pass can follow: not under torch.no_grad(), not for inputs
     # without gradients (the usual evaluation loop renders nn.Parameter tensors under no_grad)
-    optix_context.record_wanted = torch.is_grad_enabled() and any(
+    _call.record_wanted = torch.is_grad_enabled() and any(
         isinstance(t, torch.Tensor) and t.requires_grad
         for t in (ray_o, ray_d, means3D, grads3D, shs, colors_precomp, others_precomp, opacities, scales, rotations))
-    if not optix_context.record_wanted and not _transforms_active():
+    if not _call.record_wanted and not _transforms_active():
         # nothing to differentiate: the launcher without the autograd function around it
         s = tracer_settings
         args = (optix_context, training, start_from_first, ray_o, ray_d, vertices, s.bg, means3D, shs, s.sh_degree,

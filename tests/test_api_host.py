@@ -299,7 +299,7 @@ def test_a_failed_call_leaves_nothing_for_the_next_one(monkeypatch, grad):
     args = _call_args()
     args[6].requires_grad_(grad)
     args[-1] = args[-1]._replace(debug=True)
-    before = dict(vars(args[0]), record_wanted=grad, acquired=int(grad), released=int(grad))
+    before = dict(vars(args[0]), acquired=int(grad), released=int(grad))
     with pytest.raises(OSError):
         dst.trace_surfels(*args)
     assert vars(args[0]) == before
@@ -347,3 +347,31 @@ def test_bench_quotes_traffic_for_the_kernels_that_run_only():
         fwd, bwd, _ = bench.kernels_of(*grid, False)
         assert bench.traffic_of(key, "forward", fwd) and bench.traffic_of(key, "backward", bwd)
         assert bench.traffic_of(key, "forward", bench.kernels_of(*grid, True)[0]) is None
+
+
+def test_a_thread_that_evaluates_does_not_cost_another_its_record(monkeypatch):
+    """One thread trains while another renders through the same context under no_grad: whether a record is made is the
+    call's own business."""
+    import threading
+
+    import diff_surfel_tracing as dst
+    from diff_surfel_tracing import _C
+    monkeypatch.setattr(_C, "trace_surfels", _fake_launcher)
+    train, view = _call_args(), _call_args()
+    view[0] = train[0]
+    train[6].requires_grad_(True)
+
+    def evaluate():
+        with torch.no_grad():
+            dst.trace_surfels(*view)
+
+    started = dst._TraceSurfels.apply
+
+    def apply(*a):   # the other thread's call falls between the wrapper and the autograd function
+        t = threading.Thread(target=evaluate)
+        t.start()
+        t.join()
+        return started(*a)
+    monkeypatch.setattr(dst._TraceSurfels, "apply", apply)
+    dst.trace_surfels(*train)
+    assert train[0].acquired == 1
