@@ -1,6 +1,7 @@
 """Training steps of one context on two streams in turn, without the host waiting in between: the buffers kept between
 calls (records, rows of gradient sums and marks) go from stream to stream, grow with the scene and change with the
-mode, and every step's gradients are those of the step on its own."""
+mode, and every step's gradients are those of the step on its own.  (Images small enough to share nothing else: ray lists
+and images of 1536 blocks and more must not overlap on one context.)"""
 import pytest
 import torch
 
