@@ -406,8 +406,9 @@ class OptiXStateWrapper:
     def release_memory(self):
         """Give back what is kept between calls for reuse (hit records, rows of gradient sums; not a caller's own record
         storage).  The next training step allocates again."""
+        self.update_record_estimate()
         with self._pool_lock:
-            self._row_pool = []
+            self._row_pool, self._record_watch = [], []   # (a record nobody traced backward through is held there alone)
             if not self._record_fixed:
                 self._record_pool, self._record_events = [], {}
 

@@ -137,8 +137,13 @@ def test_gradient_rows_kept_between_calls_are_bounded_and_given_back(device):
     ctx.release_rows(*grown)
     assert ctx.acquire_rows(10, 660, torch.int64, "cuda:0")[0] is grown[0]   # larger than needed: serves
     ctx.release_rows(*grown)
+
+    class _Pending:                                    # a forward trace that nobody traced backward through
+        def asked(self, wait=False):
+            return None
+    ctx._record_watch.append(_Pending())
     ctx.release_memory()
-    assert _held(ctx) == 0
+    assert _held(ctx) == 0 and not ctx._record_watch
 
 
 def test_threads_never_share_a_buffer(device, monkeypatch):
