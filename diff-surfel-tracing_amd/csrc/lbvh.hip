@@ -539,7 +539,7 @@ __global__ void k_ploc_init(const float *__restrict__ vertices, const int4 *__re
     if (m == 0) {
         pb.state[0] = pb.state[1] = n;
         pb.state[2] = pb.state[3] = 0u;
-        pb.state[4] = pb.state[5] = pb.state[6] = 0u;
+        pb.state[4] = pb.state[5] = pb.state[6] = pb.state[7] = 0u;
     }
     if (m >= n) return;
     const uint32_t g = sorted_ids[m];
@@ -552,6 +552,7 @@ __global__ void k_ploc_init(const float *__restrict__ vertices, const int4 *__re
         out[3 + a] = fmaxf(fmaxf(c[0][a], c[1][a]), fmaxf(c[2][a], c[3][a]));
     }
     pb.id[0][m] = DST_LEAF_BIT | m;
+    pb.low[0][m] = m;
 }
 
 // The trace kernels widen every box and every stand-in limit by a multiple of the magnitudes of the numbers that meet
@@ -1100,7 +1101,7 @@ int ensure_capacity(dst_ctx *ctx, uint32_t P) {
     }
     ctx->tile_hist_elems = tiles * kRadix + kRadix;
     DST_HIP(ctx, hipMalloc((void **)&ctx->tile_hist, sizeof(uint32_t) * ctx->tile_hist_elems));
-    ctx->ploc_blocks = (uint32_t)((n + kPlocBlock - 1) / kPlocBlock);
+    ctx->ploc_blocks = (uint32_t)((n + kPlocOwn - 1) / kPlocOwn);
     DST_HIP(ctx, hipMalloc((void **)&ctx->ploc_state, sizeof(uint32_t) * (kPlocStateWords + 2 * ((size_t)ctx->ploc_blocks + 1))));
     DST_HIP(ctx, hipMemset(ctx->ploc_state, 0xFF, sizeof(uint32_t) * kPlocStateWords));   // depth word: "too deep" until a build says otherwise
     if (!ctx->ploc_host) DST_HIP(ctx, hipHostMalloc((void **)&ctx->ploc_host, sizeof(uint32_t) * kPlocStateWords, hipHostMallocDefault));
@@ -1132,52 +1133,47 @@ int ploc_hierarchy(dst_ctx *ctx, const float *vertices, uint32_t n, hipStream_t 
     pb.nn = words;
     pb.pre = words + (size_t)n;
     pb.lpar = words + 2 * (size_t)n;
+    pb.low[0] = words + 3 * (size_t)n;
+    pb.low[1] = words + 4 * (size_t)n;
+    pb.tsize = words + 5 * (size_t)n;
     uint32_t *tmp = reinterpret_cast<uint32_t *>(ctx->centroids);
-    pb.tc0 = tmp;
-    pb.tc1 = tmp + (size_t)n;
-    pb.tsize = tmp + 2 * (size_t)n;
-    pb.tpar = tmp + 3 * (size_t)n;
+    pb.up = tmp;
+    pb.tc0 = tmp + 2 * (size_t)n;
+    pb.tc1 = tmp + 3 * (size_t)n;
     pb.state = ctx->ploc_state;
     pb.n_blocks = ctx->ploc_blocks;
     hipLaunchKernelGGL(k_ploc_init, grid_for(n), dim3(kBlock), 0, stream, vertices, reinterpret_cast<const int4 *>(ctx->quad_ids),
                        ctx->vals[0], pb, n);
+    // As many launches as leave few enough for one workgroup if each leaves three fifths of the clusters (an eighth merges
+    // per round on the scenes measured here); one that finds no more to do takes 4 us.  Then the layout, without waiting
+    // for the count: its kernels find nothing to do unless the rounds came to an end.
     int it = 0;
     uint32_t count = n;
-    int batch = 32;
-    while (count > kPlocTail) {
-        const dim3 grid((count + kPlocBlock - 1) / kPlocBlock);   // enough for the largest count this batch can see
+    for (;;) {
+        const dim3 grid((count + kPlocOwn - 1) / kPlocOwn);   // enough for the largest count this batch can see
+        int batch = 0;
+        for (double left = count; left > kPlocTail; left *= 0.6) ++batch;
         for (int k = 0; k < batch; ++k, ++it) {
-            hipLaunchKernelGGL(k_ploc_nn, grid, dim3(kPlocBlock), 0, stream, pb, it);
-            hipLaunchKernelGGL(k_ploc_flags, grid, dim3(kPlocBlock), 0, stream, pb, it);
+            hipLaunchKernelGGL(k_ploc_rounds, grid, dim3(kPlocBlock), 0, stream, pb, it);
             hipLaunchKernelGGL(k_ploc_scan, dim3(1), dim3(kPlocBlock), 0, stream, pb, it);
-            hipLaunchKernelGGL(k_ploc_apply, grid, dim3(kPlocBlock), 0, stream, pb, it);
         }
+        hipLaunchKernelGGL(k_ploc_tail, dim3(1), dim3(kPlocBlock), 0, stream, pb, it);
+        hipLaunchKernelGGL(k_ploc_leaf_positions, grid_for(n), dim3(kBlock), 0, stream, pb, ctx->vals[0], ctx->vals[1], n);
+        hipLaunchKernelGGL(k_ploc_node_numbers, grid_for(n - 1), dim3(kBlock), 0, stream, pb, ctx->nodes, n);
+        hipLaunchKernelGGL(k_ploc_links, grid_for(n - 1), dim3(kBlock), 0, stream, pb, ctx->nodes, ctx->node_parent, ctx->leaf_parent, n);
+        DST_HIP(ctx, hipGetLastError());
         DST_HIP(ctx, hipMemcpyAsync(ctx->ploc_host, ctx->ploc_state, sizeof(uint32_t) * kPlocStateWords, hipMemcpyDeviceToHost, stream));
         DST_HIP(ctx, hipStreamSynchronize(stream));
         const uint32_t now = ctx->ploc_host[it & 1];
+        if (now <= kPlocTail) break;
         if (now >= count || (uint32_t)it > kPlocMaxRounds) {   // no progress in a whole batch: cannot happen (every round merges)
             ctx->ploc_refused = true;
             return kPlocRefused;
         }
         count = now;
-        batch = 8;
     }
-    hipLaunchKernelGGL(k_ploc_tail, dim3(1), dim3(kPlocBlock), 0, stream, pb, it);
-    // the layout below follows the links of a finished hierarchy: make sure it is one
-    DST_HIP(ctx, hipMemcpyAsync(ctx->ploc_host, ctx->ploc_state, sizeof(uint32_t) * kPlocStateWords, hipMemcpyDeviceToHost, stream));
-    DST_HIP(ctx, hipStreamSynchronize(stream));
-    if (ctx->ploc_host[4] != 0u || ctx->ploc_host[0] != 1u || ctx->ploc_host[2] != n - 1u) {
-        ctx->ploc_refused = true;
-        return kPlocRefused;
-    }
-    hipLaunchKernelGGL(k_ploc_leaf_positions, grid_for(n), dim3(kBlock), 0, stream, pb, ctx->vals[0], ctx->vals[1], n);
-    hipLaunchKernelGGL(k_ploc_node_numbers, grid_for(n - 1), dim3(kBlock), 0, stream, pb, ctx->nodes, n);
-    hipLaunchKernelGGL(k_ploc_links, grid_for(n - 1), dim3(kBlock), 0, stream, pb, ctx->nodes, ctx->node_parent, ctx->leaf_parent, n);
-    DST_HIP(ctx, hipGetLastError());
-    DST_HIP(ctx, hipMemcpyAsync(ctx->ploc_host, ctx->ploc_state, sizeof(uint32_t) * kPlocStateWords, hipMemcpyDeviceToHost, stream));
-    DST_HIP(ctx, hipStreamSynchronize(stream));
-    if (ctx->ploc_host[4] != 0u) {   // the links did not form one hierarchy over all leaves: nothing may read its order
-        ctx->ploc_refused = true;
+    if (ctx->ploc_host[4] != 0u || ctx->ploc_host[0] != 1u || ctx->ploc_host[3] != n || ctx->ploc_host[2] + 1u >= n) {
+        ctx->ploc_refused = true;   // no hierarchy over all leaves: nothing may read its order
         return kPlocRefused;
     }
     std::swap(ctx->vals[0], ctx->vals[1]);   // the surfel ids in leaf order
