@@ -2416,12 +2416,10 @@ TraceBy row_grid(const DstParams &p, const TileGrid &t, RowGrid &g) {
         g.n_waves = t.btiles_x * t.btiles_y * kWavesPerBlock;
         return p.max_trace_depth == 0 ? TraceBy::Tiles : TraceBy::TilesThenRows;
     }
-    // Sixteen rays a wave once that leaves a thousand waves, four below: a wave's record pieces and the tail of its batch
-    // are then shared by more rays.  Four / sixteen rays a wave, us: training steps of lidar lists of 131,072 rays 1409 /
-    // 1079, 65,536 883 / 772, 32,768 584 / 624, 16,384 476 / 539; 128x128 images 546 / 909 (cube) and 363 / 506 (room);
-    // evaluated lists of 16,384 rays 204 / 310, 131,072 467 / 540.  So the line is right for training lists of some 50,000
-    // rays and more, and too low for everything else.
-    g.batch_log2 = rays >= 16384u ? 4u : 2u;
+    // Four rays a wave, one to a row: the hardware hands the next four to whichever wave slot is free.  Sixteen left one
+    // wave per SIMD on 128x128 rays (training step on the cube 804 -> 473 us with four) and let lists end with a few waves
+    // whose sixteen rays all run along the ground (131,072 lidar rays 3230 -> 2384).
+    g.batch_log2 = 2u;
     if (t.th_log2 == 0) {
         g.side_log2 = 0u;
         g.tiles_x = g.n_waves = (uint32_t)((rays + (1u << g.batch_log2) - 1u) >> g.batch_log2);
@@ -2437,14 +2435,10 @@ TraceBy row_grid(const DstParams &p, const TileGrid &t, RowGrid &g) {
 template <bool REC, bool BEYOND>
 void launch_row_fwd(const DstParams &p, const DstAccelView &acc, const RowGrid &g, const uint32_t *ray_order, hipStream_t stream) {
     const dim3 grid(BEYOND ? g.n_waves : (g.n_waves + 31u) / 32u * 32u), block(BEYOND ? kWavesPerBlock * DST_WAVE : DST_WAVE);
-    // Pieces of a record a wave takes at a time (an addition to one counter that all waves share): four where a wave has
-    // sixteen rays.  One / four / sixteen, training steps of lidar lists: 131,072 rays 1576 / 1078 / 1056 us, 32,768
-    // 717 / 625 / 626.
-    const uint32_t grab = g.batch_log2 == 4u ? 4u : 1u;
 #define DST_ROW(AUX)                                                                                                       \
     do {                                                                                                                   \
-        if (p.flags != 0u) hipLaunchKernelGGL((k_row_fwd<AUX, REC, true, BEYOND>), grid, block, 0, stream, p, acc, g, ray_order, grab); \
-        else hipLaunchKernelGGL((k_row_fwd<AUX, REC, false, BEYOND>), grid, block, 0, stream, p, acc, g, ray_order, grab);  \
+        if (p.flags != 0u) hipLaunchKernelGGL((k_row_fwd<AUX, REC, true, BEYOND>), grid, block, 0, stream, p, acc, g, ray_order); \
+        else hipLaunchKernelGGL((k_row_fwd<AUX, REC, false, BEYOND>), grid, block, 0, stream, p, acc, g, ray_order);  \
     } while (0)
     if (p.aux <= 2) DST_ROW(2);
     else if (p.aux <= 4) DST_ROW(4);
