@@ -810,13 +810,19 @@ constexpr int kColColor = 0, kColOpac = 3, kColScale = 4, kColRot = 6, kColMean 
 // The sums are doubles (deterministic mode: 64-bit fixed point).  Not for their precision: an LDS addition of floats
 // takes its lanes one after the other (measured: 3 cycles a lane, 192 for a wave, whatever the addresses), one of
 // doubles or of integers takes 8.
-constexpr int kStageBytes = kWavesPerBlock * DST_WAVE * 17 * 4;   // the waves' staging areas (GradSink)
 template <int AUXM> struct RowLayout {
     static constexpr int cols = kColAux + AUXM;
     static constexpr int stride = cols | 1;     // 8-byte words of a table row; odd: rows spread over all LDS banks
+    // A wave's staging area in words: a hit's columns (GradSink), or sixteen sums a channel of four rays (row.inc).
+    static constexpr int stage = DST_WAVE * 17 > 4 * (7 + AUXM) * 20 ? DST_WAVE * 17 : 4 * (7 + AUXM) * 20;
     // Rows of the block's table, one more taking what belongs nowhere: what DST_BWD_WAVES blocks (two: 117 rows with two
     // auxiliary channels) leave each other of a CU's 160 KB, which is given out in pieces of 1280 bytes.
-    static constexpr int rows = ((128 / DST_BWD_WAVES) * 1280 - kStageBytes - 1024) / (8 * stride) - 1;
+    static constexpr int rows = ((128 / DST_BWD_WAVES) * 1280 - kWavesPerBlock * stage * 4 - 1024) / (8 * stride) - 1;
+    // Where column `col` of surfel g lies in the caller's rows of P surfels: 64 columns a row, so that the sixteen lanes of
+    // an addition share a cache line of 64 bytes, and the auxiliary channels behind all of them.
+    static __device__ __forceinline__ size_t word(int32_t P, uint32_t g, int col) {
+        return col < kColAux ? (size_t)g * kColAux + col : (size_t)P * kColAux + (size_t)g * AUXM + (col - kColAux);
+    }
 };
 
 // ---- deterministic mode: sums in 64-bit fixed point ------------------------------------------------------
@@ -864,7 +870,7 @@ __device__ __forceinline__ bool column_live(const P &p, int col) {
 template <int AUXM, class P>
 __device__ __forceinline__ float *grad_address(const P &p, uint32_t g, int col) {
     if (p.grad_rows == nullptr) return tensor_address<AUXM>(p, g, col);
-    return column_live<AUXM>(p, col) ? p.grad_rows + (size_t)g * RowLayout<AUXM>::cols + col : nullptr;
+    return column_live<AUXM>(p, col) ? p.grad_rows + RowLayout<AUXM>::word(p.P, g, col) : nullptr;
 }
 
 // Sum of v over the 64 lanes; every lane must be active.
@@ -1005,7 +1011,7 @@ __device__ __attribute__((noinline)) void put_columns(const DstParams *p_in, uin
     auto put = [&](int col, float v) {
         if (DET) {
             if (column_live<AUXM>(p, col))
-                atomicAdd(p.det_workspace + (size_t)g * RowLayout<AUXM>::cols + col, (unsigned long long)to_fixed(v, det_shift(col)));
+                atomicAdd(p.det_workspace + RowLayout<AUXM>::word(p.P, g, col), (unsigned long long)to_fixed(v, det_shift(col)));
         } else {
             float *dst = grad_address<AUXM>(p, g, col);
             if (dst != nullptr) aadd(dst, v);
@@ -1029,15 +1035,14 @@ __device__ __attribute__((noinline)) void put_columns(const DstParams *p_in, uin
 // in LDS.  Grouping cost more than it saved: a step of these scenes composites 6 to 20 different surfels, over half the
 // steps of two of them more than sixteen, and what did not fit went column by column.)
 constexpr int kGeoCols = 16;
-// TABLE = false: every hit's columns go straight to memory (the row kernels, whose hits hardly ever share a surfel).
-template <int AUXM, bool DET, bool TABLE = true>
+template <int AUXM, bool DET>
 struct GradSink {
     // basis value of this lane's coefficient for ray M of its row (rows of one ray: the same for all)
     template <int M> static __device__ __forceinline__ float basis_of(const float (&b)[16]) { return b[M]; }
     template <int M> static __device__ __forceinline__ float basis_of(const float &b) { return b; }
     static constexpr int stride = kGeoCols + 1;   // four rays sixteen apart start in different quarters of the banks
     static constexpr int words = DST_WAVE * stride;
-    static_assert(kWavesPerBlock * words * 4 == kStageBytes, "the table's size counts on the staging areas'");
+    static_assert(words <= RowLayout<AUXM>::stage, "the table's size counts on the staging areas'");
     double *rows;        // the block's table; its last row takes what belongs nowhere
     float *stage;        // this wave's staging area
     bool did;            // this lane composited a hit in this step
@@ -1046,7 +1051,7 @@ struct GradSink {
     uint64_t wt;         // wave-uniform: lanes whose surfel has no table row (their values go to global memory)
 
     __device__ __forceinline__ void plan(uint32_t *keys) {
-        own_slot = TABLE && did ? table_slot<RowLayout<AUXM>::rows>(keys, g) : -1;
+        own_slot = did ? table_slot<RowLayout<AUXM>::rows>(keys, g) : -1;
         wt = wave_ballot(did && own_slot < 0);
     }
     // Column `col` of this lane's hit (every lane; a lane without a hit may pass anything).
@@ -1054,7 +1059,6 @@ struct GradSink {
 
     // v into column `col` (in the table's memory: word `at`).
     __device__ __forceinline__ void put(uint32_t at, int shift, float v) const {
-        if (!TABLE) return;
         if (DET) __hip_atomic_fetch_add(reinterpret_cast<long long *>(rows) + at, to_fixed(v, shift), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         else __hip_atomic_fetch_add(rows + at, (double)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
@@ -1079,7 +1083,7 @@ struct GradSink {
             if (DET || grad_rows == nullptr) {
                 put_columns<AUXM, DET>((const DstParams *)p, gm, on, geo, sh ? f3(x, y, z) : f3(0, 0, 0));
             } else if (on) {
-                float *dst = grad_rows + (size_t)gm * RowLayout<AUXM>::cols + i;
+                float *dst = grad_rows + (size_t)gm * kColAux + i;
                 aadd(dst, geo);
                 if (sh) {
                     aadd(dst + kColSh, x);
@@ -1126,8 +1130,8 @@ struct GradSink {
                     const uint32_t gs = (uint32_t)__builtin_amdgcn_ds_bpermute((src & 63) << 2, (int)g);
                     const float v = stage[(src & 63) * stride + ch];
                     if (src >= 0 && (int)ch < p->aux && v != 0.f) {
-                        if (DET) atomicAdd(p->det_workspace + (size_t)gs * RowLayout<AUXM>::cols + kColAux + ch, (unsigned long long)to_fixed(v, kDetShiftOther));
-                        else aadd(p->grad_rows != nullptr ? p->grad_rows + (size_t)gs * RowLayout<AUXM>::cols + kColAux + ch
+                        if (DET) atomicAdd(p->det_workspace + RowLayout<AUXM>::word(p->P, gs, kColAux + (int)ch), (unsigned long long)to_fixed(v, kDetShiftOther));
+                        else aadd(p->grad_rows != nullptr ? p->grad_rows + RowLayout<AUXM>::word(p->P, gs, kColAux + (int)ch)
                                                           : p->dL_dothers + (size_t)p->aux * gs + ch, v);
                     }
                     for (uint32_t q = 0; q < kRays; ++q) m &= m - 1ull;
@@ -1407,7 +1411,7 @@ __device__ __forceinline__ void table_flush(const DstParams &p, uint32_t *keys, 
             if (q == 0) continue;
             qrows[k] = 0;
             if (column_live<AUXM>(p, col))
-                atomicAdd(p.det_workspace + (size_t)g * RowLayout<AUXM>::cols + col, (unsigned long long)q);
+                atomicAdd(p.det_workspace + RowLayout<AUXM>::word(p.P, g, col), (unsigned long long)q);
         } else {
             const double v = rows[k];
             if (v == 0.0) continue;
@@ -1833,7 +1837,7 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
     __shared__ uint32_t s_keys[BWD ? kTableRows + 1 : 1];   // + the count of claimed rows
     constexpr int kTableWords = (kTableRows + 1) * RowLayout<AUXM>::stride;
     __shared__ double s_rows[BWD ? kTableWords : 1];
-    constexpr int kStageWords = GradSink<AUXM, DET>::words;
+    constexpr int kStageWords = RowLayout<AUXM>::stage;
     __shared__ float s_stage[BWD ? kWavesPerBlock * kStageWords : 1];
     uint32_t *tab_keys = s_keys;
     double *tab_rows = s_rows;
@@ -2191,7 +2195,7 @@ __global__ __launch_bounds__(kCloseThreads) void k_close_gradients(const DstPara
     constexpr uint32_t cols = RowLayout<AUXM>::cols, stride = cols | 1u;
     __shared__ float s_rows[kCloseSurfels * stride];
     __shared__ uint8_t s_on[kCloseSurfels];
-    const bool writes = p.grad_touched != nullptr;
+    const bool writes = p.grad_touched != nullptr, aux_rows = p.others_precomp != nullptr;
     const uint32_t tid = threadIdx.x, P = (uint32_t)p.P;
     for (uint32_t base = blockIdx.x * kCloseSurfels; base < P; base += gridDim.x * kCloseSurfels) {
         const uint32_t n = min(kCloseSurfels, P - base);
@@ -2203,11 +2207,14 @@ __global__ __launch_bounds__(kCloseThreads) void k_close_gradients(const DstPara
         }
         const bool any = __syncthreads_or(on ? 1 : 0) != 0;
         if (any) {
-            for (uint32_t k = tid; k < n * cols; k += kCloseThreads) {
-                const uint32_t row = k / cols, col = k - row * cols;
+            const uint32_t n_cols = aux_rows ? n * cols : n * (uint32_t)kColAux;   // (the auxiliary columns behind the others)
+            for (uint32_t k = tid; k < n_cols; k += kCloseThreads) {
+                const uint32_t rest = k - n * (uint32_t)kColAux;
+                const bool main = k < n * (uint32_t)kColAux;
+                const uint32_t row = main ? k / (uint32_t)kColAux : rest / AUXM, col = main ? k % (uint32_t)kColAux : kColAux + rest % AUXM;
                 float v = 0.f;
                 if (s_on[row] != 0u) {
-                    const size_t at = (size_t)base * cols + k;
+                    const size_t at = main ? (size_t)base * kColAux + k : (size_t)P * kColAux + (size_t)base * AUXM + rest;
                     if (DET) {
                         const long long q = (long long)p.det_workspace[at];
                         if (q != 0) {
@@ -2240,7 +2247,9 @@ __global__ __launch_bounds__(kCloseThreads) void k_close_gradients(const DstPara
         emit(p.dL_drotations, 4u, kColRot);
         emit(p.dL_dmeans3D, 3u, kColMean);
         emit(p.dL_dgrads3D, 3u, kColGrad);
-        if (p.others_precomp != nullptr || writes) emit(p.dL_dothers, (uint32_t)p.aux, kColAux);
+        if (aux_rows) emit(p.dL_dothers, (uint32_t)p.aux, kColAux);
+        else if (writes && p.dL_dothers != nullptr)   // nothing was given: zeros
+            for (uint32_t e = tid; e < n * (uint32_t)p.aux; e += kCloseThreads) p.dL_dothers[(size_t)base * p.aux + e] = 0.f;
         if (p.colors_precomp == nullptr && p.dL_dshs != nullptr && (any || writes)) {
             const uint32_t width = 3u * (uint32_t)p.M;
             float *const dst = p.dL_dshs + (size_t)base * width;
@@ -2445,8 +2454,17 @@ void launch_row_fwd(const DstParams &p, const DstAccelView &acc, const RowGrid &
     else DST_ROW(8);
 #undef DST_ROW
 }
-void launch_row_bwd(const DstParams &p, const RowGrid &g, const uint32_t *ray_order, hipStream_t stream) {
-    const dim3 grid((g.n_waves + 31u) / 32u * 32u), block(DST_WAVE);
+void launch_row_bwd(const DstParams &p, RowGrid g, const uint32_t *ray_order, hipStream_t stream) {
+    // a workgroup takes sixteen rays: a square of an image, a stretch of a list
+    g.batch_log2 = 4u;
+    if (g.tiles_y == 0u) {
+        g.n_waves = ((uint32_t)p.W + 15u) / 16u;
+    } else {
+        g.side_log2 = 2u;
+        g.tiles_x = ((uint32_t)p.W + 3u) / 4u;
+        g.n_waves = g.tiles_x * (((uint32_t)p.H + 3u) / 4u);
+    }
+    const dim3 grid(g.n_waves), block(kWavesPerBlock * DST_WAVE);
     const bool det = (p.flags & DST_FLAG_DETERMINISTIC) != 0u;
 #define DST_ROW(AUX)                                                                                        \
     do {                                                                                                    \
