@@ -83,16 +83,19 @@ def traffic_of(workload, which, kernel):
 
 def kernels_of(H, W, aux, depth, handover):
     """Names of the kernels that do a step's work with a complete hit record: (forward, backward, backward without a
-    record).  Lists (fewer than eight rows of rays) and images of up to 25,600 rays are traced ray by ray, larger images
-    by tiles of 64 rays, their reflections ray by ray; a context that can hand tiles over traces everything by tiles."""
+    record).  Lists (fewer than eight rows of rays) and images of up to 25,600 rays are traced and recorded ray by ray,
+    images of up to 65,536 traced ray by ray and recorded by tiles of 64, larger images traced by tiles, their reflections
+    ray by ray; a context that can hand tiles over traces everything by tiles."""
     a = 2 if aux <= 2 else (4 if aux <= 4 else 8)
     lists, mixed = H < 8, "true" if depth > 0 or H < 8 else "false"
     retrace = "k_trace_bwd<%d,false,%s,false>" % (a, mixed)
     if handover:
         return "k_trace_fwd<%d,true,%s,false>" % (a, mixed), "k_trace_bwd<%d,true,false,false> + k_close_gradients<%d,false>" % (a, a), retrace
     if lists or (H * W + 63) // 64 <= 400:
-        return "k_row_fwd<%d,true,false,false>" % a, "k_row_bwd<%d,false> + k_close_gradients<%d,false>" % (a, a), retrace
-    fwd = "k_trace_fwd_plain<%d,true>" % a + (" + k_row_fwd<%d,true,false,true>" % a if depth > 0 else "")
+        return "k_row_fwd<%d,true,false,0>" % a, "k_row_bwd<%d,false> + k_close_gradients<%d,false>" % (a, a), retrace
+    fwd = "k_trace_fwd_plain<%d,true>" % a + (" + k_row_fwd<%d,true,false,1>" % a if depth > 0 else "")
+    if H * W <= 65536:
+        fwd = "k_row_fwd<%d,true,false,2>" % a
     return fwd, "k_trace_bwd<%d,true,false,false> + k_close_gradients<%d,false>" % (a, a), retrace
 
 

@@ -2406,14 +2406,31 @@ void launch(const DstParams &p, const DstAccelView &acc, const TileGrid &t, cons
 }
 
 // How the rays of this grid are traced.  Tiles: a wave per 64 rays.  Rows (sixteen lanes per ray): lists, whose rays
-// are unrelated, and images so small that waves of 64 rays leave most of the chip idle.  TilesThenRows: images with
-// reflections - the primary rays as tiles, the bounces beyond as rows.
-// The line between small images and the others (400 waves: 25,600 rays), rows / tiles in us: training steps 128x128 cube
-// of 10,000 surfels 914 / 1367, 160x160 1022 / 1204, 192x192 1155 / 1138, 256x256 1761 / 1083; room of 200,000 surfels
-// 160x160 620 / 780, 192x192 725 / 675.  Evaluated, rows would still pay beyond it, with four rays a wave (below):
-// 192x192 189 / 482 and 113 / 382, 256x256 262 / 455 and 162 / 284; a record has one layout for both directions of a step,
-// and calls without one follow the same line.
+// are unrelated, and images so small that waves of 64 rays leave most of the chip idle or end with a few long ones.
+// TilesThenRows: images with reflections - the primary rays as tiles, the bounces beyond as rows.
+// Up to 25,600 rays a record is written ray by ray.  Larger images' records have the tiles' layout, which rows can write as
+// well (RowTiles), and which costs them some; images that are only evaluated need none.  Rows / tiles in us, evaluated:
+// cube of 10,000 surfels 192x192 156 / 483, 320x320 277 / 430, 400x400 387 / 393; room of 200,000 101 / 381, 218 / 252,
+// 327 / 222; sphere of 100,000 (whose limb makes tiles of a millisecond and more) 256 / 3753, 452 / 2357, 645 / 1881.
+// Training steps: cube 192x192 772 / 1137, 256x256 859 / 1083, 320x320 953 / 1025; room 419 / 672, 500 / 571, 604 / 542;
+// sphere 1007 / 4482, 1204 / 3991, 1465 / 3187.
+#ifndef DST_ROW_REC_RAYS
+#define DST_ROW_REC_RAYS 65536
+#define DST_ROW_EVAL_RAYS 102400
+#endif
+constexpr uint64_t kRowRecordedRays = DST_ROW_REC_RAYS, kRowEvaluatedRays = DST_ROW_EVAL_RAYS;
 enum class TraceBy { Tiles, Rows, TilesThenRows };
+// An image by rows: four rays a wave, one to a row; the hardware hands the next four to whichever wave slot is free.
+// Sixteen left one wave per SIMD on 128x128 rays (training step on the cube 804 -> 473 us with four) and let lists end with
+// a few waves whose sixteen rays all run along the ground (131,072 lidar rays 3230 -> 2384).
+RowGrid row_squares(const DstParams &p, RowGrid g) {
+    g.batch_log2 = 2u;
+    g.side_log2 = 1u;
+    g.tiles_x = ((uint32_t)p.W + 1u) / 2u;
+    g.tiles_y = ((uint32_t)p.H + 1u) / 2u;
+    g.n_waves = g.tiles_x * g.tiles_y;
+    return g;
+}
 TraceBy row_grid(const DstParams &p, const TileGrid &t, RowGrid &g) {
     const uint64_t rays = (uint64_t)p.H * p.W;
     g.record_header = record_header_words(rays, t.th_log2, (uint32_t)p.mtd_alloc + 1u, (uint64_t)t.btiles_x * t.btiles_y * kWavesPerBlock);
@@ -2425,29 +2442,23 @@ TraceBy row_grid(const DstParams &p, const TileGrid &t, RowGrid &g) {
         g.n_waves = t.btiles_x * t.btiles_y * kWavesPerBlock;
         return p.max_trace_depth == 0 ? TraceBy::Tiles : TraceBy::TilesThenRows;
     }
-    // Four rays a wave, one to a row: the hardware hands the next four to whichever wave slot is free.  Sixteen left one
-    // wave per SIMD on 128x128 rays (training step on the cube 804 -> 473 us with four) and let lists end with a few waves
-    // whose sixteen rays all run along the ground (131,072 lidar rays 3230 -> 2384).
-    g.batch_log2 = 2u;
     if (t.th_log2 == 0) {
+        g.batch_log2 = 2u;
         g.side_log2 = 0u;
-        g.tiles_x = g.n_waves = (uint32_t)((rays + (1u << g.batch_log2) - 1u) >> g.batch_log2);
+        g.tiles_x = g.n_waves = (uint32_t)((rays + 3u) / 4u);
         g.tiles_y = 0u;
     } else {
-        g.side_log2 = g.batch_log2 / 2u;
-        g.tiles_x = ((uint32_t)p.W + (1u << g.side_log2) - 1u) >> g.side_log2;
-        g.tiles_y = ((uint32_t)p.H + (1u << g.side_log2) - 1u) >> g.side_log2;
-        g.n_waves = g.tiles_x * g.tiles_y;
+        g = row_squares(p, g);
     }
     return TraceBy::Rows;
 }
-template <bool REC, bool BEYOND>
+template <bool REC, int KIND>
 void launch_row_fwd(const DstParams &p, const DstAccelView &acc, const RowGrid &g, const uint32_t *ray_order, hipStream_t stream) {
-    const dim3 grid(BEYOND ? g.n_waves : (g.n_waves + 31u) / 32u * 32u), block(BEYOND ? kWavesPerBlock * DST_WAVE : DST_WAVE);
+    const dim3 grid(KIND != RowRays ? g.n_waves : (g.n_waves + 31u) / 32u * 32u), block(row_waves(KIND) * DST_WAVE);
 #define DST_ROW(AUX)                                                                                                       \
     do {                                                                                                                   \
-        if (p.flags != 0u) hipLaunchKernelGGL((k_row_fwd<AUX, REC, true, BEYOND>), grid, block, 0, stream, p, acc, g, ray_order); \
-        else hipLaunchKernelGGL((k_row_fwd<AUX, REC, false, BEYOND>), grid, block, 0, stream, p, acc, g, ray_order);  \
+        if (p.flags != 0u) hipLaunchKernelGGL((k_row_fwd<AUX, REC, true, KIND>), grid, block, 0, stream, p, acc, g, ray_order); \
+        else hipLaunchKernelGGL((k_row_fwd<AUX, REC, false, KIND>), grid, block, 0, stream, p, acc, g, ray_order);  \
     } while (0)
     if (p.aux <= 2) DST_ROW(2);
     else if (p.aux <= 4) DST_ROW(4);
@@ -2620,15 +2631,19 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
         // takes 29.9 ms with OFF, 2.8 with the hand-over and 0.24 by rows, a list of 20,000 rays there 813 and 290 us, a
         // 637x1013 room with one reflection 5.5 ms against 3.5.
         if (by == TraceBy::Rows && list == nullptr && (ctx->handover_mode != DST_HANDOVER_OFF || p.max_trace_depth > 0 || t.th_log2 < 3)) {
-            if (rec) launch_row_fwd<true, false>(p, acc, rows, ray_order, stream);
-            else launch_row_fwd<false, false>(p, acc, rows, ray_order, stream);
+            if (rec) launch_row_fwd<true, RowRays>(p, acc, rows, ray_order, stream);
+            else launch_row_fwd<false, RowRays>(p, acc, rows, ray_order, stream);
+        } else if (by != TraceBy::Rows && list == nullptr && ctx->handover_mode != DST_HANDOVER_OFF &&
+                   (uint64_t)p.H * p.W <= (rec ? kRowRecordedRays : kRowEvaluatedRays)) {
+            if (rec) launch_row_fwd<true, RowTiles>(p, acc, rows, ray_order, stream);
+            else launch_row_fwd<false, RowRays>(p, acc, row_squares(p, rows), ray_order, stream);
         } else if (by == TraceBy::TilesThenRows && list == nullptr) {
             if (rec) {
                 launch<false, true>(p, acc, t, ray_order, stream, nullptr, nullptr, 0u, true);
-                launch_row_fwd<true, true>(p, acc, rows, ray_order, stream);
+                launch_row_fwd<true, RowBeyond>(p, acc, rows, ray_order, stream);
             } else {
                 launch<false, false>(p, acc, t, ray_order, stream, nullptr, nullptr, 0u, true);
-                launch_row_fwd<false, true>(p, acc, rows, ray_order, stream);
+                launch_row_fwd<false, RowBeyond>(p, acc, rows, ray_order, stream);
             }
         } else
         for (int pass = 0; pass < (list != nullptr ? 2 : 1); ++pass) {

@@ -115,3 +115,45 @@ def test_reflections_of_images_traced_by_tiles(oracle, depth, aux, mode):
         for k, v in runs[1][0]["grads_gpu"].items():
             assert v is None or np.array_equal(v.view(np.uint32), runs[2][0]["grads_gpu"][k].view(np.uint32)), k
         assert np.array_equal(runs[0][1]["wet"], runs[1][1]["wet"])
+
+
+@pytest.mark.parametrize("size,depth,aux,det", [(264, 1, 2, False), (264, 3, 8, True), (328, 2, 4, False)])
+def test_tiles_then_rows_on_images_beyond_the_small_ones(oracle, size, depth, aux, det):
+    """First bounce by tiles, the others by rows, with a record (264x264) and without one (328x328)."""
+    import diff_surfel_tracing as dst
+    sc = S.scene_room(P=12000, seed=20 + depth, aux=aux, half=1.5)
+    sc["others_precomp"][:, 0] = sc["others_precomp"][:, 0] * 0.8 + 0.1
+    o, d = S.pinhole_rays(size, size, 70.0, (-0.6, -0.3, 0.15), (0.9, 0.45, -0.15))
+    rows, cols = slice(120, 140), slice(100, 124)
+    kw = dict(max_trace_depth=depth, specular_threshold=0.1)
+    tracer = dst.SurfelTracer()
+    tracer.deterministic = det
+    ug, ref, refg, refg64 = window_reference(oracle, sc, o, d, aux, rows, cols, **kw)
+    for step in range(2):
+        out, g = gpu_trace(tracer, sc, o, d, upstream=ug, build=(step == 0), **kw)
+        check_window(out, g, ref, refg, refg64, rows, cols, "step %d " % step)
+    assert tracer.optix_context._record_watch[-1].complete()
+    out, _ = gpu_trace(tracer, sc, o, d, build=False, **kw)
+    assert_forward_exact({k: v[rows, cols] for k, v in out.items() if k != "wet"}, ref)
+
+
+@pytest.mark.parametrize("n", [15, 16, 17, 33, 63, 64, 65, 124, 125, 130, 190, 300])
+def test_a_ray_goes_on_from_what_its_last_walk_left(oracle, n):
+    """Stacks of n faint quads, some at one depth, in front of a list of rays: chunks that end at the stack's end, kept quads
+    that just fit a row's memory or do not, and rays that graze the quads' edges."""
+    import diff_surfel_tracing as dst
+    from test_gpu_parity import check_case
+    gen = torch.Generator().manual_seed(n)
+    means = torch.stack([0.02 * torch.randn(n, generator=gen), 0.02 * torch.randn(n, generator=gen),
+                         1.0 + torch.floor(12.0 * torch.rand(n, generator=gen)) / 4.0], dim=-1)
+    means[::2, 2] += 0.001 * torch.arange(n)[::2]
+    rot = torch.zeros(n, 4)
+    rot[:, 0] = 1.0
+    # (scales unequal: a round quad has no gradient about its normal, only its rounding)
+    sc = {"means3D": means, "scales": torch.tensor([[0.1, 0.06]]).repeat(n, 1), "rotations": rot,
+          "opacities": 0.01 + 0.05 * torch.rand(n, 1, generator=gen), "shs": 0.3 * torch.randn(n, 16, 3, generator=gen)}
+    sc["vertices"], sc["faces"] = S.get_triangles(sc["means3D"], sc["scales"], sc["rotations"])
+    o = torch.zeros(1, 96, 3)
+    d = torch.nn.functional.normalize(torch.cat([0.12 * torch.randn(1, 96, 2, generator=gen), torch.ones(1, 96, 1)], dim=-1), dim=-1)
+    d[0, :16, 0] = 0.3 / 1.0      # past or along the nearest quads' edges
+    check_case(oracle, dst.SurfelTracer(), sc, o, d.contiguous())
