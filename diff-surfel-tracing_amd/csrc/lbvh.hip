@@ -352,8 +352,8 @@ __global__ void k_radix_hist(const uint32_t *__restrict__ keys, uint32_t *__rest
 }
 
 // Exclusive scan of the tile counters in two steps: block d scans the row of digit d (one counter per tile) in place
-// and leaves the row's total in row_total[d]; a second, tiny kernel turns the 256 totals into the digits' start
-// positions, which the scatter adds to a tile's entry.  (One block walking all 256 x tiles counters took 0.14 ms per
+// and leaves the row's total in row_total[d]; the scatter's workgroups each turn the 256 totals into the digits' start
+// positions, which they add to a tile's entry (a launch for it took 4.5 us a pass).  (One block walking all 256 x tiles counters took 0.14 ms per
 // pass at a million keys: a fifth of the whole build.)
 __global__ void k_scan_rows(uint32_t *tile_hist, uint32_t *row_total, uint32_t n_tiles) {
     __shared__ uint32_t wave_sum[1024 / DST_WAVE];
@@ -382,27 +382,27 @@ __global__ void k_scan_rows(uint32_t *tile_hist, uint32_t *row_total, uint32_t n
     }
     if (t == 0) row_total[blockIdx.x] = carry_s;
 }
-__global__ void k_scan_digits(uint32_t *row_total) {   // one block of kRadix threads, in place, exclusive
-    __shared__ uint32_t s[kRadix];
-    const uint32_t t = threadIdx.x;
-    s[t] = row_total[t];
-    __syncthreads();
-    for (uint32_t off = 1; off < kRadix; off <<= 1) {
-        const uint32_t add = t >= off ? s[t - off] : 0u;
-        __syncthreads();
-        s[t] += add;
-        __syncthreads();
-    }
-    row_total[t] = s[t] - row_total[t];
-}
-
 __global__ void k_radix_scatter(const uint32_t *__restrict__ keys_in, const uint32_t *__restrict__ vals_in,
                                 uint32_t *__restrict__ keys_out, uint32_t *__restrict__ vals_out,
-                                const uint32_t *__restrict__ tile_hist, const uint32_t *__restrict__ digit_start,
+                                const uint32_t *__restrict__ tile_hist, const uint32_t *__restrict__ row_total,
                                 uint32_t n, uint32_t n_tiles, int shift) {
     __shared__ uint32_t base[kBlock / DST_WAVE][kRadix];
+    __shared__ uint32_t digit_start[kRadix], part[kBlock / DST_WAVE];
     const int w = threadIdx.x / DST_WAVE, lane = threadIdx.x % DST_WAVE;
     const uint32_t tile = blockIdx.x * (kBlock / DST_WAVE) + w;
+    static_assert(kBlock == kRadix, "a thread per digit");
+    const uint32_t mine = row_total[threadIdx.x];
+    uint32_t upto = mine;
+#pragma unroll
+    for (int off = 1; off < DST_WAVE; off <<= 1) {
+        const uint32_t below = __shfl_up(upto, off);
+        if (lane >= off) upto += below;
+    }
+    if (lane == DST_WAVE - 1) part[w] = upto;
+    __syncthreads();
+    for (int k = 0; k < w; ++k) upto += part[k];
+    digit_start[threadIdx.x] = upto - mine;
+    __syncthreads();
     if (tile < n_tiles)
         for (int d = lane; d < kRadix; d += DST_WAVE) base[w][d] = tile_hist[(size_t)d * n_tiles + tile] + digit_start[d];
     __syncthreads();
@@ -727,6 +727,43 @@ __device__ __forceinline__ void wave_range_boxes(const float (&c)[4][3], bool va
     box_store(rb.pbox + 6 * (size_t)i, pre);
     box_store(rb.sbox + 6 * (size_t)i, suf);
     if (lane == DST_WAVE - 1 || i == n - 1u) box_store(rb.table + 6 * (size_t)(i / kRangeBlock), pre);   // level 0: whole blocks
+}
+// The first kRangeLow levels in one launch: a workgroup takes 1024 blocks and the 1023 behind them through LDS, joining
+// neighbours twice as far apart from level to level.  (A launch per level took 4.6 us each, ten of a refit's fourteen.)
+constexpr int kRangeLow = 10;
+constexpr uint32_t kRangeSpan = 1u << kRangeLow;
+__global__ __launch_bounds__(1024) void k_range_table_low(float *table, uint32_t n_blocks) {
+    __shared__ float s_box[6][2u * kRangeSpan];
+    const uint32_t t = threadIdx.x, from = blockIdx.x * kRangeSpan;
+    float box[2][6];
+    for (uint32_t h = 0; h < 2u; ++h) {
+        const uint32_t b = from + h * kRangeSpan + t;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            box[h][k] = b < n_blocks ? table[6 * (size_t)b + k] : (k < 3 ? INFINITY : -INFINITY);
+            s_box[k][h * kRangeSpan + t] = box[h][k];
+        }
+    }
+    __syncthreads();
+    for (int level = 1; level <= kRangeLow && (2u << (level - 1)) <= n_blocks; ++level) {
+        const uint32_t half = 1u << (level - 1);
+        for (uint32_t h = 0; h < 2u; ++h) {
+            const uint32_t at = h * kRangeSpan + t + half;
+            if (at < 2u * kRangeSpan) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    box[h][k] = fminf(box[h][k], s_box[k][at]);
+                    box[h][3 + k] = fmaxf(box[h][3 + k], s_box[3 + k][at]);
+                }
+            }
+        }
+        __syncthreads();
+        for (uint32_t h = 0; h < 2u; ++h)
+#pragma unroll
+            for (int k = 0; k < 6; ++k) s_box[k][h * kRangeSpan + t] = box[h][k];
+        __syncthreads();
+        if (from + t + 2u * half <= n_blocks) box_store(table + ((size_t)level * n_blocks + from + t) * 6, box[0]);
+    }
 }
 // table[level][b] = union of blocks b .. b + 2^level - 1 (entries that would run past the last block stay unused)
 __global__ void k_range_table_level(float *table, uint32_t n_blocks, int level) {
@@ -1198,18 +1235,17 @@ uint32_t *dst_static_scratch(const dst_ctx *ctx) {
 }
 
 // Stable LSD radix sort of (key, value) pairs, 32-bit keys, four 8-bit passes; the sorted pairs end in buffer 0.
-// tile_hist holds 256 counters per 1024 keys and 256 more for the digits' start positions (dst_sort_hist_elems).  Used by the BVH build (Morton codes) and by the ray ordering.
+// tile_hist holds 256 counters per 1024 keys and 256 more for the digits' totals (dst_sort_hist_elems).  Used by the BVH build (Morton codes) and by the ray ordering.
 void dst_sort_pairs(uint32_t *keys[2], uint32_t *vals[2], uint32_t *tile_hist, uint32_t n, hipStream_t stream) {
     const uint32_t tiles = (n + kTile - 1) / kTile;
     const uint32_t tile_blocks = (tiles + (kBlock / DST_WAVE) - 1) / (kBlock / DST_WAVE);
     int src = 0;
     for (int shift = 0; shift < 32; shift += kRadixBits) {
         hipLaunchKernelGGL(k_radix_hist, dim3(tile_blocks), dim3(kBlock), 0, stream, keys[src], tile_hist, n, tiles, shift);
-        uint32_t *digit_start = tile_hist + (size_t)tiles * kRadix;   // kRadix words behind the tile counters
-        hipLaunchKernelGGL(k_scan_rows, dim3(kRadix), dim3(1024), 0, stream, tile_hist, digit_start, tiles);
-        hipLaunchKernelGGL(k_scan_digits, dim3(1), dim3(kRadix), 0, stream, digit_start);
+        uint32_t *row_total = tile_hist + (size_t)tiles * kRadix;   // kRadix words behind the tile counters
+        hipLaunchKernelGGL(k_scan_rows, dim3(kRadix), dim3(1024), 0, stream, tile_hist, row_total, tiles);
         hipLaunchKernelGGL(k_radix_scatter, dim3(tile_blocks), dim3(kBlock), 0, stream, keys[src], vals[src],
-                           keys[1 - src], vals[1 - src], tile_hist, digit_start, n, tiles, shift);
+                           keys[1 - src], vals[1 - src], tile_hist, row_total, n, tiles, shift);
         src = 1 - src;
     }
 }
@@ -1336,7 +1372,9 @@ int dst_lbvh_build(dst_ctx *ctx, const float *vertices, uint32_t n_vertices, con
                            ctx->leaves, ctx->pre, rb, rebuild ? nullptr : ctx->bounds, ctx->bounds, n);
     if (by_ranges) {
         const uint32_t n_blocks = (n + kRangeBlock - 1) / kRangeBlock;
-        for (int level = 1; (2u << (level - 1)) <= n_blocks; ++level)
+        if (n_blocks > 1u)
+            hipLaunchKernelGGL(k_range_table_low, dim3((n_blocks + kRangeSpan - 1u) / kRangeSpan), dim3(1024), 0, stream, ctx->range_table, n_blocks);
+        for (int level = kRangeLow + 1; (2u << (level - 1)) <= n_blocks; ++level)
             hipLaunchKernelGGL(k_range_table_level, grid_for(n_blocks), dim3(kBlock), 0, stream, ctx->range_table, n_blocks, level);
         if (n > 1)
             hipLaunchKernelGGL(k_fit_ranges, grid_for(n - 1), dim3(kBlock), 0, stream, ctx->nodes, rb, n_blocks, n - 1);
