@@ -101,6 +101,9 @@ class _TraceSurfels(torch.autograd.Function):
             raise
         ctx.hit_record = record
 
+        # (outputs that the loss does not use: their gradients would each be filled with zeros before every backward trace,
+        # the largest, mid_val's, with 0.27 GB on a 1080p image, for nobody to read)
+        ctx.set_materialize_grads(False)
         ctx.tracer_settings = s
         ctx.optix_context = optix_context
         ctx.start_from_first = start_from_first
@@ -117,6 +120,12 @@ class _TraceSurfels(torch.autograd.Function):
         s = ctx.tracer_settings
         (ray_o, ray_d, vertices, means3D, shs, colors_precomp, others_precomp, opacities, scales, rotations,
          cov3Ds_precomp, out_rgb, out_dpt, out_acc, out_norm, out_dist, out_aux, mid_val) = ctx.saved_tensors
+        grad_out_rgb, grad_out_dpt, grad_out_acc, grad_out_norm, grad_out_aux = (
+            torch.zeros_like(out) if grad is None else grad
+            for grad, out in ((grad_out_rgb, out_rgb), (grad_out_dpt, out_dpt), (grad_out_acc, out_acc),
+                              (grad_out_norm, out_norm), (grad_out_aux, out_aux)))
+        if grad_out_dist is None:   # (nothing flows back from the distortion)
+            grad_out_dist = _placeholder(out_rgb.device)
         args = (ctx.optix_context, ctx.start_from_first, ray_o, ray_d, vertices, s.bg, means3D, shs, s.sh_degree,
                 colors_precomp, others_precomp, opacities, scales, s.scale_modifier, rotations,
                 cov3Ds_precomp) + _settings_args(s) + (
