@@ -120,8 +120,8 @@ typedef struct DstParams {
     unsigned long long *det_workspace;
     /* optional gradient rows (no counterpart in the reference): dst_det_workspace_words(P, aux, 1) floats of device
      * memory, zero-filled by the caller before each backward call.  When non-NULL (and not in the deterministic
-     * mode) the backward trace sums the per-surfel gradients in this buffer, where the columns of one surfel lie
-     * side by side in one row, and a closing kernel of the same call adds the rows to the dL_d* tensors below.
+     * mode) the backward trace sums the per-surfel gradients in this buffer, where the 64 columns of one surfel lie
+     * side by side in one row (the auxiliary channels behind all rows), and a closing kernel of the same call adds the rows to the dL_d* tensors below.
      * Same results up to the order of the float additions; faster, because a hit's 66-72 atomic additions then go
      * to a few consecutive cache lines instead of one line in each of seven tensors. */
     float *grad_rows;
