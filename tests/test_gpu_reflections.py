@@ -157,3 +157,31 @@ def test_a_ray_goes_on_from_what_its_last_walk_left(oracle, n):
     d = torch.nn.functional.normalize(torch.cat([0.12 * torch.randn(1, 96, 2, generator=gen), torch.ones(1, 96, 1)], dim=-1), dim=-1)
     d[0, :16, 0] = 0.3 / 1.0      # past or along the nearest quads' edges
     check_case(oracle, dst.SurfelTracer(), sc, o, d.contiguous())
+
+
+@pytest.mark.parametrize("blocks", [16, 17])
+def test_a_list_whose_record_is_one_block_short(oracle, blocks):
+    """512 rays, 128 waves: their first pieces fill sixteen blocks of the record, the few pieces that two waves ask for
+    beyond those lie in a seventeenth, of which nobody gets the first piece.  With sixteen blocks the record has to be
+    known to be incomplete, with seventeen it is replayed."""
+    import diff_surfel_tracing as dst
+    from test_gpu_parity import check_case
+    gen = torch.Generator().manual_seed(17)
+    n = 40
+    means = torch.stack([0.02 * torch.randn(n, generator=gen), 0.02 * torch.randn(n, generator=gen), 1.0 + 0.05 * torch.arange(n)], dim=-1)
+    rot = torch.zeros(n, 4)
+    rot[:, 0] = 1.0
+    sc = {"means3D": means, "scales": torch.tensor([[0.3, 0.2]]).repeat(n, 1), "rotations": rot,
+          "opacities": 0.01 + 0.05 * torch.rand(n, 1, generator=gen), "shs": 0.3 * torch.randn(n, 16, 3, generator=gen)}
+    sc["vertices"], sc["faces"] = S.get_triangles(sc["means3D"], sc["scales"], sc["rotations"])
+    o = torch.zeros(1, 512, 3)
+    d = torch.cat([0.02 * torch.randn(1, 512, 2, generator=gen), torch.ones(1, 512, 1)], dim=-1)
+    d[:, 8:] *= -1.0      # the first two waves' rays meet everything, the others nothing
+    tracer = dst.SurfelTracer()
+    ctx = tracer.optix_context
+    ctx.record_blocks_per_wave = (blocks - 0.5) / dst._C.HitRecord.layout(1, 512, 0, 1.0)[3]
+    ctx.update_record_estimate = lambda: None
+    ref, _ = check_case(oracle, tracer, sc, o, torch.nn.functional.normalize(d, dim=-1).contiguous())
+    assert (ref["n_proc"].reshape(-1)[:8] > 32).all() and not ref["n_proc"].reshape(-1)[8:].any()
+    rec = ctx._record_watch[-1]
+    assert rec.blocks == blocks and rec.requested_blocks() == 17 and rec.complete() == (blocks == 17)
