@@ -274,7 +274,8 @@ __device__ __forceinline__ float safe_inv(float d) {
     return 1.0f / v;
 }
 
-__device__ __forceinline__ RaySlab make_slab(F3 o, F3 d, float max_abs) {
+// (`reach`: how large the numbers are that the ray's origin was made from, where it has been moved up along the ray.)
+__device__ __forceinline__ RaySlab make_slab(F3 o, F3 d, float max_abs, float reach = 0.f) {
     RaySlab s;
     s.ix = safe_inv(d.x);
     s.iy = safe_inv(d.y);
@@ -285,7 +286,7 @@ __device__ __forceinline__ RaySlab make_slab(F3 o, F3 d, float max_abs) {
     // The quad test works in origin-relative fp32 coordinates, so it can accept a ray that passes
     // a few ulps of (|o| + |vertex|) outside the quad; boxes are widened by well above that: by 4e-6 |o| here,
     // and by 4e-6 of the quad's own largest coordinate where the boxes are made (lbvh.hip, kBoxPad).
-    float oa = __builtin_fmaxf(__builtin_fabsf(o.x), __builtin_fmaxf(__builtin_fabsf(o.y), __builtin_fabsf(o.z)));
+    float oa = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(o.x), reach), __builtin_fmaxf(__builtin_fabsf(o.y), __builtin_fabsf(o.z)));
     s.max_abs = max_abs;
     float pad = 4e-6f * oa;
     s.wx = pad * __builtin_fabsf(s.ix);

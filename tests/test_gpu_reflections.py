@@ -185,3 +185,40 @@ def test_a_list_whose_record_is_one_block_short(oracle, blocks):
     assert (ref["n_proc"].reshape(-1)[:8] > 32).all() and not ref["n_proc"].reshape(-1)[8:].any()
     rec = ctx._record_watch[-1]
     assert rec.blocks == blocks and rec.requested_blocks() == 17 and rec.complete() == (blocks == 17)
+
+
+def _pairs_of_quads(n, gen, along, apart):
+    """`n` pairs of faint quads across the z axis, each pair at one place, the next 0.02 further on (a pair is one leaf group
+    of the hierarchy, with a flat box).  Their low x sides lie along the line x = along * z, `apart` from it at random, and they
+    end within their Gaussian there, so that every one of them shows."""
+    z = 1.0 + 0.02 * torch.arange(n).repeat_interleave(2)
+    side = along * z + apart * torch.randn(n, generator=gen).repeat_interleave(2)
+    means = torch.stack([side + 0.5, torch.zeros(2 * n), z], dim=-1)
+    rot = torch.zeros(2 * n, 4)
+    rot[:, 0] = 1.0
+    sc = {"means3D": means, "scales": torch.tensor([[0.6, 0.5]]).repeat(2 * n, 1), "rotations": rot,
+          "opacities": 0.01 + 0.01 * torch.rand(2 * n, 1, generator=gen), "shs": 0.3 * torch.randn(2 * n, 16, 3, generator=gen)}
+    corner = torch.tensor([[-0.5, -0.6, 0.0], [-0.5, 0.6, 0.0], [0.5, -0.6, 0.0], [0.5, 0.6, 0.0]])
+    sc["vertices"] = (means[:, None, :] + corner).reshape(-1, 3).contiguous()
+    sc["faces"] = S.get_triangles(sc["means3D"], sc["scales"], sc["rotations"])[1]
+    return sc
+
+
+@pytest.mark.parametrize("distance", [3.0, 300.0, 3000.0, 30000.0])
+def test_rays_from_far_away_along_the_sides_of_quads(oracle, distance):
+    """A chunk's origin carries the rounding of the ray's own, however close to the scene it lies: chunks of a ray that comes
+    from thousands of scene sizes away look along lines that far apart, and what one of them passes by another may meet.  The
+    first walk keeps more than fits a row's memory, the second one what the others go on from."""
+    import diff_surfel_tracing as dst
+    gen = torch.Generator().manual_seed(int(distance))
+    ulp = distance * 2.0 ** -24
+    sc = _pairs_of_quads(80, gen, 0.7, 4.0 * ulp)
+    R = 2048
+    d = torch.nn.functional.normalize(torch.tensor([0.7, 0.05, 1.0]), dim=0).expand(1, R, 3).contiguous()
+    at = torch.stack([0.7 * 2.0 + 4.0 * ulp * torch.randn(R, generator=gen), 0.1 * torch.randn(R, generator=gen), torch.full((R,), 2.0)], dim=-1)
+    o = (at.double() - (distance * (1.0 + 0.2 * torch.rand(R, 1, generator=gen))).double() * d[0].double()).float()[None].contiguous()
+    s = oracle_scene(oracle, sc, o, d)
+    ref = oracle.forward(s, oracle.HITS_BRUTE_LEXI)
+    assert (ref["n_proc"] > 40).sum() > R // 8
+    out, _ = gpu_trace(dst.SurfelTracer(), sc, o, d)
+    assert_forward_exact(out, ref)
