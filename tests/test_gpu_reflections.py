@@ -222,3 +222,28 @@ def test_rays_from_far_away_along_the_sides_of_quads(oracle, distance):
     assert (ref["n_proc"] > 40).sum() > R // 8
     out, _ = gpu_trace(dst.SurfelTracer(), sc, o, d)
     assert_forward_exact(out, ref)
+
+
+@pytest.mark.parametrize("length", [1.0, 1e-3, 1e-5])
+def test_short_directions_along_quads_of_one_plane(oracle, length):
+    """Directions need not be of length one.  Sixty quads of one plane, met at a slant, and as many of another behind it: which
+    of them lie behind a chunk's origin is a matter of the origin's rounding, which does not shrink with the direction."""
+    import diff_surfel_tracing as dst
+    gen = torch.Generator().manual_seed(7)
+    n, R = 120, 1024
+    normal = torch.nn.functional.normalize(torch.tensor([-0.6, 0.2, 1.0]), dim=0)
+    q = torch.nn.functional.normalize(torch.stack([1 + normal[2], -normal[1], normal[0], torch.tensor(0.0)]), dim=0)   # z into the normal
+    sc = {"scales": 0.3 + 0.1 * torch.rand(n, 2, generator=gen), "rotations": q.expand(n, 4).contiguous(),
+          "opacities": 0.02 + 0.02 * torch.rand(n, 1, generator=gen), "shs": 0.3 * torch.randn(n, 16, 3, generator=gen)}
+    x = torch.nn.functional.normalize(torch.tensor([1.0, 0.0, 0.6]), dim=0)      # in the plane
+    y = torch.linalg.cross(normal, x)
+    centre = torch.where((torch.arange(n) < n // 2)[:, None], torch.tensor([2.0, 1.0, 2.0]), torch.tensor([3.0, 1.5, 3.0]))
+    sc["means3D"] = (centre + 0.1 * torch.randn(n, 1, generator=gen) * x + 0.1 * torch.randn(n, 1, generator=gen) * y).contiguous()
+    sc["vertices"], sc["faces"] = S.get_triangles(sc["means3D"], sc["scales"], sc["rotations"])
+    o = (0.05 * torch.randn(1, R, 3, generator=gen)).contiguous()
+    d = length * torch.nn.functional.normalize(torch.tensor([2.0, 1.0, 2.0]) + 0.1 * torch.randn(1, R, 3, generator=gen), dim=-1)
+    s = oracle_scene(oracle, sc, o, d.contiguous())
+    ref = oracle.forward(s, oracle.HITS_BRUTE_LEXI)
+    assert (ref["n_proc"] > 16).sum() > R // 2
+    out, _ = gpu_trace(dst.SurfelTracer(), sc, o, d.contiguous())
+    assert_forward_exact(out, ref)
