@@ -539,7 +539,7 @@ __global__ void k_ploc_init(const float *__restrict__ vertices, const int4 *__re
     if (m == 0) {
         pb.state[0] = pb.state[1] = n;
         pb.state[2] = pb.state[3] = 0u;
-        pb.state[4] = pb.state[5] = pb.state[6] = pb.state[7] = 0u;
+        pb.state[4] = pb.state[5] = pb.state[6] = pb.state[7] = pb.state[8] = 0u;
     }
     if (m >= n) return;
     const uint32_t g = sorted_ids[m];
@@ -1138,7 +1138,7 @@ int ensure_capacity(dst_ctx *ctx, uint32_t P) {
     }
     ctx->tile_hist_elems = tiles * kRadix + kRadix;
     DST_HIP(ctx, hipMalloc((void **)&ctx->tile_hist, sizeof(uint32_t) * ctx->tile_hist_elems));
-    ctx->ploc_blocks = (uint32_t)((n + kPlocOwn - 1) / kPlocOwn);
+    ctx->ploc_blocks = (uint32_t)((n + ploc_own(4) - 1) / ploc_own(4));
     DST_HIP(ctx, hipMalloc((void **)&ctx->ploc_state, sizeof(uint32_t) * (kPlocStateWords + 2 * ((size_t)ctx->ploc_blocks + 1))));
     DST_HIP(ctx, hipMemset(ctx->ploc_state, 0xFF, sizeof(uint32_t) * kPlocStateWords));   // depth word: "too deep" until a build says otherwise
     if (!ctx->ploc_host) DST_HIP(ctx, hipHostMalloc((void **)&ctx->ploc_host, sizeof(uint32_t) * kPlocStateWords, hipHostMallocDefault));
@@ -1181,18 +1181,20 @@ int ploc_hierarchy(dst_ctx *ctx, const float *vertices, uint32_t n, hipStream_t 
     pb.n_blocks = ctx->ploc_blocks;
     hipLaunchKernelGGL(k_ploc_init, grid_for(n), dim3(kBlock), 0, stream, vertices, reinterpret_cast<const int4 *>(ctx->quad_ids),
                        ctx->vals[0], pb, n);
-    // As many launches as leave few enough for one workgroup if each leaves three fifths of the clusters (an eighth merges
-    // per round on the scenes measured here); one that finds no more to do takes 4 us.  Then the layout, without waiting
-    // for the count: its kernels find nothing to do unless the rounds came to an end.
+    // As many launches as leave few enough for one workgroup if a round leaves seven eighths of the clusters, as it does on the
+    // scenes measured here, or a little more (three rounds 0.69, four 0.6); one that finds no more to do takes 4 us.  Then the
+    // layout, without waiting for the count: its kernels find nothing to do unless the rounds came to an end.
     int it = 0;
     uint32_t count = n;
     for (;;) {
-        const dim3 grid((count + kPlocOwn - 1) / kPlocOwn);   // enough for the largest count this batch can see
-        int batch = 0;
-        for (double left = count; left > kPlocTail; left *= 0.6) ++batch;
-        for (int k = 0; k < batch; ++k, ++it) {
-            hipLaunchKernelGGL(k_ploc_rounds, grid, dim3(kPlocBlock), 0, stream, pb, it);
-            hipLaunchKernelGGL(k_ploc_scan, dim3(1), dim3(kPlocBlock), 0, stream, pb, it);
+        for (double left = count; left > kPlocTail; ++it) {
+            const bool many = left > kPlocMany;
+            const uint32_t own = many ? ploc_own(3) : ploc_own(4);
+            const dim3 grid((count + own - 1) / own);   // enough for the largest count this batch can see
+            if (many) hipLaunchKernelGGL(k_ploc_rounds<3>, grid, dim3(kPlocBlock), 0, stream, pb, it);
+            else hipLaunchKernelGGL(k_ploc_rounds<4>, grid, dim3(kPlocBlock), 0, stream, pb, it);
+            hipLaunchKernelGGL(k_ploc_scan, dim3(1), dim3(kPlocBlock), 0, stream, pb, it, own);
+            left *= many ? 0.69 : 0.6;
         }
         hipLaunchKernelGGL(k_ploc_tail, dim3(1), dim3(kPlocBlock), 0, stream, pb, it);
         hipLaunchKernelGGL(k_ploc_leaf_positions, grid_for(n), dim3(kBlock), 0, stream, pb, ctx->vals[0], ctx->vals[1], n);

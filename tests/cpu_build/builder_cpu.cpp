@@ -253,6 +253,185 @@ void run_case(uint32_t P, int kind, bool agglomerate, uint32_t seed) {
     std::free(ctx.ploc_host);
 }
 
+// ---- the rounds of the agglomeration, several to a launch on a window of the clusters, against rounds over all of them -------
+struct Cluster { float lo, hi; uint32_t id, low, size; };   // a box (lo,lo,lo) .. (hi,hi,hi)
+struct Merge { uint32_t c0, c1, size; };
+bool operator==(const Merge &a, const Merge &b) { return a.c0 == b.c0 && a.c1 == b.c1 && a.size == b.size; }
+
+void whole_round(std::vector<Cluster> &c, std::vector<Merge> &made) {
+    const int n = (int)c.size();
+    auto area = [&](int i, int j) {
+        const float e = std::max(c[i].hi, c[j].hi) - std::min(c[i].lo, c[j].lo);
+        return e * e + e * e + e * e;
+    };
+    std::vector<int> nn(n);
+    for (int i = 0; i < n; ++i) {
+        float best = INFINITY;
+        nn[i] = i;
+        for (int d = 1; d <= kPlocRadius; ++d) {
+            const float up = i + d < n ? area(i, i + d) : INFINITY, down = i >= d ? area(i, i - d) : INFINITY;
+            const bool lower = down < up || (down == up && i >= d && c[i - d].low * 2654435761u < c[i].low * 2654435761u);
+            if ((lower ? down : up) < best) {
+                best = lower ? down : up;
+                nn[i] = lower ? i - d : i + d;
+            }
+        }
+    }
+    std::vector<Cluster> next;
+    for (int i = 0; i < n; ++i) {
+        const int j = nn[i];
+        if (j == i || nn[j] != i) { next.push_back(c[i]); continue; }
+        if (j < i) continue;
+        const uint32_t node = c[j].low - 1u;
+        made[node] = {c[i].id, c[j].id, c[i].size + c[j].size};
+        next.push_back({std::min(c[i].lo, c[j].lo), std::max(c[i].hi, c[j].hi), node, c[i].low, made[node].size});
+    }
+    c.swap(next);
+}
+
+struct PlocTest {   // the buffers of ploc_hierarchy
+    std::vector<float> box[2];
+    std::vector<uint32_t> words[11];
+    PlocBufs pb;
+    explicit PlocTest(uint32_t n) {
+        for (auto &b : box) b.assign(6 * (size_t)n, NAN);
+        for (auto &w : words) w.assign(2 * (size_t)n + 64, 0xDEADBEEFu);
+        pb.box[0] = box[0].data();
+        pb.box[1] = box[1].data();
+        uint32_t **to[] = {&pb.id[0], &pb.id[1], &pb.low[0], &pb.low[1], &pb.nn, &pb.pre, &pb.tc0, &pb.tc1, &pb.tsize, &pb.up, &pb.lpar};
+        for (int k = 0; k < 11; ++k) *to[k] = words[k].data();
+        pb.n_blocks = (n + ploc_own(4) - 1) / ploc_own(4);
+        state.assign(kPlocStateWords + 2 * ((size_t)pb.n_blocks + 1), 0u);
+        pb.state = state.data();
+    }
+    std::vector<uint32_t> state;
+};
+
+// `rounds`: 3 or 4 to a launch; 0: in turn
+void check_rounds(std::vector<Cluster> c, int rounds, const char *what) {
+    const uint32_t n = (uint32_t)c.size();
+    PlocTest t(n);
+    for (uint32_t i = 0; i < n; ++i) {
+        for (int k = 0; k < 3; ++k) {
+            t.box[0][6 * (size_t)i + k] = c[i].lo;
+            t.box[0][6 * (size_t)i + 3 + k] = c[i].hi;
+        }
+        t.pb.id[0][i] = c[i].id = DST_LEAF_BIT | i;
+        t.pb.low[0][i] = c[i].low = i;
+        c[i].size = 1u;
+    }
+    t.state[0] = t.state[1] = n;
+    int it = 0;
+    for (; t.state[it & 1] > kPlocTail && it < 200; ++it) {
+        const int r = rounds != 0 ? rounds : 3 + it % 2;
+        const uint32_t own = ploc_own(r);
+        if (r == 3) hipLaunchKernelGGL(k_ploc_rounds<3>, dim3((n + own - 1) / own), dim3(kPlocBlock), 0, nullptr, t.pb, it);
+        else hipLaunchKernelGGL(k_ploc_rounds<4>, dim3((n + own - 1) / own), dim3(kPlocBlock), 0, nullptr, t.pb, it);
+        hipLaunchKernelGGL(k_ploc_scan, dim3(1), dim3(kPlocBlock), 0, nullptr, t.pb, it, own);
+    }
+    hipLaunchKernelGGL(k_ploc_tail, dim3(1), dim3(kPlocBlock), 0, nullptr, t.pb, it);
+    std::vector<Merge> want(n - 1);
+    while (c.size() > 1) whole_round(c, want);
+    uint32_t off = 0;
+    for (uint32_t k = 0; k + 1 < n; ++k) off += Merge{t.pb.tc0[k], t.pb.tc1[k], t.pb.tsize[k]} == want[k] ? 0u : 1u;
+    CHECK(off == 0u && t.state[0] == 1u && t.state[3] == n, "%s: %u of %u merges differ from rounds over all clusters", what, off, n - 1);
+    std::printf("rounds %-40s %u clusters, %d launches, %u merges off\n", what, n, it, off);
+}
+void check_rounds(const std::vector<float> &at, int rounds, const char *what) {
+    std::vector<Cluster> c;
+    for (float t : at) c.push_back({t, t, 0u, 0u, 0u});
+    check_rounds(c, rounds, what);
+}
+
+// An order in which news travels as far as it can in four rounds: what lies 289 places beyond position `edge` (233 before
+// it, `before`) decides about a merge of the cluster next to the edge.  Everything lies in tight groups of eight, each at a
+// site of its own, that halve their number in every round; eight clusters a round merge across the edge (a merged cluster
+// goes on in the lower one's place, so those beyond the edge lose eight, those before it none); and in every round there
+// are three clusters eight places apart, a, b and c, of which b takes c where c is (still) alone, and a where not.
+std::vector<float> far_reaching_order(uint32_t n, uint32_t edge, bool before) {
+    const float in_group[8] = {0.f, 0.05f, 0.3f, 0.35f, 1.5f, 1.55f, 1.8f, 1.85f};
+    uint32_t site = 0;
+    std::vector<float> beyond, inside;   // places from the edge on, away from it and into the other side
+    auto group = [&](std::vector<float> &to, uint32_t points, float where) {
+        for (uint32_t k = 0; k < points; ++k) to.push_back(where + in_group[k]);
+    };
+    auto elsewhere = [&](std::vector<float> &to, uint32_t points) { group(to, points, 100.f * (float)(site++ % 60)); };
+    const float home = 7000.f, a3 = home - 34.f, b3 = home - 25.f, a2 = home - 18.f, b2 = home - 12.f, a1 = home - 7.f, b1 = home - 3.f;
+    if (before) {
+        group(inside, 8, a3);
+    } else {
+        // the last eight clusters before the edge, the edge's side first; what they merge with beyond it in rounds 0, 1 and 2
+        float u[8];
+        for (int k = 0; k < 8; ++k) u[k] = k == 7 ? a3 : 6100.f + 100.f * (float)k;
+        for (int k = 7; k >= 0; --k) inside.push_back(u[k]);
+        for (int k = 0; k < 8; ++k) beyond.push_back(u[k] + 0.05f);
+        for (int k = 0; k < 8; ++k) group(beyond, 2, u[k] + 0.3f);
+        for (int k = 0; k < 8; ++k) group(beyond, 4, u[k] + 0.9f);
+    }
+    for (int k = 0; k < 15; ++k) {
+        if (k == 7) group(beyond, 8, b3);
+        else elsewhere(beyond, 8);
+    }
+    auto seven = [&](uint32_t points) {   // seven clusters of a round
+        for (int k = 0; k < 3; ++k) elsewhere(beyond, 2 * points);
+        elsewhere(beyond, points);
+    };
+    group(beyond, 4, a2);
+    seven(4);
+    group(beyond, 4, b2);
+    seven(4);
+    group(beyond, 2, a1);
+    seven(2);
+    group(beyond, 2, b1);
+    seven(2);
+    beyond.push_back(home);
+    seven(1);
+    beyond.push_back(home + 2.f);
+    seven(1);
+    beyond.push_back(home + 3.9f);
+    std::vector<float> at(n);
+    for (uint32_t i = 0; i < n; ++i) at[i] = 100.f * (float)((i / 8u) % 60) + 30.f + in_group[i % 8u];   // (all else)
+    for (uint32_t k = 0; k < beyond.size(); ++k) at[before ? edge - 1u - k : edge + k] = beyond[k];
+    for (uint32_t k = 0; k < inside.size(); ++k) at[before ? edge + k : edge - 1u - k] = inside[k];
+    return at;
+}
+
+void check_windows() {
+    char what[96];
+    for (int before = 0; before < 2; ++before)
+        for (uint32_t k = 1; k < 4; k += 2) {
+            std::snprintf(what, sizeof(what), "four, far-reaching %s %u", before ? "before" : "beyond", k * ploc_own(4));
+            check_rounds(far_reaching_order(3000, k * ploc_own(4), before != 0), 4, what);
+            // three rounds: what the first of the four leaves, with the edge where it then lies
+            bool found = false;
+            for (uint32_t edge = 2 * k * ploc_own(3) - 24; !found && edge < 2 * k * ploc_own(3) + 24; ++edge) {
+                std::vector<Cluster> c;
+                for (float t : far_reaching_order(6000, edge, before != 0)) c.push_back({t, t, 0u, (uint32_t)c.size(), 1u});
+                std::vector<Merge> made(c.size());
+                whole_round(c, made);
+                uint32_t at = 0;
+                while (c[at].low < edge) ++at;
+                found = at == k * ploc_own(3);
+                if (!found) continue;
+                std::snprintf(what, sizeof(what), "three, far-reaching %s %u", before ? "before" : "beyond", at);
+                check_rounds(c, 3, what);
+            }
+            CHECK(found, "no order with an edge at %u", k * ploc_own(3));
+        }
+    std::mt19937 rng(5);
+    for (uint32_t n : {1025u, 2900u, 5000u}) {
+        for (int kind = 0; kind < 3; ++kind) {   // even, clustered, equal
+            std::vector<float> at(n);
+            for (float &t : at) {
+                t = std::uniform_real_distribution<float>(0.f, 1000.f)(rng);
+                if (kind == 1) t = std::round(t / 50.f) * 50.f + std::exp2(-(float)(rng() % 12u)) * t / 100.f;
+                if (kind == 2) t = std::round(t / 200.f);
+            }
+            for (int rounds : {0, 3, 4}) check_rounds(at, rounds, kind == 0 ? "even" : (kind == 1 ? "clustered" : "equal"));
+        }
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -262,6 +441,7 @@ int main(int argc, char **argv) {
         std::printf(failures ? "FAILED: %d checks\n" : "ALL OK\n", failures);
         return failures ? 1 : 0;
     }
+    check_windows();
     const bool quick = argc > 1 && std::string(argv[1]) == "quick";
     const uint32_t sizes[] = {1, 2, 3, 63, 64, 65, 100, 1024, 1025, 2500, 5000};
     for (int agg = 1; agg >= 0; --agg) {
