@@ -1158,8 +1158,8 @@ uint32_t *g_refit_scratch_ptr[kMaxDevices] = {};
 
 // Hierarchy by agglomeration (see above).  Scratch comes from buffers that are idle between the sort and the leaf
 // records: the range boxes (cluster boxes, per-cluster words), the centroids (temporary nodes), the sort's second
-// value buffer and the fit's arrival counters (cluster ids).  Reads the cluster count back every few rounds, to know
-// when one workgroup can finish; leaves the sorted surfel ids of the new leaf order in ctx->vals[0].
+// value buffer and the fit's arrival counters (cluster ids).  Waits for the stream behind the layout, once unless the
+// rounds merge unusually little; leaves the sorted surfel ids of the new leaf order in ctx->vals[0].
 int ploc_hierarchy(dst_ctx *ctx, const float *vertices, uint32_t n, hipStream_t stream) {
     PlocBufs pb;
     pb.box[0] = ctx->range_pbox;
@@ -1198,7 +1198,7 @@ int ploc_hierarchy(dst_ctx *ctx, const float *vertices, uint32_t n, hipStream_t 
         }
         hipLaunchKernelGGL(k_ploc_tail, dim3(1), dim3(kPlocBlock), 0, stream, pb, it);
         hipLaunchKernelGGL(k_ploc_leaf_positions, grid_for(n), dim3(kBlock), 0, stream, pb, ctx->vals[0], ctx->vals[1], n);
-        hipLaunchKernelGGL(k_ploc_node_numbers, grid_for(n - 1), dim3(kBlock), 0, stream, pb, ctx->nodes, n);
+        hipLaunchKernelGGL(k_ploc_node_numbers, grid_for(n), dim3(kBlock), 0, stream, pb, ctx->vals[0], ctx->vals[1], ctx->nodes, n);
         hipLaunchKernelGGL(k_ploc_links, grid_for(n - 1), dim3(kBlock), 0, stream, pb, ctx->nodes, ctx->node_parent, ctx->leaf_parent, n);
         DST_HIP(ctx, hipGetLastError());
         DST_HIP(ctx, hipMemcpyAsync(ctx->ploc_host, ctx->ploc_state, sizeof(uint32_t) * kPlocStateWords, hipMemcpyDeviceToHost, stream));

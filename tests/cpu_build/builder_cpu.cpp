@@ -343,6 +343,44 @@ void check_rounds(const std::vector<float> &at, int rounds, const char *what) {
     check_rounds(c, rounds, what);
 }
 
+// The layout of 200 leaves over links of which one or two are not those of a hierarchy, though the counts at its root are: a
+// build has to find out (state[4]), whatever the buffers held before.
+void check_broken_links() {
+    const uint32_t n = 200;
+    for (int kind = 0; kind < 4; ++kind) {   // none; a leaf in another's place; a node in another's; a leaf on its sibling's side
+        PlocTest t(n);
+        std::mt19937 rng(3);
+        for (uint32_t i = 0; i < n; ++i) {
+            for (int k = 0; k < 6; ++k) t.box[0][6 * (size_t)i + k] = std::uniform_real_distribution<float>(0.f, 1.f)(rng) * (k % 3 == 0);
+            for (int k = 0; k < 3; ++k) t.box[0][6 * (size_t)i + 3 + k] = t.box[0][6 * (size_t)i + k] + 0.01f;
+            t.pb.id[0][i] = DST_LEAF_BIT | i;
+            t.pb.low[0][i] = i;
+        }
+        t.state[0] = t.state[1] = n;
+        hipLaunchKernelGGL(k_ploc_tail, dim3(1), dim3(kPlocBlock), 0, nullptr, t.pb, 0);
+        const uint32_t root = t.state[2];
+        if (kind == 1) t.pb.lpar[7] = t.pb.lpar[150];
+        if (kind == 2) {   // two nodes of one size
+            for (uint32_t a = 0, done = 0; a + 1 < n && !done; ++a)
+                for (uint32_t b = a + 1; b + 1 < n && !done; ++b)
+                    if (t.pb.tsize[a] == t.pb.tsize[b] && a != root && b != root) {
+                        t.pb.up[2 * a] = t.pb.up[2 * b];
+                        done = 1;
+                    }
+        }
+        if (kind == 3) t.pb.lpar[20] ^= 1u;
+        std::vector<uint32_t> in(n), out(n, 0xFFFFFFFFu), node_parent(n), leaf_parent(n);
+        for (uint32_t i = 0; i < n; ++i) in[i] = (i * 77u) % n;
+        for (uint32_t i = 0; i < n; ++i) out[i] = DST_LEAF_BIT | i;
+        std::vector<DstNode> nodes(n - 1);
+        hipLaunchKernelGGL(k_ploc_leaf_positions, dim3(1), dim3(kBlock), 0, nullptr, t.pb, in.data(), out.data(), n);
+        hipLaunchKernelGGL(k_ploc_node_numbers, dim3(1), dim3(kBlock), 0, nullptr, t.pb, in.data(), out.data(), nodes.data(), n);
+        hipLaunchKernelGGL(k_ploc_links, dim3(1), dim3(kBlock), 0, nullptr, t.pb, nodes.data(), node_parent.data(), leaf_parent.data(), n);
+        CHECK(t.state[0] == 1u && t.state[3] == n, "broken links %d: one cluster of %u", kind, n);
+        CHECK((t.state[4] != 0u) == (kind != 0), "broken links %d: %u", kind, t.state[4]);
+    }
+}
+
 // An order in which news travels as far as it can in four rounds: what lies 289 places beyond position `edge` (233 before
 // it, `before`) decides about a merge of the cluster next to the edge.  Everything lies in tight groups of eight, each at a
 // site of its own, that halve their number in every round; eight clusters a round merge across the edge (a merged cluster
@@ -442,6 +480,7 @@ int main(int argc, char **argv) {
         return failures ? 1 : 0;
     }
     check_windows();
+    check_broken_links();
     const bool quick = argc > 1 && std::string(argv[1]) == "quick";
     const uint32_t sizes[] = {1, 2, 3, 63, 64, 65, 100, 1024, 1025, 2500, 5000};
     for (int agg = 1; agg >= 0; --agg) {
