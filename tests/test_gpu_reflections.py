@@ -159,6 +159,33 @@ def test_a_ray_goes_on_from_what_its_last_walk_left(oracle, n):
     check_case(oracle, dst.SurfelTracer(), sc, o, d.contiguous())
 
 
+@pytest.mark.parametrize("n,batches", [(60, 1), (140, 1), (400, 1), (400, 9)])
+def test_rays_with_and_without_room_share_a_wave(oracle, n, batches):
+    """One ray of every four meets a stack of n quads, more than its row has room to keep where n is large; its neighbours meet
+    a dozen or three dozen, or nothing.  Once one ray of a wave has no room, none of the wave's walks keeps anything any more
+    until all have ended.  (A list of 2304 rays is traced in an order of its own.)"""
+    import diff_surfel_tracing as dst
+    from test_gpu_parity import check_case
+    gen = torch.Generator().manual_seed(n)
+    sizes, x = [n, 12, 36], [0.0, 4.0, 8.0]
+    means = torch.cat([torch.stack([x[k] + 0.02 * torch.randn(m, generator=gen), 0.02 * torch.randn(m, generator=gen),
+                                    1.0 + 3.0 * torch.rand(m, generator=gen)], dim=-1) for k, m in enumerate(sizes)])
+    P = means.shape[0]
+    rot = torch.zeros(P, 4)
+    rot[:, 0] = 1.0
+    sc = {"means3D": means, "scales": torch.tensor([[0.1, 0.06]]).repeat(P, 1), "rotations": rot,
+          "opacities": 0.01 + 0.03 * torch.rand(P, 1, generator=gen), "shs": 0.3 * torch.randn(P, 16, 3, generator=gen)}
+    sc["vertices"], sc["faces"] = S.get_triangles(sc["means3D"], sc["scales"], sc["rotations"])
+    R = 256 * batches
+    o = torch.zeros(1, R, 3)
+    o[0, :, 0] = torch.tensor(x + [12.0]).repeat(R // 4)
+    o[0, :, :2] += 0.02 * torch.randn(R, 2, generator=gen)
+    d = torch.nn.functional.normalize(torch.cat([0.01 * torch.randn(1, R, 2, generator=gen), torch.ones(1, R, 1)], dim=-1), dim=-1)
+    ref, _ = check_case(oracle, dst.SurfelTracer(), sc, o, d.contiguous())
+    proc = ref["n_proc"].reshape(-1, 4)
+    assert (proc[:, 0] > 0.5 * n).mean() > 0.9 and (proc[:, 1] <= 12).all() and (proc[:, 3] == 0).all()
+
+
 @pytest.mark.parametrize("blocks", [16, 17])
 def test_a_list_whose_record_is_one_block_short(oracle, blocks):
     """512 rays, 128 waves: their first pieces fill sixteen blocks of the record, the few pieces that two waves ask for
