@@ -2577,7 +2577,7 @@ uint64_t dst_hit_record_layout(int32_t H, int32_t W, int32_t mtd_alloc, uint32_t
     const TileGrid t = tile_grid(H, W);
     const uint64_t waves = (uint64_t)t.btiles_x * t.btiles_y * kWavesPerBlock;
     const uint64_t header = record_header_words((uint64_t)H * W, t.th_log2, (uint32_t)mtd_alloc + 1u, waves);
-    if (header_words) *header_words = header;
+    if (header_words) *header_words = record_order_at((uint64_t)H * W, t.th_log2, (uint32_t)mtd_alloc + 1u, waves);
     if (n_waves) *n_waves = (uint32_t)waves;
     return header + (uint64_t)blocks * kRecBlockWords;
 }

@@ -152,13 +152,13 @@ class HitRecord:
     replay them instead of walking the BVH again (see `hit_record` in include/dst_api.h).  `storage` is a
     caller- or pool-owned int64 tensor that is at least `words_needed(...)` long."""
 
-    _layouts = {}   # (H, W, mtd_alloc) -> (header words, waves, words of a block)
+    _layouts = {}   # (H, W, mtd_alloc) -> (header words, waves, words without blocks, words of a block)
     _slots = []     # free words of pinned host memory for the request counts (note_request)
     _late = []      # words given up before their copy had come: looked at again when new ones are needed
 
     @classmethod
     def layout(cls, H, W, mtd_alloc, blocks_per_wave):
-        """(words of the whole buffer, header words, blocks, waves) for an (H,W) ray grid."""
+        """(words of the whole buffer, header words to be zeroed, blocks, waves) for an (H,W) ray grid."""
         known = cls._layouts.get((H, W, mtd_alloc))
         if known is None:
             header, waves = C.c_uint64(0), C.c_uint32(0)
@@ -167,10 +167,10 @@ class HitRecord:
             per_block = lib.dst_hit_record_layout(H, W, mtd_alloc, 1, None, None) - words
             if len(cls._layouts) >= 256:
                 cls._layouts.clear()
-            known = cls._layouts[(H, W, mtd_alloc)] = (int(header.value), max(1, waves.value), int(per_block))
-        header, n_waves, per_block = known
+            known = cls._layouts[(H, W, mtd_alloc)] = (int(header.value), max(1, waves.value), int(words), int(per_block))
+        header, n_waves, bare, per_block = known
         blocks = max(1, int(n_waves * blocks_per_wave) + 1)
-        return (header + blocks * per_block if per_block else 0), header, blocks, n_waves
+        return (bare + blocks * per_block if per_block else 0), header, blocks, n_waves
 
     def __init__(self, H, W, mtd_alloc, blocks_per_wave, device, storage=None):
         words, header, self.blocks, self.n_waves = self.layout(H, W, mtd_alloc, blocks_per_wave)

@@ -100,8 +100,11 @@ typedef struct DstParams {
      * call.  Word 0 then holds the number of blocks the forward trace asked for.  If that exceeds
      * hit_record_blocks the record is incomplete: the backward trace sees this ON THE DEVICE and walks the BVH
      * again instead (the host need not look at the record between the two calls; it may read word 0 later to
-     * size the next record; at most 2^26 - 1 blocks of a record are used).  Word 1 counts chains a replay found broken: it stays 0 unless the buffer was
-     * not written by a forward trace with the same grid, depth and a zeroed header. */
+     * size the next record; at most 2^26 - 1 blocks of a record are used).  Word 1 counts chains a replay found
+     * broken: it stays 0 unless the buffer was not written by a forward trace with the same grid, depth and a zeroed
+     * header.  The record of a ray list (fewer than eight rows) of 2048 rays and more also carries the order in which the
+     * rays were traced, and the backward trace takes it from there, also where the record is incomplete: it may only be
+     * given a record that a forward trace of the same grid and depth has been given before. */
     uint64_t *hit_record;
     uint32_t hit_record_blocks;
     uint32_t flags;               /* DST_FLAG_* */
@@ -267,8 +270,8 @@ int dst_trace_info(dst_ctx *ctx, DstTraceInfo *info);
 int dst_set_handover(dst_ctx *ctx, int mode, uint32_t steps);
 
 /* Size in 8-byte words of a hit record with room for `blocks` chunk blocks, for an (H,W) ray grid traced with
- * `mtd_alloc`.  Also returns the words of the header the caller must zero-fill, and the number of waves the
- * grid is traced with (a forward trace at depth 0 asks for about 3-6 blocks per wave). */
+ * `mtd_alloc`.  Also returns the words at its front that the caller must zero-fill (a list's order of rays, behind them, needs
+ * no zeros), and the number of waves the grid is traced with (a forward trace at depth 0 asks for about 3-6 blocks per wave). */
 uint64_t dst_hit_record_layout(int32_t H, int32_t W, int32_t mtd_alloc, uint32_t blocks, uint64_t *header_words,
                                uint32_t *n_waves);
 

@@ -334,6 +334,9 @@ def test_record_headers_hold_the_directory_in_use(binding, H, W):
     assert header <= 4 + waves + 2 and words > header
     assert binding.HitRecord.layout(160, 160, 1, 4.0)[1] >= 3 + 160 * 160
     assert binding.HitRecord.layout(1, 131072, 1, 4.0)[1] >= 3 + 131072
+    # the order of a list's rays lies between the words to be zeroed and the first block
+    words, header, blocks, _ = binding.HitRecord.layout(1, 131072, 1, 4.0)
+    assert header < 3 + 131072 + 2 and words >= header + 131072 // 2 + blocks * 42 * 7 * 8
 
 
 def test_bench_quotes_traffic_for_the_kernels_that_run_only():
