@@ -1,6 +1,8 @@
-"""Images large enough to be traced by tiles, whose reflections are traced ray by ray (k_row_fwd<BEYOND>), against the
-oracle: per-ray outputs bit-identical, gradients within the usual bar.  The oracle follows a window of the image; upstream
-gradients are zero outside of it, so that the per-surfel sums are the window's alone."""
+"""Reflections of images too large to be recorded ray by ray, against the oracle: per-ray outputs bit-identical, gradients
+within the usual bar.  Mid-size images are traced ray by ray from the start (k_row_fwd<RowTiles> with a record, <RowRays>
+without), larger ones by tiles, their reflections ray by ray (<RowBeyond>); HANDOVER_OFF has the latter at mid sizes too, so
+that the tests below run on both paths.  The oracle follows a window of the image; upstream gradients are zero outside of it,
+so that the per-surfel sums are the window's alone."""
 import numpy as np
 import pytest
 import torch
@@ -9,7 +11,16 @@ import dst_scenes as S
 from helpers import GRAD_REL, assert_forward_exact, assert_gradients, gpu_trace, oracle_scene, upstream
 
 pytestmark = pytest.mark.gpu
-H, W = 152, 176          # 418 waves: above the sizes that are traced ray by ray from the start
+H, W = 152, 176          # 418 waves: above the sizes that are recorded ray by ray
+PATHS = pytest.mark.parametrize("path", ["rows", "tiles_then_rows"])
+
+
+def tracer_by(path):
+    import diff_surfel_tracing as dst
+    tracer = dst.SurfelTracer()
+    if path == "tiles_then_rows":
+        tracer.optix_context.set_handover(dst._C.HANDOVER_OFF)
+    return tracer
 
 
 def window_reference(oracle, sc, o, d, aux, rows, cols, **kw):
@@ -53,17 +64,17 @@ def translucent_corridor(n=720, seed=5):
     return sc
 
 
-def test_a_long_way_through_translucent_surfels_is_recorded(oracle):
+@PATHS
+def test_a_long_way_through_translucent_surfels_is_recorded(oracle, path):
     """Some fifty chunks of sixteen entries behind the mirror: the record of the second step has room for them all, is
     complete, and stays the size it is; replay and re-trace both give the oracle's gradients."""
-    import diff_surfel_tracing as dst
     sc = translucent_corridor()
     o, d = S.pinhole_rays(H, W, 40.0, (0.0, 0.0, 0.0), (1.0, 0.0, 0.0))
     rows, cols = slice(60, 76), slice(70, 94)
     kw = dict(max_trace_depth=1, specular_threshold=0.4)
     ug, ref, refg, refg64 = window_reference(oracle, sc, o, d, 2, rows, cols, **kw)
     assert ref["n_proc"].max() > 16 * 40 and ref["n_con"].mean() > 100
-    tracer = dst.SurfelTracer()
+    tracer = tracer_by(path)
     ctx = tracer.optix_context
     sizes = []
     for step in range(4):
@@ -76,11 +87,11 @@ def test_a_long_way_through_translucent_surfels_is_recorded(oracle):
     assert sizes[1] == sizes[2] == sizes[3]
 
 
+@PATHS
 @pytest.mark.parametrize("depth,aux,mode", [(1, 2, "plain"), (1, 4, "det"), (2, 8, "norec"), (3, 2, "plain"), (3, 4, "colors"),
                                             (1, 3, "colors_det"), (2, 2, "half"), (1, 8, "distortion"), (3, 8, "det"),
                                             (2, 4, "norows")])
-def test_reflections_of_images_traced_by_tiles(oracle, depth, aux, mode):
-    import diff_surfel_tracing as dst
+def test_reflections_of_mid_size_images(oracle, depth, aux, mode, path):
     from test_gpu_parity import check_case
     sc = S.scene_room(P=12000, seed=depth + aux, aux=aux, half=1.5)
     sc["others_precomp"][:, 0] = sc["others_precomp"][:, 0] * 0.8 + 0.1    # the reference divides by the specular
@@ -89,7 +100,7 @@ def test_reflections_of_images_traced_by_tiles(oracle, depth, aux, mode):
         del sc["shs"]
     o, d = S.pinhole_rays(H, W, 70.0, (-0.6, -0.3, 0.15), (0.9, 0.45, -0.15))
     kw = dict(max_trace_depth=depth, specular_threshold=0.0 if depth == 3 else 0.1, bg=(0.3, 0.1, 0.2))
-    tracer = dst.SurfelTracer()
+    tracer = tracer_by(path)
     ctx = tracer.optix_context
     tracer.deterministic = mode.endswith("det")
     seen, call = sc, tracer

@@ -21,11 +21,13 @@ def step(tracer, st, g, o, d, ug, leaf):
     return dict(zip(names, torch.autograd.grad(losses, [leaf[k] for k in names], [ug[k] for k in ("rgb", "dpt", "acc", "norm", "aux")])))
 
 
-@pytest.mark.parametrize("size", [(48, 64), (152, 176)])
-def test_two_streams_in_turn(size):
+@pytest.mark.parametrize("size,handover", [((48, 64), True), ((152, 176), True), ((152, 176), False)])
+def test_two_streams_in_turn(size, handover):
     import diff_surfel_tracing as dst
     H, W = size
     tracer = dst.SurfelTracer()
+    if not handover:   # the larger image by tiles
+        tracer.optix_context.set_handover(dst._C.HANDOVER_OFF)
     st = settings(dst, H, W, DEV)
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
     views = [tuple(t.to(DEV) for t in S.rays_cube(H, W, view=v)) for v in range(4)]
@@ -56,13 +58,16 @@ def test_two_streams_in_turn(size):
     assert not tracer.optix_context._row_pool and not tracer.optix_context._record_pool
 
 
-@pytest.mark.parametrize("size,depth", [((48, 64), 0), ((152, 176), 1)])
-def test_a_captured_training_step_can_be_replayed(size, depth):
+@pytest.mark.parametrize("size,depth,handover", [((48, 64), 0, True), ((152, 176), 1, True), ((152, 176), 1, False)])
+def test_a_captured_training_step_can_be_replayed(size, depth, handover):
     """Forward and backward recorded into a graph: every replay gives the eager gradients, with eager training steps in
-    between, one of them in two halves around the replay (the graph's record and rows are its own)."""
+    between, one of them in two halves around the replay (the graph's record and rows are its own).  (Without the hand-over the
+    larger image's first bounce is traced by tiles, its reflections by rows.)"""
     import diff_surfel_tracing as dst
     H, W = size
     tracer = dst.SurfelTracer()
+    if not handover:
+        tracer.optix_context.set_handover(dst._C.HANDOVER_OFF)
     st = settings(dst, H, W, DEV, max_trace_depth=depth, specular_threshold=0.1)
     g = {k: v.to(DEV) for k, v in S.scene_room(P=6000, seed=1, aux=2, half=1.5).items()}
     g["others_precomp"][:, 0] = g["others_precomp"][:, 0] * 0.8 + 0.1
