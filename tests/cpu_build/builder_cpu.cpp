@@ -492,6 +492,7 @@ int main(int argc, char **argv) {
         run_case(3000, 2, agg != 0, 6);
         run_case(3000, 3, agg != 0, 7);
         run_case(4000, 4, agg != 0, 8);
+        if (!quick) run_case(110000, 0, agg != 0, 9);   // range table of two workgroups; three rounds to a launch, then four
     }
     std::printf(failures ? "FAILED: %d checks\n" : "ALL OK\n", failures);
     return failures ? 1 : 0;
