@@ -164,6 +164,7 @@ int dst_trace_forward(dst_ctx *ctx, const DstParams *p, void *stream) {
     int rc = check_common(ctx, p);
     if (rc) return rc;
     if (p->training && !p->a_weights) return dst_fail(ctx, DST_E_INVALID, "training needs a_weights");
+    if (reinterpret_cast<uintptr_t>(p->scratch) & 127u) return dst_fail(ctx, DST_E_INVALID, "scratch must be aligned to 128 bytes");
     if ((p->flags & DST_FLAG_SH_HALF) && (!p->shs || !p->shs_half))
         return dst_fail(ctx, DST_E_INVALID, "DST_FLAG_SH_HALF needs shs and its binary16 copy shs_half");
     return dst_launch_trace(ctx, *p, false, (hipStream_t)stream);

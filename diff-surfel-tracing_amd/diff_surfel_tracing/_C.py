@@ -40,7 +40,7 @@ class DstParams(C.Structure):
         + [(n, _FP) for n in ("dL_dray_o", "dL_dray_d", "dL_dmeans3D", "dL_dgrads3D", "dL_dshs", "dL_dcolors",
                               "dL_dothers", "dL_dopacities", "dL_dscales", "dL_drotations")]
         + [("shs_half", _FP), ("grad_touched", _FP), ("hit_record_asked", _FP), ("dist_channels", C.c_int32),
-           ("reserved", C.c_int32)]
+           ("reserved", C.c_int32), ("scratch", _FP)]
     )
 
 
@@ -63,7 +63,7 @@ HANDOVER_OFF, HANDOVER_AUTO, HANDOVER_ALWAYS = 0, 1, 2
 EXPORTS = ("dst_create", "dst_destroy", "dst_build_accel", "dst_trace_forward", "dst_trace_backward",
            "dst_last_error", "dst_accel_info", "dst_accel_download", "dst_version", "dst_sizeof_params",
            "dst_hit_record_layout", "dst_refit_accel_static", "dst_refit_from_surfels",
-           "dst_det_workspace_words", "dst_pack_sh_half", "dst_trace_info", "dst_set_handover", "dst_det_out_of_range")
+           "dst_det_workspace_words", "dst_trace_scratch_bytes", "dst_pack_sh_half", "dst_trace_info", "dst_set_handover", "dst_det_out_of_range")
 
 _lib = None
 
@@ -96,6 +96,8 @@ def load_library():
     L.dst_set_handover.argtypes = [C.c_void_p, C.c_int, C.c_uint32]
     L.dst_det_workspace_words.restype = C.c_uint64
     L.dst_det_workspace_words.argtypes = [C.c_int32, C.c_int32, C.c_int]
+    L.dst_trace_scratch_bytes.restype = C.c_uint64
+    L.dst_trace_scratch_bytes.argtypes = [C.c_int32, C.c_int32, C.c_int32]
     L.dst_pack_sh_half.argtypes = [C.c_void_p, C.c_void_p, C.c_uint64, C.c_void_p]
     L.dst_version.restype = C.c_char_p
     L.dst_sizeof_params.restype = C.c_size_t
@@ -537,6 +539,26 @@ def _common_params(ray_o, ray_d, vertices, background, means3D, shs, degree, col
     return p, t
 
 
+_scratch_bytes = {}   # (P, H, W) -> dst_trace_scratch_bytes
+
+
+def _scratch(p, keep):
+    """The forward call's scratch memory (DstParams.scratch): of the current stream's, given back when the call is done."""
+    key = (p.P, p.H, p.W)
+    size = _scratch_bytes.get(key)
+    if size is None:
+        if len(_scratch_bytes) >= 256:
+            _scratch_bytes.clear()
+        size = _scratch_bytes[key] = load_library().dst_trace_scratch_bytes(*key)
+    if size == 0:
+        return
+    try:
+        keep["scratch"] = torch.empty(size, dtype=torch.uint8, device=keep["means3D"].device)
+    except torch.OutOfMemoryError:   # (the same results without it)
+        return
+    p.scratch = keep["scratch"].data_ptr()
+
+
 def trace_surfels(ctx, training, start_from_first, ray_o, ray_d, vertices, background, means3D, shs, degree,
                   colors_precomp, others_precomp, opacities, scales, scale_modifier, rotations, transMat_precomp,
                   viewmatrix, projmatrix, campos, prefiltered, debug, max_trace_depth, specular_threshold,
@@ -577,6 +599,8 @@ def trace_surfels(ctx, training, start_from_first, ray_o, ray_d, vertices, backg
     if getattr(ctx, "distortion", False):
         p.flags |= FLAG_DISTORTION
     _use_sh_half(ctx, p, keep)
+    if p.flags == 0:   # (the kernels with the rare options have no use for it)
+        _scratch(p, keep)
     if events is not None:
         events[0].record()
     _check(ctx, load_library().dst_trace_forward(ctx.handle, C.byref(p), _stream()))

@@ -153,6 +153,10 @@ typedef struct DstParams {
     uint64_t *hit_record_asked;
     int32_t dist_channels;        /* forward: channels of out_dist: 1 (the distortion alone), or 3 (also 0: three) */
     int32_t reserved;
+    /* forward, optional: device memory, aligned to 128 bytes, dst_trace_scratch_bytes(P, H, W) of it, in which the call keeps
+     * what it derives from the surfels' parameters before it traces (contents before and after the call mean nothing).  Same
+     * results bit for bit, faster; NULL: everything is derived anew at every hit. */
+    void *scratch;
 } DstParams;
 
 /* Shape of the current acceleration structure, for tests and tools. */
@@ -274,6 +278,10 @@ int dst_set_handover(dst_ctx *ctx, int mode, uint32_t steps);
  * no zeros), and the number of waves the grid is traced with (a forward trace at depth 0 asks for about 3-6 blocks per wave). */
 uint64_t dst_hit_record_layout(int32_t H, int32_t W, int32_t mtd_alloc, uint32_t blocks, uint64_t *header_words,
                                uint32_t *n_waves);
+
+/* Size in bytes of DstParams.scratch for a forward trace of P surfels over an (H,W) ray grid; 0 where the call has no use for
+ * any (lists and small images, or far fewer rays than surfels). */
+uint64_t dst_trace_scratch_bytes(int32_t P, int32_t H, int32_t W);
 
 /* Words (8 bytes each) of DstParams.det_workspace for a forward (backward = 0: one per surfel) or a backward
  * call (one per surfel and gradient column: 16 + aux table columns + 48 SH columns). */

@@ -1,0 +1,79 @@
+"""The forward trace's scratch memory (DstParams.scratch): hits evaluated from records of the surfels that the call makes
+first.  Outputs and hit records have to be those of the same call without scratch memory bit for bit, whatever the
+scales (quotients by them are formed from their reciprocals in the records, and divided out where that does not hold)."""
+import pytest
+import torch
+
+import dst_scenes as S
+from diff_surfel_tracing import _C
+
+pytestmark = pytest.mark.gpu
+
+
+def both(monkeypatch, tracer, sc, o, d, depth=0, aux=0, training=False):
+    """(outputs with scratch memory, without)"""
+    g = {k: v.cuda() for k, v in sc.items()}
+    e, bg, eye = torch.empty(0, device="cuda"), torch.zeros(3, device="cuda"), torch.eye(4, device="cuda")
+    others = torch.rand(sc["means3D"].shape[0], aux, generator=torch.Generator().manual_seed(3)).cuda() if aux else e
+    out = []
+    for use in (True, False):
+        if not use:
+            monkeypatch.setattr(_C, "_scratch", lambda p, keep: None)
+        elif not _C.load_library().dst_trace_scratch_bytes(sc["means3D"].shape[0], o.shape[0], o.shape[1]):
+            pytest.fail("this size has no scratch memory")
+        out.append([x for x in _C.trace_surfels(
+            tracer.optix_context, training, True, o.cuda(), d.cuda(), g["vertices"], bg, g["means3D"], g["shs"], 3, e, others,
+            g["opacities"], g["scales"], 1.0, g["rotations"], e, eye, eye, bg, False, False, depth, 0.1) if x is not None])
+        torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("depth,aux", [(0, 0), (0, 3), (1, 2), (1, 8)])
+def test_records_change_no_bit(monkeypatch, depth, aux):
+    import diff_surfel_tracing as dst
+    tracer = dst.SurfelTracer()
+    sc = S.scene_room(P=30011, seed=4)
+    o, d = S.rays_room(259, 331)
+    tracer.build_acceleration_structure(sc["vertices"].cuda(), sc["faces"].cuda(), rebuild=True)
+    with_, without = both(monkeypatch, tracer, sc, o, d, depth, aux)
+    for a, b in zip(with_, without):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
+@pytest.mark.parametrize("factor", [0.0, 1e-42, 1e-20, 2.0 ** -40, 0.99 * 2.0 ** -40, 1.0, 2.0 ** 40, 1.01 * 2.0 ** 40, 1e20, 3e38,
+                                    -1.0, float("inf"), float("nan")])
+def test_scales_of_any_size(monkeypatch, factor):
+    """The quads stay what they are; the scales the trace is given are theirs times `factor`, on every third surfel."""
+    import diff_surfel_tracing as dst
+    tracer = dst.SurfelTracer()
+    sc = S.scene_room(P=20000, seed=5)
+    o, d = S.rays_room(257, 257)
+    tracer.build_acceleration_structure(sc["vertices"].cuda(), sc["faces"].cuda(), rebuild=True)
+    sc["scales"][::3] *= factor
+    if factor in (2.0 ** -40, 2.0 ** 40):   # the edges of the reciprocals' range
+        sc["scales"][::3] = factor
+    sc["means3D"][1::50] = 1e30             # far too large to divide by way of a reciprocal
+    with_, without = both(monkeypatch, tracer, sc, o, d)
+    for a, b in zip(with_, without):
+        same = (a.view(torch.int32) == b.view(torch.int32)) | (torch.isnan(a) & torch.isnan(b))
+        assert bool(same.all())
+
+
+def test_misaligned_scratch_is_refused():
+    import diff_surfel_tracing as dst
+    tracer = dst.SurfelTracer()
+    sc = S.scene_cube(P=64, seed=0)
+    tracer.build_acceleration_structure(sc["vertices"].cuda(), sc["faces"].cuda(), rebuild=True)
+    def shifted(p, keep):
+        keep["scratch"] = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
+        p.scratch = keep["scratch"].data_ptr() + 64
+    before, _C._scratch = _C._scratch, shifted
+    try:
+        with pytest.raises(RuntimeError, match="aligned"):
+            o, d = S.rays_cube(16, 16)
+            e, bg, eye = torch.empty(0, device="cuda"), torch.zeros(3, device="cuda"), torch.eye(4, device="cuda")
+            g = {k: v.cuda() for k, v in sc.items()}
+            _C.trace_surfels(tracer.optix_context, False, True, o.cuda(), d.cuda(), g["vertices"], bg, g["means3D"], g["shs"], 3,
+                             e, e, g["opacities"], g["scales"], 1.0, g["rotations"], e, eye, eye, bg, False, False, 0, 0.0)
+    finally:
+        _C._scratch = before
