@@ -106,3 +106,21 @@ class _HalfSeen:
 
     def __call__(self, *a, shs=None, **k):
         return self._tracer(*a, shs=shs + (self._shs.to(shs.device) - shs.detach()), **k)
+
+
+@pytest.mark.parametrize("aux,det", [(2, False), (4, True), (8, False)])
+@pytest.mark.parametrize("P", [1, 3, 4, 5, 107, 112, 113, 240])
+def test_gradient_table_edges(oracle, P, aux, det):
+    """One 16x16 block before P faint surfels that all of its rays meet: its table of gradients (104 to 112 rows, in groups
+    of four) takes few of them, all, or no more than it has rows for."""
+    sc = {k: v.clone() for k, v in S.scene_cube(P=P, seed=P, aux=aux).items()}
+    gen = torch.Generator().manual_seed(P)
+    sc["means3D"] = torch.cat([2.0 + 0.01 * torch.arange(P)[:, None].float(), 0.05 * torch.randn(P, 2, generator=gen)], 1)
+    q = torch.tensor([0.7071, 0.0, 0.7071, 0.0]) + 0.05 * torch.randn(P, 4, generator=gen)   # facing along x
+    sc["rotations"] = q / q.norm(dim=1, keepdim=True)
+    sc["scales"] = 0.5 + 0.2 * torch.rand(P, 2, generator=gen)
+    sc["opacities"] = 0.02 + 0.02 * torch.rand(P, 1, generator=gen)
+    sc["vertices"], sc["faces"] = S.get_triangles(sc["means3D"], sc["scales"], sc["rotations"])
+    o, d = S.pinhole_rays(16, 16, 10.0, (0.0, 0.0, 0.0), (1.0, 0.0, 0.0))
+    ref, _ = check_case(oracle, tile_tracer(deterministic=det), sc, o, d)
+    assert ref["n_con"].min() >= 0.9 * P   # (a ray in ten is outside some splat)
