@@ -35,7 +35,7 @@ struct DstWideChild {
     float lo[3];
     uint32_t ref;             // wide node index, or leaf-group reference
     float hi[3];
-    uint32_t used;            // 1, or 0 for an unused slot
+    uint32_t used;            // 0: an unused slot; else 1 + where its box stands in the binary hierarchy (2 * node + side)
 };
 // The same words by coordinate, for the checks of a finished hierarchy (host only: the kernels read whole children).
 template <typename T, int WORD>
@@ -47,7 +47,7 @@ struct DstWideCount {
     uint32_t words[8 * DST_WIDE];
     operator uint32_t() const {
         uint32_t n = 0;
-        for (int k = 0; k < DST_WIDE; ++k) n += words[8 * k + 7];
+        for (int k = 0; k < DST_WIDE; ++k) n += words[8 * k + 7] != 0u ? 1u : 0u;
         return n;
     }
 };

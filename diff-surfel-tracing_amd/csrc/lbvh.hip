@@ -776,41 +776,65 @@ __global__ void k_range_table_level(float *table, uint32_t n_blocks, int level) 
     box_join(box, hi);
     box_store(table + ((size_t)level * n_blocks + b) * 6, box);
 }
-__device__ __forceinline__ void range_box(const RangeBoxes &rb, uint32_t n_blocks, uint32_t a, uint32_t b, float (&box)[6]) {
-    const uint32_t ba = a / kRangeBlock, bb = b / kRangeBlock;
-    if (ba == bb) {
-        const float *src = rb.lbox + 6 * (size_t)a;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) box[k] = src[k];
-        for (uint32_t j = a + 1u; j <= b; ++j) box_join(box, rb.lbox + 6 * (size_t)j);
-        return;
-    }
-    const float *s = rb.sbox + 6 * (size_t)a;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) box[k] = s[k];
-    box_join(box, rb.pbox + 6 * (size_t)b);
-    if (bb > ba + 1u) {
-        const uint32_t x = ba + 1u, y = bb - 1u;
-        const int l = 31 - __clz(y - x + 1u);
-        box_join(box, rb.table + ((size_t)l * n_blocks + x) * 6);
-        box_join(box, rb.table + ((size_t)l * n_blocks + (y + 1u - (1u << l))) * 6);
-    }
-}
-// Fit by look-up: node i's children cover leaves first..split and split+1..last (split = the child reference itself,
-// see k_karras).
-__global__ void k_fit_ranges(DstNode *nodes, RangeBoxes rb, uint32_t n_blocks, uint32_t n_internal) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_internal) return;
-    DstNode &nd = nodes[i];
-    const uint32_t first = nd.first, last = nd.last, split = nd.c0 & ~DST_LEAF_BIT;
-    float b0[6], b1[6];
-    range_box(rb, n_blocks, first, split, b0);
-    range_box(rb, n_blocks, split + 1u, last, b1);
+// Fit by look-up: the box of leaf i and the box of node i go to their parents' records, two entries of one line each.  A node
+// takes its number from its first or its last leaf, so a node inside one block of 64 leaves lies inside the block of the
+// wave it falls to, which holds the unions of 2^l leaves from every leaf on in LDS: two look-ups, as for the others in memory.
+// (A node looking up its two children's boxes, leaf by leaf inside a block: up to 62 trips that the wave waits for; refit of 2M
+// surfels 186 -> 95 us, build of 1M 91 -> 46.)  Bound by memory: a line read and written a node, 24 bytes a leaf.
+constexpr int kFitLevels = 6, kFitThreads = 256;
+__global__ __launch_bounds__(kFitThreads) void k_fit_ranges(DstNode *nodes, const uint32_t *__restrict__ node_parent,
+                                                            const uint32_t *__restrict__ leaf_parent, RangeBoxes rb,
+                                                            uint32_t n_blocks, uint32_t n) {
+    __shared__ float s_box[kFitThreads / DST_WAVE][kFitLevels][6][DST_WAVE];
+    const uint32_t i = blockIdx.x * kFitThreads + threadIdx.x, lane = threadIdx.x % DST_WAVE, wave = threadIdx.x / DST_WAVE;
+    float box[6], leaf[6];
+    const float2 *src = reinterpret_cast<const float2 *>(rb.lbox + 6 * (size_t)min(i, n - 1u));
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        nd.lo0[k] = b0[k]; nd.hi0[k] = b0[3 + k];
-        nd.lo1[k] = b1[k]; nd.hi1[k] = b1[3 + k];
+        const float2 v = src[k];
+        leaf[2 * k] = v.x;
+        leaf[2 * k + 1] = v.y;
     }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) s_box[wave][0][k][lane] = box[k] = i < n ? leaf[k] : (k < 3 ? INFINITY : -INFINITY);
+#pragma unroll
+    for (int l = 1; l < kFitLevels; ++l) {
+        __syncthreads();   // (a wave reads its own boxes alone, so these cost little)
+        const uint32_t half = 1u << (l - 1);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            const float other = lane + half < (uint32_t)DST_WAVE ? s_box[wave][l - 1][k][lane + half] : box[k];
+            box[k] = k < 3 ? fminf(box[k], other) : fmaxf(box[k], other);
+            s_box[wave][l][k][lane] = box[k];
+        }
+    }
+    __syncthreads();
+    if (i >= n) return;
+    auto put = [&](uint32_t to, const float (&b)[6]) { box_store((to & 1u) != 0u ? nodes[to >> 1].lo1 : nodes[to >> 1].lo0, b); };
+    put(leaf_parent[i], leaf);
+    if (i >= n - 1u || node_parent[i] == DST_NO_PARENT) return;   // (the root's box is nobody's)
+    const uint32_t first = nodes[i].first, last = nodes[i].last, bf = first / kRangeBlock, bl = last / kRangeBlock;
+    if (bf == bl) {
+        const int l = min(31 - __clz(last - first + 1u), kFitLevels - 1);   // (64 leaves: twice 32)
+        const uint32_t at0 = first % kRangeBlock, at1 = (last + 1u - (1u << l)) % kRangeBlock;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            const float u = s_box[wave][l][k][at0], v = s_box[wave][l][k][at1];
+            box[k] = k < 3 ? fminf(u, v) : fmaxf(u, v);
+        }
+    } else {
+        const float *from = rb.sbox + 6 * (size_t)first;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) box[k] = from[k];
+        box_join(box, rb.pbox + 6 * (size_t)last);
+        if (bl > bf + 1u) {
+            const uint32_t x = bf + 1u, y = bl - 1u;
+            const int l = 31 - __clz(y - x + 1u);
+            box_join(box, rb.table + ((size_t)l * n_blocks + x) * 6);
+            box_join(box, rb.table + ((size_t)l * n_blocks + (y + 1u - (1u << l))) * 6);
+        }
+    }
+    put(node_parent[i], box);
 }
 
 // Is this quad far smaller than the scene (DstBounds::small_quads)?  `scale` = the scene's size as set by the last build.
@@ -837,12 +861,13 @@ __global__ void k_leaf_fill(const float *__restrict__ vertices, const int4 *__re
                             DstBounds *__restrict__ count_small, uint32_t n) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const bool valid = i < n;   // every lane stays for the wave-wide scans of the boxes
+    // (quad_ids == nullptr: known to be rows 4g..4g+3, so 16 bytes a quad need not be gathered)
     float c[4][3] = {};
     float mabs = 0.f;
     bool small = false;
     if (valid) {
         const uint32_t g = sorted_ids[i];
-        load_corners(vertices, quad_ids[g], g, c);
+        load_corners(vertices, quad_ids != nullptr ? quad_ids[g] : make_int4((int)(4u * g), (int)(4u * g + 1u), (int)(4u * g + 2u), (int)(4u * g + 3u)), g, c);
         write_leaf(c, g, i, leaves, pre);
         small = quad_is_small(c, __uint_as_float(count_small->scale));
 #pragma unroll
@@ -855,18 +880,45 @@ __global__ void k_leaf_fill(const float *__restrict__ vertices, const int4 *__re
     count_small_quads(small, count_small);
 }
 
-// The same for a refit straight from the surfel parameters: the four corners of surfel g are
+// For a refit straight from the surfel parameters: the four corners of surfel g are
 //   v_k = (mean + a_k * (sx * R[:,0])) + b_k * (sy * R[:,1]),  (a,b) = (-3,3), (-3,-3), (3,3), (3,-3),
 // R the rotation of the quaternion (w,x,y,z) divided by its norm sqrt(((w*w + x*x) + y*y) + z*z): the quads of
 // the 2DGS convention (reference example/utils/gaussian_utils.py:176-210), every operation in fp32, rounded once,
-// in exactly this order (this file is compiled without contraction).  Optionally writes the corners to
-// `vertices_out` (4P,3) in the canonical order (rows 4g..4g+3) for the trace calls, and reduces the largest
-// |coordinate| the trace kernels size their padding with.
+// in exactly this order (this file is compiled without contraction).
+__device__ __forceinline__ void surfel_corners(const float *__restrict__ means, const float *__restrict__ scales,
+                                               const float *__restrict__ rotations, uint32_t g, float (&c)[4][3]) {
+    const float q0 = rotations[4 * (size_t)g], q1 = rotations[4 * (size_t)g + 1], q2 = rotations[4 * (size_t)g + 2],
+                q3 = rotations[4 * (size_t)g + 3];
+    const float nrm = sqrtf(((q0 * q0 + q1 * q1) + q2 * q2) + q3 * q3);
+    const float w = q0 / nrm, x = q1 / nrm, y = q2 / nrm, z = q3 / nrm;
+    const float sx = scales[2 * (size_t)g], sy = scales[2 * (size_t)g + 1];
+    const float u[3] = {(1.f - 2.f * (y * y + z * z)) * sx, (2.f * (x * y + w * z)) * sx, (2.f * (x * z - w * y)) * sx};
+    const float v[3] = {(2.f * (x * y - w * z)) * sy, (1.f - 2.f * (x * x + z * z)) * sy, (2.f * (y * z + w * x)) * sy};
+    const float m[3] = {means[3 * (size_t)g], means[3 * (size_t)g + 1], means[3 * (size_t)g + 2]};
+    const float sa[4] = {-3.f, -3.f, 3.f, 3.f}, sb[4] = {3.f, -3.f, 3.f, -3.f};
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int a = 0; a < 3; ++a) c[k][a] = (m[a] + sa[k] * u[a]) + sb[k] * v[a];
+}
+// The corners of all surfels as a vertex buffer, rows 4g..4g+3, in the surfels' order; k_leaf_fill then takes them from there.
+// (Made in leaf order, they came from four gathers and went out scattered: 2M surfels 305 us, now 52 + 202.)
+__global__ void k_surfel_quads(const float *__restrict__ means, const float *__restrict__ scales, const float *__restrict__ rotations,
+                               float *__restrict__ vertices_out, uint32_t n) {
+    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= n) return;
+    float c[4][3];
+    surfel_corners(means, scales, rotations, g, c);
+    float4 *dst = reinterpret_cast<float4 *>(vertices_out + 12 * (size_t)g);   // 48 bytes per surfel
+    dst[0] = make_float4(c[0][0], c[0][1], c[0][2], c[1][0]);
+    dst[1] = make_float4(c[1][1], c[1][2], c[2][0], c[2][1]);
+    dst[2] = make_float4(c[2][2], c[3][0], c[3][1], c[3][2]);
+}
+// Leaf records from the surfel parameters themselves, for callers that want no vertex buffer.
 __global__ void k_leaf_fill_from_surfels(const float *__restrict__ means, const float *__restrict__ scales,
                                          const float *__restrict__ rotations, const uint32_t *__restrict__ sorted_ids,
                                          DstLeaf *__restrict__ leaves, DstLeafPre *__restrict__ pre,
-                                         float *__restrict__ vertices_out, DstBounds *__restrict__ bounds,
-                                         RangeBoxes rb, uint32_t n) {
+                                         DstBounds *__restrict__ bounds, RangeBoxes rb, uint32_t n) {
     float mabs = 0.f;
     // wave-uniform trip count: every lane stays for the wave-wide scans of the boxes
     for (uint32_t base = blockIdx.x * blockDim.x + (threadIdx.x & ~(DST_WAVE - 1u)); base < n; base += gridDim.x * blockDim.x) {
@@ -874,30 +926,13 @@ __global__ void k_leaf_fill_from_surfels(const float *__restrict__ means, const 
         const bool valid = i < n;
         float c[4][3] = {};
         if (valid) {
-        const uint32_t g = sorted_ids[i];
-        const float q0 = rotations[4 * (size_t)g], q1 = rotations[4 * (size_t)g + 1], q2 = rotations[4 * (size_t)g + 2],
-                    q3 = rotations[4 * (size_t)g + 3];
-        const float nrm = sqrtf(((q0 * q0 + q1 * q1) + q2 * q2) + q3 * q3);
-        const float w = q0 / nrm, x = q1 / nrm, y = q2 / nrm, z = q3 / nrm;
-        const float sx = scales[2 * (size_t)g], sy = scales[2 * (size_t)g + 1];
-        const float u[3] = {(1.f - 2.f * (y * y + z * z)) * sx, (2.f * (x * y + w * z)) * sx, (2.f * (x * z - w * y)) * sx};
-        const float v[3] = {(2.f * (x * y - w * z)) * sy, (1.f - 2.f * (x * x + z * z)) * sy, (2.f * (y * z + w * x)) * sy};
-        const float m[3] = {means[3 * (size_t)g], means[3 * (size_t)g + 1], means[3 * (size_t)g + 2]};
-        const float sa[4] = {-3.f, -3.f, 3.f, 3.f}, sb[4] = {3.f, -3.f, 3.f, -3.f};
+            const uint32_t g = sorted_ids[i];
+            surfel_corners(means, scales, rotations, g, c);
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+            for (int k = 0; k < 4; ++k)
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                c[k][a] = (m[a] + sa[k] * u[a]) + sb[k] * v[a];
-                mabs = finite_max(mabs, fabsf(c[k][a]));
-            }
-        if (vertices_out != nullptr) {
-            float4 *dst = reinterpret_cast<float4 *>(vertices_out + 12 * (size_t)g);   // 48 bytes per surfel
-            dst[0] = make_float4(c[0][0], c[0][1], c[0][2], c[1][0]);
-            dst[1] = make_float4(c[1][1], c[1][2], c[2][0], c[2][1]);
-            dst[2] = make_float4(c[2][2], c[3][0], c[3][1], c[3][2]);
-        }
-        write_leaf(c, g, i, leaves, pre);
+                for (int a = 0; a < 3; ++a) mabs = finite_max(mabs, fabsf(c[k][a]));
+            write_leaf(c, g, i, leaves, pre);
         }
         count_small_quads(valid && quad_is_small(c, __uint_as_float(bounds->scale)), bounds);
         if (rb.lbox != nullptr) wave_range_boxes(c, valid, i, n, rb);
@@ -998,23 +1033,24 @@ __device__ __forceinline__ void child_refs(const DstNode &nd, uint32_t &r0, uint
 // looking inside them at once saves the visit (6 to 9 % fewer node visits on the scenes measured).  A step of the
 // second kind may go down a single level of the binary hierarchy, so the walks' stacks (128 entries, three deferred
 // children per step) bound its use to hierarchies of at most kAreaCollapseDepth levels; the grandchildren rule goes
-// down two levels per step and serves up to kMaxDepth.  The choice depends on the boxes, so a refit may make it anew.
+// down two levels per step and serves up to kMaxDepth.  Builds choose; a refit keeps what its build chose and renews the
+// boxes, whose places in the binary hierarchy the nodes remember (k_refit_wide).
 constexpr uint32_t kAreaCollapseDepth = 42;
 __global__ void k_widen(const DstNode *__restrict__ nodes, DstWideNode *__restrict__ wide, uint32_t n_internal,
                         const uint32_t *__restrict__ depth_word) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_internal) return;
     const DstNode nd = nodes[i];
-    if (nd.last - nd.first + 1u <= DST_GROUP) return;   // inside a leaf group: never visited
+    if (nd.last - nd.first + 1u <= DST_GROUP) {   // inside a leaf group: never visited
+        wide[i].child[0].used = 0u;
+        return;
+    }
     const bool by_area = depth_word != nullptr && *depth_word <= kAreaCollapseDepth;
-    DstWideNode w;
+    float4 *const out = reinterpret_cast<float4 *>(&wide[i]);   // (two of a child, as DstWideChild has them)
     uint32_t k = 0;
-    auto put = [&](const float *lo, const float *hi, uint32_t ref) {
-        DstWideChild &c = w.child[k];
-        c.lo[0] = lo[0]; c.lo[1] = lo[1]; c.lo[2] = lo[2];
-        c.hi[0] = hi[0]; c.hi[1] = hi[1]; c.hi[2] = hi[2];
-        c.ref = ref;
-        c.used = 1u;
+    auto put = [&](const float *lo, const float *hi, uint32_t ref, uint32_t place) {
+        out[2u * k] = make_float4(lo[0], lo[1], lo[2], __uint_as_float(ref));
+        out[2u * k + 1u] = make_float4(hi[0], hi[1], hi[2], __uint_as_float(place + 1u));
         ++k;
     };
     uint32_t own[2];
@@ -1025,67 +1061,94 @@ __global__ void k_widen(const DstNode *__restrict__ nodes, DstWideNode *__restri
         for (int s = 0; s < 2; ++s) {
             const uint32_t r = own[s];
             if (r & DST_LEAF_BIT) {
-                put(los[s], his[s], r);
+                put(los[s], his[s], r, 2u * i + (uint32_t)s);
             } else {
                 const DstNode ch = nodes[r];
                 uint32_t g0, g1;
                 child_refs(ch, g0, g1);
-                put(ch.lo0, ch.hi0, g0);
-                put(ch.lo1, ch.hi1, g1);
+                put(ch.lo0, ch.hi0, g0, 2u * r);
+                put(ch.lo1, ch.hi1, g1, 2u * r + 1u);
             }
         }
     } else {
-        float lo[DST_WIDE][3], hi[DST_WIDE][3];
-        uint32_t ref[DST_WIDE];   // traversal references, in the order of the leaves below them
-        int m = 2;
+        // (every index is known when compiling: arrays that are indexed by a variable live in memory; 1M surfels 126 -> 50 us)
+        struct Child { float box[6]; uint32_t ref, place; };   // ref: traversal reference; place: whose box it is
+        Child ch[DST_WIDE] = {};
+        auto entry = [&](const DstNode &from, uint32_t at, bool side, uint32_t ref) {
+            Child c;
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            lo[0][a] = nd.lo0[a]; hi[0][a] = nd.hi0[a];
-            lo[1][a] = nd.lo1[a]; hi[1][a] = nd.hi1[a];
-        }
-        ref[0] = own[0];
-        ref[1] = own[1];
-        while (m < DST_WIDE) {
+            for (int a = 0; a < 3; ++a) {
+                c.box[a] = side ? from.lo1[a] : from.lo0[a];
+                c.box[3 + a] = side ? from.hi1[a] : from.hi0[a];
+            }
+            c.ref = ref;
+            c.place = 2u * at + (side ? 1u : 0u);
+            return c;
+        };
+        auto choose = [](bool b, const Child &x, const Child &y) {
+            Child c;
+#pragma unroll
+            for (int a = 0; a < 6; ++a) c.box[a] = b ? x.box[a] : y.box[a];
+            c.ref = b ? x.ref : y.ref;
+            c.place = b ? x.place : y.place;
+            return c;
+        };
+        ch[0] = entry(nd, i, false, own[0]);
+        ch[1] = entry(nd, i, true, own[1]);
+        int m = 2;   // in the order of the leaves below them
+#pragma unroll
+        for (int step = 0; step < DST_WIDE - 2; ++step) {
             int best = -1;
             float best_area = -1.f;
-            for (int c = 0; c < m; ++c) {
-                if (ref[c] & DST_LEAF_BIT) continue;
-                const float dx = hi[c][0] - lo[c][0], dy = hi[c][1] - lo[c][1], dz = hi[c][2] - lo[c][2];
+            uint32_t opened = 0u;
+#pragma unroll
+            for (int c = 0; c < 2 + step; ++c) {
+                if (c >= m || (ch[c].ref & DST_LEAF_BIT)) continue;
+                const float dx = ch[c].box[3] - ch[c].box[0], dy = ch[c].box[4] - ch[c].box[1], dz = ch[c].box[5] - ch[c].box[2];
                 float area = dx * dy + dy * dz + dz * dx;
                 if (!(area >= 0.f)) area = INFINITY;   // a box of non-finite corners: open it
                 if (area > best_area) {
                     best_area = area;
                     best = c;
+                    opened = ch[c].ref;
                 }
             }
             if (best < 0) break;
-            const DstNode ch = nodes[ref[best]];
-            for (int c = m; c > best + 1; --c) {   // make room behind the opened child
+            const DstNode in = nodes[opened];
+            uint32_t r0, r1;
+            child_refs(in, r0, r1);
+            const Child c0 = entry(in, opened, false, r0), c1 = entry(in, opened, true, r1);
 #pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    lo[c][a] = lo[c - 1][a];
-                    hi[c][a] = hi[c - 1][a];
-                }
-                ref[c] = ref[c - 1];
+            for (int c = 2 + step; c >= 0; --c) {   // the opened one makes room for its two
+                if (c >= 1) ch[c] = choose(c > best + 1, ch[c - 1], ch[c]);
+                ch[c] = choose(c == best, c0, choose(c == best + 1, c1, ch[c]));
             }
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                lo[best][a] = ch.lo0[a]; hi[best][a] = ch.hi0[a];
-                lo[best + 1][a] = ch.lo1[a]; hi[best + 1][a] = ch.hi1[a];
-            }
-            child_refs(ch, ref[best], ref[best + 1]);
             ++m;
         }
-        for (int c = 0; c < m; ++c) put(lo[c], hi[c], ref[c]);
+#pragma unroll
+        for (int c = 0; c < DST_WIDE; ++c)
+            if (c < m) put(ch[c].box, ch[c].box + 3, ch[c].ref, ch[c].place);
     }
-    for (; k < DST_WIDE; ++k) {
-        DstWideChild &c = w.child[k];
-        c.lo[0] = c.lo[1] = c.lo[2] = INFINITY;
-        c.hi[0] = c.hi[1] = c.hi[2] = -INFINITY;
-        c.ref = DST_LEAF_BIT;   // would be a harmless one-quad group, never another node
-        c.used = 0u;
+    for (; k < DST_WIDE; ++k) {   // a reference that would be a harmless one-quad group, never another node
+        out[2u * k] = make_float4(INFINITY, INFINITY, INFINITY, __uint_as_float(DST_LEAF_BIT));
+        out[2u * k + 1u] = make_float4(-INFINITY, -INFINITY, -INFINITY, __uint_as_float(0u));
     }
-    wide[i] = w;
+}
+
+// A refit's boxes into the traversal nodes, a thread per child.  (Collapsing anew: 2M surfels 199 us, now 98.)
+__global__ void k_refit_wide(const DstNode *__restrict__ nodes, DstWideNode *__restrict__ wide, uint32_t n_internal) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t / DST_WIDE >= n_internal || wide[t / DST_WIDE].child[0].used == 0u) return;
+    DstWideChild &c = wide[t / DST_WIDE].child[t % DST_WIDE];
+    const uint32_t place = c.used - 1u;
+    if (place >= 2u * n_internal) return;   // an unused slot
+    const DstNode &nd = nodes[place / 2u];
+    const float *from = (place & 1u) != 0u ? nd.lo1 : nd.lo0;   // low corner, then high corner
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        c.lo[a] = from[a];
+        c.hi[a] = from[3 + a];
+    }
 }
 
 inline dim3 grid_for(uint32_t n, int block = kBlock) { return dim3((n + block - 1) / block); }
@@ -1314,10 +1377,13 @@ int dst_lbvh_build(dst_ctx *ctx, const float *vertices, uint32_t n_vertices, con
 
     hipLaunchKernelGGL(k_init_bounds, dim3(1), dim3(64), 0, stream, ctx->bounds);
     const dim3 setup_grid(std::min<uint32_t>(grid_for(n).x, 1024u));   // 4 blocks per CU, each thread takes several surfels
-    if (surfels != nullptr) {
-        // refit from the surfel parameters: corners, leaf records and the coordinate bound in one kernel
+    if (surfels != nullptr && surfels->vertices_out != nullptr) {   // refit from the surfel parameters: first their corners
+        hipLaunchKernelGGL(k_surfel_quads, grid_for(n), dim3(kBlock), 0, stream, surfels->means, surfels->scales,
+                           surfels->rotations, surfels->vertices_out, n);
+        vertices = surfels->vertices_out;
+    } else if (surfels != nullptr) {
         hipLaunchKernelGGL(k_leaf_fill_from_surfels, setup_grid, dim3(kBlock), 0, stream, surfels->means, surfels->scales,
-                           surfels->rotations, ctx->vals[0], ctx->leaves, ctx->pre, surfels->vertices_out, ctx->bounds, rb, n);
+                           surfels->rotations, ctx->vals[0], ctx->leaves, ctx->pre, ctx->bounds, rb, n);
     } else if (rebuild)
         hipLaunchKernelGGL(k_quad_setup, setup_grid, dim3(kBlock), 0, stream, vertices, n_vertices, triangles,
                            quad_ids, centroids, ctx->bounds, n);
@@ -1369,8 +1435,8 @@ int dst_lbvh_build(dst_ctx *ctx, const float *vertices, uint32_t n_vertices, con
             hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(kBlock), 0, stream, ctx->leaf_parent, DST_NO_PARENT, 1u);
         }
     }
-    if (surfels == nullptr)
-        hipLaunchKernelGGL(k_leaf_fill, grid_for(n), dim3(kBlock), 0, stream, vertices, quad_ids, ctx->vals[0],
+    if (vertices != nullptr)
+        hipLaunchKernelGGL(k_leaf_fill, grid_for(n), dim3(kBlock), 0, stream, vertices, !rebuild && ctx->canonical ? nullptr : quad_ids, ctx->vals[0],
                            ctx->leaves, ctx->pre, rb, rebuild ? nullptr : ctx->bounds, ctx->bounds, n);
     if (by_ranges) {
         const uint32_t n_blocks = (n + kRangeBlock - 1) / kRangeBlock;
@@ -1379,14 +1445,16 @@ int dst_lbvh_build(dst_ctx *ctx, const float *vertices, uint32_t n_vertices, con
         for (int level = kRangeLow + 1; (2u << (level - 1)) <= n_blocks; ++level)
             hipLaunchKernelGGL(k_range_table_level, grid_for(n_blocks), dim3(kBlock), 0, stream, ctx->range_table, n_blocks, level);
         if (n > 1)
-            hipLaunchKernelGGL(k_fit_ranges, grid_for(n - 1), dim3(kBlock), 0, stream, ctx->nodes, rb, n_blocks, n - 1);
+            hipLaunchKernelGGL(k_fit_ranges, grid_for(n, kFitThreads), dim3(kFitThreads), 0, stream, ctx->nodes, ctx->node_parent, ctx->leaf_parent, rb, n_blocks, n);
     } else {
         hipLaunchKernelGGL(k_fill_u32, grid_for(n), dim3(kBlock), 0, stream, fit_flags, 0u, n);
         if (vertices == nullptr) return dst_fail(ctx, DST_E_INVALID, "the fit by arrival counters reads the corners from a vertex buffer");
         hipLaunchKernelGGL(k_fit, dim3((n + kFitBlock - 1) / kFitBlock), dim3(kFitBlock), 0, stream, ctx->nodes, ctx->node_parent, ctx->leaf_parent,
                            fit_flags, vertices, quad_ids, ctx->vals[0], n);
     }
-    if (n > DST_GROUP)
+    if (n > DST_GROUP && !rebuild)
+        hipLaunchKernelGGL(k_refit_wide, grid_for(DST_WIDE * (n - 1)), dim3(kBlock), 0, stream, ctx->nodes, ctx->wide, n - 1);
+    else if (n > DST_GROUP)
         hipLaunchKernelGGL(k_widen, grid_for(n - 1), dim3(kBlock), 0, stream, ctx->nodes, ctx->wide, n - 1, ctx->ploc_state + 5);
     DST_HIP(ctx, hipGetLastError());
 

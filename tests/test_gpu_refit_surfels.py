@@ -81,3 +81,39 @@ def test_refit_from_surfels_needs_canonical_quads_and_matching_sizes(tracer):
     tracer.build_acceleration_structure(v, f, True)
     out = tracer.refit_from_surfels(*args)
     assert out.shape == (4 * P, 3)
+
+
+@pytest.mark.parametrize("P", [1, 2, 3, 4, 63, 64, 65, 127, 128, 129, 257, 4097, 66000])
+def test_refits_keep_the_traversal_nodes_of_their_build(oracle, P):
+    """Sizes around the blocks of 64 leaves that the fit works in: after a build every refit (from a vertex buffer, from the
+    surfels with and without corners asked for, and the one that allocates nothing) renews the boxes of the traversal
+    nodes that the build chose.  Boxes as exact unions, and traces as the oracle's."""
+    import ctypes as C
+
+    import diff_surfel_tracing as dst
+    from diff_surfel_tracing import _C
+    lib = _C.load_library()
+    tracer = dst.SurfelTracer()
+    sc = S.scene_cube(P=P, seed=P)
+    o, d = S.rays_cube(24, 24, view=1)
+    gpu_trace(tracer, sc, o, d)
+    handle, stream = tracer.optix_context.handle, C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for frame, way in enumerate(("vertices", "surfels", "no corners", "static", "vertices")):
+        sc = {k: v.clone() for k, v in sc.items()}
+        sc["means3D"] = -sc["means3D"].roll(1, 0)      # no surfel stays near where it was
+        v = torch.from_numpy(corners_as_stated(sc["means3D"].numpy(), sc["scales"].numpy(), sc["rotations"].numpy()))
+        sc["vertices"] = v
+        dev = [sc[k].cuda().contiguous() for k in ("means3D", "scales", "rotations")]
+        if way == "vertices":
+            tracer.build_acceleration_structure(v.cuda(), sc["faces"].cuda(), False)
+        elif way == "surfels":
+            tracer.refit_from_surfels(*dev)
+        elif way == "no corners":
+            assert lib.dst_refit_from_surfels(handle, *(x.data_ptr() for x in dev), P, None, stream) == 0
+        else:
+            vg = v.cuda()
+            assert lib.dst_refit_accel_static(handle, vg.data_ptr(), 4 * P, stream) == 0
+        if P > 1:
+            check_tree(*download(tracer), v.numpy())
+        out, _ = gpu_trace(tracer, sc, o, d, build=False)
+        assert_forward_exact(out, oracle.forward(oracle_scene(oracle, sc, o, d), oracle.HITS_BVH_LEXI))
