@@ -103,6 +103,7 @@ struct DstBounds {          // device-resident reduction targets, order-preservi
     uint32_t scale;         // raw bits of a float: size of the scene's bulk (set by a build, kept by refits); what ray
                             // origins are compared with (rays_run_together, ray keys) - not a bound on anything
     uint32_t small_quads;   // quads with edges below kDstSmallQuad of that size, counted by every build and refit
+    uint32_t layers;        // raw bits of a float, set by a build: the quads' area over the surface of the centroids' box
 };
 // Quads this much smaller than the scene are smaller than a pixel at usual resolutions (a 1080p pixel at half the
 // scene's size away is about 5e-4 of it wide); a context whose last build counted kDstSmallQuadsMin of them traces
@@ -186,6 +187,7 @@ struct dst_ctx {
     uint32_t *det_host = nullptr;      // pinned host copy of the deterministic mode's out-of-range count
     void *core_box = nullptr;          // device: the box the two-level Morton keys are laid over (lbvh.hip)
     float scene_lo[3] = {0, 0, 0}, scene_hi[3] = {0, 0, 0}, max_abs = 0;
+    float layers = 0;                  // as of the last build (DstBounds::layers)
 };
 
 static inline bool dst_handover_active(const dst_ctx *ctx) {

@@ -39,6 +39,12 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+__device__ __forceinline__ float wave_total(float v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    return v;
+}
+
 __global__ void k_init_bounds(DstBounds *b) {
     if (threadIdx.x == 0) {
         for (int a = 0; a < 3; ++a) { b->lo[a] = 0xFFFFFFFFu; b->hi[a] = 0u; }
@@ -98,12 +104,13 @@ __device__ __forceinline__ void load_corners(const float *__restrict__ vertices,
 // the coordinate bound from the kernel that writes the leaf records.
 __global__ void k_quad_setup(const float *__restrict__ vertices, uint32_t n_vertices,
                              const int32_t *__restrict__ triangles, int4 *__restrict__ quad_ids,
-                             float4 *__restrict__ centroids, DstBounds *__restrict__ bounds, uint32_t P) {
+                             float4 *__restrict__ centroids, DstBounds *__restrict__ bounds, float *__restrict__ block_area,
+                             uint32_t P) {
     // grid-stride: a block ends with seven atomics on the same seven words, and those are served one by one,
     // so each block takes many surfels
     __shared__ float s_lo[kBlock / DST_WAVE][3], s_hi[kBlock / DST_WAVE][3];
     float cen[3] = {INFINITY, INFINITY, INFINITY}, cenh[3] = {-INFINITY, -INFINITY, -INFINITY};
-    float mabs = 0.f;
+    float mabs = 0.f, area = 0.f;
     for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < P; g += gridDim.x * blockDim.x) {
         float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
         const int32_t *t = triangles + (size_t)g * 6;   // 24 bytes per surfel: three 8-byte loads where the buffer allows
@@ -136,6 +143,10 @@ __global__ void k_quad_setup(const float *__restrict__ vertices, uint32_t n_vert
                 mabs = finite_max(mabs, fabsf(c[k][a]));
             }
         }
+        const float ab[3] = {c[1][0] - c[0][0], c[1][1] - c[0][1], c[1][2] - c[0][2]}, ac[3] = {c[2][0] - c[0][0], c[2][1] - c[0][1], c[2][2] - c[0][2]};
+        const float nx = ab[1] * ac[2] - ab[2] * ac[1], ny = ab[2] * ac[0] - ab[0] * ac[2], nz = ab[0] * ac[1] - ab[1] * ac[0];
+        const float quad = sqrtf(nx * nx + ny * ny + nz * nz);
+        if (quad < INFINITY) area += quad;
         float4 c4;
         c4.x = 0.5f * (lo[0] + hi[0]);
         c4.y = 0.5f * (lo[1] + hi[1]);
@@ -152,6 +163,8 @@ __global__ void k_quad_setup(const float *__restrict__ vertices, uint32_t n_vert
         cen[a] = wave_min(cen[a]);
         cenh[a] = wave_max(cenh[a]);
     }
+    __shared__ float s_area[kBlock / DST_WAVE];
+    area = wave_total(area);
     const int w = threadIdx.x / DST_WAVE;
     if ((threadIdx.x & (DST_WAVE - 1)) == 0) {
 #pragma unroll
@@ -159,8 +172,14 @@ __global__ void k_quad_setup(const float *__restrict__ vertices, uint32_t n_vert
             s_lo[w][a] = cen[a];
             s_hi[w][a] = cenh[a];
         }
+        s_area[w] = area;
     }
     __syncthreads();
+    if (threadIdx.x == 3) {
+        float sum = 0.f;
+        for (int k = 0; k < (int)(blockDim.x / DST_WAVE); ++k) sum += s_area[k];
+        block_area[blockIdx.x] = sum;
+    }
     if (threadIdx.x < 3) {
         const int a = threadIdx.x;
         float l = INFINITY, h = -INFINITY;
@@ -284,9 +303,16 @@ __global__ void k_core_cut(CoreBox *core) {
     core->s0[a] = core->s1[a] = core->s2[a] = 0ull;
 }
 
-// Size of the scene's bulk: the largest coordinate of the keys' box (two-level keys: the cut box), else of any vertex.
-__global__ void k_scene_scale(DstBounds *bounds, const CoreBox *core) {
+// Size of the scene's bulk: the largest coordinate of the keys' box (two-level keys: the cut box), else of any vertex.  And how
+// often its quads cover its walls: their area (k_quad_setup: by blocks) over the surface of the centroids' box.  One wave.
+__global__ void k_scene_scale(DstBounds *bounds, const CoreBox *core, const float *__restrict__ block_area, uint32_t n_blocks) {
+    float area = 0.f;
+    for (uint32_t k = threadIdx.x; k < n_blocks; k += DST_WAVE) area += block_area[k];
+    area = wave_total(area);
     if (threadIdx.x != 0) return;
+    float e[3];
+    for (int a = 0; a < 3; ++a) e[a] = ord2f(bounds->hi[a]) - ord2f(bounds->lo[a]);
+    bounds->layers = __float_as_uint(area / (2.f * (e[0] * e[1] + e[1] * e[2] + e[2] * e[0])));
     float m = __uint_as_float(bounds->max_abs);
     if (core != nullptr) {
         float c = 0.f;
@@ -1386,7 +1412,7 @@ int dst_lbvh_build(dst_ctx *ctx, const float *vertices, uint32_t n_vertices, con
                            surfels->rotations, ctx->vals[0], ctx->leaves, ctx->pre, ctx->bounds, rb, n);
     } else if (rebuild)
         hipLaunchKernelGGL(k_quad_setup, setup_grid, dim3(kBlock), 0, stream, vertices, n_vertices, triangles,
-                           quad_ids, centroids, ctx->bounds, n);
+                           quad_ids, centroids, ctx->bounds, reinterpret_cast<float *>(ctx->tile_hist), n);   // (idle until the sort)
 
     if (rebuild) {
         if (ctx->fine_keys) {
@@ -1399,7 +1425,7 @@ int dst_lbvh_build(dst_ctx *ctx, const float *vertices, uint32_t n_vertices, con
                                    centroids, core, n);
                 hipLaunchKernelGGL(k_core_cut, dim3(1), dim3(64), 0, stream, core);
             }
-            hipLaunchKernelGGL(k_scene_scale, dim3(1), dim3(64), 0, stream, ctx->bounds, core);
+            hipLaunchKernelGGL(k_scene_scale, dim3(1), dim3(64), 0, stream, ctx->bounds, core, reinterpret_cast<const float *>(ctx->tile_hist), setup_grid.x);
             hipLaunchKernelGGL(k_morton_fine, grid_for(n), dim3(kBlock), 0, stream, centroids, core, ctx->keys[0],
                                lo_of, hi_of, ctx->vals[0], n);
             dst_sort_pairs(ctx->keys, ctx->vals, ctx->tile_hist, n, stream);
@@ -1407,7 +1433,7 @@ int dst_lbvh_build(dst_ctx *ctx, const float *vertices, uint32_t n_vertices, con
             dst_sort_pairs(ctx->keys, ctx->vals, ctx->tile_hist, n, stream);   // stable: equal cells stay in `lo` order
             hipLaunchKernelGGL(k_gather_u32, grid_for(n), dim3(kBlock), 0, stream, ctx->keys[1], lo_of, ctx->vals[0], n);
         } else {
-            hipLaunchKernelGGL(k_scene_scale, dim3(1), dim3(64), 0, stream, ctx->bounds, (const CoreBox *)nullptr);
+            hipLaunchKernelGGL(k_scene_scale, dim3(1), dim3(64), 0, stream, ctx->bounds, (const CoreBox *)nullptr, reinterpret_cast<const float *>(ctx->tile_hist), setup_grid.x);
             hipLaunchKernelGGL(k_morton, grid_for(n), dim3(kBlock), 0, stream, centroids, ctx->bounds, ctx->keys[0],
                                ctx->vals[0], n);
             dst_sort_pairs(ctx->keys, ctx->vals, ctx->tile_hist, n, stream);   // the sorted pairs end in buffer 0
@@ -1479,6 +1505,7 @@ int dst_lbvh_build(dst_ctx *ctx, const float *vertices, uint32_t n_vertices, con
             ctx->scene_hi[a] = ord2f(ctx->bounds_host->hi[a]);
         }
         std::memcpy(&ctx->max_abs, &ctx->bounds_host->max_abs, 4);
+        std::memcpy(&ctx->layers, &ctx->bounds_host->layers, 4);
         ctx->small_quads = ctx->bounds_host->small_quads;
         ctx->small_quads_refits = ctx->refits;
         ctx->small_quads_asked = false;

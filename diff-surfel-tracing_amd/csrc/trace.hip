@@ -1951,6 +1951,60 @@ __global__ __launch_bounds__(1024) void k_block_order(const uint32_t *__restrict
     }
 }
 
+// Order of the blocks of a forward trace: those that look long first, so that no tile of a millisecond begins when the chip
+// is about to run dry.  What a block will cost is guessed from how many leaf groups lie in the way of its rays, from the
+// boxes alone: a wave walks down for sixty-four of its 256 rays (the outermost among them) as the tiles' waves will, without
+// quads, windows or distances.  A guess that is off costs time and nothing else.  (It goes with the time of the block's longest
+// tile at 0.75 to 0.9 on the scenes measured; of an 800x800 sphere's 10,000 tiles the last to begin ran from 0.6 to 1.75 ms.)
+constexpr uint32_t kCostMax = 2047u;   // leaf groups counted; a wave stops there
+__device__ __forceinline__ uint32_t block_cost(const DstParams &p, const DstAccelView &acc, uint32_t block, uint32_t btiles_x, lds_u32 area) {
+    const uint32_t lane = __lane_id(), bx = block % btiles_x, by = block / btiles_x;
+    const uint32_t px = 16u * bx + (lane & 7u) * 15u / 7u, py = 16u * by + (lane >> 3) * 15u / 7u;
+    const bool inside = px < (uint32_t)p.W && py < (uint32_t)p.H;
+    const size_t r = inside ? (size_t)py * p.W + px : 0;
+    const F3 o = ld3(p.ray_o + 3 * r), d = ld3(p.ray_d + 3 * r);
+    const float dmax = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(d.x), __builtin_fabsf(d.y)), __builtin_fabsf(d.z));
+    const bool usable = inside && (__builtin_fabsf(o.x) + __builtin_fabsf(o.y)) + __builtin_fabsf(o.z) < INFINITY && dmax > 0.f &&
+                        (__builtin_fabsf(d.x) + __builtin_fabsf(d.y)) + __builtin_fabsf(d.z) < INFINITY;
+    const uint64_t todo = wave_ballot(usable);
+    uint32_t count = 0u;
+    if (todo != 0ull && !(acc.root & DST_LEAF_BIT)) {
+        const int lead = __builtin_ctzll(todo);
+        const float lx = lane_value(d.x, lead), ly = lane_value(d.y, lead), lz = lane_value(d.z, lead);
+        const float ax_ = __builtin_fabsf(lx), ay_ = __builtin_fabsf(ly), az_ = __builtin_fabsf(lz);
+        const uint32_t ax = (ax_ >= ay_ && ax_ >= az_) ? 0u : (ay_ >= az_ ? 1u : 2u);
+        const float sg = (ax == 0u ? lx : (ax == 1u ? ly : lz)) > 0.f ? 1.0f : -1.0f;
+        const bool mine = usable && dmax <= kBwMaxSlope * (sg * axis_of(d, ax));   // (rays apart from the first: not looked at)
+        const BundleLds lds = {area};
+        (void)bundle_begin(lds.base, ax, sg, o, d, mine, __uint_as_float(acc.bounds->scale));
+        count = bundle_count({acc.leaves, acc.wide, acc.n_leaves, acc.root}, lds, kCostMax);
+    }
+    return count;
+}
+// Counting sort by that guess, in one workgroup; blocks of equal cost keep their neighbourhood, 1024 at a time.
+__global__ __launch_bounds__(1024) void k_cost_order(const uint32_t *__restrict__ cost, uint32_t n_blocks, uint32_t *__restrict__ order) {
+    constexpr uint32_t kClasses = 128u;
+    __shared__ uint32_t s_count[kClasses], s_base[kClasses];
+    auto cost_class = [&](uint32_t j) { return kClasses - 1u - min(cost[j] / ((kCostMax + 1u) / kClasses), kClasses - 1u); };   // 0: the longest
+    if (threadIdx.x < kClasses) s_count[threadIdx.x] = 0u;
+    __syncthreads();
+    for (uint32_t j = threadIdx.x; j < n_blocks; j += blockDim.x) atomicAdd(&s_count[cost_class(j)], 1u);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t run = 0u;
+        for (uint32_t c = 0; c < kClasses; ++c) {
+            s_base[c] = run;
+            run += s_count[c];
+        }
+    }
+    __syncthreads();
+    for (uint32_t base = 0; base < n_blocks; base += blockDim.x) {
+        const uint32_t j = base + threadIdx.x;
+        if (j < n_blocks) order[atomicAdd(&s_base[cost_class(j)], 1u)] = j;
+        __syncthreads();
+    }
+}
+
 // Tile hand-over (forward).  A bundle walk lists and tests what any of its 64 rays may need, one candidate after the
 // other.  Over geometry much finer than the ray spacing (a dense cloud of surfels far smaller than a pixel) that is the
 // whole content of the tile's frustum, wanted by one ray at best, and a single wave walks for milliseconds while the chip
@@ -2018,7 +2072,8 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
     // vertical neighbours and meet the same BVH nodes in that XCD's own L2 (row-major order over a 120-block-wide image
     // gives an XCD blocks eight columns apart).  The last strip may be narrower; its blocks are spread over all XCDs
     // like the others.  The launcher chooses the width, and has the figures (launch()).
-    if (BWD && block_order != nullptr) bid = block_order[bid];   // replay: the longest blocks first (k_block_order)
+    // the longest blocks first (replay: k_block_order; forward: k_cost_order)
+    if (block_order != nullptr) bid = bid < btiles_x * ((tiles_y + 1u) / 2u) ? block_order[bid] : bid;
     uint32_t bx, by;
     static_assert(!HAND || (!BWD && kFwdWavesPerBlock == 1), "tiles are handed over by forward kernels of one wave per workgroup");
     const bool taker = HAND && MIXED && handover != nullptr && hand_arg == 0u;
@@ -2309,8 +2364,9 @@ void k_trace_fwd(const DstParams p, const DstAccelView acc, int tw_log2, int th_
 template <int AUXM, bool REC, bool PACK>
 __global__ __launch_bounds__(kFwdWavesPerBlock *DST_WAVE) __attribute__((amdgpu_waves_per_eu(DST_FWD_WAVES, DST_FWD_WAVES)))
 void k_trace_fwd_plain(const DstParams p, const DstAccelView acc, int tw_log2, int th_log2, uint32_t tiles_x,
-                       uint32_t tiles_y, uint32_t btiles_x, const uint32_t *ray_order, uint32_t strip_width) {
-    trace_body<false, AUXM, REC, false, false, false, PACK>(p, acc, tw_log2, th_log2, tiles_x, tiles_y, btiles_x, ray_order, strip_width, nullptr, nullptr, 0u);
+                       uint32_t tiles_y, uint32_t btiles_x, const uint32_t *ray_order, uint32_t strip_width,
+                       const uint32_t *block_order) {
+    trace_body<false, AUXM, REC, false, false, false, PACK>(p, acc, tw_log2, th_log2, tiles_x, tiles_y, btiles_x, ray_order, strip_width, block_order, nullptr, 0u);
 }
 template <int AUXM, bool REC, bool MIXED, bool DET>
 __global__ __launch_bounds__(kWavesPerBlock *DST_WAVE) __attribute__((amdgpu_waves_per_eu(DST_BWD_WAVES, DST_BWD_WAVES)))
@@ -2320,10 +2376,8 @@ void k_trace_bwd(const DstParams p, const DstAccelView acc, int tw_log2, int th_
     trace_body<true, AUXM, REC, MIXED, DET, false, false>(p, acc, tw_log2, th_log2, tiles_x, tiles_y, btiles_x, ray_order, strip_width, block_order, nullptr, 0u);
 }
 
-// Surfel records, a thread per surfel: 40 bytes in, 64 out.
-__global__ __launch_bounds__(256) void k_surfel_records(const DstParams p) {
-    const uint32_t g = blockIdx.x * 256u + threadIdx.x;
-    if (g >= (uint32_t)p.P) return;
+// Surfel record of surfel g: 40 bytes in, 64 out.
+__device__ __forceinline__ void surfel_record(const DstParams &p, uint32_t g) {
     const F3 mean = ld3(p.means3D + 3 * (size_t)g);
     const float sx = p.scales[2 * (size_t)g], sy = p.scales[2 * (size_t)g + 1];
     const float *qp = p.rotations + 4 * (size_t)g;
@@ -2338,6 +2392,23 @@ __global__ __launch_bounds__(256) void k_surfel_records(const DstParams p) {
     out[1] = v4f{R[1].x, R[1].y, R[1].z, -dot(R[1], mean)};
     out[2] = v4f{R[2].x, R[2].y, R[2].z, p.opacities[g]};
     out[3] = v4f{sx, sy, inverse(sx), inverse(sy)};
+}
+// What a forward trace prepares, in one launch: the blocks' costs (a wave each, first, as they take longest) and the surfels'
+// records (a thread each).
+constexpr uint32_t kPrepareWaves = 4u;
+__global__ __launch_bounds__(kPrepareWaves *DST_WAVE) void k_prepare(const DstParams p, const DstAccelView acc, uint32_t btiles_x, uint32_t *cost,
+                                                                     uint32_t n_blocks) {
+    __shared__ uint32_t s_lds[kPrepareWaves * (kBwStateWords + kBwStack)];
+    const uint32_t of_cost = (n_blocks + kPrepareWaves - 1u) / kPrepareWaves;
+    if (blockIdx.x < of_cost) {
+        const uint32_t wave = uni(threadIdx.x / DST_WAVE), block = blockIdx.x * kPrepareWaves + wave;
+        if (block >= n_blocks) return;
+        const uint32_t count = block_cost(p, acc, block, btiles_x, (lds_u32)s_lds + wave * (kBwStateWords + kBwStack));
+        if (__lane_id() == 0u) cost[block] = count;
+    } else {
+        const uint32_t g = (blockIdx.x - of_cost) * kPrepareWaves * DST_WAVE + threadIdx.x;
+        if (g < (uint32_t)p.P) surfel_record(p, g);
+    }
 }
 
 #include "row.inc"
@@ -2545,10 +2616,10 @@ void launch(const DstParams &p, const DstAccelView &acc, const TileGrid &t, cons
                                t.tw_log2, t.th_log2, t.tiles_x, t.tiles_y, t.btiles_x, ray_order, strip, block_order);    \
         else if (!(MIXED) && p.flags == 0u && handover == nullptr && p.scratch != nullptr && (AUX) < 8)            \
             hipLaunchKernelGGL((k_trace_fwd_plain<AUX, REC, (AUX) < 8>), grid, block, 0, stream, p, acc, t.tw_log2, \
-                               t.th_log2, t.tiles_x, t.tiles_y, t.btiles_x, ray_order, strip);                            \
+                               t.th_log2, t.tiles_x, t.tiles_y, t.btiles_x, ray_order, strip, block_order);               \
         else if (!(MIXED) && p.flags == 0u && handover == nullptr)                                                 \
             hipLaunchKernelGGL((k_trace_fwd_plain<AUX, REC, false>), grid, block, 0, stream, p, acc, t.tw_log2,           \
-                               t.th_log2, t.tiles_x, t.tiles_y, t.btiles_x, ray_order, strip);                            \
+                               t.th_log2, t.tiles_x, t.tiles_y, t.btiles_x, ray_order, strip, block_order);               \
         else if (p.flags != 0u)                                                                                    \
             hipLaunchKernelGGL((k_trace_fwd<AUX, REC, MIXED, true>), grid, block, 0, stream, p, acc, t.tw_log2,    \
                                t.th_log2, t.tiles_x, t.tiles_y, t.btiles_x, ray_order, strip, handover, hand_arg);        \
@@ -2652,10 +2723,45 @@ void launch_row_bwd(const DstParams &p, RowGrid g, const uint32_t *ray_order, hi
 #undef DST_ROW
 }
 
-// Records where the kernels that read them are launched next: plain tiles, and rows beyond them.
-void make_records(const DstParams &p, hipStream_t stream) {
-    if (p.scratch == nullptr || p.flags != 0u) return;
-    hipLaunchKernelGGL(k_surfel_records, dim3(((uint32_t)p.P + 255u) / 256u), dim3(256), 0, stream, p);
+// What a forward trace keeps in its scratch memory: the surfels' records, and behind them the guessed cost of every block and
+// the order that follows from it.  Records are worth their pass where there are no more than four surfels to a ray (0.03 ns a
+// surfel against 0.09 a ray of the 1080p room), the order on grids of up to 4095 blocks: larger ones keep the chip full to the
+// end (1280x720 room of 300,000 surfels, 3600 blocks: 504 / 503 us without and with, of a million 1903 / 1708), and a single
+// launch in front of them more than pays for it only where tiles take long, which is where quads cover the scene many times
+// over (DstBounds::layers).  Without / with, us: 800x800 sphere of 100,000 (20 layers) 1588 / 1124, 600x600 of 30,000 (6) 378 /
+// 297, 500x500 of 20,000 (4) 204 / 218; room of a million (29) 640x360 1163 / 918, 960x540 1395 / 1175, of 200,000 (6) 640x360
+// 183 / 173, of 100,000 (3) 121 / 119, of 50,000 (1.4) 83 / 90, 480x270 63 / 75.  Records of that last room cost it 1 us.
+constexpr uint64_t kOrderedBlocks = 4095u;
+constexpr float kOrderedLayers = 5.0f, kRecordedLayers = 2.0f;
+struct ScratchLayout {
+    uint64_t records, blocks;   // 0: none
+    ScratchLayout(int32_t P, int32_t H, int32_t W) : records(0), blocks(0) {
+        const uint64_t rays = (uint64_t)std::max(H, 0) * (uint64_t)std::max(W, 0);
+        if (P <= 0 || H < kThinRows || rays <= kRowRecordedRays) return;
+        const TileGrid t = tile_grid(H, W);
+        if (rays >= (uint64_t)P / 4u) records = (uint64_t)P;
+        if ((uint64_t)t.btiles_x * t.btiles_y <= kOrderedBlocks) blocks = (uint64_t)t.btiles_x * t.btiles_y;
+    }
+    uint64_t bytes() const { return sizeof(DstSurfel) * records + 2u * sizeof(uint32_t) * blocks; }
+};
+// Made where the kernels that read it are launched next, plain tiles and the rows beyond them.  Returns the order of the blocks
+// (nullptr: as they lie), and takes from p.scratch what these kernels shall not look for.
+const uint32_t *make_scratch(const dst_ctx *ctx, DstParams &p, const DstAccelView &acc, const TileGrid &t, hipStream_t stream) {
+    if (p.scratch == nullptr || p.flags != 0u) return nullptr;
+    ScratchLayout s(p.P, p.H, p.W);
+    if (ctx->layers < kOrderedLayers) s.blocks = 0u;   // (no number, of a scene on a line: many)
+    if (ctx->layers < kRecordedLayers) s.records = 0u;
+    if (s.records == 0u && s.blocks == 0u) {
+        p.scratch = nullptr;
+        return nullptr;
+    }
+    uint32_t *const cost = reinterpret_cast<uint32_t *>(reinterpret_cast<DstSurfel *>(p.scratch) + s.records), *const order = cost + s.blocks;
+    const uint32_t n_blocks = (uint32_t)s.blocks, threads = kPrepareWaves * DST_WAVE;
+    const uint32_t grid = (n_blocks + kPrepareWaves - 1u) / kPrepareWaves + ((uint32_t)s.records + threads - 1u) / threads;
+    hipLaunchKernelGGL(k_prepare, dim3(grid), dim3(threads), 0, stream, p, acc, t.btiles_x, cost, n_blocks);
+    if (n_blocks != 0u) hipLaunchKernelGGL(k_cost_order, dim3(1), dim3(1024), 0, stream, cost, n_blocks, order);
+    if (s.records == 0u) p.scratch = nullptr;
+    return n_blocks != 0u ? order : nullptr;
 }
 
 void launch_close(const DstParams &p, uint32_t *out_of_range, hipStream_t stream) {
@@ -2688,13 +2794,7 @@ uint64_t dst_det_workspace_words(int32_t P, int32_t aux, int backward) {
     return (uint64_t)P * cols;
 }
 
-// Worth it on images that tiles trace, with at least half as many rays as surfels: a record takes 0.03 ns to make, and spares
-// a ray of the 1080p room 0.09.
-uint64_t dst_trace_scratch_bytes(int32_t P, int32_t H, int32_t W) {
-    if (P <= 0 || H < kThinRows || W <= 0) return 0;
-    const uint64_t rays = (uint64_t)H * W;
-    return rays > kRowRecordedRays && rays >= (uint64_t)P / 2u ? sizeof(DstSurfel) * (uint64_t)P : 0u;
-}
+uint64_t dst_trace_scratch_bytes(int32_t P, int32_t H, int32_t W) { return ScratchLayout(P, H, W).bytes(); }
 
 uint64_t dst_hit_record_layout(int32_t H, int32_t W, int32_t mtd_alloc, uint32_t blocks, uint64_t *header_words,
                                uint32_t *n_waves) {
@@ -2824,20 +2924,20 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
             if (rec) launch_row_fwd<true, RowTiles>(p, acc, rows, ray_order, stream);
             else launch_row_fwd<false, RowRays>(p, acc, row_squares(p, rows), ray_order, stream);
         } else if (by == TraceBy::TilesThenRows && list == nullptr) {
-            make_records(p, stream);
+            const uint32_t *const order = make_scratch(ctx, p, acc, t, stream);
             if (rec) {
-                launch<false, true>(p, acc, t, ray_order, stream, nullptr, nullptr, 0u, true);
+                launch<false, true>(p, acc, t, ray_order, stream, order, nullptr, 0u, true);
                 launch_row_fwd<true, RowBeyond>(p, acc, rows, ray_order, stream);
             } else {
-                launch<false, false>(p, acc, t, ray_order, stream, nullptr, nullptr, 0u, true);
+                launch<false, false>(p, acc, t, ray_order, stream, order, nullptr, 0u, true);
                 launch_row_fwd<false, RowBeyond>(p, acc, rows, ray_order, stream);
             }
         } else
         for (int pass = 0; pass < (list != nullptr ? 2 : 1); ++pass) {
             const uint32_t arg = pass == 0 ? steps : 0u;
-            if (list == nullptr && t.th_log2 == 3) make_records(p, stream);
-            if (rec) launch<false, true>(p, acc, t, ray_order, stream, nullptr, list, arg);
-            else launch<false, false>(p, acc, t, ray_order, stream, nullptr, list, arg);
+            const uint32_t *const order = list == nullptr && t.th_log2 == 3 ? make_scratch(ctx, p, acc, t, stream) : nullptr;
+            if (rec) launch<false, true>(p, acc, t, ray_order, stream, order, list, arg);
+            else launch<false, false>(p, acc, t, ray_order, stream, order, list, arg);
         }
         if (det && p.training && p.a_weights != nullptr)
             hipLaunchKernelGGL(k_det_finish_weights, dim3(1024), dim3(256), 0, stream, p, out_of_range);

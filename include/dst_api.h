@@ -154,8 +154,8 @@ typedef struct DstParams {
     int32_t dist_channels;        /* forward: channels of out_dist: 1 (the distortion alone), or 3 (also 0: three) */
     int32_t reserved;
     /* forward, optional: device memory, aligned to 128 bytes, dst_trace_scratch_bytes(P, H, W) of it, in which the call keeps
-     * what it derives from the surfels' parameters before it traces (contents before and after the call mean nothing).  Same
-     * results bit for bit, faster; NULL: everything is derived anew at every hit. */
+     * what it prepares before it traces: what depends on a surfel alone, and an order for the image's tiles (contents before
+     * and after the call mean nothing).  Same results bit for bit, faster; NULL: neither is made. */
     void *scratch;
 } DstParams;
 
@@ -280,7 +280,7 @@ uint64_t dst_hit_record_layout(int32_t H, int32_t W, int32_t mtd_alloc, uint32_t
                                uint32_t *n_waves);
 
 /* Size in bytes of DstParams.scratch for a forward trace of P surfels over an (H,W) ray grid; 0 where the call has no use for
- * any (lists and small images, or far fewer rays than surfels). */
+ * any (lists, small images, and the largest with far fewer rays than surfels). */
 uint64_t dst_trace_scratch_bytes(int32_t P, int32_t H, int32_t W);
 
 /* Words (8 bytes each) of DstParams.det_workspace for a forward (backward = 0: one per surfel) or a backward

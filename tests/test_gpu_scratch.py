@@ -1,5 +1,5 @@
-"""The forward trace's scratch memory (DstParams.scratch): hits evaluated from records of the surfels that the call makes
-first.  Outputs and hit records have to be those of the same call without scratch memory bit for bit, whatever the
+"""The forward trace's scratch memory (DstParams.scratch): hits evaluated from records of the surfels, and blocks traced in
+the order of a cost guessed for them, both of which the call makes first.  Outputs and hit records have to be those of the same call without scratch memory bit for bit, whatever the
 scales (quotients by them are formed from their reciprocals in the records, and divided out where that does not hold)."""
 import pytest
 import torch
@@ -28,12 +28,33 @@ def both(monkeypatch, tracer, sc, o, d, depth=0, aux=0, training=False):
     return out
 
 
+def view(H, W):
+    return S.pinhole_rays(H, W, 70.0, (-0.6, -0.3, 0.15), (0.9, 0.45, -0.15))
+
+
+@pytest.mark.parametrize("H,W", [(8, 8221), (4111, 16), (257, 256), (1040, 1008), (1040, 1024)])
+@pytest.mark.parametrize("P,half", [(3000, 0.4), (250000, 1.5)])
+def test_every_block_is_traced_once(monkeypatch, H, W, P, half):
+    """One row and one column of blocks, an odd one, the largest grid whose blocks are ordered and one larger; fewer surfels
+    than rays, and so many that only the order is made."""
+    import diff_surfel_tracing as dst
+    tracer = dst.SurfelTracer()
+    sc = S.scene_room(P=P, seed=6, half=half)
+    o, d = S.pinhole_rays(H, W, 70.0, (-0.4 * half, -0.2 * half, 0.1 * half), (0.6 * half, 0.3 * half, -0.1 * half))
+    tracer.build_acceleration_structure(sc["vertices"].cuda(), sc["faces"].cuda(), rebuild=True)
+    with_, without = both(monkeypatch, tracer, sc, o, d, training=True)
+    assert without[0].std() > 0.01
+    for a, b in zip(with_[:-1], without[:-1]):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+    torch.testing.assert_close(with_[-1], without[-1], rtol=1e-4, atol=1e-4)   # blending weights: sums in another order
+
+
 @pytest.mark.parametrize("depth,aux", [(0, 0), (0, 3), (1, 2), (1, 8)])
 def test_records_change_no_bit(monkeypatch, depth, aux):
     import diff_surfel_tracing as dst
     tracer = dst.SurfelTracer()
-    sc = S.scene_room(P=30011, seed=4)
-    o, d = S.rays_room(259, 331)
+    sc = S.scene_room(P=30011, seed=4, half=1.5)
+    o, d = view(259, 331)
     tracer.build_acceleration_structure(sc["vertices"].cuda(), sc["faces"].cuda(), rebuild=True)
     with_, without = both(monkeypatch, tracer, sc, o, d, depth, aux)
     for a, b in zip(with_, without):
@@ -46,8 +67,8 @@ def test_scales_of_any_size(monkeypatch, factor):
     """The quads stay what they are; the scales the trace is given are theirs times `factor`, on every third surfel."""
     import diff_surfel_tracing as dst
     tracer = dst.SurfelTracer()
-    sc = S.scene_room(P=20000, seed=5)
-    o, d = S.rays_room(257, 257)
+    sc = S.scene_room(P=20000, seed=5, half=1.5)
+    o, d = view(257, 257)
     tracer.build_acceleration_structure(sc["vertices"].cuda(), sc["faces"].cuda(), rebuild=True)
     sc["scales"][::3] *= factor
     if factor in (2.0 ** -40, 2.0 ** 40):   # the edges of the reciprocals' range
