@@ -597,10 +597,33 @@ __device__ __forceinline__ float quad_magnitude(const float (&c)[4][3]) {
     return m;
 }
 
-// Leaf record + conservative stand-in of one quad (corners c[0..3] = A,B,C,D, surfel id g) at leaf position i.
+// Consecutive rows of WORDS words, one a thread, out to memory as they lie: through LDS, so that neighbouring lanes write
+// neighbouring words.  All threads of the block (kBlock of them) take part; `rows` of them have one.  (From the threads that
+// made them, a store of a wave touches 64 cache lines and takes 224 cycles of a CU, 158 like this: k_leaf_fill of 2M surfels
+// 203 -> 166 us, of 1M 105 -> 90, k_surfel_quads of 2M 52 -> 44.)
+constexpr uint32_t kStageWords = 24;
+template <int WORDS>
+__device__ __forceinline__ void block_store(float *stage, const float (&row)[WORDS], float *__restrict__ dst, uint32_t rows) {
+    static_assert(WORDS % 2 == 0 && WORDS <= (int)kStageWords, "pieces of eight or sixteen bytes");
+    constexpr bool WIDE = WORDS % 4 == 0;
+    constexpr uint32_t kPieces = WORDS / (WIDE ? 4 : 2);
+    __syncthreads();   // (what lay there before is out)
+    float *mine = stage + (size_t)threadIdx.x * WORDS;
+#pragma unroll
+    for (uint32_t k = 0; k < kPieces; ++k) {
+        if (WIDE) reinterpret_cast<float4 *>(mine)[k] = make_float4(row[4 * k], row[4 * k + 1], row[(4 * k + 2) % WORDS], row[(4 * k + 3) % WORDS]);
+        else reinterpret_cast<float2 *>(mine)[k] = make_float2(row[2 * k], row[2 * k + 1]);
+    }
+    __syncthreads();
+    for (uint32_t e = threadIdx.x; e < rows * kPieces; e += kBlock) {
+        if (WIDE) reinterpret_cast<float4 *>(dst)[e] = reinterpret_cast<const float4 *>(stage)[e];
+        else reinterpret_cast<float2 *>(dst)[e] = reinterpret_cast<const float2 *>(stage)[e];
+    }
+}
+
+// Leaf record + conservative stand-in of one quad (corners c[0..3] = A,B,C,D, surfel id g), as DstLeaf and DstLeafPre have them.
 // The plane normals use the fused form the hit test is defined with: cross(x,y).x = fma(x.y, y.z, -(x.z*y.y)), ...
-__device__ __forceinline__ void write_leaf(const float (&c)[4][3], uint32_t g, uint32_t i, DstLeaf *__restrict__ leaves,
-                                           DstLeafPre *__restrict__ pre) {
+__device__ __forceinline__ void make_leaf(const float (&c)[4][3], uint32_t g, float (&out)[24], float (&pr)[16]) {
     auto cross_f = [](const float *x, const float *y, float *out) {
         out[0] = __builtin_fmaf(x[1], y[2], -(x[2] * y[1]));
         out[1] = __builtin_fmaf(x[2], y[0], -(x[0] * y[2]));
@@ -619,7 +642,6 @@ __device__ __forceinline__ void write_leaf(const float (&c)[4][3], uint32_t g, u
     cross_f(f1, f2, n1);
     cross_f(e2, e3, n2);
     const float c1 = __builtin_fmaf(n1[2], e1[2], __builtin_fmaf(n1[1], e1[1], n1[0] * e1[0]));
-    float out[24];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         out[a] = c[0][a];
@@ -635,9 +657,6 @@ __device__ __forceinline__ void write_leaf(const float (&c)[4][3], uint32_t g, u
     out[23] = 0.f;   // largest coordinate of an edge vector
 #pragma unroll
     for (int a = 0; a < 3; ++a) out[23] = fmaxf(out[23], fmaxf(fmaxf(fabsf(e1[a]), fabsf(e2[a])), fabsf(e3[a])));
-    float4 *dst = reinterpret_cast<float4 *>(&leaves[i]);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) dst[k] = make_float4(out[4 * k], out[4 * k + 1], out[4 * k + 2], out[4 * k + 3]);
 
     // the conservative stand-in (see DstLeafPre): mean plane, averaged half edges, their dual vectors
     float cen[3], nrm[3], h1[3], h2[3];
@@ -683,7 +702,6 @@ __device__ __forceinline__ void write_leaf(const float (&c)[4][3], uint32_t g, u
     const float rad_padded = rad + kPlanePad * mag;
     const bool ok = isfinite(mfu) && isfinite(lim0) && isfinite(tdev) && isfinite(rad_padded) && isfinite(cen[0] + cen[1] + cen[2]) &&
                     isfinite(nrm[0] + nrm[1] + nrm[2]) && nl > 0.f;
-    float pr[16];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         pr[a] = ok ? cen[a] : 0.f;
@@ -695,9 +713,6 @@ __device__ __forceinline__ void write_leaf(const float (&c)[4][3], uint32_t g, u
     pr[13] = ok ? lim0 : INFINITY;
     pr[14] = ok ? tdev : INFINITY;
     pr[15] = ok ? rad_padded : INFINITY;
-    float4 *pdst = reinterpret_cast<float4 *>(&pre[i]);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) pdst[k] = make_float4(pr[4 * k], pr[4 * k + 1], pr[4 * k + 2], pr[4 * k + 3]);
 }
 
 // ---- boxes of leaf ranges without climbing the tree ---------------------------------------------------------
@@ -726,9 +741,10 @@ __device__ __forceinline__ void box_store(float *dst, const float (&b)[6]) {
     d[1] = make_float2(b[2], b[3]);
     d[2] = make_float2(b[4], b[5]);
 }
-// Called by ALL 64 lanes of a wave whose lane l holds leaf position base + l (`valid`: that position exists).
-__device__ __forceinline__ void wave_range_boxes(const float (&c)[4][3], bool valid, uint32_t i, uint32_t n,
-                                                 const RangeBoxes &rb) {
+// Called by ALL threads of a block whose thread t holds leaf position i = base + t, base a multiple of kBlock (`valid`: that
+// position exists).
+__device__ __forceinline__ void block_range_boxes(float *stage, const float (&c)[4][3], bool valid, uint32_t i, uint32_t n,
+                                                  const RangeBoxes &rb) {
     const uint32_t lane = threadIdx.x % DST_WAVE;
     float box[6], pre[6], suf[6];
     const float pad = kBoxPad * quad_magnitude(c);
@@ -748,11 +764,11 @@ __device__ __forceinline__ void wave_range_boxes(const float (&c)[4][3], bool va
             if ((int)lane + off < DST_WAVE) suf[k] = k < 3 ? fminf(suf[k], down) : fmaxf(suf[k], down);
         }
     }
-    if (!valid) return;
-    box_store(rb.lbox + 6 * (size_t)i, box);
-    box_store(rb.pbox + 6 * (size_t)i, pre);
-    box_store(rb.sbox + 6 * (size_t)i, suf);
-    if (lane == DST_WAVE - 1 || i == n - 1u) box_store(rb.table + 6 * (size_t)(i / kRangeBlock), pre);   // level 0: whole blocks
+    const uint32_t base = i - threadIdx.x, rows = min(n - base, (uint32_t)kBlock);
+    block_store(stage, box, rb.lbox + 6 * (size_t)base, rows);
+    block_store(stage, pre, rb.pbox + 6 * (size_t)base, rows);
+    block_store(stage, suf, rb.sbox + 6 * (size_t)base, rows);
+    if (valid && (lane == DST_WAVE - 1 || i == n - 1u)) box_store(rb.table + 6 * (size_t)(i / kRangeBlock), pre);   // level 0: whole blocks
 }
 // The first kRangeLow levels in one launch: a workgroup takes 1024 blocks and the 1023 behind them through LDS, joining
 // neighbours twice as far apart from level to level.  (A launch per level took 4.6 us each, ten of a refit's fourteen.)
@@ -885,23 +901,26 @@ __global__ void k_leaf_fill(const float *__restrict__ vertices, const int4 *__re
                             const uint32_t *__restrict__ sorted_ids, DstLeaf *__restrict__ leaves,
                             DstLeafPre *__restrict__ pre, RangeBoxes rb, DstBounds *__restrict__ bounds,
                             DstBounds *__restrict__ count_small, uint32_t n) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = i < n;   // every lane stays for the wave-wide scans of the boxes
+    __shared__ alignas(16) float s_stage[kBlock * kStageWords];
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x, base = blockIdx.x * kBlock, rows = min(n - base, (uint32_t)kBlock);
+    const bool valid = i < n;   // every thread stays for the stores, and for the scans of the boxes
     // (quad_ids == nullptr: known to be rows 4g..4g+3, so 16 bytes a quad need not be gathered)
-    float c[4][3] = {};
+    float c[4][3] = {}, leaf[24] = {}, stand_in[16] = {};
     float mabs = 0.f;
     bool small = false;
     if (valid) {
         const uint32_t g = sorted_ids[i];
         load_corners(vertices, quad_ids != nullptr ? quad_ids[g] : make_int4((int)(4u * g), (int)(4u * g + 1u), (int)(4u * g + 2u), (int)(4u * g + 3u)), g, c);
-        write_leaf(c, g, i, leaves, pre);
+        make_leaf(c, g, leaf, stand_in);
         small = quad_is_small(c, __uint_as_float(count_small->scale));
 #pragma unroll
         for (int k = 0; k < 4; ++k)
 #pragma unroll
             for (int a = 0; a < 3; ++a) mabs = finite_max(mabs, fabsf(c[k][a]));
     }
-    if (rb.lbox != nullptr) wave_range_boxes(c, valid, i, n, rb);
+    block_store(s_stage, leaf, reinterpret_cast<float *>(leaves + base), rows);
+    block_store(s_stage, stand_in, reinterpret_cast<float *>(pre + base), rows);
+    if (rb.lbox != nullptr) block_range_boxes(s_stage, c, valid, i, n, rb);
     if (bounds != nullptr) block_max_abs(mabs, bounds);   // a refit: the coordinate bound of the moved quads
     count_small_quads(small, count_small);
 }
@@ -928,29 +947,29 @@ __device__ __forceinline__ void surfel_corners(const float *__restrict__ means, 
         for (int a = 0; a < 3; ++a) c[k][a] = (m[a] + sa[k] * u[a]) + sb[k] * v[a];
 }
 // The corners of all surfels as a vertex buffer, rows 4g..4g+3, in the surfels' order; k_leaf_fill then takes them from there.
-// (Made in leaf order, they came from four gathers and went out scattered: 2M surfels 305 us, now 52 + 202.)
+// (Made in leaf order, they came from four gathers and went out scattered: 2M surfels 305 us, now 44 + 166.)
 __global__ void k_surfel_quads(const float *__restrict__ means, const float *__restrict__ scales, const float *__restrict__ rotations,
                                float *__restrict__ vertices_out, uint32_t n) {
-    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= n) return;
-    float c[4][3];
-    surfel_corners(means, scales, rotations, g, c);
-    float4 *dst = reinterpret_cast<float4 *>(vertices_out + 12 * (size_t)g);   // 48 bytes per surfel
-    dst[0] = make_float4(c[0][0], c[0][1], c[0][2], c[1][0]);
-    dst[1] = make_float4(c[1][1], c[1][2], c[2][0], c[2][1]);
-    dst[2] = make_float4(c[2][2], c[3][0], c[3][1], c[3][2]);
+    __shared__ alignas(16) float s_stage[kBlock * 12];
+    const uint32_t base = blockIdx.x * kBlock, g = base + threadIdx.x;
+    float c[4][3] = {}, row[12];
+    if (g < n) surfel_corners(means, scales, rotations, g, c);
+#pragma unroll
+    for (int k = 0; k < 12; ++k) row[k] = c[k / 3][k % 3];
+    block_store(s_stage, row, vertices_out + 12 * (size_t)base, min(n - base, (uint32_t)kBlock));
 }
 // Leaf records from the surfel parameters themselves, for callers that want no vertex buffer.
 __global__ void k_leaf_fill_from_surfels(const float *__restrict__ means, const float *__restrict__ scales,
                                          const float *__restrict__ rotations, const uint32_t *__restrict__ sorted_ids,
                                          DstLeaf *__restrict__ leaves, DstLeafPre *__restrict__ pre,
                                          DstBounds *__restrict__ bounds, RangeBoxes rb, uint32_t n) {
+    __shared__ alignas(16) float s_stage[kBlock * kStageWords];
     float mabs = 0.f;
-    // wave-uniform trip count: every lane stays for the wave-wide scans of the boxes
-    for (uint32_t base = blockIdx.x * blockDim.x + (threadIdx.x & ~(DST_WAVE - 1u)); base < n; base += gridDim.x * blockDim.x) {
-        const uint32_t i = base + (threadIdx.x & (DST_WAVE - 1u));
+    // a trip count for the whole block: every thread stays for the stores, and for the scans of the boxes
+    for (uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
+        const uint32_t i = base + threadIdx.x, rows = min(n - base, (uint32_t)kBlock);
         const bool valid = i < n;
-        float c[4][3] = {};
+        float c[4][3] = {}, leaf[24] = {}, stand_in[16] = {};
         if (valid) {
             const uint32_t g = sorted_ids[i];
             surfel_corners(means, scales, rotations, g, c);
@@ -958,10 +977,12 @@ __global__ void k_leaf_fill_from_surfels(const float *__restrict__ means, const 
             for (int k = 0; k < 4; ++k)
 #pragma unroll
                 for (int a = 0; a < 3; ++a) mabs = finite_max(mabs, fabsf(c[k][a]));
-            write_leaf(c, g, i, leaves, pre);
+            make_leaf(c, g, leaf, stand_in);
         }
+        block_store(s_stage, leaf, reinterpret_cast<float *>(leaves + base), rows);
+        block_store(s_stage, stand_in, reinterpret_cast<float *>(pre + base), rows);
         count_small_quads(valid && quad_is_small(c, __uint_as_float(bounds->scale)), bounds);
-        if (rb.lbox != nullptr) wave_range_boxes(c, valid, i, n, rb);
+        if (rb.lbox != nullptr) block_range_boxes(s_stage, c, valid, i, n, rb);
     }
     mabs = wave_max(mabs);
     if ((threadIdx.x & (DST_WAVE - 1)) == 0 && mabs > 0.f && mabs < INFINITY)
@@ -988,7 +1009,7 @@ __global__ __launch_bounds__(kFitBlock) void k_fit(DstNode *nodes, const uint32_
     float c[4][3];
     const uint32_t g = sorted_ids[i];
     load_corners(vertices, quad_ids[g], g, c);   // (the leaf records hold edge vectors, not the corners)
-    const float pad = kBoxPad * quad_magnitude(c);   // as in wave_range_boxes: the two fits give the same bits
+    const float pad = kBoxPad * quad_magnitude(c);   // as in block_range_boxes: the two fits give the same bits
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         box[a] = fminf(fminf(c[0][a], c[1][a]), fminf(c[2][a], c[3][a])) - pad;
