@@ -408,7 +408,7 @@ struct RayPre {
 __device__ __forceinline__ RayPre make_pre(F3 o, F3 d, float max_abs) {
     RayPre r;
     const float oa = __builtin_fmaxf(__builtin_fabsf(o.x), __builtin_fmaxf(__builtin_fabsf(o.y), __builtin_fabsf(o.z)));
-    const float S = oa;   // the ray's share; the quad's own coordinates are in its limits already (lbvh.hip, write_leaf)
+    const float S = oa;   // the ray's share; the quad's own coordinates are in its limits already (lbvh.hip, make_leaf)
     const float dl = __builtin_sqrtf(d.x * d.x + d.y * d.y + d.z * d.z);
     r.inv_dl = 1.0f / dl;
     r.padw = 1.5e-4f * S;
@@ -2414,91 +2414,112 @@ __global__ __launch_bounds__(kPrepareWaves *DST_WAVE) void k_prepare(const DstPa
 #include "row.inc"
 
 // Closing kernel of a backward trace: the per-surfel sums (gradient rows, or the deterministic mode's fixed point) to the
-// caller's tensors.  A workgroup takes kCloseSurfels surfels at a time through LDS: rows in as they lie, tensors out as
+// caller's tensors.  A workgroup takes kCloseSurfels surfels through LDS: rows in as they lie, tensors out as
 // they lie, 16 bytes a lane for the SH gradient.  Bound by memory.  With p.grad_touched it writes the tensors (a caller
 // has nothing to fill), reads the marked surfels' rows alone (a view meets a third of a room's surfels, a LiDAR frame a
 // tenth of its scene's) and clears what it read, so that the rows stay zero between calls; without, it adds to them.
 // (2M surfels, 4 auxiliary channels: rows filled 0.1 ms + tensors filled 0.1 ms + closing 0.24 ms before.)
-// (Surfels a workgroup takes at a time, 32 / 64 / 128: 2M surfels, 4 channels 205 / 182 / 202 us, 1M 97 / 84 / 93.)
+// (A workgroup for every 64 surfels, and all it reads asked for at once: one that goes on to the next 64 waits for its stores,
+// which memory counts with its loads.  8192 workgroups that go on / one for each:
+// 2M surfels, 4 channels 181 / 127 us, 1M, 2 channels 84 / 66, 500,000, 8 channels 101 / 64.)
 constexpr uint32_t kCloseSurfels = 64, kCloseThreads = 256;
 template <int AUXM, bool DET>
 __global__ __launch_bounds__(kCloseThreads) void k_close_gradients(const DstParams p, uint32_t *out_of_range) {
     constexpr uint32_t cols = RowLayout<AUXM>::cols, stride = cols | 1u;
+    static_assert(kCloseSurfels == DST_WAVE && kColAux == DST_WAVE, "a bit per surfel, a lane per column");
+    constexpr uint32_t kWaves = kCloseThreads / DST_WAVE, kMain = kCloseSurfels / kWaves, kAux = (kCloseSurfels * AUXM + kCloseThreads - 1u) / kCloseThreads;
     __shared__ float s_rows[kCloseSurfels * stride];
-    __shared__ uint8_t s_on[kCloseSurfels];
+    __shared__ uint64_t s_on;   // whose rows are read
     const bool writes = p.grad_touched != nullptr, aux_rows = p.others_precomp != nullptr;
     const uint32_t tid = threadIdx.x, P = (uint32_t)p.P;
-    for (uint32_t base = blockIdx.x * kCloseSurfels; base < P; base += gridDim.x * kCloseSurfels) {
-        const uint32_t n = min(kCloseSurfels, P - base);
-        bool on = false;
-        if (tid < n) {
-            on = !writes || p.grad_touched[base + tid] != 0u;
-            s_on[tid] = on ? 1u : 0u;
-            if (writes && on) p.grad_touched[base + tid] = 0u;
+    const uint32_t base = blockIdx.x * kCloseSurfels, n = min(kCloseSurfels, P - base);
+    if (tid < DST_WAVE) {
+        const bool on = tid < n && (!writes || p.grad_touched[base + tid] != 0u);
+        const uint64_t mask = wave_ballot(on);
+        if (writes && on) p.grad_touched[base + tid] = 0u;
+        if (tid == 0u) s_on = mask;
+    }
+    __syncthreads();
+    const uint64_t on = s_on;
+    const bool any = on != 0ull;
+    if (any) {
+        // a wave's rows, sixteen of 64 columns, and a thread's share of the auxiliary columns behind them: all asked for at once
+        typedef typename std::conditional<DET, long long, float>::type Sum;
+        Sum *const sums = DET ? (Sum *)p.det_workspace : (Sum *)p.grad_rows;
+        Sum *const from = sums + (size_t)base * kColAux, *const from_aux = sums + (size_t)P * kColAux + (size_t)base * AUXM;
+        const uint32_t wave = uni(tid / DST_WAVE), lane = tid % DST_WAVE;
+        Sum main[kMain], aux[kAux];
+        auto has = [&](uint32_t row) { return ((on >> row) & 1ull) != 0ull; };
+#pragma unroll
+        for (uint32_t j = 0; j < kMain; ++j) {
+            const uint32_t row = wave + kWaves * j;
+            main[j] = 0;
+            if (has(row)) main[j] = from[row * DST_WAVE + lane];
         }
-        const bool any = __syncthreads_or(on ? 1 : 0) != 0;
-        if (any) {
-            const uint32_t n_cols = aux_rows ? n * cols : n * (uint32_t)kColAux;   // (the auxiliary columns behind the others)
-            for (uint32_t k = tid; k < n_cols; k += kCloseThreads) {
-                const uint32_t rest = k - n * (uint32_t)kColAux;
-                const bool main = k < n * (uint32_t)kColAux;
-                const uint32_t row = main ? k / (uint32_t)kColAux : rest / AUXM, col = main ? k % (uint32_t)kColAux : kColAux + rest % AUXM;
-                float v = 0.f;
-                if (s_on[row] != 0u) {
-                    const size_t at = main ? (size_t)base * kColAux + k : (size_t)P * kColAux + (size_t)base * AUXM + rest;
-                    if (DET) {
-                        const long long q = (long long)p.det_workspace[at];
-                        if (q != 0) {
-                            if (det_out_of_range(q)) atomicAdd(out_of_range, 1u);
-                            v = from_fixed(q, det_shift((int)col));
-                            if (writes) p.det_workspace[at] = 0ull;
-                        }
-                    } else {
-                        v = p.grad_rows[at];
-                        if (writes && v != 0.f) p.grad_rows[at] = 0.f;
-                    }
-                }
-                s_rows[row * stride + col] = v;
-            }
-            __syncthreads();
+#pragma unroll
+        for (uint32_t j = 0; j < kAux; ++j) {
+            const uint32_t k = tid + j * kCloseThreads;
+            aux[j] = 0;
+            if (aux_rows && k < kCloseSurfels * AUXM && has(k / AUXM)) aux[j] = from_aux[k];
         }
-        auto put = [&](float *dst, float v) {
-            if (writes) *dst = v;
-            else if (v != 0.f) *dst += v;
-        };
-        // `width` columns from `col0` on of every surfel to the tensor `dst` (width, .)
-        auto emit = [&](float *dst, uint32_t width, uint32_t col0) {
-            if (dst == nullptr || (!any && !writes)) return;
-            for (uint32_t e = tid; e < n * width; e += kCloseThreads)
-                put(dst + (size_t)base * width + e, any ? s_rows[(e / width) * stride + col0 + e % width] : 0.f);
-        };
-        emit(p.dL_dcolors, 3u, kColColor);
-        emit(p.dL_dopacities, 1u, kColOpac);
-        emit(p.dL_dscales, 2u, kColScale);
-        emit(p.dL_drotations, 4u, kColRot);
-        emit(p.dL_dmeans3D, 3u, kColMean);
-        emit(p.dL_dgrads3D, 3u, kColGrad);
-        if (aux_rows) emit(p.dL_dothers, (uint32_t)p.aux, kColAux);
-        else if (writes && p.dL_dothers != nullptr)   // nothing was given: zeros
-            for (uint32_t e = tid; e < n * (uint32_t)p.aux; e += kCloseThreads) p.dL_dothers[(size_t)base * p.aux + e] = 0.f;
-        if (p.colors_precomp == nullptr && p.dL_dshs != nullptr && (any || writes)) {
-            const uint32_t width = 3u * (uint32_t)p.M;
-            float *const dst = p.dL_dshs + (size_t)base * width;
-            // element r of a surfel is coefficient r / 3, channel r % 3 (coefficients past the sixteenth have no gradient)
-            auto of = [&](uint32_t row, uint32_t r) { return any && r < 48u ? s_rows[row * stride + kColSh + 16u * (r % 3u) + r / 3u] : 0.f; };
-            if (writes && width == 48u && (reinterpret_cast<uintptr_t>(p.dL_dshs) & 15u) == 0u) {
-                for (uint32_t e = tid; e < n * 12u; e += kCloseThreads) {
-                    const uint32_t row = e / 12u, r = 4u * (e - row * 12u);
-                    reinterpret_cast<float4 *>(dst)[e] = make_float4(of(row, r), of(row, r + 1u), of(row, r + 2u), of(row, r + 3u));
-                }
+        // `sum` of column `col`; the row is left empty
+        auto take = [&](Sum sum, Sum *at, uint32_t col) {
+            if (sum == 0) return 0.f;
+            if (writes) *at = 0;
+            if constexpr (DET) {
+                if (det_out_of_range(sum)) atomicAdd(out_of_range, 1u);
+                return from_fixed(sum, det_shift((int)col));
             } else {
-                for (uint32_t e = tid; e < n * width; e += kCloseThreads) {
-                    const uint32_t row = e / width;
-                    put(dst + e, of(row, e - row * width));
-                }
+                return sum;
             }
+        };
+#pragma unroll
+        for (uint32_t j = 0; j < kMain; ++j) {
+            const uint32_t row = wave + kWaves * j;
+            s_rows[row * stride + lane] = take(main[j], from + row * DST_WAVE + lane, lane);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kAux; ++j) {
+            const uint32_t k = tid + j * kCloseThreads;
+            if (aux_rows && k < kCloseSurfels * AUXM) s_rows[(k / AUXM) * stride + kColAux + k % AUXM] = take(aux[j], from_aux + k, kColAux + k % AUXM);
         }
         __syncthreads();
+    }
+    auto put = [&](float *dst, float v) {
+        if (writes) *dst = v;
+        else if (v != 0.f) *dst += v;
+    };
+    // `width` columns from `col0` on of every surfel to the tensor `dst` (width, .)
+    auto emit = [&](float *dst, uint32_t width, uint32_t col0) {
+        if (dst == nullptr || (!any && !writes)) return;
+        for (uint32_t e = tid; e < n * width; e += kCloseThreads)
+            put(dst + (size_t)base * width + e, any ? s_rows[(e / width) * stride + col0 + e % width] : 0.f);
+    };
+    emit(p.dL_dcolors, 3u, kColColor);
+    emit(p.dL_dopacities, 1u, kColOpac);
+    emit(p.dL_dscales, 2u, kColScale);
+    emit(p.dL_drotations, 4u, kColRot);
+    emit(p.dL_dmeans3D, 3u, kColMean);
+    emit(p.dL_dgrads3D, 3u, kColGrad);
+    if (aux_rows) emit(p.dL_dothers, (uint32_t)p.aux, kColAux);
+    else if (writes && p.dL_dothers != nullptr)   // nothing was given: zeros
+        for (uint32_t e = tid; e < n * (uint32_t)p.aux; e += kCloseThreads) p.dL_dothers[(size_t)base * p.aux + e] = 0.f;
+    if (p.colors_precomp == nullptr && p.dL_dshs != nullptr && (any || writes)) {
+        const uint32_t width = 3u * (uint32_t)p.M;
+        float *const dst = p.dL_dshs + (size_t)base * width;
+        // element r of a surfel is coefficient r / 3, channel r % 3 (coefficients past the sixteenth have no gradient)
+        auto of = [&](uint32_t row, uint32_t r) { return any && r < 48u ? s_rows[row * stride + kColSh + 16u * (r % 3u) + r / 3u] : 0.f; };
+        if (writes && width == 48u && (reinterpret_cast<uintptr_t>(p.dL_dshs) & 15u) == 0u) {
+            for (uint32_t e = tid; e < n * 12u; e += kCloseThreads) {
+                const uint32_t row = e / 12u, r = 4u * (e - row * 12u);
+                reinterpret_cast<float4 *>(dst)[e] = make_float4(of(row, r), of(row, r + 1u), of(row, r + 2u), of(row, r + 3u));
+            }
+        } else {
+            for (uint32_t e = tid; e < n * width; e += kCloseThreads) {
+                const uint32_t row = e / width;
+                put(dst + e, of(row, e - row * width));
+            }
+        }
     }
 }
 __global__ void k_det_finish_weights(const DstParams p, uint32_t *out_of_range) {
@@ -2767,7 +2788,7 @@ const uint32_t *make_scratch(const dst_ctx *ctx, DstParams &p, const DstAccelVie
 void launch_close(const DstParams &p, uint32_t *out_of_range, hipStream_t stream) {
     const bool det = (p.flags & DST_FLAG_DETERMINISTIC) != 0u;
     if (!det && p.grad_rows == nullptr) return;   // the sums are in the caller's tensors already
-    const dim3 grid(std::min<uint32_t>(((uint32_t)p.P + kCloseSurfels - 1u) / kCloseSurfels, 8192u)), block(kCloseThreads);
+    const dim3 grid(((uint32_t)p.P + kCloseSurfels - 1u) / kCloseSurfels), block(kCloseThreads);
 #define DST_CLOSE(AUX)                                                                                              \
     do {                                                                                                            \
         if (det) hipLaunchKernelGGL((k_close_gradients<AUX, true>), grid, block, 0, stream, p, out_of_range);       \

@@ -126,6 +126,20 @@ def test_gradient_table_edges(oracle, P, aux, det):
     assert ref["n_con"].min() >= 0.9 * P   # (a ray in ten is outside some splat)
 
 
+@pytest.mark.parametrize("aux,det", [(0, False), (3, True), (8, False)])
+@pytest.mark.parametrize("P", [63, 64, 65, 129])
+def test_closing_edges(oracle, P, aux, det):
+    """Sizes around the 64 surfels that the closing kernel takes at a time, every other surfel met by no ray: the oracle's
+    gradients, and again from rows that the call before left empty."""
+    sc = {k: v.clone() for k, v in S.scene_cube(P=P, seed=P, aux=aux).items()}
+    sc["means3D"][1::2, 2] += 50.0
+    sc["vertices"], sc["faces"] = S.get_triangles(sc["means3D"], sc["scales"], sc["rotations"])
+    tracer = tile_tracer(deterministic=det)
+    for _ in range(2):
+        ref, _ = check_case(oracle, tracer, sc, *view("cube"))
+        assert np.abs(ref["grads_gpu"]["means3D"][0::2]).max() > 0.0 and not ref["grads_gpu"]["means3D"][1::2].any()
+
+
 @pytest.mark.parametrize("kind,fov", [("cube", 20.0), ("cube", 140.0), ("room", 70.0), ("lidar", 110.0)])
 @pytest.mark.parametrize("shrink,shift", [(1.0, 0.0), (1.0 / 30.0, 0.0), (20.0, 0.0), (1.0, 3e4)])
 def test_rays_of_one_origin(kind, fov, shrink, shift):
