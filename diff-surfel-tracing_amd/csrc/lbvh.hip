@@ -1307,6 +1307,7 @@ int ploc_hierarchy(dst_ctx *ctx, const float *vertices, uint32_t n, hipStream_t 
             left *= many ? 0.69 : 0.6;
         }
         hipLaunchKernelGGL(k_ploc_tail, dim3(1), dim3(kPlocBlock), 0, stream, pb, it);
+        if (n > kPlocBig) hipLaunchKernelGGL(k_ploc_big_nodes, grid_for(n - 1), dim3(kBlock), 0, stream, pb, n);
         hipLaunchKernelGGL(k_ploc_leaf_positions, grid_for(n), dim3(kBlock), 0, stream, pb, ctx->vals[0], ctx->vals[1], n);
         hipLaunchKernelGGL(k_ploc_node_numbers, grid_for(n), dim3(kBlock), 0, stream, pb, ctx->vals[0], ctx->vals[1], ctx->nodes, n);
         hipLaunchKernelGGL(k_ploc_links, grid_for(n - 1), dim3(kBlock), 0, stream, pb, ctx->nodes, ctx->node_parent, ctx->leaf_parent, n);

@@ -343,10 +343,10 @@ void check_rounds(const std::vector<float> &at, int rounds, const char *what) {
     check_rounds(c, rounds, what);
 }
 
-// The layout of 200 leaves over links of which one or two are not those of a hierarchy, though the counts at its root are: a
+// The layout of `n` leaves over links of which one or two are not those of a hierarchy, though the counts at its root are: a
 // build has to find out (state[4]), whatever the buffers held before.
-void check_broken_links() {
-    const uint32_t n = 200;
+void check_broken_links(uint32_t n) {
+    const dim3 grid((n + kBlock - 1) / kBlock);
     for (int kind = 0; kind < 4; ++kind) {   // none; a leaf in another's place; a node in another's; a leaf on its sibling's side
         PlocTest t(n);
         std::mt19937 rng(3);
@@ -373,9 +373,10 @@ void check_broken_links() {
         for (uint32_t i = 0; i < n; ++i) in[i] = (i * 77u) % n;
         for (uint32_t i = 0; i < n; ++i) out[i] = DST_LEAF_BIT | i;
         std::vector<DstNode> nodes(n - 1);
-        hipLaunchKernelGGL(k_ploc_leaf_positions, dim3(1), dim3(kBlock), 0, nullptr, t.pb, in.data(), out.data(), n);
-        hipLaunchKernelGGL(k_ploc_node_numbers, dim3(1), dim3(kBlock), 0, nullptr, t.pb, in.data(), out.data(), nodes.data(), n);
-        hipLaunchKernelGGL(k_ploc_links, dim3(1), dim3(kBlock), 0, nullptr, t.pb, nodes.data(), node_parent.data(), leaf_parent.data(), n);
+        hipLaunchKernelGGL(k_ploc_big_nodes, grid, dim3(kBlock), 0, nullptr, t.pb, n);
+        hipLaunchKernelGGL(k_ploc_leaf_positions, grid, dim3(kBlock), 0, nullptr, t.pb, in.data(), out.data(), n);
+        hipLaunchKernelGGL(k_ploc_node_numbers, grid, dim3(kBlock), 0, nullptr, t.pb, in.data(), out.data(), nodes.data(), n);
+        hipLaunchKernelGGL(k_ploc_links, grid, dim3(kBlock), 0, nullptr, t.pb, nodes.data(), node_parent.data(), leaf_parent.data(), n);
         CHECK(t.state[0] == 1u && t.state[3] == n, "broken links %d: one cluster of %u", kind, n);
         CHECK((t.state[4] != 0u) == (kind != 0), "broken links %d: %u", kind, t.state[4]);
     }
@@ -480,9 +481,11 @@ int main(int argc, char **argv) {
         return failures ? 1 : 0;
     }
     check_windows();
-    check_broken_links();
+    check_broken_links(200);
+    check_broken_links(900);   // with big nodes
     const bool quick = argc > 1 && std::string(argv[1]) == "quick";
     const uint32_t sizes[] = {1, 2, 3, 63, 64, 65, 100, 1024, 1025, 2500, 5000};
+    for (uint32_t P : {kPlocBig, kPlocBig + 1, kPlocBig + 2}) run_case(P, 0, true, 11 + P);   // the root the one big node
     for (int agg = 1; agg >= 0; --agg) {
         for (uint32_t P : sizes) {
             if (quick && P > 2500) continue;
