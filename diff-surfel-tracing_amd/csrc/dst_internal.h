@@ -215,7 +215,7 @@ int dst_lbvh_build(dst_ctx *ctx, const float *vertices, uint32_t n_vertices, con
 int dst_static_scratch_init(dst_ctx *ctx);
 uint32_t *dst_static_scratch(const dst_ctx *ctx);
 void dst_lbvh_free(dst_ctx *ctx);
-void dst_sort_pairs(uint32_t *keys[2], uint32_t *vals[2], uint32_t *tile_hist, uint32_t n, hipStream_t stream);
+void dst_sort_pairs(uint32_t *keys[2], uint32_t *vals[2], uint32_t *tile_hist, uint32_t n, hipStream_t stream, int bits = 32);
 size_t dst_sort_hist_elems(uint32_t n);
 // trace.hip
 int dst_launch_trace(dst_ctx *ctx, const DstParams &p, bool backward, hipStream_t stream);

@@ -2018,10 +2018,19 @@ __global__ __launch_bounds__(1024) void k_cost_order(const uint32_t *__restrict_
 // made, word 3 = not the list's: sums of the deterministic mode found out of range (its closing kernels count there),
 // entries ((by * btiles_x + bx) * 4 + wave) from word 4.  A wave that finds the list full starts again without a limit.
 constexpr uint32_t kHandHeader = kDstHandoverHeader, kHandCap = kDstHandoverCap;
+// Ray lists that are traced in an order of their own: by tiles (contexts that hand tiles over, the re-tracing backward) from
+// kOrderMinRays on, by rows from kOrderMinByRows on.  Sixteen lanes share a ray in rows and a wave has four rays, so unrelated
+// ones cost little, and the sort (110 us of thirteen launches with 32 bits a key, half of that with 16) gains that much only
+// where a long list's rays go apart.  In the rays' order / sorted by 16 / by 32 bits, us a call: unrelated rays in a room of
+// 300,000 surfels, 5,000 110 / 158 / 206, 19,000 113 / 175 / 211, 131,072 400 / 418 / 489, 262,144 707 / 710, 400,000 1049 / 973 /
+// 1092; of a million surfels, 262,144 2020 / 1961; lidar frames of 131,072 rays 108 / 182 / 223 (200,000 surfels), 315 / 378 /
+// 434 (two million), with the step's backward 925 / 979 / 1053.
+constexpr uint32_t kOrderMinRays = 2048, kOrderMinByRows = 262144;
+
 template <bool BWD, int AUXM, bool REC, bool MIXED, bool DET, bool HAND, bool PACK>
 __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelView &acc, int tw_log2, int th_log2,
                                            uint32_t tiles_x, uint32_t tiles_y, uint32_t btiles_x,
-                                           const uint32_t *__restrict__ ray_order, uint32_t strip_width,
+                                           const uint32_t *ray_order, uint32_t strip_width,
                                            const uint32_t *__restrict__ block_order, uint32_t *handover,
                                            uint32_t hand_arg) {
     // a block = 2x2 wave tiles (16x16 pixels for the usual 8x8 tile): neighbouring rays share surfels, which
@@ -2053,6 +2062,7 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
     if (BWD && p.hit_record != nullptr) {
         const bool complete = p.hit_record[0] <= (uint64_t)p.hit_record_blocks;
         if (REC != complete || (REC && (uint32_t)p.hit_record[2] != 0u)) return;
+        if (!REC && (uint32_t)p.hit_record[2] != 0u && (uint32_t)p.W < kOrderMinByRows) ray_order = nullptr;   // (rows left none)
     }
     if (BWD) {
         table_clear_keys<AUXM, DET>(s_keys);
@@ -2532,9 +2542,10 @@ __global__ void k_det_finish_weights(const DstParams p, uint32_t *out_of_range) 
 
 // Sort key of a ray of a ray list, so that the 64 rays of a wave run side by side: the cell of the origin on a
 // 32^3 grid over the scene (15 bits), then the direction as a Morton code of its octahedral map (2 x 8 bits).
+// `by_rows`: sixteen bits, half the sort: an 8^3 grid and the seven highest of the direction's.
 // Rays that cannot be keyed (NaN, zero direction) get key 0.
 __global__ void k_ray_keys(const float *__restrict__ ray_o, const float *__restrict__ ray_d, const DstBounds *bounds,
-                           uint32_t *__restrict__ keys, uint32_t *__restrict__ vals, uint32_t n) {
+                           uint32_t *__restrict__ keys, uint32_t *__restrict__ vals, uint32_t n, int by_rows) {
     const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= n) return;
     const float ext = __uint_as_float(bounds->scale);
@@ -2565,7 +2576,8 @@ __global__ void k_ray_keys(const float *__restrict__ ray_o, const float *__restr
         };
         dir = (spread8(qu) << 1) | spread8(qv);
     }
-    keys[r] = (cell << 16) | dir;
+    const uint32_t coarse = ((cell >> 6) & 0x1C0u) | ((cell >> 4) & 0x38u) | ((cell >> 2) & 7u);   // three bits of each axis' five
+    keys[r] = by_rows ? (coarse << 7) | (dir >> 9) : (cell << 16) | dir;
     vals[r] = r;
 }
 
@@ -2580,9 +2592,8 @@ struct TileGrid {
 };
 
 // 8x8 pixel tiles per wave, 2x2 tiles per block.  A thin grid (H < 8: a (B,N,3) ray list) is one flat list of
-// H*W rays in tiles of 1x64, traced in a coherent order of its own (k_ray_keys).
+// H*W rays in tiles of 1x64, traced in a coherent order of its own where that pays (k_ray_keys).
 constexpr int kThinRows = 8;
-constexpr uint32_t kOrderMinRays = 2048;   // shorter lists are traced as they come
 TileGrid tile_grid(int H, int W) {
     TileGrid t;
     if (H < kThinRows) {
@@ -2841,10 +2852,23 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
         return DST_OK;
     }
     DstParams p = p_in;
-    const uint32_t *ray_order = nullptr;
+    if (!backward) {
+        // Refits count the small quads too, on the device; the count comes over behind the first forward trace after
+        // a refit (a 4-byte copy on this stream, nobody waits for it) and serves the traces after that one.
+        if (ctx->bounds_host != nullptr && ctx->bounds != nullptr) {
+            if (ctx->small_quads_asked) ctx->small_quads = *(volatile const uint32_t *)&ctx->bounds_host->small_quads;
+            if (ctx->small_quads_refits != ctx->refits) {
+                DST_HIP(ctx, hipMemcpyAsync(&ctx->bounds_host->small_quads, &ctx->bounds->small_quads, sizeof(uint32_t),
+                                            hipMemcpyDeviceToHost, stream));
+                ctx->small_quads_refits = ctx->refits;
+                ctx->small_quads_asked = true;
+            }
+        }
+    }
+    const uint32_t *ray_order = nullptr, *row_order = nullptr;   // row_order: of a list traced by rows
     if (p.H < kThinRows) {
-        // a ray list: flat, and (when it is long enough to matter) in an order that puts similar rays in one wave.
-        // Forward and backward derive the same order from the same rays, or the backward trace takes it from the record.
+        // a ray list: flat, and (when it is long enough to matter: kOrderMinByRows) in an order that puts similar rays in one
+        // wave.  The backward trace takes it from the record, and without a record makes its own.
         if ((uint64_t)p.H * p.W > 0x7FFFFFFFull) return dst_fail(ctx, DST_E_INVALID, "ray grid too large");
         p.W = p.H * p.W;
         p.H = 1;
@@ -2854,9 +2878,11 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
             const TileGrid t = tile_grid(1, p.W);
             kept = reinterpret_cast<uint32_t *>(p.hit_record + record_order_at(n, t.th_log2, (uint32_t)p.mtd_alloc + 1u, (uint64_t)t.btiles_x * t.btiles_y * kWavesPerBlock));
         }
+        const bool by_rows = backward ? kept != nullptr : !(kFwdWavesPerBlock == 1 && dst_handover_active(ctx));
         if (n >= kOrderMinRays && backward && kept != nullptr) {
-            ray_order = kept;
-        } else if (n >= kOrderMinRays) {
+            ray_order = kept;   // (what the forward trace left there; nobody looks where it left nothing)
+            if (n >= kOrderMinByRows) row_order = kept;
+        } else if (n >= (by_rows ? kOrderMinByRows : kOrderMinRays)) {
             if (n > ctx->ray_capacity) {
                 for (int k = 0; k < 2; ++k) {
                     if (ctx->ray_keys[k]) (void)hipFree(ctx->ray_keys[k]);
@@ -2875,9 +2901,9 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
             }
             uint32_t *vals[2] = {kept != nullptr ? kept : ctx->ray_vals[0], ctx->ray_vals[1]};
             hipLaunchKernelGGL(k_ray_keys, dim3((n + 255u) / 256u), dim3(256), 0, stream, p.ray_o, p.ray_d, ctx->bounds,
-                               ctx->ray_keys[0], vals[0], n);
-            dst_sort_pairs(ctx->ray_keys, vals, ctx->ray_hist, n, stream);
-            ray_order = vals[0];
+                               ctx->ray_keys[0], vals[0], n, by_rows ? 1 : 0);
+            dst_sort_pairs(ctx->ray_keys, vals, ctx->ray_hist, n, stream, by_rows ? 16 : 32);
+            ray_order = row_order = vals[0];
         }
     }
     const TileGrid t = tile_grid(p.H, p.W);
@@ -2897,7 +2923,7 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
     if (backward) {
         const uint32_t n_blocks = t.btiles_x * t.btiles_y;
         // the kernel that fits the record (complete, written ray by ray or wave by wave; incomplete) does the work
-        if (rec && by == TraceBy::Rows) launch_row_bwd(p, rows, ray_order, stream);
+        if (rec && by == TraceBy::Rows) launch_row_bwd(p, rows, row_order, stream);
         if (rec && n_blocks < kOrderMinBlocks) {
             launch<true, true>(p, acc, t, ray_order, stream);
         } else if (rec) {
@@ -2918,17 +2944,6 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
         launch<true, false>(p, acc, t, ray_order, stream);           // else this one does (it returns at once otherwise)
         launch_close(p, out_of_range, stream);
     } else {
-        // Refits count the small quads too, on the device; the count comes over behind the first forward trace after
-        // a refit (a 4-byte copy on this stream, nobody waits for it) and serves the traces after that one.
-        if (ctx->bounds_host != nullptr && ctx->bounds != nullptr) {
-            if (ctx->small_quads_asked) ctx->small_quads = *(volatile const uint32_t *)&ctx->bounds_host->small_quads;
-            if (ctx->small_quads_refits != ctx->refits) {
-                DST_HIP(ctx, hipMemcpyAsync(&ctx->bounds_host->small_quads, &ctx->bounds->small_quads, sizeof(uint32_t),
-                                            hipMemcpyDeviceToHost, stream));
-                ctx->small_quads_refits = ctx->refits;
-                ctx->small_quads_asked = true;
-            }
-        }
         const uint32_t steps = std::max<uint32_t>(ctx->handover_steps, 1u);
         // the second launch of each pair traces the tiles the first one handed over (usually none: it leaves at once)
         uint32_t *const list = (kFwdWavesPerBlock == 1 && dst_handover_active(ctx)) ? ctx->handover : nullptr;
@@ -2938,8 +2953,8 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
         // takes 29.9 ms with OFF, 2.8 with the hand-over and 0.24 by rows, a list of 20,000 rays there 813 and 290 us, a
         // 637x1013 room with one reflection 5.5 ms against 3.5.
         if (by == TraceBy::Rows && list == nullptr && (ctx->handover_mode != DST_HANDOVER_OFF || p.max_trace_depth > 0 || t.th_log2 < 3)) {
-            if (rec) launch_row_fwd<true, RowRays>(p, acc, rows, ray_order, stream);
-            else launch_row_fwd<false, RowRays>(p, acc, rows, ray_order, stream);
+            if (rec) launch_row_fwd<true, RowRays>(p, acc, rows, row_order, stream);
+            else launch_row_fwd<false, RowRays>(p, acc, rows, row_order, stream);
         } else if (by != TraceBy::Rows && list == nullptr && ctx->handover_mode != DST_HANDOVER_OFF &&
                    (uint64_t)p.H * p.W <= (rec ? kRowRecordedRays : kRowEvaluatedRays)) {
             if (rec) launch_row_fwd<true, RowTiles>(p, acc, rows, ray_order, stream);

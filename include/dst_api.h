@@ -102,9 +102,9 @@ typedef struct DstParams {
      * again instead (the host need not look at the record between the two calls; it may read word 0 later to
      * size the next record; at most 2^26 - 1 blocks of a record are used).  Word 1 counts chains a replay found
      * broken: it stays 0 unless the buffer was not written by a forward trace with the same grid, depth and a zeroed
-     * header.  The record of a ray list (fewer than eight rows) of 2048 rays and more also carries the order in which the
-     * rays were traced, and the backward trace takes it from there, also where the record is incomplete: it may only be
-     * given a record that a forward trace of the same grid and depth has been given before. */
+     * header.  The record of a ray list (fewer than eight rows) of 2048 rays and more also has room for an order of the
+     * rays; where the forward trace made one, the backward trace takes it from there, also where the record is
+     * incomplete: it may only be given a record that a forward trace of the same grid and depth has been given before. */
     uint64_t *hit_record;
     uint32_t hit_record_blocks;
     uint32_t flags;               /* DST_FLAG_* */
