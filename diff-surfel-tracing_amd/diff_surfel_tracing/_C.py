@@ -510,32 +510,31 @@ def _common_params(ray_o, ray_d, vertices, background, means3D, shs, degree, col
                    start_from_first):
     if means3D.dim() != 2 or means3D.size(1) != 3:
         raise RuntimeError("means3D must have dimensions (num_points, 3)")
-    t = {
-        "ray_o": _cuda_f32(ray_o, "ray_o"), "ray_d": _cuda_f32(ray_d, "ray_d"),
-        "vertices": _cuda_f32(vertices, "vertices"), "background": _cuda_f32(background, "background"),
-        "means3D": _cuda_f32(means3D, "means3D"), "shs": _cuda_f32(shs, "shs"),
-        "colors_precomp": _cuda_f32(colors_precomp, "colors_precomp"),
-        "others_precomp": _cuda_f32(others_precomp, "others_precomp"),
-        "opacities": _cuda_f32(opacities, "opacities"), "scales": _cuda_f32(scales, "scales"),
-        "rotations": _cuda_f32(rotations, "rotations"),
-    }
+    # (one look at each of eleven tensors, and their addresses with it)
+    p, t, f32, Tensor = DstParams(), {}, torch.float32, torch.Tensor
+    for name, x in (("ray_o", ray_o), ("ray_d", ray_d), ("vertices", vertices), ("background", background),
+                    ("means3D", means3D), ("shs", shs), ("colors_precomp", colors_precomp),
+                    ("others_precomp", others_precomp), ("opacities", opacities), ("scales", scales),
+                    ("rotations", rotations)):
+        if not (isinstance(x, Tensor) and x.is_cuda and x.dtype is f32 and x.is_contiguous()):
+            x = _cuda_f32(x, name)
+        t[name] = x
+        if x.numel() != 0:
+            setattr(p, name, x.data_ptr())
     if t["ray_o"].dim() != 3 or t["ray_o"].size(2) != 3 or t["ray_d"].shape != t["ray_o"].shape:
         raise RuntimeError("ray_o and ray_d must have the same dimensions (H, W, 3) or (B, P, 3)")
     if t["scales"].numel() == 0 or t["rotations"].numel() == 0:
         raise RuntimeError("scales and rotations are required (a precomputed 3D covariance is not consumed by "
                            "the tracer)")
-    p = DstParams()
     p.P, p.H, p.W = means3D.size(0), t["ray_o"].size(0), t["ray_o"].size(1)
     p.D = int(degree)
-    p.M = t["shs"].size(1) if t["shs"].numel() != 0 else 0
-    p.aux = t["others_precomp"].size(1) if t["others_precomp"].numel() != 0 else DEFAULT_AUX_CHANNELS
+    p.M = t["shs"].size(1) if p.shs else 0
+    p.aux = t["others_precomp"].size(1) if p.others_precomp else DEFAULT_AUX_CHANNELS
     p.max_trace_depth = int(max_trace_depth)
     p.mtd_alloc = max(DEFAULT_MAX_TRACE_DEPTH, p.max_trace_depth)
     p.start_from_first = int(bool(start_from_first))
     p.specular_threshold = float(specular_threshold)
     p.scale_modifier = float(scale_modifier)
-    for name, ten in t.items():
-        setattr(p, name, _ptr(ten))
     return p, t
 
 
@@ -599,7 +598,7 @@ def trace_surfels(ctx, training, start_from_first, ray_o, ray_d, vertices, backg
     if getattr(ctx, "distortion", False):
         p.flags |= FLAG_DISTORTION
     _use_sh_half(ctx, p, keep)
-    if p.flags == 0:   # (the kernels with the rare options have no use for it)
+    if p.flags == 0 and _scratch_bytes.get((P, H, W)) != 0:   # (the kernels with the rare options have no use for it)
         _scratch(p, keep)
     if events is not None:
         events[0].record()
