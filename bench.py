@@ -92,10 +92,11 @@ def kernels_of(H, W, aux, depth, handover):
     if handover:
         return "k_trace_fwd<%d,true,%s,false>" % (a, mixed), "k_trace_bwd<%d,true,false,false> + k_close_gradients<%d,false>" % (a, a), retrace
     if lists or (H * W + 63) // 64 <= 400:
-        return "k_row_fwd<%d,true,false,0>" % a, "k_row_bwd<%d,false> + k_close_gradients<%d,false>" % (a, a), retrace
-    fwd = "k_trace_fwd_plain<%d,true>" % a + (" + k_row_fwd<%d,true,false,1>" % a if depth > 0 else "")
+        return "k_row_fwd<%d,true,false,0,false>" % a, "k_row_bwd<%d,false> + k_close_gradients<%d,false>" % (a, a), retrace
+    # (the last argument: hits evaluated from records of the surfels, as on all workloads of this size here)
+    fwd = "k_trace_fwd_plain<%d,true,%s>" % (a, "true" if a < 8 else "false") + (" + k_row_fwd<%d,true,false,1,true>" % a if depth > 0 else "")
     if H * W <= 65536:
-        fwd = "k_row_fwd<%d,true,false,2>" % a
+        fwd = "k_row_fwd<%d,true,false,2,false>" % a
     return fwd, "k_trace_bwd<%d,true,false,false> + k_close_gradients<%d,false>" % (a, a), retrace
 
 
