@@ -1347,14 +1347,13 @@ uint32_t *dst_static_scratch(const dst_ctx *ctx) {
     return (ctx->device >= 0 && ctx->device < kMaxDevices) ? g_refit_scratch_ptr[ctx->device] : nullptr;
 }
 
-// Stable LSD radix sort of (key, value) pairs by the lowest `bits` (16 or 32) bits of the keys, eight a pass; the sorted pairs
-// end in buffer 0.
+// Stable LSD radix sort of (key, value) pairs, 32-bit keys, four 8-bit passes; the sorted pairs end in buffer 0.
 // tile_hist holds 256 counters per 1024 keys and 256 more for the digits' totals (dst_sort_hist_elems).  Used by the BVH build (Morton codes) and by the ray ordering.
-void dst_sort_pairs(uint32_t *keys[2], uint32_t *vals[2], uint32_t *tile_hist, uint32_t n, hipStream_t stream, int bits) {
+void dst_sort_pairs(uint32_t *keys[2], uint32_t *vals[2], uint32_t *tile_hist, uint32_t n, hipStream_t stream) {
     const uint32_t tiles = (n + kTile - 1) / kTile;
     const uint32_t tile_blocks = (tiles + (kBlock / DST_WAVE) - 1) / (kBlock / DST_WAVE);
     int src = 0;
-    for (int shift = 0; shift < bits; shift += kRadixBits) {
+    for (int shift = 0; shift < 32; shift += kRadixBits) {
         hipLaunchKernelGGL(k_radix_hist, dim3(tile_blocks), dim3(kBlock), 0, stream, keys[src], tile_hist, n, tiles, shift);
         uint32_t *row_total = tile_hist + (size_t)tiles * kRadix;   // kRadix words behind the tile counters
         hipLaunchKernelGGL(k_scan_rows, dim3(kRadix), dim3(1024), 0, stream, tile_hist, row_total, tiles);

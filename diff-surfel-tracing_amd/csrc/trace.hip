@@ -2018,14 +2018,13 @@ __global__ __launch_bounds__(1024) void k_cost_order(const uint32_t *__restrict_
 // made, word 3 = not the list's: sums of the deterministic mode found out of range (its closing kernels count there),
 // entries ((by * btiles_x + bx) * 4 + wave) from word 4.  A wave that finds the list full starts again without a limit.
 constexpr uint32_t kHandHeader = kDstHandoverHeader, kHandCap = kDstHandoverCap;
-// Ray lists that are traced in an order of their own: by tiles (contexts that hand tiles over, the re-tracing backward) from
-// kOrderMinRays on, by rows from kOrderMinByRows on.  Sixteen lanes share a ray in rows and a wave has four rays, so unrelated
-// ones cost little, and the sort (110 us of thirteen launches with 32 bits a key, half of that with 16) gains that much only
-// where a long list's rays go apart.  In the rays' order / sorted by 16 / by 32 bits, us a call: unrelated rays in a room of
-// 300,000 surfels, 5,000 110 / 158 / 206, 19,000 113 / 175 / 211, 131,072 400 / 418 / 489, 262,144 707 / 710, 400,000 1049 / 973 /
-// 1092; of a million surfels, 262,144 2020 / 1961; lidar frames of 131,072 rays 108 / 182 / 223 (200,000 surfels), 315 / 378 /
-// 434 (two million), with the step's backward 925 / 979 / 1053.
-constexpr uint32_t kOrderMinRays = 2048, kOrderMinByRows = 262144;
+// Ray lists that are traced in an order of their own: by tiles (contexts that hand tiles over, the backward trace without a
+// record) from kOrderMinRays on, by rows from kOrderMinByRows on, where it pays (k_list_look, which has the figures).  A record
+// that turned out too small is traced again by tiles: in the rows' order from kOrderManyRays on.  (In the rays' order / in the
+// rows', us a training step: pixels of one camera, shuffled, 65,536 6381 / 6511 in a room of a million, 5188 / 6276 at a
+// sphere of 100,000, 131,072 8636 / 8016 and 6305 / 6427, 262,144 16,472 / 13,022 and 12,479 / 8731; unrelated rays, 131,072
+// 2282 / 2614 in a room of 300,000, 262,144 13,531 / 12,925 in one of a million.)
+constexpr uint32_t kOrderMinRays = 2048, kOrderMinByRows = 65536, kOrderManyRays = 262144;
 
 template <bool BWD, int AUXM, bool REC, bool MIXED, bool DET, bool HAND, bool PACK>
 __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelView &acc, int tw_log2, int th_log2,
@@ -2062,7 +2061,7 @@ __device__ __forceinline__ void trace_body(const DstParams &p, const DstAccelVie
     if (BWD && p.hit_record != nullptr) {
         const bool complete = p.hit_record[0] <= (uint64_t)p.hit_record_blocks;
         if (REC != complete || (REC && (uint32_t)p.hit_record[2] != 0u)) return;
-        if (!REC && (uint32_t)p.hit_record[2] != 0u && (uint32_t)p.W < kOrderMinByRows) ray_order = nullptr;   // (rows left none)
+        if (!REC && (uint32_t)p.hit_record[2] != 0u && (uint32_t)p.W < kOrderManyRays) ray_order = nullptr;   // (written by rows)
     }
     if (BWD) {
         table_clear_keys<AUXM, DET>(s_keys);
@@ -2540,45 +2539,160 @@ __global__ void k_det_finish_weights(const DstParams p, uint32_t *out_of_range) 
     }
 }
 
+// Direction of a ray as a Morton code of its octahedral map (2 x 8 bits); 0 for one that has none (NaN, zero).
+__device__ __forceinline__ uint32_t direction_code(const float *d) {
+    const float l1 = fabsf(d[0]) + fabsf(d[1]) + fabsf(d[2]);
+    if (!(l1 > 0.f && l1 < INFINITY)) return 0u;
+    float u = d[0] / l1, v = d[1] / l1;
+    if (d[2] < 0.f) {   // fold the lower hemisphere over the square's corners
+        const float fu = (1.f - fabsf(v)) * (u >= 0.f ? 1.f : -1.f), fv = (1.f - fabsf(u)) * (v >= 0.f ? 1.f : -1.f);
+        u = fu;
+        v = fv;
+    }
+    uint32_t qu = (uint32_t)fminf(fmaxf((u * 0.5f + 0.5f) * 256.f, 0.f), 255.f);
+    uint32_t qv = (uint32_t)fminf(fmaxf((v * 0.5f + 0.5f) * 256.f, 0.f), 255.f);
+    auto spread8 = [](uint32_t x) {
+        x = (x | (x << 4)) & 0x0F0Fu;
+        x = (x | (x << 2)) & 0x3333u;
+        x = (x | (x << 1)) & 0x5555u;
+        return x;
+    };
+    return (spread8(qu) << 1) | spread8(qv);
+}
+// Cell of an origin on a grid of 2^(3 LOG2) cells over the scene; outside (and NaN): the nearest one.
+template <int LOG2>
+__device__ __forceinline__ uint32_t origin_cell(const float *o, const DstBounds *bounds) {
+    const float ext = __uint_as_float(bounds->scale), half = 0.5f * (float)(1 << LOG2);
+    const float inv = ext > 0.f ? half / ext : 0.f;
+    uint32_t cell = 0u;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) cell = (cell << LOG2) | (uint32_t)fminf(fmaxf(o[a] * inv + half, 0.f), 2.f * half - 1.f);   // NaN -> 0
+    return cell;
+}
+
 // Sort key of a ray of a ray list, so that the 64 rays of a wave run side by side: the cell of the origin on a
-// 32^3 grid over the scene (15 bits), then the direction as a Morton code of its octahedral map (2 x 8 bits).
-// `by_rows`: sixteen bits, half the sort: an 8^3 grid and the seven highest of the direction's.
-// Rays that cannot be keyed (NaN, zero direction) get key 0.
+// 32^3 grid over the scene (15 bits), then the direction's code.
 __global__ void k_ray_keys(const float *__restrict__ ray_o, const float *__restrict__ ray_d, const DstBounds *bounds,
-                           uint32_t *__restrict__ keys, uint32_t *__restrict__ vals, uint32_t n, int by_rows) {
+                           uint32_t *__restrict__ keys, uint32_t *__restrict__ vals, uint32_t n) {
     const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= n) return;
-    const float ext = __uint_as_float(bounds->scale);
-    const float inv = ext > 0.f ? 16.0f / ext : 0.f;
-    uint32_t cell = 0u, dir = 0u;
-    float d[3], l1 = 0.f;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        const float c = fminf(fmaxf(ray_o[3 * (size_t)r + a] * inv + 16.0f, 0.f), 31.f);   // NaN -> 0
-        cell = (cell << 5) | (uint32_t)c;
-        d[a] = ray_d[3 * (size_t)r + a];
-        l1 += fabsf(d[a]);
-    }
-    if (l1 > 0.f && l1 < INFINITY) {
-        float u = d[0] / l1, v = d[1] / l1;
-        if (d[2] < 0.f) {   // fold the lower hemisphere over the square's corners
-            const float fu = (1.f - fabsf(v)) * (u >= 0.f ? 1.f : -1.f), fv = (1.f - fabsf(u)) * (v >= 0.f ? 1.f : -1.f);
-            u = fu;
-            v = fv;
-        }
-        uint32_t qu = (uint32_t)fminf(fmaxf((u * 0.5f + 0.5f) * 256.f, 0.f), 255.f);
-        uint32_t qv = (uint32_t)fminf(fmaxf((v * 0.5f + 0.5f) * 256.f, 0.f), 255.f);
-        auto spread8 = [](uint32_t x) {
-            x = (x | (x << 4)) & 0x0F0Fu;
-            x = (x | (x << 2)) & 0x3333u;
-            x = (x | (x << 1)) & 0x5555u;
-            return x;
-        };
-        dir = (spread8(qu) << 1) | spread8(qv);
-    }
-    const uint32_t coarse = ((cell >> 6) & 0x1C0u) | ((cell >> 4) & 0x38u) | ((cell >> 2) & 7u);   // three bits of each axis' five
-    keys[r] = by_rows ? (coarse << 7) | (dir >> 9) : (cell << 16) | dir;
+    keys[r] = (origin_cell<5>(ray_o + 3 * (size_t)r, bounds) << 16) | direction_code(ray_d + 3 * (size_t)r);
     vals[r] = r;
+}
+
+// Order of a list traced by rows, in the call's scratch memory and in three launches: is the list in order as it comes
+// (k_list_look), how many rays have each key (k_list_count, whose last workgroup makes of these where the keys' rays begin), the
+// order (k_list_place).  The keys' sixteen bits go to what tells the rays apart: as many as it takes to tell the cells of
+// an 8^3 grid that origins lie in, the rest to the direction.  A camera's rays have all sixteen for it.  Rays of one key
+// follow in no order.  A list that comes in order (neighbours with nearly the same ray: a sensor's frame, rows of an image) keeps it,
+// and rays from more than kListPlaces cells are unrelated and gain only by the number: from kOrderManyRays on.
+// Bound by latency: 8 us to look, 28 to count 131,072 rays, 5 to place them; 17 in all for a list that keeps its order.
+// As the rays come / like this, us evaluated and us a training step:
+//   pixels of one camera, shuffled: room of a million surfels, 32,768 835 / 709 and 1454 / 1180, 65,536 1315 / 1084 and 2421 /
+//   1755, 131,072 2293 / 1862 and 4350 / 3028; of 300,000, 32,768 179 / 218 and 430 / 430, 131,072 482 / 558 and 1116 / 1022;
+//   sphere of 100,000, 65,536 616 / 417 and 1167 / 900, 131,072 1005 / 662 and 1963 / 1469
+//   of 32 cameras, shuffled: room of a million, 65,536 876 / 740 and 1646 / 1426, 131,072 1531 / 1177 and 2772 / 2281
+//   unrelated rays, sorted all the same: room of a million, 131,072 1261 / 1286 and 2392 / 2390, 262,144 2254 / 2160 and 4252 / 4086
+//   a sensor's frame in order, sorted all the same: 131,072 of two million surfels 148 / 266 and 567 / 677; kept 167 and 587
+// (A list of fewer than 65,536 rays loses by it in as many scenes as it gains.)
+constexpr uint32_t kListKeys = 65536u, kListCells = 512u, kListLooks = kListCells, kListThreads = 1024u, kListPlaces = 128u;
+struct ListHead {
+    uint32_t sorts;                // 0: as the rays come
+    uint32_t direction_bits;
+    uint32_t finished;             // workgroups that have counted their rays
+    uint32_t pad[29];
+    uint32_t place[kListCells];    // of a cell: its number among those where rays begin
+    uint32_t start[kListKeys];     // rays of a key, then the place of its first
+};
+__global__ __launch_bounds__(kListLooks) void k_list_look(const float *__restrict__ ray_o, const float *__restrict__ ray_d, const DstBounds *bounds,
+                                                            ListHead *__restrict__ head, uint32_t n) {
+    if (blockIdx.x != 0u) {
+        head->start[(blockIdx.x - 1u) * kListLooks + threadIdx.x] = 0u;
+        return;
+    }
+    // places all over the list, and at each a ray and the next one
+    __shared__ uint32_t s_cells[kListCells / 32u];
+    const uint32_t tid = threadIdx.x, at = (uint32_t)((uint64_t)tid * (n - 1u) / kListLooks);
+    if (tid < kListCells / 32u) s_cells[tid] = 0u;
+    __syncthreads();
+    const float *o = ray_o + 3 * (size_t)at, *d = ray_d + 3 * (size_t)at;   // (the next ray's lie behind them)
+    const uint32_t cell = origin_cell<3>(o, bounds);
+    atomicOr(&s_cells[cell / 32u], 1u << (cell % 32u));
+    const F3 d0 = ld3(d), d1 = ld3(d + 3), c = cross(d0, d1);
+    const float off = fmaxf(fmaxf(fabsf(o[3] - o[0]), fabsf(o[4] - o[1])), fabsf(o[5] - o[2]));
+    // a sixteenth of a radian, and of the scene's size
+    const bool alike = dot(c, c) <= (1.f / 256.f) * (dot(d0, d0) * dot(d1, d1)) && dot(d0, d1) > 0.f && off <= (1.f / 16.f) * __uint_as_float(bounds->scale);
+    const uint32_t n_alike = (uint32_t)__syncthreads_count(alike ? 1 : 0);
+    uint32_t before = 0u, all = 0u;
+    for (uint32_t w = 0u; w < kListCells / 32u; ++w) {
+        if (w < tid / 32u) before += (uint32_t)__popc(s_cells[w]);
+        all += (uint32_t)__popc(s_cells[w]);
+    }
+    const uint32_t bits = all <= 1u ? 0u : 32u - (uint32_t)__clz(all - 1u);
+    const uint32_t mine = s_cells[tid / 32u], bit = 1u << (tid % 32u);
+    // (a cell that no ray looked at begins in: with one of the others)
+    head->place[tid] = (mine & bit) != 0u ? before + (uint32_t)__popc(mine & (bit - 1u)) : tid & ((1u << bits) - 1u);
+    if (tid == 0u) {
+        head->sorts = n_alike < kListLooks / 4u * 3u && (all <= kListPlaces || n >= kOrderManyRays) ? 1u : 0u;
+        head->direction_bits = 16u - bits;
+        head->finished = 0u;
+    }
+}
+__global__ __launch_bounds__(kListThreads) void k_list_count(const float *__restrict__ ray_o, const float *__restrict__ ray_d, const DstBounds *bounds,
+                                                             ListHead *head, uint32_t *__restrict__ keys, uint32_t *__restrict__ ranks, uint32_t n) {
+    if (head->sorts == 0u) return;
+    __shared__ uint32_t s_last, s_sum[kListThreads / DST_WAVE];
+    const uint32_t tid = threadIdx.x, r = blockIdx.x * kListThreads + tid, bits = head->direction_bits;
+    if (r < n) {
+        const uint32_t key = (head->place[origin_cell<3>(ray_o + 3 * (size_t)r, bounds)] << bits) | (direction_code(ray_d + 3 * (size_t)r) >> (16u - bits));
+        keys[r] = key;
+        ranks[r] = atomicAdd(&head->start[key], 1u);
+    }
+    __syncthreads();
+    if (tid == 0u) {   // (one fence for the workgroup: one for every wave made this 60 us of 131,072 rays)
+        __threadfence();
+        s_last = atomicAdd(&head->finished, 1u) == gridDim.x - 1u ? 1u : 0u;
+    }
+    __syncthreads();
+    if (s_last == 0u) return;
+    __threadfence();
+    // a wave's stretch of the keys, sixteen bytes a lane at a time
+    constexpr uint32_t kSteps = kListKeys / (4u * kListThreads);
+    const uint32_t lane = tid % DST_WAVE, wave = tid / DST_WAVE;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 *const from = reinterpret_cast<u32x4 *>(head->start) + (size_t)wave * kSteps * DST_WAVE + lane;
+    u32x4 count[kSteps];
+    uint32_t upto[kSteps], sum = 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < kSteps; ++k) count[k] = from[k * DST_WAVE];
+#pragma unroll
+    for (uint32_t k = 0; k < kSteps; ++k) {
+        const uint32_t mine = (count[k].x + count[k].y) + (count[k].z + count[k].w);
+        uint32_t run = mine;
+#pragma unroll
+        for (uint32_t off = 1u; off < (uint32_t)DST_WAVE; off <<= 1) {
+            const uint32_t other = __shfl_up(run, off);
+            if (lane >= off) run += other;
+        }
+        upto[k] = sum + run - mine;
+        sum += __shfl(run, DST_WAVE - 1);
+    }
+    if (lane == 0u) s_sum[wave] = sum;
+    __syncthreads();
+    uint32_t base = 0u;
+    for (uint32_t w = 0u; w < wave; ++w) base += s_sum[w];
+#pragma unroll
+    for (uint32_t k = 0; k < kSteps; ++k) {
+        const uint32_t a = base + upto[k], b = a + count[k].x, c = b + count[k].y;
+        from[k * DST_WAVE] = u32x4{a, b, c, c + count[k].z};
+    }
+}
+// (head == nullptr: no scratch memory)
+__global__ __launch_bounds__(kListThreads) void k_list_place(const ListHead *__restrict__ head, const uint32_t *__restrict__ keys, const uint32_t *__restrict__ ranks,
+                                                             uint32_t *__restrict__ order, uint32_t n) {
+    const uint32_t r = blockIdx.x * kListThreads + threadIdx.x;
+    if (r >= n) return;
+    order[head != nullptr && head->sorts != 0u ? head->start[keys[r]] + ranks[r] : r] = r;
 }
 
 __global__ void k_pack_half(const float *__restrict__ src, uint16_t *__restrict__ dst, uint64_t n) {
@@ -2592,7 +2706,7 @@ struct TileGrid {
 };
 
 // 8x8 pixel tiles per wave, 2x2 tiles per block.  A thin grid (H < 8: a (B,N,3) ray list) is one flat list of
-// H*W rays in tiles of 1x64, traced in a coherent order of its own where that pays (k_ray_keys).
+// H*W rays in tiles of 1x64, traced in a coherent order of its own where that pays (k_ray_keys, k_list_look).
 constexpr int kThinRows = 8;
 TileGrid tile_grid(int H, int W) {
     TileGrid t;
@@ -2755,7 +2869,7 @@ void launch_row_bwd(const DstParams &p, RowGrid g, const uint32_t *ray_order, hi
 #undef DST_ROW
 }
 
-// What a forward trace keeps in its scratch memory: the surfels' records, and behind them the guessed cost of every block and
+// What a forward trace keeps in its scratch memory.  Of a list: what its order is made with (k_list_look).  Of an image: the surfels' records, and behind them the guessed cost of every block and
 // the order that follows from it.  Records are worth their pass where there are no more than four surfels to a ray (0.03 ns a
 // surfel against 0.09 a ray of the 1080p room), the order on grids of up to 4095 blocks: larger ones keep the chip full to the
 // end (1280x720 room of 300,000 surfels, 3600 blocks: 504 / 503 us without and with, of a million 1903 / 1708), and a single
@@ -2766,16 +2880,36 @@ void launch_row_bwd(const DstParams &p, RowGrid g, const uint32_t *ray_order, hi
 constexpr uint64_t kOrderedBlocks = 4095u;
 constexpr float kOrderedLayers = 5.0f, kRecordedLayers = 2.0f;
 struct ScratchLayout {
-    uint64_t records, blocks;   // 0: none
-    ScratchLayout(int32_t P, int32_t H, int32_t W) : records(0), blocks(0) {
+    uint64_t records, blocks, list;   // 0: none
+    ScratchLayout(int32_t P, int32_t H, int32_t W) : records(0), blocks(0), list(0) {
         const uint64_t rays = (uint64_t)std::max(H, 0) * (uint64_t)std::max(W, 0);
+        if (P > 0 && H < kThinRows && rays >= kOrderMinByRows) list = rays;
         if (P <= 0 || H < kThinRows || rays <= kRowRecordedRays) return;
         const TileGrid t = tile_grid(H, W);
         if (rays >= (uint64_t)P / 4u) records = (uint64_t)P;
         if ((uint64_t)t.btiles_x * t.btiles_y <= kOrderedBlocks) blocks = (uint64_t)t.btiles_x * t.btiles_y;
     }
-    uint64_t bytes() const { return sizeof(DstSurfel) * records + 2u * sizeof(uint32_t) * blocks; }
+    uint64_t bytes() const {
+        return list != 0u ? sizeof(ListHead) + 3u * sizeof(uint32_t) * list : sizeof(DstSurfel) * records + 2u * sizeof(uint32_t) * blocks;
+    }
 };
+// The order of a list traced by rows: in `kept`, the record's room for it (from kOrderMinByRows rays on the backward trace counts
+// on finding one there), or else in the scratch memory.  Without scratch memory as the rays come (nullptr: the same).
+const uint32_t *order_list(const dst_ctx *ctx, const DstParams &p, uint32_t n, uint32_t *kept, hipStream_t stream) {
+    ListHead *const head = reinterpret_cast<ListHead *>(p.scratch);
+    if (head == nullptr && kept == nullptr) return nullptr;
+    const dim3 grid((n + kListThreads - 1u) / kListThreads), block(kListThreads);
+    uint32_t *keys = nullptr, *ranks = nullptr, *order = kept;
+    if (head != nullptr) {
+        keys = reinterpret_cast<uint32_t *>(head + 1);
+        ranks = keys + n;
+        if (order == nullptr) order = ranks + n;
+        hipLaunchKernelGGL(k_list_look, dim3(1u + kListKeys / kListLooks), dim3(kListLooks), 0, stream, p.ray_o, p.ray_d, ctx->bounds, head, n);
+        hipLaunchKernelGGL(k_list_count, grid, block, 0, stream, p.ray_o, p.ray_d, ctx->bounds, head, keys, ranks, n);
+    }
+    hipLaunchKernelGGL(k_list_place, grid, block, 0, stream, head, keys, ranks, order, n);
+    return order;
+}
 // Made where the kernels that read it are launched next, plain tiles and the rows beyond them.  Returns the order of the blocks
 // (nullptr: as they lie), and takes from p.scratch what these kernels shall not look for.
 const uint32_t *make_scratch(const dst_ctx *ctx, DstParams &p, const DstAccelView &acc, const TileGrid &t, hipStream_t stream) {
@@ -2868,7 +3002,7 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
     const uint32_t *ray_order = nullptr, *row_order = nullptr;   // row_order: of a list traced by rows
     if (p.H < kThinRows) {
         // a ray list: flat, and (when it is long enough to matter: kOrderMinByRows) in an order that puts similar rays in one
-        // wave.  The backward trace takes it from the record, and without a record makes its own.
+        // wave.  The backward trace takes it from the record, and without a record makes its own (kOrderMinRays).
         if ((uint64_t)p.H * p.W > 0x7FFFFFFFull) return dst_fail(ctx, DST_E_INVALID, "ray grid too large");
         p.W = p.H * p.W;
         p.H = 1;
@@ -2878,11 +3012,13 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
             const TileGrid t = tile_grid(1, p.W);
             kept = reinterpret_cast<uint32_t *>(p.hit_record + record_order_at(n, t.th_log2, (uint32_t)p.mtd_alloc + 1u, (uint64_t)t.btiles_x * t.btiles_y * kWavesPerBlock));
         }
-        const bool by_rows = backward ? kept != nullptr : !(kFwdWavesPerBlock == 1 && dst_handover_active(ctx));
-        if (n >= kOrderMinRays && backward && kept != nullptr) {
-            ray_order = kept;   // (what the forward trace left there; nobody looks where it left nothing)
+        const bool by_rows = !backward && !(kFwdWavesPerBlock == 1 && dst_handover_active(ctx));
+        if (backward && kept != nullptr) {   // (what the forward trace left there; nobody looks where it left nothing)
+            if (n >= kOrderMinRays) ray_order = kept;
             if (n >= kOrderMinByRows) row_order = kept;
-        } else if (n >= (by_rows ? kOrderMinByRows : kOrderMinRays)) {
+        } else if (by_rows) {
+            if (n >= kOrderMinByRows) row_order = order_list(ctx, p, n, kept, stream);
+        } else if (n >= kOrderMinRays) {
             if (n > ctx->ray_capacity) {
                 for (int k = 0; k < 2; ++k) {
                     if (ctx->ray_keys[k]) (void)hipFree(ctx->ray_keys[k]);
@@ -2901,9 +3037,9 @@ int dst_launch_trace(dst_ctx *ctx, const DstParams &p_in, bool backward, hipStre
             }
             uint32_t *vals[2] = {kept != nullptr ? kept : ctx->ray_vals[0], ctx->ray_vals[1]};
             hipLaunchKernelGGL(k_ray_keys, dim3((n + 255u) / 256u), dim3(256), 0, stream, p.ray_o, p.ray_d, ctx->bounds,
-                               ctx->ray_keys[0], vals[0], n, by_rows ? 1 : 0);
-            dst_sort_pairs(ctx->ray_keys, vals, ctx->ray_hist, n, stream, by_rows ? 16 : 32);
-            ray_order = row_order = vals[0];
+                               ctx->ray_keys[0], vals[0], n);
+            dst_sort_pairs(ctx->ray_keys, vals, ctx->ray_hist, n, stream);
+            ray_order = vals[0];
         }
     }
     const TileGrid t = tile_grid(p.H, p.W);

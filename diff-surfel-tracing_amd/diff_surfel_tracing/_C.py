@@ -598,7 +598,7 @@ def trace_surfels(ctx, training, start_from_first, ray_o, ray_d, vertices, backg
     if getattr(ctx, "distortion", False):
         p.flags |= FLAG_DISTORTION
     _use_sh_half(ctx, p, keep)
-    if p.flags == 0 and _scratch_bytes.get((P, H, W)) != 0:   # (the kernels with the rare options have no use for it)
+    if (p.flags == 0 or H < 8) and _scratch_bytes.get((P, H, W)) != 0:   # (images' kernels with the rare options do without)
         _scratch(p, keep)
     if events is not None:
         events[0].record()

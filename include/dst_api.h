@@ -102,9 +102,9 @@ typedef struct DstParams {
      * again instead (the host need not look at the record between the two calls; it may read word 0 later to
      * size the next record; at most 2^26 - 1 blocks of a record are used).  Word 1 counts chains a replay found
      * broken: it stays 0 unless the buffer was not written by a forward trace with the same grid, depth and a zeroed
-     * header.  The record of a ray list (fewer than eight rows) of 2048 rays and more also has room for an order of the
-     * rays; where the forward trace made one, the backward trace takes it from there, also where the record is
-     * incomplete: it may only be given a record that a forward trace of the same grid and depth has been given before. */
+     * header.  The record of a ray list (fewer than eight rows) also has room for an order of the rays; where the forward
+     * trace made one, the backward trace takes it from there, also where the record is incomplete: it may only be given a
+     * record that a forward trace of the same grid and depth has been given before. */
     uint64_t *hit_record;
     uint32_t hit_record_blocks;
     uint32_t flags;               /* DST_FLAG_* */
@@ -154,8 +154,8 @@ typedef struct DstParams {
     int32_t dist_channels;        /* forward: channels of out_dist: 1 (the distortion alone), or 3 (also 0: three) */
     int32_t reserved;
     /* forward, optional: device memory, aligned to 128 bytes, dst_trace_scratch_bytes(P, H, W) of it, in which the call keeps
-     * what it prepares before it traces: what depends on a surfel alone, and an order for the image's tiles (contents before
-     * and after the call mean nothing).  Same results bit for bit, faster; NULL: neither is made. */
+     * what it prepares before it traces: what depends on a surfel alone and an order for the image's tiles, or a long list's
+     * order of rays (contents before and after the call mean nothing).  Same results bit for bit, faster; NULL: none is made. */
     void *scratch;
 } DstParams;
 
@@ -280,7 +280,7 @@ uint64_t dst_hit_record_layout(int32_t H, int32_t W, int32_t mtd_alloc, uint32_t
                                uint32_t *n_waves);
 
 /* Size in bytes of DstParams.scratch for a forward trace of P surfels over an (H,W) ray grid; 0 where the call has no use for
- * any (lists, small images, and the largest with far fewer rays than surfels). */
+ * any (lists of fewer than 65,536 rays, small images, and the largest with far fewer rays than surfels). */
 uint64_t dst_trace_scratch_bytes(int32_t P, int32_t H, int32_t W);
 
 /* Words (8 bytes each) of DstParams.det_workspace for a forward (backward = 0: one per surfel) or a backward
