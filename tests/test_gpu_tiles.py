@@ -169,3 +169,28 @@ def test_rays_of_one_origin(kind, fov, shrink, shift):
            for x in (o, moved)]
     for a, b in zip(*out):
         assert torch.equal(a.cpu()[same].view(torch.int32), b.cpu()[same].view(torch.int32))
+
+
+@pytest.mark.parametrize("H_,W_,fov", [(24, 16, 2.0), (40, 48, 35.0), (33, 17, 8.0)])
+def test_limb_of_a_sphere(H_, W_, fov):
+    """Tiles whose way is full of quads that their edges leave out none of (a bundle that has looked at many for nothing looks at
+    edges no more), and tiles beside them that quads are left out for: the same bits with one ray of every tile moved a
+    little, for which the edges are not looked at."""
+    from diff_surfel_tracing import _C
+    sc = S.scene_sphere(P=60000, seed=3)
+    # along the tangent from the eye: the limb crosses the image from top to bottom
+    o, d = S.pinhole_rays(H_, W_, fov, (4.0, 0.0, 0.0), (0.25, 0.968, 0.0) if fov < 30 else (0.0, 0.0, 0.0))
+    moved = o.clone()
+    moved[3::8, 5::8] += 1e-3
+    same = torch.ones(H_, W_, dtype=torch.bool)
+    same[3::8, 5::8] = False
+    tracer = tile_tracer()
+    tracer.build_acceleration_structure(sc["vertices"].cuda(), sc["faces"].cuda(), rebuild=True)
+    g = {k: v.cuda() for k, v in sc.items()}
+    e, bg, eye4 = torch.empty(0, device="cuda"), torch.zeros(3, device="cuda"), torch.eye(4, device="cuda")
+    out = [_C.trace_surfels(tracer.optix_context, False, True, x.cuda(), d.cuda(), g["vertices"], bg, g["means3D"], g["shs"], 3, e, e,
+                            g["opacities"], g["scales"], 1.0, g["rotations"], e, eye4, eye4, bg, False, False, 0, 0.0)[:6]
+           for x in (o, moved)]
+    assert out[0][2].max() > 0.9
+    for a, b in zip(*out):
+        assert torch.equal(a.cpu()[same].view(torch.int32), b.cpu()[same].view(torch.int32))
