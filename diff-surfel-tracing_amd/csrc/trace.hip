@@ -2729,6 +2729,11 @@ TileGrid tile_grid(int H, int W) {
     return t;
 }
 
+// Tiles evaluate hits from the surfels' records with up to this many auxiliary channels.  (With eight, from the tensors / from
+// records, us evaluated and recorded: 1080p room of a million 2549 / 2601 and 2970 / 2981, 1280x720 room of 300,000 582 / 591 and
+// 710 / 716, 640x480 of 100,000 145 / 151 and 196 / 198, 800x800 sphere of 100,000 1347 / 1304 and 1519 / 1444.)
+constexpr int kPackedAux = 4;
+
 // `handover` / `hand_arg`: see trace_body (forward only; hand_arg steps = 0 launches the takers of the listed tiles).
 template <bool BWD, bool REC>
 void launch(const DstParams &p, const DstAccelView &acc, const TileGrid &t, const uint32_t *ray_order, hipStream_t stream,
@@ -2760,8 +2765,8 @@ void launch(const DstParams &p, const DstAccelView &acc, const TileGrid &t, cons
         else if (BWD)                                                                                              \
             hipLaunchKernelGGL((k_trace_bwd<AUX, REC, (MIXED) && !REC, false>), grid, block, 0, stream, p, acc,     \
                                t.tw_log2, t.th_log2, t.tiles_x, t.tiles_y, t.btiles_x, ray_order, strip, block_order);    \
-        else if (!(MIXED) && p.flags == 0u && handover == nullptr && p.scratch != nullptr && (AUX) < 8)            \
-            hipLaunchKernelGGL((k_trace_fwd_plain<AUX, REC, (AUX) < 8>), grid, block, 0, stream, p, acc, t.tw_log2, \
+        else if (!(MIXED) && p.flags == 0u && handover == nullptr && p.scratch != nullptr && (AUX) <= kPackedAux)  \
+            hipLaunchKernelGGL((k_trace_fwd_plain<AUX, REC, ((AUX) <= kPackedAux)>), grid, block, 0, stream, p, acc, t.tw_log2, \
                                t.th_log2, t.tiles_x, t.tiles_y, t.btiles_x, ray_order, strip, block_order);               \
         else if (!(MIXED) && p.flags == 0u && handover == nullptr)                                                 \
             hipLaunchKernelGGL((k_trace_fwd_plain<AUX, REC, false>), grid, block, 0, stream, p, acc, t.tw_log2,           \
@@ -2889,6 +2894,15 @@ struct ScratchLayout {
         if (rays >= (uint64_t)P / 4u) records = (uint64_t)P;
         if ((uint64_t)t.btiles_x * t.btiles_y <= kOrderedBlocks) blocks = (uint64_t)t.btiles_x * t.btiles_y;
     }
+    // Of these, what the kernels that trace this call read.
+    ScratchLayout(const dst_ctx *ctx, const DstParams &p) : ScratchLayout(p.P, p.H, p.W) {
+        const bool hands = kFwdWavesPerBlock == 1 && dst_handover_active(ctx);
+        const bool by_rows = ctx->handover_mode != DST_HANDOVER_OFF && (uint64_t)p.H * p.W <= (p.hit_record != nullptr ? kRowRecordedRays : kRowEvaluatedRays);
+        if (hands) list = 0u;
+        if (hands || by_rows || p.flags != 0u) records = blocks = 0u;
+        if (ctx->layers < kOrderedLayers) blocks = 0u;   // (no number, of a scene on a line: many)
+        if (ctx->layers < kRecordedLayers || (p.aux > kPackedAux && p.max_trace_depth == 0)) records = 0u;
+    }
     uint64_t bytes() const {
         return list != 0u ? sizeof(ListHead) + 3u * sizeof(uint32_t) * list : sizeof(DstSurfel) * records + 2u * sizeof(uint32_t) * blocks;
     }
@@ -2913,10 +2927,8 @@ const uint32_t *order_list(const dst_ctx *ctx, const DstParams &p, uint32_t n, u
 // Made where the kernels that read it are launched next, plain tiles and the rows beyond them.  Returns the order of the blocks
 // (nullptr: as they lie), and takes from p.scratch what these kernels shall not look for.
 const uint32_t *make_scratch(const dst_ctx *ctx, DstParams &p, const DstAccelView &acc, const TileGrid &t, hipStream_t stream) {
-    if (p.scratch == nullptr || p.flags != 0u) return nullptr;
-    ScratchLayout s(p.P, p.H, p.W);
-    if (ctx->layers < kOrderedLayers) s.blocks = 0u;   // (no number, of a scene on a line: many)
-    if (ctx->layers < kRecordedLayers) s.records = 0u;
+    if (p.scratch == nullptr) return nullptr;
+    const ScratchLayout s(ctx, p);
     if (s.records == 0u && s.blocks == 0u) {
         p.scratch = nullptr;
         return nullptr;
@@ -2961,6 +2973,7 @@ uint64_t dst_det_workspace_words(int32_t P, int32_t aux, int backward) {
 }
 
 uint64_t dst_trace_scratch_bytes(int32_t P, int32_t H, int32_t W) { return ScratchLayout(P, H, W).bytes(); }
+uint64_t dst_trace_scratch_needed(const dst_ctx *ctx, const DstParams *p) { return ctx != nullptr && p != nullptr ? ScratchLayout(ctx, *p).bytes() : 0u; }
 
 uint64_t dst_hit_record_layout(int32_t H, int32_t W, int32_t mtd_alloc, uint32_t blocks, uint64_t *header_words,
                                uint32_t *n_waves) {

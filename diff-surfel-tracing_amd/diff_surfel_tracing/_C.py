@@ -63,7 +63,8 @@ HANDOVER_OFF, HANDOVER_AUTO, HANDOVER_ALWAYS = 0, 1, 2
 EXPORTS = ("dst_create", "dst_destroy", "dst_build_accel", "dst_trace_forward", "dst_trace_backward",
            "dst_last_error", "dst_accel_info", "dst_accel_download", "dst_version", "dst_sizeof_params",
            "dst_hit_record_layout", "dst_refit_accel_static", "dst_refit_from_surfels",
-           "dst_det_workspace_words", "dst_trace_scratch_bytes", "dst_pack_sh_half", "dst_trace_info", "dst_set_handover", "dst_det_out_of_range")
+           "dst_det_workspace_words", "dst_trace_scratch_bytes",
+           "dst_trace_scratch_needed", "dst_pack_sh_half", "dst_trace_info", "dst_set_handover", "dst_det_out_of_range")
 
 _lib = None
 
@@ -98,6 +99,8 @@ def load_library():
     L.dst_det_workspace_words.argtypes = [C.c_int32, C.c_int32, C.c_int]
     L.dst_trace_scratch_bytes.restype = C.c_uint64
     L.dst_trace_scratch_bytes.argtypes = [C.c_int32, C.c_int32, C.c_int32]
+    L.dst_trace_scratch_needed.restype = C.c_uint64
+    L.dst_trace_scratch_needed.argtypes = [C.c_void_p, C.POINTER(DstParams)]
     L.dst_pack_sh_half.argtypes = [C.c_void_p, C.c_void_p, C.c_uint64, C.c_void_p]
     L.dst_version.restype = C.c_char_p
     L.dst_sizeof_params.restype = C.c_size_t
@@ -549,6 +552,8 @@ def _scratch(p, keep):
         if len(_scratch_bytes) >= 256:
             _scratch_bytes.clear()
         size = _scratch_bytes[key] = load_library().dst_trace_scratch_bytes(*key)
+    if size != 0:
+        size = load_library().dst_trace_scratch_needed(keep["context"].handle, C.byref(p))
     if size == 0:
         return
     try:
@@ -598,7 +603,8 @@ def trace_surfels(ctx, training, start_from_first, ray_o, ray_d, vertices, backg
     if getattr(ctx, "distortion", False):
         p.flags |= FLAG_DISTORTION
     _use_sh_half(ctx, p, keep)
-    if (p.flags == 0 or H < 8) and _scratch_bytes.get((P, H, W)) != 0:   # (images' kernels with the rare options do without)
+    if (p.flags == 0 or H < 8) and _scratch_bytes.get((P, H, W)) != 0:   # (images' kernels with the rare options take none)
+        keep["context"] = ctx
         _scratch(p, keep)
     if events is not None:
         events[0].record()

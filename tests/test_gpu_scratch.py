@@ -10,6 +10,21 @@ from diff_surfel_tracing import _C
 pytestmark = pytest.mark.gpu
 
 
+RECORD_BYTES = 64   # of a surfel
+
+
+def layers(vertices):
+    """How often the quads cover the surface of the box of their centres."""
+    q = vertices.reshape(-1, 4, 3).double()
+    area = torch.linalg.cross(q[:, 1] - q[:, 0], q[:, 2] - q[:, 0]).norm(dim=1).sum()
+    e = (0.5 * (q.amin(1) + q.amax(1))).amax(0) - (0.5 * (q.amin(1) + q.amax(1))).amin(0)
+    return float(area / (2 * (e[0] * e[1] + e[1] * e[2] + e[2] * e[0])))
+
+
+def blocks_of(o):
+    return ((o.shape[0] + 15) // 16) * ((o.shape[1] + 15) // 16)
+
+
 def both(monkeypatch, tracer, sc, o, d, depth=0, aux=0, training=False):
     """(outputs with scratch memory, without)"""
     g = {k: v.cuda() for k, v in sc.items()}
@@ -59,6 +74,43 @@ def test_records_change_no_bit(monkeypatch, depth, aux):
     with_, without = both(monkeypatch, tracer, sc, o, d, depth, aux)
     for a, b in zip(with_, without):
         assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
+@pytest.mark.parametrize("case", ["eight channels", "rows", "hand-over", "one layer", "options"])
+def test_nothing_is_made_that_no_kernel_reads(monkeypatch, case):
+    """No memory is taken for it, and where a caller gives all that the size could want, none of it is written."""
+    import diff_surfel_tracing as dst
+    tracer = dst.SurfelTracer()
+    P = 3000 if case == "one layer" else 30011
+    sc = S.scene_room(P=P, seed=4, half=0.4 if case == "one layer" else 1.5)
+    assert (layers(sc["vertices"]) < 1.8) == (case == "one layer")
+    o, d = view(256, 399) if case == "rows" else view(331, 317)   # 102,144 rays; 104,927
+    tracer.build_acceleration_structure(sc["vertices"].cuda(), sc["faces"].cuda(), rebuild=True)
+    if case == "hand-over":
+        tracer.optix_context.set_handover(_C.HANDOVER_ALWAYS, 4000)
+    if case == "options":
+        tracer.optix_context.distortion = True
+    read = 8 * blocks_of(o) if case == "eight channels" else 0    # the order
+    given = []
+
+    def all_of_it(p, keep):
+        size = _C.load_library().dst_trace_scratch_bytes(p.P, p.H, p.W)
+        assert size == RECORD_BYTES * P + 8 * blocks_of(o)
+        assert _C.load_library().dst_trace_scratch_needed(tracer.optix_context.handle, _C.C.byref(p)) == (0 if p.flags else read)
+        given.append(torch.full((size,), 0xA5, dtype=torch.uint8, device="cuda"))
+        keep["scratch"], p.scratch = given[0], given[0].data_ptr()
+
+    monkeypatch.setattr(_C, "_scratch", all_of_it)
+    g = {k: v.cuda() for k, v in sc.items()}
+    e, bg, eye = torch.empty(0, device="cuda"), torch.zeros(3, device="cuda"), torch.eye(4, device="cuda")
+    others = torch.rand(P, 8).cuda() if case == "eight channels" else e
+    out = _C.trace_surfels(tracer.optix_context, False, True, o.cuda(), d.cuda(), g["vertices"], bg, g["means3D"], g["shs"], 3, e,
+                           others, g["opacities"], g["scales"], 1.0, g["rotations"], e, eye, eye, bg, False, False, 0, 0.0)
+    assert out[0].std() > 0.01
+    if case == "options":
+        assert not given
+    else:
+        assert bool((given[0][read:] == 0xA5).all())
 
 
 @pytest.mark.parametrize("factor", [0.0, 1e-42, 1e-20, 2.0 ** -40, 0.99 * 2.0 ** -40, 1.0, 2.0 ** 40, 1.01 * 2.0 ** 40, 1e20, 3e38,
