@@ -1,6 +1,7 @@
 """The forward trace's scratch memory (DstParams.scratch): hits evaluated from records of the surfels, and blocks traced in
-the order of a cost guessed for them, both of which the call makes first.  Outputs and hit records have to be those of the same call without scratch memory bit for bit, whatever the
-scales (quotients by them are formed from their reciprocals in the records, and divided out where that does not hold)."""
+the order of a cost guessed for them, both of which the call makes first.  Outputs, and what a record lets the backward trace
+replay, have to be those of the same call without scratch memory bit for bit, whatever the scales (quotients by them are
+formed from their reciprocals in the records, and divided out where that does not hold)."""
 import pytest
 import torch
 
@@ -25,53 +26,78 @@ def blocks_of(o):
     return ((o.shape[0] + 15) // 16) * ((o.shape[1] + 15) // 16)
 
 
-def both(monkeypatch, tracer, sc, o, d, depth=0, aux=0, training=False):
-    """(outputs with scratch memory, without)"""
+def both(monkeypatch, tracer, sc, o, d, depth=0, aux=0, training=False, record=False):
+    """(outputs with scratch memory, without, bytes of it).  With `record`, behind the outputs the number of blocks that were
+    asked for in a hit record, and the rays' gradients as replayed from it."""
     g = {k: v.cuda() for k, v in sc.items()}
     e, bg, eye = torch.empty(0, device="cuda"), torch.zeros(3, device="cuda"), torch.eye(4, device="cuda")
     others = torch.rand(sc["means3D"].shape[0], aux, generator=torch.Generator().manual_seed(3)).cuda() if aux else e
-    out = []
+    real, taken, out, (H, W) = _C._scratch, [], [], o.shape[:2]
+
+    def spy(p, keep):
+        real(p, keep)
+        taken.append(keep["scratch"].numel() if "scratch" in keep else 0)
+
+    args = (True, o.cuda(), d.cuda(), g["vertices"], bg, g["means3D"], g["shs"], 3, e, others, g["opacities"], g["scales"], 1.0,
+            g["rotations"], e, eye, eye, bg, False, False, depth, 0.1)
+    if not _C.load_library().dst_trace_scratch_bytes(sc["means3D"].shape[0], H, W):
+        pytest.fail("this size has no scratch memory")
     for use in (True, False):
-        if not use:
-            monkeypatch.setattr(_C, "_scratch", lambda p, keep: None)
-        elif not _C.load_library().dst_trace_scratch_bytes(sc["means3D"].shape[0], o.shape[0], o.shape[1]):
-            pytest.fail("this size has no scratch memory")
-        out.append([x for x in _C.trace_surfels(
-            tracer.optix_context, training, True, o.cuda(), d.cuda(), g["vertices"], bg, g["means3D"], g["shs"], 3, e, others,
-            g["opacities"], g["scales"], 1.0, g["rotations"], e, eye, eye, bg, False, False, depth, 0.1) if x is not None])
+        monkeypatch.setattr(_C, "_scratch", spy if use else lambda p, keep: None)
+        rec = _C.HitRecord(H, W, max(1, depth), 16.0, torch.device("cuda")) if record else None
+        res = [x for x in _C.trace_surfels(tracer.optix_context, training, *args, hit_record=rec) if x is not None]
+        if record:
+            gen = torch.Generator().manual_seed(8)
+            ups = [torch.randn(x.shape, generator=gen).cuda() for x in res[:6]]
+            asked = rec.words[:1].clone()
+            assert int(asked) <= rec.blocks
+            grads = _C.trace_surfels_backward(tracer.optix_context, *args, *res[:7], *ups, hit_record=rec)[:2]
+            assert grads[1].abs().max() > 0
+            res[7:7] = [asked.to(torch.int32), *grads]
+        out.append(res)
         torch.cuda.synchronize()
-    return out
+    monkeypatch.setattr(_C, "_scratch", real)
+    return out[0], out[1], taken[0]
 
 
 def view(H, W):
     return S.pinhole_rays(H, W, 70.0, (-0.6, -0.3, 0.15), (0.9, 0.45, -0.15))
 
 
-@pytest.mark.parametrize("H,W", [(8, 8221), (4111, 16), (257, 256), (1040, 1008), (1040, 1024)])
-@pytest.mark.parametrize("P,half", [(3000, 0.4), (250000, 1.5)])
-def test_every_block_is_traced_once(monkeypatch, H, W, P, half):
-    """One row and one column of blocks, an odd one, the largest grid whose blocks are ordered and one larger; fewer surfels
-    than rays, and so many that only the order is made."""
+@pytest.mark.parametrize("H,W,P,makes", [
+    # one row and one column of blocks, an odd one, the largest grid whose blocks are ordered; fewer surfels than rays
+    (8, 8221, 30011, "both"), (4111, 16, 30011, "both"), (257, 256, 30011, "both"), (1040, 1008, 30011, "both"),
+    (1040, 1024, 30011, "records"),                                 # one block row more
+    (257, 256, 10007, "records"),                                   # quads that cover the room three times
+    (8, 8221, 300000, "order"), (4111, 16, 300000, "order"), (257, 256, 300000, "order"),   # four surfels to a ray and more
+])
+def test_every_block_is_traced_once(monkeypatch, H, W, P, makes):
+    """Outputs, what is recorded and what is replayed from it: the same bits with the blocks' order and the records of the
+    surfels, with either alone, and with neither."""
     import diff_surfel_tracing as dst
     tracer = dst.SurfelTracer()
-    sc = S.scene_room(P=P, seed=6, half=half)
-    o, d = S.pinhole_rays(H, W, 70.0, (-0.4 * half, -0.2 * half, 0.1 * half), (0.6 * half, 0.3 * half, -0.1 * half))
+    sc = S.scene_room(P=P, seed=6, half=1.5)
+    o, d = view(H, W)
+    assert (layers(sc["vertices"]) > 5.5) == (P != 10007) and layers(sc["vertices"]) > 2.5
     tracer.build_acceleration_structure(sc["vertices"].cuda(), sc["faces"].cuda(), rebuild=True)
-    with_, without = both(monkeypatch, tracer, sc, o, d, training=True)
+    with_, without, size = both(monkeypatch, tracer, sc, o, d, training=True, record=True)
+    assert size == (0 if makes == "order" else RECORD_BYTES * P) + (0 if makes == "records" else 8 * blocks_of(o))
     assert without[0].std() > 0.01
     for a, b in zip(with_[:-1], without[:-1]):
         assert torch.equal(a.view(torch.int32), b.view(torch.int32))
     torch.testing.assert_close(with_[-1], without[-1], rtol=1e-4, atol=1e-4)   # blending weights: sums in another order
 
 
-@pytest.mark.parametrize("depth,aux", [(0, 0), (0, 3), (1, 2), (1, 8)])
-def test_records_change_no_bit(monkeypatch, depth, aux):
+@pytest.mark.parametrize("record", [False, True])
+@pytest.mark.parametrize("depth,aux", [(0, 0), (0, 3), (0, 8), (1, 2), (1, 8)])
+def test_records_change_no_bit(monkeypatch, depth, aux, record):
     import diff_surfel_tracing as dst
     tracer = dst.SurfelTracer()
     sc = S.scene_room(P=30011, seed=4, half=1.5)
-    o, d = view(259, 331)
+    o, d = view(331, 317)
     tracer.build_acceleration_structure(sc["vertices"].cuda(), sc["faces"].cuda(), rebuild=True)
-    with_, without = both(monkeypatch, tracer, sc, o, d, depth, aux)
+    with_, without, size = both(monkeypatch, tracer, sc, o, d, depth, aux, record=record)
+    assert size == (RECORD_BYTES * 30011 if aux <= 4 or depth else 0) + 8 * blocks_of(o)
     for a, b in zip(with_, without):
         assert torch.equal(a.view(torch.int32), b.view(torch.int32))
 
@@ -120,33 +146,36 @@ def test_scales_of_any_size(monkeypatch, factor):
     import diff_surfel_tracing as dst
     tracer = dst.SurfelTracer()
     sc = S.scene_room(P=20000, seed=5, half=1.5)
-    o, d = view(257, 257)
+    o, d = view(257, 407)
     tracer.build_acceleration_structure(sc["vertices"].cuda(), sc["faces"].cuda(), rebuild=True)
     sc["scales"][::3] *= factor
     if factor in (2.0 ** -40, 2.0 ** 40):   # the edges of the reciprocals' range
         sc["scales"][::3] = factor
     sc["means3D"][1::50] = 1e30             # far too large to divide by way of a reciprocal
-    with_, without = both(monkeypatch, tracer, sc, o, d)
+    with_, without, size = both(monkeypatch, tracer, sc, o, d)
+    assert size > RECORD_BYTES * 20000
     for a, b in zip(with_, without):
         same = (a.view(torch.int32) == b.view(torch.int32)) | (torch.isnan(a) & torch.isnan(b))
         assert bool(same.all())
 
 
-def test_misaligned_scratch_is_refused():
+def test_misaligned_scratch_is_refused(monkeypatch):
     import diff_surfel_tracing as dst
     tracer = dst.SurfelTracer()
     sc = S.scene_cube(P=64, seed=0)
     tracer.build_acceleration_structure(sc["vertices"].cuda(), sc["faces"].cuda(), rebuild=True)
+    o, d = S.rays_cube(257, 407)
+    called = []
+
     def shifted(p, keep):
         keep["scratch"] = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
         p.scratch = keep["scratch"].data_ptr() + 64
-    before, _C._scratch = _C._scratch, shifted
-    try:
-        with pytest.raises(RuntimeError, match="aligned"):
-            o, d = S.rays_cube(16, 16)
-            e, bg, eye = torch.empty(0, device="cuda"), torch.zeros(3, device="cuda"), torch.eye(4, device="cuda")
-            g = {k: v.cuda() for k, v in sc.items()}
-            _C.trace_surfels(tracer.optix_context, False, True, o.cuda(), d.cuda(), g["vertices"], bg, g["means3D"], g["shs"], 3,
-                             e, e, g["opacities"], g["scales"], 1.0, g["rotations"], e, eye, eye, bg, False, False, 0, 0.0)
-    finally:
-        _C._scratch = before
+        called.append(p.scratch)
+
+    monkeypatch.setattr(_C, "_scratch", shifted)
+    e, bg, eye = torch.empty(0, device="cuda"), torch.zeros(3, device="cuda"), torch.eye(4, device="cuda")
+    g = {k: v.cuda() for k, v in sc.items()}
+    with pytest.raises(RuntimeError, match="aligned"):
+        _C.trace_surfels(tracer.optix_context, False, True, o.cuda(), d.cuda(), g["vertices"], bg, g["means3D"], g["shs"], 3,
+                         e, e, g["opacities"], g["scales"], 1.0, g["rotations"], e, eye, eye, bg, False, False, 0, 0.0)
+    assert called
