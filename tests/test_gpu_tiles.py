@@ -109,10 +109,10 @@ class _HalfSeen:
 
 
 @pytest.mark.parametrize("aux,det", [(2, False), (4, True), (8, False)])
-@pytest.mark.parametrize("P", [1, 3, 4, 5, 107, 112, 113, 240])
+@pytest.mark.parametrize("P", [1, 3, 4, 5, 100, 101, 107, 108, 109, 112, 113, 240])
 def test_gradient_table_edges(oracle, P, aux, det):
-    """One 16x16 block before P faint surfels that all of its rays meet: its table of gradients (104 to 112 rows, in groups
-    of four) takes few of them, all, or no more than it has rows for."""
+    """One 16x16 block before P faint surfels that all of its rays meet: its table of gradients (112, 108 or 100 rows with two, four or
+    eight auxiliary channels, in groups of four) takes few of them, all, or no more than it has rows for."""
     sc = {k: v.clone() for k, v in S.scene_cube(P=P, seed=P, aux=aux).items()}
     gen = torch.Generator().manual_seed(P)
     sc["means3D"] = torch.cat([2.0 + 0.01 * torch.arange(P)[:, None].float(), 0.05 * torch.randn(P, 2, generator=gen)], 1)
