@@ -2610,9 +2610,11 @@ __global__ __launch_bounds__(kListLooks) void k_list_look(const float *__restric
         head->start[(blockIdx.x - 1u) * kListLooks + threadIdx.x] = 0u;
         return;
     }
-    // places all over the list, and at each a ray and the next one
+    // places all over the list, one in every stretch of it, and at each a ray and the next one.  (Not at even distances: of an
+    // image that is some power of two wide, row after row, every other one would be the end of a row.)
     __shared__ uint32_t s_cells[kListCells / 32u];
-    const uint32_t tid = threadIdx.x, at = (uint32_t)((uint64_t)tid * (n - 1u) / kListLooks);
+    const uint32_t tid = threadIdx.x, within = (tid * 2654435769u) >> 16;   // in its stretch, in 1 / 65536
+    const uint32_t at = (uint32_t)((((uint64_t)tid << 16) | within) * (n - 1u) / (kListLooks << 16));
     if (tid < kListCells / 32u) s_cells[tid] = 0u;
     __syncthreads();
     const float *o = ray_o + 3 * (size_t)at, *d = ray_d + 3 * (size_t)at;   // (the next ray's lie behind them)

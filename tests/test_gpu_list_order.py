@@ -59,6 +59,9 @@ def _pixels(n, seed, cameras=1):
 def _list(kind, n):
     if kind in ("one place", "twenty places"):
         return _pixels(n, 1, 1 if kind == "one place" else 20)
+    if kind.startswith("rows of"):   # an image, row after row
+        w = int(kind.split()[-1])
+        return tuple(x.reshape(1, -1, 3)[:, :n].contiguous() for x in S.pinhole_rays((n + w - 1) // w, w, 70.0, (-0.6, -0.3, 0.15), (0.9, 0.45, -0.15)))
     if kind == "in order":
         a = torch.arange(n) * (6.2831853 / 2048)
         el = torch.floor(torch.arange(n) / 2048.0) * 0.01 - 0.3
@@ -87,7 +90,8 @@ def room():
 
 @pytest.mark.parametrize("kind,n,sorts", [
     ("one place", 65535, None), ("one place", 65536, True), ("one place", 66560, True), ("one place", 66561, True), ("one place", 300001, True),
-    ("twenty places", 100003, True), ("in order", 65536, False), ("in order", 262147, False), ("unrelated", 131071, False),
+    ("twenty places", 100003, True), ("in order", 65536, False),
+    ("rows of 256", 65536, False), ("rows of 512", 131072, False), ("rows of 1024", 131072, False), ("rows of 100", 70000, False), ("in order", 262147, False), ("unrelated", 131071, False),
     ("unrelated", 262144, True)])
 def test_which_lists_are_sorted(room, kind, n, sorts):
     """The order that the record of a list keeps has every ray once; it is the rays' own for lists that come in order, and
