@@ -2586,7 +2586,7 @@ __global__ void k_ray_keys(const float *__restrict__ ray_o, const float *__restr
 // an 8^3 grid that origins lie in, the rest to the direction.  A camera's rays have all sixteen for it.  Rays of one key
 // follow in no order.  A list that comes in order (neighbours with nearly the same ray: a sensor's frame, rows of an image) keeps it,
 // and rays from more than kListPlaces cells are unrelated and gain only by the number: from kOrderManyRays on.
-// Bound by latency: 8 us to look, 28 to count 131,072 rays, 5 to place them; 17 in all for a list that keeps its order.
+// Bound by latency: 6 us to look, 28 to count 131,072 rays, 5 to place them; 13 in all for a list that keeps its order.
 // As the rays come / like this, us evaluated and us a training step:
 //   pixels of one camera, shuffled: room of a million surfels, 32,768 835 / 709 and 1454 / 1180, 65,536 1315 / 1084 and 2421 /
 //   1755, 131,072 2293 / 1862 and 4350 / 3028; of 300,000, 32,768 179 / 218 and 430 / 430, 131,072 482 / 558 and 1116 / 1022;
@@ -2595,6 +2595,12 @@ __global__ void k_ray_keys(const float *__restrict__ ray_o, const float *__restr
 //   unrelated rays, sorted all the same: room of a million, 131,072 1261 / 1286 and 2392 / 2390, 262,144 2254 / 2160 and 4252 / 4086
 //   a sensor's frame in order, sorted all the same: 131,072 of two million surfels 148 / 266 and 567 / 677; kept 167 and 587
 // (A list of fewer than 65,536 rays loses by it in as many scenes as it gains.)
+// Where quads cover the scene a few times at most (DstBounds::layers), a list of fewer than 262,144 rays that is only evaluated
+// is not looked at.  As the rays come / like this, us evaluated, pixels of one camera, shuffled: room of 50,000 (1.4 layers), 65,536
+// 97 / 118, 131,072 162 / 192, of 100,000 (2.9) 108 / 123 and 189 / 207, of 150,000 (4.3) 150 / 159 and 266 / 257, sphere of 30,000
+// (6.1) 125 / 109 and 279 / 203; frames of a sensor, shuffled, 131,072 of 600,000 surfels (0.8) 211 / 196, of two million
+// (2.5) 460 / 391, 65,536 62 / 90 and 90 / 104; 131,072 in order 165 / 174 and 331 / 339.  Training steps gain there too: 271 / 270
+// and 467 / 462, 300 / 286 and 534 / 515, 620 / 518, 1324 / 1027, and lose in order 493 / 500 and 950 / 955.
 constexpr uint32_t kListKeys = 65536u, kListCells = 512u, kListLooks = kListCells, kListThreads = 1024u, kListPlaces = 128u;
 struct ListHead {
     uint32_t sorts;                // 0: as the rays come
@@ -2612,19 +2618,23 @@ __global__ __launch_bounds__(kListLooks) void k_list_look(const float *__restric
     }
     // places all over the list, one in every stretch of it, and at each a ray and the next one.  (Not at even distances: of an
     // image that is some power of two wide, row after row, every other one would be the end of a row.)
-    __shared__ uint32_t s_cells[kListCells / 32u];
+    __shared__ uint32_t s_cells[kListCells / 32u], s_alike;
     const uint32_t tid = threadIdx.x, within = (tid * 2654435769u) >> 16;   // in its stretch, in 1 / 65536
     const uint32_t at = (uint32_t)((((uint64_t)tid << 16) | within) * (n - 1u) / (kListLooks << 16));
     if (tid < kListCells / 32u) s_cells[tid] = 0u;
-    __syncthreads();
+    if (tid == 0u) s_alike = 0u;
     const float *o = ray_o + 3 * (size_t)at, *d = ray_d + 3 * (size_t)at;   // (the next ray's lie behind them)
     const uint32_t cell = origin_cell<3>(o, bounds);
-    atomicOr(&s_cells[cell / 32u], 1u << (cell % 32u));
     const F3 d0 = ld3(d), d1 = ld3(d + 3), c = cross(d0, d1);
     const float off = fmaxf(fmaxf(fabsf(o[3] - o[0]), fabsf(o[4] - o[1])), fabsf(o[5] - o[2]));
     // a sixteenth of a radian, and of the scene's size
     const bool alike = dot(c, c) <= (1.f / 256.f) * (dot(d0, d0) * dot(d1, d1)) && dot(d0, d1) > 0.f && off <= (1.f / 16.f) * __uint_as_float(bounds->scale);
-    const uint32_t n_alike = (uint32_t)__syncthreads_count(alike ? 1 : 0);
+    const uint64_t wave_alike = wave_ballot(alike);
+    __syncthreads();
+    atomicOr(&s_cells[cell / 32u], 1u << (cell % 32u));
+    if (__lane_id() == 0u) atomicAdd(&s_alike, (uint32_t)__popcll(wave_alike));
+    __syncthreads();
+    const uint32_t n_alike = s_alike;
     uint32_t before = 0u, all = 0u;
     for (uint32_t w = 0u; w < kListCells / 32u; ++w) {
         if (w < tid / 32u) before += (uint32_t)__popc(s_cells[w]);
@@ -2902,7 +2912,7 @@ struct ScratchLayout {
     ScratchLayout(const dst_ctx *ctx, const DstParams &p) : ScratchLayout(p.P, p.H, p.W) {
         const bool hands = kFwdWavesPerBlock == 1 && dst_handover_active(ctx);
         const bool by_rows = ctx->handover_mode != DST_HANDOVER_OFF && (uint64_t)p.H * p.W <= (p.hit_record != nullptr ? kRowRecordedRays : kRowEvaluatedRays);
-        if (hands) list = 0u;
+        if (hands || (p.hit_record == nullptr && list < kOrderManyRays && ctx->layers < kOrderedLayers)) list = 0u;
         if (hands || by_rows || p.flags != 0u) records = blocks = 0u;
         if (ctx->layers < kOrderedLayers) blocks = 0u;   // (no number, of a scene on a line: many)
         if (ctx->layers < kRecordedLayers || (p.aux > kPackedAux && p.max_trace_depth == 0)) records = 0u;
@@ -2914,7 +2924,7 @@ struct ScratchLayout {
 // The order of a list traced by rows: in `kept`, the record's room for it (from kOrderMinByRows rays on the backward trace counts
 // on finding one there), or else in the scratch memory.  Without scratch memory as the rays come (nullptr: the same).
 const uint32_t *order_list(const dst_ctx *ctx, const DstParams &p, uint32_t n, uint32_t *kept, hipStream_t stream) {
-    ListHead *const head = reinterpret_cast<ListHead *>(p.scratch);
+    ListHead *const head = ScratchLayout(ctx, p).list != 0u ? reinterpret_cast<ListHead *>(p.scratch) : nullptr;
     if (head == nullptr && kept == nullptr) return nullptr;
     const dim3 grid((n + kListThreads - 1u) / kListThreads), block(kListThreads);
     uint32_t *keys = nullptr, *ranks = nullptr, *order = kept;

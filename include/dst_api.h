@@ -283,8 +283,8 @@ uint64_t dst_hit_record_layout(int32_t H, int32_t W, int32_t mtd_alloc, uint32_t
  * any (lists of fewer than 65,536 rays, small images, and the largest with far fewer rays than surfels). */
 uint64_t dst_trace_scratch_bytes(int32_t P, int32_t H, int32_t W);
 /* The same for this one forward call, all of whose other fields are set: what the kernels that will trace it make use of (of
- * images with more than four auxiliary channels and no reflections no surfels' records, of images traced by rows or by contexts
- * that hand tiles over nothing).  Never more than dst_trace_scratch_bytes. */
+ * images with more than four auxiliary channels and no reflections no surfels' records, of images traced by rows, of calls of
+ * contexts that hand tiles over and of long lists that are only evaluated in thin scenes nothing).  Never more than dst_trace_scratch_bytes. */
 uint64_t dst_trace_scratch_needed(const dst_ctx *ctx, const DstParams *p);
 
 /* Words (8 bytes each) of DstParams.det_workspace for a forward (backward = 0: one per surfel) or a backward

@@ -151,6 +151,32 @@ def test_order_changes_no_bit(monkeypatch, room, kind):
     assert torch.equal(order.cpu(), torch.arange(n, dtype=torch.int32))   # (a record has one in any case: the backward trace reads it)
 
 
+@pytest.mark.parametrize("surfels,n,record,looks", [(20000, 65535, True, False), (20000, 65536, False, True), (4000, 65536, False, False),
+                                                    (4000, 65536, True, True), (4000, 262143, False, False), (4000, 262144, False, True)])
+def test_which_lists_are_looked_at(monkeypatch, surfels, n, record, looks):
+    """Long ones, in thin scenes (a room covered 1.3 times instead of 6) longer ones where nothing is recorded.  The others
+    take no memory for it and come as they are, with the same results."""
+    from diff_surfel_tracing import _C
+    import diff_surfel_tracing as dst
+    sc = S.scene_room(P=surfels, seed=3, half=1.5)
+    tracer = dst.SurfelTracer()
+    tracer.build_acceleration_structure(sc["vertices"].cuda(), sc["faces"].cuda(), rebuild=True)
+    real, taken = _C._scratch, []
+
+    def spy(p, keep):
+        real(p, keep)
+        taken.append(bool(p.scratch))
+
+    o, d = _list("one place", n)
+    out = []
+    for scratch in (spy, lambda p, keep: None):
+        monkeypatch.setattr(_C, "_scratch", scratch)
+        out.append(_forward(tracer, sc, o, d, _C.HitRecord(1, n, 1, 4.0, torch.device("cuda")) if record else None))
+    assert taken in ([], [False]) if not looks else taken == [True]
+    for a, b in zip(*out):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
 def test_deterministic_sums_know_no_order(room):
     """Fixed-point sums of a sorted list: the same bits from run to run, wherever its rays stand."""
     tracer, sc = room
