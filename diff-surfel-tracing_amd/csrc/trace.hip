@@ -2886,15 +2886,15 @@ void launch_row_bwd(const DstParams &p, RowGrid g, const uint32_t *ray_order, hi
 #undef DST_ROW
 }
 
-// What a forward trace keeps in its scratch memory.  Of a list: what its order is made with (k_list_look).  Of an image: the surfels' records, and behind them the guessed cost of every block and
-// the order that follows from it.  Records are worth their pass where there are no more than four surfels to a ray (0.03 ns a
-// surfel against 0.09 a ray of the 1080p room), the order on grids that are walked row by row, as the guess numbers their blocks
-// (block_cost, block_of_position; larger grids are walked in strips, where it has not been tried.  3600 blocks, a 1280x720
-// room: of 300,000 surfels 504 / 503 us without and with, of a million 1903 / 1708), and a single
-// launch in front of them more than pays for it only where tiles take long, which is where quads cover the scene many times
-// over (DstBounds::layers).  Without / with, us: 800x800 sphere of 100,000 (20 layers) 1588 / 1124, 600x600 of 30,000 (6) 378 /
-// 297, 500x500 of 20,000 (4) 204 / 218; room of a million (29) 640x360 1163 / 918, 960x540 1395 / 1175, of 200,000 (6) 640x360
-// 183 / 173, of 100,000 (3) 121 / 119, of 50,000 (1.4) 83 / 90, 480x270 63 / 75.  Records of that last room cost it 1 us.
+// What a forward trace keeps in its scratch memory.  Of a list: what its order is made with (k_list_look).  Of an image: the
+// surfels' records, and behind them the guessed cost of every block and the order that follows from it.  Records are worth their
+// pass where there are no more than four surfels to a ray (0.03 ns a surfel against 0.09 a ray of the 1080p room), the order on
+// grids that are walked row by row, as the guess numbers their blocks (block_cost, block_of_position; larger grids are walked in
+// strips, where it has not been tried.  3600 blocks, a 1280x720 room: of 300,000 surfels 504 / 503 us without and with, of a million
+// 1903 / 1708), and a single launch in front of them more than pays for it only where tiles take long, which is where quads cover
+// the scene many times over (DstBounds::layers).  Without / with, us: 800x800 sphere of 100,000 (20 layers) 1588 / 1124, 600x600 of
+// 30,000 (6) 378 / 297, 500x500 of 20,000 (4) 204 / 218; room of a million (29) 640x360 1163 / 918, 960x540 1395 / 1175, of 200,000
+// (6) 640x360 183 / 173, of 100,000 (3) 121 / 119, of 50,000 (1.4) 83 / 90, 480x270 63 / 75.  Records of that last room cost it 1 us.
 constexpr uint64_t kOrderedBlocks = 4095u;
 static_assert(kOrderedBlocks < kStripMinBlocks, "the guessed costs' blocks are numbered row by row, those of a launch in strips by strips");
 constexpr float kOrderedLayers = 5.0f, kRecordedLayers = 2.0f;
